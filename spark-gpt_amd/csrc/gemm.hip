@@ -860,6 +860,31 @@ SFP8_DEV void stage_bf16_half8(uint8_t* lds, const floatx16 (&acc)[4][2], float 
   }
 }
 
+// The 128 x 128 tile (TileShape<true>): 4 waves of 64 x 64, the whole bf16
+// tile staged at once (stride kSmallStride: consecutive rows shift by 4
+// banks) and written as 256-byte rows.
+constexpr int kSmallStride = 272;
+SFP8_DEV void stage_bf16_small(uint8_t* lds, const floatx16 (&acc)[2][2], float s) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
+  const int fr = lane & 31, g = lane >> 5, cb = 64 * wn + 32 * g;
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb) {
+    const int lr = 64 * wm + 32 * tb + fr;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      uint32_t w0[4], w1[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        w0[i] = pack2_bf16(acc[tb][nb][2 * i] * s, acc[tb][nb][2 * i + 1] * s);
+        w1[i] = pack2_bf16(acc[tb][nb][8 + 2 * i] * s, acc[tb][nb][8 + 2 * i + 1] * s);
+      }
+      uint8_t* q = lds + lr * kSmallStride + (cb + 16 * nb) * 2;
+      store16(q, w0);
+      store16(q + 16, w1);
+    }
+  }
+}
+
 // Tile row held in staging row lr of pass p.
 SFP8_DEV int half_tile_row(int lr, int p) { return 128 * (lr >> 6) + 64 * p + (lr & 63); }
 
@@ -925,6 +950,75 @@ SFP8_DEV void write_bf16_half_res(const uint8_t* lds, int p, int64_t m0, int64_t
   }
 }
 
+// The staged 128 x 128 tile to out[t, n] (bf16, leading dimension ld), rows
+// m0.. below T, columns below N; with RES the bf16 residual rv (requested by
+// load_res_small) is added first: out = bf16(res + staged).
+SFP8_DEV void load_res_small(__amdgpu_buffer_rsrc_t rres, int64_t n0, int64_t D, intx4 (&rv)[8]) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int idx = (int)threadIdx.x + 256 * k;
+    rv[k] = __builtin_amdgcn_raw_buffer_load_b128(rres, (uint32_t)(((idx >> 4) * D + n0 + 8 * (idx & 15)) * 2), 0, kNT);
+  }
+}
+template <bool RES>
+SFP8_DEV void write_bf16_small(const uint8_t* lds, int64_t m0, int64_t n0, int64_t T, int64_t N, int64_t ld,
+                               const intx4 (&rv)[8], uint16_t* __restrict__ out) {
+  const __amdgpu_buffer_rsrc_t ro = make_rsrc(out + m0 * ld, (T - m0) * ld * 2);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int idx = (int)threadIdx.x + 256 * k;
+    const int lr = idx >> 4, c = idx & 15;
+    intx4 o = *reinterpret_cast<const intx4*>(lds + lr * kSmallStride + c * 16);
+    if constexpr (RES) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t a = (uint32_t)rv[k][i], b = (uint32_t)o[i];
+        o[i] = (int)pack2_bf16(__uint_as_float(b << 16) + __uint_as_float(a << 16),
+                               __uint_as_float(b & 0xffff0000u) + __uint_as_float(a & 0xffff0000u));
+      }
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(o, ro, bf16_out_off(m0 + lr, n0 + 8 * c, m0, T, N, ld), 0, 0);
+  }
+}
+
+// The two tile shapes of the GEMMs below: 256 x 256 by 8 waves, one
+// work-group per CU, or (SMALL) 128 x 128 by 4 waves, two per CU.  The B
+// rows of both are permuted by plain_col_nb<2>.
+template <bool SMALL>
+struct TileShape {
+  static constexpr int kM = SMALL ? 128 : 256;
+  static constexpr int kThreads = SMALL ? 256 : 512;
+  static constexpr int kMinWaves = SMALL ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
+  static constexpr int kWN = SMALL ? 2 : 4, kTB = SMALL ? 2 : 4;
+  template <bool BF16, int FA, int FB>
+  using Loop = MainLoop<BF16, FA, FB, false, 2, kStages, 0, false, false, kWN, kTB, kM>;
+  static constexpr int kLds = Loop<true, 0, 0>::kLds;
+  // the plan's tile of tile row tm, and that tile row's valid rows of it
+  static SFP8_DEV int plan_tile(int tm) { return SMALL ? tm >> 1 : tm; }
+  static SFP8_DEV int plan_skip(int tm) { return SMALL ? 128 * (tm & 1) : 0; }
+};
+
+// A tile's accumulators times s, as bf16, to out[t, n] (leading dimension N)
+// for rows u0.. below uend and columns n0.. below N.
+template <bool SMALL>
+SFP8_DEV void store_bf16_tile(uint8_t* lds, const floatx16 (&acc)[TileShape<SMALL>::kTB][2], float s, int64_t u0,
+                              int64_t n0, int64_t uend, int64_t N, uint16_t* __restrict__ out) {
+  if constexpr (SMALL) {
+    const intx4 none[8] = {};
+    stage_bf16_small(lds, acc, s);
+    __syncthreads();
+    write_bf16_small<false>(lds, u0, n0, uend, N, N, none, out);
+  } else {
+    stage_bf16_half8<0>(lds, acc, s);
+    __syncthreads();
+    write_bf16_half<512>(lds, 0, u0, n0, uend, N, N, out);
+    __syncthreads();
+    stage_bf16_half8<1>(lds, acc, s);
+    __syncthreads();
+    write_bf16_half<512>(lds, 1, u0, n0, uend, N, N, out);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // (a7) down forward + residual (spark-gpt train.py:1019-1046):
 //   y = bf16(res + bf16(acc / (s2 * q_d)))
@@ -932,33 +1026,45 @@ SFP8_DEV void write_bf16_half_res(const uint8_t* lds, int p, int64_t m0, int64_t
 // its rows(tm) valid rows to y rows urow(tm).. (expert order, unpadded);
 // W_down8 of expert e at wd8 + e * w_estride, its scale wscale[e] (the dense
 // call passes wscale + 1: [q_gu, q_d]).
-__global__ __launch_bounds__(512, 1) void down_fwd_kernel(
+template <bool SMALL>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void down_fwd_kernel(
     const uint8_t* __restrict__ h8, const uint8_t* __restrict__ wd8, const uint16_t* __restrict__ res,
     int64_t T, int64_t D, int64_t I, const float* __restrict__ scale, const float* __restrict__ wscale,
     uint16_t* __restrict__ y, int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan,
     int64_t w_estride) {
+  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
   int64_t u0 = 0, urows = 0;
   if (plan) {
     const MoePlan P{plan};
-    if (tm >= P.ntiles()) return;  // work-group uniform
-    const int e = P.expert(tm);
+    const int pt = TS::plan_tile(tm);
+    if (pt >= P.ntiles()) return;  // work-group uniform
+    const int e = P.expert(pt);
     wd8 += e * w_estride;
     wscale += e;
-    u0 = P.urow(tm);
-    urows = P.rows(tm);
+    u0 = P.urow(pt) + TS::plan_skip(tm);
+    urows = P.rows(pt) - TS::plan_skip(tm);
+    if (urows <= 0) return;  // nothing but padding rows, which have no output
   }
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
-  floatx16 acc[4][2];
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  floatx16 acc[TS::kTB][2];
   // K-slab operands: h8 [I/64][ldt][64], wd8 [I/64][slab_rows(D)][64]
   const int64_t dp = slab_rows(D);
-  MainLoop<false, kFmtE4M3, kFmtE4M3, false, 2, kStages, 0, false, false, 4>::run(
+  TS::template Loop<false, kFmtE4M3, kFmtE4M3>::run(
       lds, h8 + m0 * kStage, I * ldt - m0 * kStage, [=](int r) { return r * kStage; }, (int)(ldt * kStage),
       wd8 + n0 * kStage, I * dp - n0 * kStage, [=](int r) { return plain_col_nb<2>(r) * kStage; },
       (int)(dp * kStage), (int)(I / kStage), acc);
   const float deq = 1.0f / (scale[2] * wscale[0]);
+  if constexpr (SMALL) {
+    intx4 rv[8];
+    if (!plan) load_res_small(make_rsrc(res + m0 * D, (T - m0) * D * 2), n0, D, rv);
+    stage_bf16_small(lds, acc, deq);
+    __syncthreads();
+    if (plan) write_bf16_small<false>(lds, u0, n0, u0 + urows, D, D, rv, y);
+    else write_bf16_small<true>(lds, m0, n0, T, D, D, rv, y);
+  } else {
   if (plan) {
     // expert rows, no residual: out rounded to bf16 (train.py:1377-1378 stores acc / (s2 q_d) as bf16)
     stage_bf16_half8<0>(lds, acc, deq);
@@ -986,6 +1092,7 @@ __global__ __launch_bounds__(512, 1) void down_fwd_kernel(
   stage_bf16_half8<1>(lds, acc, deq);
   __syncthreads();
   write_bf16_half_res<512>(lds, 1, m0, n0, T, D, rv1, y);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1272,42 +1379,40 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
 // With a MoE plan: tile row tm of padded expert order writes its rows(tm)
 // valid rows to dxn rows urow(tm).. (expert order, unpadded); W8^T of
 // expert e at w8t + e * w_estride, its scale wscale[e].
-__global__ __launch_bounds__(512, 1) void gateup_dgrad_kernel(
+template <bool SMALL>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void gateup_dgrad_kernel(
     const uint8_t* __restrict__ dgu8, const uint8_t* __restrict__ w8t, int64_t T, int64_t D, int64_t I,
     const float* __restrict__ scale, const float* __restrict__ wscale, uint16_t* __restrict__ dxn,
     int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t w_estride) {
+  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   const int64_t K = 2 * I;
   const int64_t dp = slab_rows(D);
   int tm, tn;
   // backwards: the dgrad wrote d_gu8 in forward order (0.304 -> 0.302 ms)
   tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn, true);
-  int64_t u0 = (int64_t)tm * kTile, uend = T;  // output rows of this tile
+  int64_t u0 = (int64_t)tm * TS::kM, uend = T;  // output rows of this tile
   if (plan) {
     const MoePlan P{plan};
-    if (tm >= P.ntiles()) return;  // work-group uniform
-    const int e = P.expert(tm);
+    const int pt = TS::plan_tile(tm);
+    if (pt >= P.ntiles()) return;  // work-group uniform
+    const int e = P.expert(pt);
     w8t += e * w_estride;
     wscale += e;
-    u0 = P.urow(tm);
-    uend = u0 + P.rows(tm);
+    u0 = P.urow(pt) + TS::plan_skip(tm);
+    uend = P.urow(pt) + P.rows(pt);
+    if (u0 >= uend) return;  // nothing but padding rows, which have no output
   }
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
-  floatx16 acc[4][2];
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  floatx16 acc[TS::kTB][2];
   // K-slab operands: dgu8 [2I/64][ldt][64], w8t [2I/64][slab_rows(D)][64]
-  MainLoop<false, kFmtE5M2, kFmtE4M3, false, 2, kStages, 0, false, false, 4>::run(
+  TS::template Loop<false, kFmtE5M2, kFmtE4M3>::run(
       lds, dgu8 + m0 * kStage, K * ldt - m0 * kStage, [=](int r) { return r * kStage; }, (int)(ldt * kStage),
       w8t + n0 * kStage, K * dp - n0 * kStage, [=](int r) { return plain_col_nb<2>(r) * kStage; },
       (int)(dp * kStage), (int)(K / kStage), acc);
   // the scales are read after the K loop, so that nothing is held across it
   const float sab = (1.0f / scale[3]) * (1.0f / wscale[0]);  // both powers of two
-  stage_bf16_half8<0>(lds, acc, sab);
-  __syncthreads();
-  write_bf16_half<512>(lds, 0, u0, n0, uend, D, D, dxn);
-  __syncthreads();
-  stage_bf16_half8<1>(lds, acc, sab);
-  __syncthreads();
-  write_bf16_half<512>(lds, 1, u0, n0, uend, D, D, dxn);
+  store_bf16_tile<SMALL>(lds, acc, sab, u0, n0, uend, D, dxn);
 }
 
 // ---------------------------------------------------------------------------
@@ -1692,34 +1797,32 @@ __global__ __launch_bounds__(512, 1) void bf16_swiglu_fwd_kernel(
 // valid rows to out rows urow(tm).. (expert order); B of expert e at
 // b + e * b_estride (bytes).
 // 8 waves (two per SIMD), each 128 x 64.
-__global__ __launch_bounds__(512, 1) void bf16_gemm_kernel(
+template <bool SMALL>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void bf16_gemm_kernel(
     const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int64_t T, int64_t N, int64_t Kb, int64_t lda,
     uint16_t* __restrict__ out, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t b_estride) {
+  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   const int64_t bp = slab_rows(N);
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
-  int64_t u0 = (int64_t)tm * kTile, uend = T;  // output rows of this tile
+  int64_t u0 = (int64_t)tm * TS::kM, uend = T;  // output rows of this tile
   if (plan) {
     const MoePlan P{plan};
-    if (tm >= P.ntiles()) return;  // work-group uniform
-    b += P.expert(tm) * b_estride;
-    u0 = P.urow(tm);
-    uend = u0 + P.rows(tm);
+    const int pt = TS::plan_tile(tm);
+    if (pt >= P.ntiles()) return;  // work-group uniform
+    b += P.expert(pt) * b_estride;
+    u0 = P.urow(pt) + TS::plan_skip(tm);
+    uend = P.urow(pt) + P.rows(pt);
+    if (u0 >= uend) return;  // nothing but padding rows, which have no output
   }
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
-  floatx16 acc[4][2];
-  MainLoop<true, 0, 0, false, 2, kStages, 0, false, false, 4>::run(
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  floatx16 acc[TS::kTB][2];
+  TS::template Loop<true, 0, 0>::run(
       lds, a + m0 * kStage, Kb * lda - m0 * kStage, [=](int r) { return r * kStage; }, (int)(lda * kStage),
       b + n0 * kStage, Kb * bp - n0 * kStage, [=](int r) { return plain_col_nb<2>(r) * kStage; }, (int)(bp * kStage),
       (int)(Kb / kStage), acc);
-  stage_bf16_half8<0>(lds, acc, 1.0f);
-  __syncthreads();
-  write_bf16_half<512>(lds, 0, u0, n0, uend, N, N, out);
-  __syncthreads();
-  stage_bf16_half8<1>(lds, acc, 1.0f);
-  __syncthreads();
-  write_bf16_half<512>(lds, 1, u0, n0, uend, N, N, out);
+  store_bf16_tile<SMALL>(lds, acc, 1.0f, u0, n0, uend, N, out);
 }
 
 // The bf16 weight gradient's reduction: out[m, n] = bf16(sum over s
@@ -1862,6 +1965,40 @@ inline int64_t wgrad_chunk(int64_t ldt, int64_t s) {
 }  // namespace
 
 namespace {
+// Whether an M x N output is computed in 128 x 128 tiles (two work-groups per
+// CU) instead of 256 x 256 ones (one per CU): when the larger tiles would
+// leave half of the 256 CUs or more without one.  A CU runs its tile at the
+// same speed however many others are idle, so the quarter tiles, spread over
+// up to four times the CUs, win until they fill the chip; from then on their
+// K loop, with twice the LDS-DMA bytes per FLOP, is the slower one.  Measured
+// (us, 256 -> 128 tiles, at 16, 80, 128 and 192 tiles of 256 x 256, D = 1024,
+// I = 3072): down forward 29 -> 14, 32 -> 24, 36 -> 32, 40 -> 44; gate/up
+// dgrad 49 -> 26, 50 -> 38, 55 -> 45, 62 -> 71; bf16 dgrad 91 -> 46, 94 -> 73,
+// 99 -> 88, 125 -> 135.  At 320 tiles (a second round of 64) the two differ by
+// less than a tenth either way, and the larger ones stay.
+inline bool use_small_tiles(int64_t M, int64_t N) {
+  constexpr int64_t kCUs = 256;
+  return (int64_t)cdiv(M, kTile) * cdiv(N, kTile) <= kCUs / 2;
+}
+
+// A GEMM's tile shape over an M x N output, and its launch.
+struct Tiling {
+  bool small;
+  int m, n, lds;  // tile rows and columns, dynamic LDS
+  dim3 grid, block;
+};
+inline Tiling tiling(int64_t M, int64_t N) {
+  Tiling t;
+  t.small = use_small_tiles(M, N);
+  const int tile = t.small ? TileShape<true>::kM : TileShape<false>::kM;
+  t.m = cdiv(M, tile);
+  t.n = cdiv(N, tile);
+  t.lds = t.small ? TileShape<true>::kLds : TileShape<false>::kLds;
+  t.grid = dim3((unsigned)(t.m * t.n));
+  t.block = dim3((unsigned)(t.small ? TileShape<true>::kThreads : TileShape<false>::kThreads));
+  return t;
+}
+
 // The split partials ws[split][tile] (one 256 x 256 fp32 tile each, in
 // accumulator order of wgrad_kernel<.., kWgradWaves>) of the FP8 weight
 // gradient; TRA / TRB: that operand is the row K-slab of the token-major
@@ -1935,12 +2072,13 @@ int sfp8_gemm_down_fwd(const void* h8, const void* wd8, const void* res, int64_t
   if (!fits32(ldt, I) || !fits32(slab_rows(D), I) || !fits32(kTile, 2 * D)) return kErrBadShape;
   if (!al16(h8) || !al16(wd8) || !al16(res) || !al16(y)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const int tiles_m = cdiv(T, kTile), tiles_n = cdiv(D, kTile);
-  int rc = prep(down_fwd_kernel, kMainLds);
+  const Tiling tl = tiling(T, D);
+  const auto kern = tl.small ? down_fwd_kernel<true> : down_fwd_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(down_fwd_kernel, dim3(tiles_m * tiles_n), dim3(512), kMainLds, (hipStream_t)stream,
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
                      (const uint8_t*)h8, (const uint8_t*)wd8, (const uint16_t*)res, T, D, I, scale, wscale + 1,
-                     (uint16_t*)y, ldt, tiles_m, tiles_n, (const int*)nullptr, (int64_t)0);
+                     (uint16_t*)y, ldt, tl.m, tl.n, (const int*)nullptr, (int64_t)0);
   return status();
 }
 
@@ -1975,12 +2113,13 @@ int sfp8_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t T, int64_t
   if (!fits32(ldt, 2 * I) || !fits32(slab_rows(D), 2 * I) || !fits32(kTile, 2 * D)) return kErrBadShape;
   if (!al16(dgu8) || !al16(w8t) || !al16(dxn)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const int tiles_m = cdiv(T, kTile), tiles_n = cdiv(D, kTile);
-  int rc = prep(gateup_dgrad_kernel, kMainLds);
+  const Tiling tl = tiling(T, D);
+  const auto kern = tl.small ? gateup_dgrad_kernel<true> : gateup_dgrad_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(gateup_dgrad_kernel, dim3(tiles_m * tiles_n), dim3(512), kMainLds, (hipStream_t)stream,
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
                      (const uint8_t*)dgu8, (const uint8_t*)w8t, T, D, I, scale, wscale, (uint16_t*)dxn, ldt,
-                     tiles_m, tiles_n, (const int*)nullptr, (int64_t)0);
+                     tl.m, tl.n, (const int*)nullptr, (int64_t)0);
   return status();
 }
 
@@ -2125,12 +2264,13 @@ int sfp8_moe_gemm_down_fwd(const void* h8, const void* wd8, int64_t E, int64_t D
   if (!moe_shape(E, D, I, ldp) || R < 0 || !fits32(ldp, I) || !fits32(slab_rows(D), I) || !fits32(kTile, 2 * D))
     return kErrBadShape;
   if (!al16(h8) || !al16(wd8) || !al16(out)) return kErrBadAlignment;
-  const int tiles_m = (int)(ldp / kTile), tiles_n = cdiv(D, kTile);
-  int rc = prep(down_fwd_kernel, kMainLds);
+  const Tiling tl = tiling(ldp, D);
+  const auto kern = tl.small ? down_fwd_kernel<true> : down_fwd_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(down_fwd_kernel, dim3(tiles_m * tiles_n), dim3(512), kMainLds, (hipStream_t)stream,
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
                      (const uint8_t*)h8, (const uint8_t*)wd8, (const uint16_t*)nullptr, R, D, I, scale, q_d,
-                     (uint16_t*)out, ldp, tiles_m, tiles_n, plan, I * slab_rows(D));
+                     (uint16_t*)out, ldp, tl.m, tl.n, plan, I * slab_rows(D));
   return status();
 }
 
@@ -2163,12 +2303,13 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
       !fits32(kTile, 2 * D))
     return kErrBadShape;
   if (!al16(dgu8) || !al16(w8t) || !al16(dx)) return kErrBadAlignment;
-  const int tiles_m = (int)(ldp / kTile), tiles_n = cdiv(D, kTile);
-  int rc = prep(gateup_dgrad_kernel, kMainLds);
+  const Tiling tl = tiling(ldp, D);
+  const auto kern = tl.small ? gateup_dgrad_kernel<true> : gateup_dgrad_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(gateup_dgrad_kernel, dim3(tiles_m * tiles_n), dim3(512), kMainLds, (hipStream_t)stream,
-                     (const uint8_t*)dgu8, (const uint8_t*)w8t, R, D, I, scale, q_gu, (uint16_t*)dx, ldp, tiles_m,
-                     tiles_n, plan, 2 * I * slab_rows(D));
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
+                     (const uint8_t*)dgu8, (const uint8_t*)w8t, R, D, I, scale, q_gu, (uint16_t*)dx, ldp, tl.m,
+                     tl.n, plan, 2 * I * slab_rows(D));
   return status();
 }
 
@@ -2292,12 +2433,13 @@ int bf16_swiglu_launch(const void* x, const void* w, int64_t T, int64_t D, int64
 }
 
 int bf16_gemm_launch(const void* a, const void* b, int64_t T, int64_t N, int64_t K, int64_t lda, void* out,
-                     const int* plan, int tiles_m, hipStream_t st) {
-  const int tiles_n = cdiv(N, kTile);
-  int rc = prep(bf16_gemm_kernel, kMainLds);
+                     const int* plan, hipStream_t st) {
+  const Tiling tl = tiling(plan ? lda : T, N);
+  const auto kern = tl.small ? bf16_gemm_kernel<true> : bf16_gemm_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(bf16_gemm_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(512), kMainLds, st,
-                     (const uint8_t*)a, (const uint8_t*)b, T, N, 2 * K, lda, (uint16_t*)out, tiles_m, tiles_n, plan,
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st,
+                     (const uint8_t*)a, (const uint8_t*)b, T, N, 2 * K, lda, (uint16_t*)out, tl.m, tl.n, plan,
                      plan ? 2 * K * slab_rows(N) : 0);
   return status();
 }
@@ -2332,7 +2474,7 @@ int sfp8_bf16_gemm(const void* a, const void* b, int64_t T, int64_t N, int64_t K
   if (!fits32(lda, 2 * K) || !fits32(slab_rows(N), 2 * K) || !fits32(kTile, 2 * N)) return kErrBadShape;
   if (!al16(a) || !al16(b) || !al16(out)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  return bf16_gemm_launch(a, b, T, N, K, lda, out, nullptr, cdiv(T, kTile), (hipStream_t)stream);
+  return bf16_gemm_launch(a, b, T, N, K, lda, out, nullptr, (hipStream_t)stream);
 }
 
 int sfp8_bf16_moe_gemm(const void* a, const void* b, int64_t E, int64_t N, int64_t K, const int* plan, int64_t ldp,
@@ -2342,7 +2484,7 @@ int sfp8_bf16_moe_gemm(const void* a, const void* b, int64_t E, int64_t N, int64
   if (!fits32(ldp, 2 * K) || !fits32(slab_rows(N), 2 * K)) return kErrBadShape;
   if (!al16(a) || !al16(b) || !al16(out)) return kErrBadAlignment;
   if (ldp == 0) return kOk;
-  return bf16_gemm_launch(a, b, 0, N, K, ldp, out, plan, (int)(ldp / kTile), (hipStream_t)stream);
+  return bf16_gemm_launch(a, b, 0, N, K, ldp, out, plan, (hipStream_t)stream);
 }
 
 int64_t sfp8_bf16_wgrad_splits(int64_t M, int64_t N, int64_t ldt) { return wgrad_splits_doubling(M, N, 2 * ldt); }

@@ -1,13 +1,17 @@
 // Pipelined MFMA main loop for C = A * B^T with K-contiguous A and B rows
 // (gfx950).
 //
-// Tile: 256 A rows x 32*NB*WN B rows, one work-group of (8/TB) x WN waves;
+// Tile: TM A rows x 32*NB*WN B rows, one work-group of TM/(32*TB) x WN waves;
 // each wave owns 32*TB A rows x 32*NB B rows as TB x NB MFMA 32x32
 // accumulators (fp32, 16*TB*NB registers per lane).  The GEMMs here use
 // 8 waves (two per SIMD) of 128 x 64 (TB = 4, NB = 2, WN = 4) per 256 x 256
 // tile, or of 64 x 64 (TB = 2, NB = 2, WN = 2) per 256 x 128 tile, so that
 // one wave's stage waits and barriers are covered by the other's MFMAs; 4
-// waves of 128 x 128 (NB = 4, WN = 2) remain available.
+// waves of 128 x 128 (NB = 4, WN = 2) remain available.  The 128 x 128 tile
+// (TM = 128: 4 waves of 64 x 64, a 64 KiB ring) lets two work-groups share a
+// CU, one's epilogue and waits under the other's MFMAs: a quarter of the
+// work per tile, for shapes with too few 256 x 256 tiles or a short K.  Every
+// tile shape adds the same products in the same K order to each output.
 //
 // K advances in 64-byte stages through a ring of STAGES LDS buffers, each A
 // (16 KiB) + B (64*NB*64 bytes); A stages first, then B stages.
@@ -118,15 +122,17 @@ SFP8_DEV void sched_interleave_valu() {
 // transposing read as possibly aliasing any LDS DMA it knows to be in flight
 // and would wait for all of it first; the stage waits and barriers already
 // order every read after its stage's DMA.
-// TB = A blocks of 32 rows per wave: 4 (two wave rows of 128) or 2 (four
-// wave rows of 64; only the fragment, DMA and MFMA pieces, not run()).
+// TB = A blocks of 32 rows per wave: 4 (two wave rows of 128) or 2 (two wave
+// rows of 64 of a TM = 128 tile, or four of a TM = 256 one: then only the
+// fragment, DMA and MFMA pieces, not run()).
 template <bool BF16, int FMT_A, int FMT_B, bool PAIRED, int NB = 4, int STAGES = kStages, int PRE = 0,
-          bool TR_A = false, bool TR_B = false, int WN = 2, int TB = 4>
+          bool TR_A = false, bool TR_B = false, int WN = 2, int TB = 4, int TM = kTile>
 struct MainLoop {
   static_assert(TB == 4 || TB == 2, "2 or 4 A blocks per wave");
-  static constexpr int kWM = 8 / TB;                        // wave rows
+  static constexpr int kWM = TM / (32 * TB);                // wave rows
+  static constexpr int kStageA = TM * kStage;               // bytes of A per stage
   static constexpr int kWaves = kWM * WN;
-  static_assert(!(TR_A || TR_B) || (!PAIRED && 32 * NB * WN == 256), "transposing reads: plain, 256 x 256");
+  static_assert(!(TR_A || TR_B) || (!PAIRED && 32 * NB * WN == TM), "transposing reads: plain, square tiles");
   static constexpr bool kTr = TR_A || TR_B;
   using Rsrc = typename std::conditional<kTr, intx4, __amdgpu_buffer_rsrc_t>::type;
   static SFP8_DEV Rsrc rsrc(const void* base, int64_t bytes) {
@@ -149,7 +155,7 @@ struct MainLoop {
   static constexpr int kStageB = kTileN * kStage;
   static constexpr int kLdsB = STAGES * kStageA;           // start of the B stages
   static constexpr int kLds = STAGES * (kStageA + kStageB);
-  static constexpr int kDmaA = 16 / kWaves;                // A DMA instructions per wave per stage
+  static constexpr int kDmaA = TM / 16 / kWaves;           // A DMA instructions per wave per stage
   static constexpr int kDmaB = kTileN / 16 / kWaves;
   static constexpr int kDma = kDmaA + kDmaB;               // DMA instructions per wave per stage
   using Acc = floatx16[TB][NB];
@@ -160,7 +166,7 @@ struct MainLoop {
                                 Rsrc rb, const uint32_t (&voff_a)[4], const uint32_t (&voff_b)[NB],
                                 int soff_a, int soff_b, int wave) {
     if (j < kDmaA) {
-      uint8_t* dst = lds + buf * kStageA + ((kTile / kWaves) * wave + 16 * j) * kStage;
+      uint8_t* dst = lds + buf * kStageA + ((TM / kWaves) * wave + 16 * j) * kStage;
       dma16(dst, ra, voff_a[j], soff_a);
     } else {
       uint8_t* dst = lds + kLdsB + buf * kStageB + ((kTileN / kWaves) * wave + 16 * (j - kDmaA)) * kStage;
@@ -312,7 +318,7 @@ struct MainLoop {
   // fragments over 3 MFMAs and then the DMA over 3.
   static constexpr int kSchedPre = 2;
   static_assert(TB != 4 || kMfma >= kSchedPre + (4 + NB) / 2 + (4 + NB) / 2, "stage too short for the schedule");
-  static SFP8_DEV void stage(uint8_t* lds, const Frag& cur, Frag& nxt, Acc& acc, int dma_buf, int ld, int rd_buf,
+  static SFP8_DEV void stage_large(uint8_t* lds, const Frag& cur, Frag& nxt, Acc& acc, int dma_buf, int ld, int rd_buf,
                              Rsrc ra, Rsrc rb, const uint32_t (&voff_a)[4],
                              const uint32_t (&voff_b)[NB], int a_sstride, int b_sstride, const uint32_t (&aoff)[8],
                              const uint32_t (&boff)[8], int wave) {
@@ -420,6 +426,54 @@ struct MainLoop {
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  // The stage of a 64 x 64 wave (TB = NB = 2): 4 fp8 MFMAs of 64 cycles or 8
+  // bf16 ones of 32, four fragments and four DMA instructions.  The first
+  // MFMAs go ahead of the barrier; a[0] and b[0] are read first (the next
+  // stage starts with them), the DMA goes out with the later MFMAs.  Two
+  // work-groups share a CU, so the waits of one run under the MFMAs of the
+  // other and the order inside a stage matters little.
+  template <int LO, int HI, int R0, int R1, int J0, int J1>
+  static SFP8_DEV void small_group(uint8_t* lds, const Frag& cur, Frag& nxt, Acc& acc, int dma_buf, int rd_buf,
+                                   Rsrc ra, Rsrc rb, const uint32_t (&voff_a)[4], const uint32_t (&voff_b)[NB],
+                                   int sa, int sb, const uint32_t (&aoff)[8], const uint32_t (&boff)[8], int wave) {
+    mfma_range<LO, HI>(cur, acc);
+    if constexpr (R0 >= 0) read_frag<R0>(lds, rd_buf, aoff, boff, nxt);
+    if constexpr (R1 >= 0) read_frag<R1>(lds, rd_buf, aoff, boff, nxt);
+#pragma unroll
+    for (int j = J0; j < J1; ++j) load_one(j, lds, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  static SFP8_DEV void stage_small(uint8_t* lds, const Frag& cur, Frag& nxt, Acc& acc, int dma_buf, int ld,
+                                   int rd_buf, Rsrc ra, Rsrc rb, const uint32_t (&voff_a)[4],
+                                   const uint32_t (&voff_b)[NB], int a_sstride, int b_sstride,
+                                   const uint32_t (&aoff)[8], const uint32_t (&boff)[8], int wave) {
+    static_assert(TB != 2 || NB == 2, "64 x 64 per wave");
+    constexpr int Q = kMfma / 4;  // MFMAs per group
+    mfma_range<0, Q>(cur, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kDma * (STAGES - 3)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const int sa = ld * a_sstride, sb = ld * b_sstride;
+    small_group<Q, 2 * Q, 0, TB, 0, 0>(lds, cur, nxt, acc, dma_buf, rd_buf, ra, rb, voff_a, voff_b, sa, sb, aoff,
+                                       boff, wave);
+    small_group<2 * Q, 3 * Q, TB + 1, 1, 0, kDma / 2>(lds, cur, nxt, acc, dma_buf, rd_buf, ra, rb, voff_a, voff_b,
+                                                      sa, sb, aoff, boff, wave);
+    small_group<3 * Q, 4 * Q, -1, -1, kDma / 2, kDma>(lds, cur, nxt, acc, dma_buf, rd_buf, ra, rb, voff_a, voff_b,
+                                                      sa, sb, aoff, boff, wave);
+  }
+
+  static SFP8_DEV void stage(uint8_t* lds, const Frag& cur, Frag& nxt, Acc& acc, int dma_buf, int ld, int rd_buf,
+                             Rsrc ra, Rsrc rb, const uint32_t (&voff_a)[4], const uint32_t (&voff_b)[NB],
+                             int a_sstride, int b_sstride, const uint32_t (&aoff)[8], const uint32_t (&boff)[8],
+                             int wave) {
+    if constexpr (TB == 2)
+      stage_small(lds, cur, nxt, acc, dma_buf, ld, rd_buf, ra, rb, voff_a, voff_b, a_sstride, b_sstride, aoff, boff,
+                  wave);
+    else
+      stage_large(lds, cur, nxt, acc, dma_buf, ld, rd_buf, ra, rb, voff_a, voff_b, a_sstride, b_sstride, aoff, boff,
+                  wave);
+  }
+
   // a_bytes/b_bytes: bytes available from a_base/b_base (range-checked);
   // a_rowoff(r)/b_rowoff(r): byte offset of tile row r from the base within
   // one K stage; a_sstride/b_sstride: bytes from one 64-byte K stage to the
@@ -428,7 +482,7 @@ struct MainLoop {
   template <class ARow, class BRow>
   static SFP8_DEV void run(uint8_t* lds, const uint8_t* a_base, int64_t a_bytes, ARow a_rowoff, int a_sstride,
                            const uint8_t* b_base, int64_t b_bytes, BRow b_rowoff, int b_sstride, int nk, Acc& acc) {
-    static_assert(TB == 4, "run() schedules four A blocks per wave");
+    static_assert(kWM == 2, "run() places two wave rows");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave & 1, wn = wave >> 1;
     const Rsrc ra = rsrc(a_base, a_bytes);
@@ -446,7 +500,7 @@ struct MainLoop {
         BF16 ? (uint32_t)((lane & 3) << 4) : (uint32_t)(((lane & 3) ^ (((lane >> 4) & 1) << 1)) << 4);
 #pragma unroll
     for (int j = 0; j < kDmaA; ++j)
-      voff_a[j] = (uint32_t)a_rowoff((kTile / kWaves) * wave + 16 * j + (lane >> 2)) + (TR_A ? chunk_tr : chunk);
+      voff_a[j] = (uint32_t)a_rowoff((TM / kWaves) * wave + 16 * j + (lane >> 2)) + (TR_A ? chunk_tr : chunk);
 #pragma unroll
     for (int j = 0; j < kDmaB; ++j)
       voff_b[j] = (uint32_t)b_rowoff((kTileN / kWaves) * wave + 16 * j + (lane >> 2)) + (TR_B ? chunk_tr : chunk);
@@ -456,7 +510,7 @@ struct MainLoop {
     uint32_t aoff[8], boff[8];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      aoff[h] = (uint32_t)((128 * wm + fr) * kStage + (((2 * g + h) ^ sw) << 4));
+      aoff[h] = (uint32_t)((32 * TB * wm + fr) * kStage + (((2 * g + h) ^ sw) << 4));
       boff[h] = (uint32_t)(kLdsB + (BLayout<PAIRED, NB, WN>::kWaveStride * wn + fr) * kStage + (((2 * g + h) ^ sw) << 4));
     }
     if constexpr (kTr && BF16) {
@@ -471,7 +525,7 @@ struct MainLoop {
       for (int q = 0; q < 4; ++q) {
         const int tok = 16 * (G >> 1) + 4 * q + (j >> 2);
         const uint32_t cb = (uint32_t)(32 * (G & 1) + 8 * (j & 3));
-        if constexpr (TR_A) aoff[q] = (uint32_t)((128 * wm + tok) * kStage) + cb;
+        if constexpr (TR_A) aoff[q] = (uint32_t)((32 * TB * wm + tok) * kStage) + cb;
         if constexpr (TR_B) boff[q] = (uint32_t)((32 * NB * wn + tok) * kStage) + cb;
       }
     } else if constexpr (kTr) {
@@ -488,13 +542,13 @@ struct MainLoop {
         for (int k1 = 0; k1 < 2; ++k1) {
           const int rr = 32 * gh + 8 * q + bq;  // row within the 64-row slab
           const uint32_t cb = (uint32_t)((((2 * k1 + gc) ^ (((rr >> 2) & 1) << 1)) << 4) + 8 * hb);
-          if constexpr (TR_A) aoff[2 * q + k1] = (uint32_t)((128 * wm + rr) * kStage) + cb;
+          if constexpr (TR_A) aoff[2 * q + k1] = (uint32_t)((32 * TB * wm + rr) * kStage) + cb;
           if constexpr (TR_B) boff[2 * q + k1] = (uint32_t)((32 * NB * wn + rr) * kStage) + cb;
         }
       }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j) acc[i][j] = floatx16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
                                                         0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};

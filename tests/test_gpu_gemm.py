@@ -368,3 +368,34 @@ def test_wgrad_rows_equals_token_contiguous(dev, M, N, T, splits):
     assert torch.equal(ops.wgrad_rows(a_rows, b_rows, M, N, sa, sb), ref)
     assert torch.equal(ops.wgrad_rows(a_rows, b_t, M, N, sa, sb, b_rows=False), ref)
     assert torch.equal(ops.wgrad_rows(a_t, b_rows, M, N, sa, sb, a_rows=False), ref)
+
+
+# The bf16-output GEMMs run 128 x 128 tiles up to 128 tiles of 256 x 256 and
+# the larger tiles from 129 on: both sides of that line in rows and in
+# columns, one row past a tile of either shape, widths that end inside one,
+# the shortest K.
+@pytest.mark.parametrize("T,D,I", [(1, 128, 128), (128, 272, 128), (129, 128, 384), (257, 400, 256),
+                                   (32768, 256, 128), (32769, 256, 128), (8192, 1024, 128), (8193, 1040, 128)])
+def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
+    """Integer operands: every product and sum is exact in fp32 (at most
+    64 * 768 < 2^24), so the rounded result of either tile shape is known."""
+    g = torch.Generator(device=dev).manual_seed(T + D + I)
+    ldt = sg.ops.ldt_of(T)
+
+    def ints(rows, cols, dtype):
+        return torch.randint(-8, 9, (rows, cols), generator=g, device=dev).float().to(dtype)
+
+    def padded(x):
+        return sg.ops.to_slab(torch.cat([x, torch.zeros(ldt - T, x.shape[1], device=dev).to(x.dtype)]))
+
+    one = torch.ones(5, device=dev)
+    h8, wd8, res = ints(T, I, E4), ints(D, I, E4), ints(T, D, torch.bfloat16)
+    y = sg.ops.down_fwd(padded(h8), sg.ops.to_slab(wd8), res, one, one[:2])
+    prod = (h8.float() @ wd8.float().t()).bfloat16()
+    assert torch.equal(y, (res.float() + prod.float()).bfloat16())
+    dgu8, w8t = ints(T, 2 * I, E5), ints(D, 2 * I, E4)
+    dxn = sg.ops.gateup_dgrad(padded(dgu8), sg.ops.to_slab(w8t), one, one[:2], T, D)
+    assert torch.equal(dxn, (dgu8.float() @ w8t.float().t()).bfloat16())
+    a, b = ints(T, 2 * I, torch.bfloat16), ints(D, 2 * I, torch.bfloat16)
+    out = sg.ops.bf16_gemm(padded(a), sg.ops.to_slab(b), T, D, 2 * I)
+    assert torch.equal(out, (a.float() @ b.float().t()).bfloat16())
