@@ -404,29 +404,18 @@ def time_stack(T: int, D: int, I: int, L: int, steps: int, warmup: int) -> dict:
 
 
 def launch_name(sym: str, a, D: int, I: int) -> str:
-    """Kernel name of a C-ABI launch (symbol, its arguments)."""
-    if sym == "sfp8_weight_quant":
-        return "weight_quant_gu" if a[1] == 2 * I else "weight_quant_down"
-    if sym == "sfp8_gemm_wgrad":
-        return "wgrad_down" if a[4] == D else "wgrad_gateup"
-    if sym == "sfp8_gemm_wgrad_rows":
-        return "wgrad_down" if a[6] == D else "wgrad_gateup"
-    if sym == "sfp8_weight_quant_experts":
-        return "weight_quant_gu" if a[2] == 2 * I else "weight_quant_down"
-    if sym == "sfp8_moe_gemm_wgrad":
-        return "moe_wgrad_down" if a[4] == D else "moe_wgrad_gateup"
-    if sym == "sfp8_moe_gemm_wgrad_rows":
-        return "moe_wgrad_down" if a[6] == D else "moe_wgrad_gateup"
-    if sym == "sfp8_moe_rows_quant":
-        return "moe_gather_quant_x" if a[11] == 0 else "moe_quant_dout"
-    return {"sfp8_norm_quant": "norm_quant", "sfp8_gemm_gateup_swiglu_fwd": "gateup_swiglu_fwd",
-            "sfp8_gemm_down_fwd": "down_fwd", "sfp8_gemm_down_dgrad_swiglu": "down_dgrad_swiglu_bf16",
-            "sfp8_gemm_gateup_dgrad": "gateup_dgrad", "sfp8_norm_bwd": "norm_bwd",
-            "sfp8_update_scales": "update_scales", "sfp8_block_weight_quant": "post_step_quant",
-            "sfp8_moe_plan": "moe_plan",
-            "sfp8_moe_gemm_gateup_swiglu_fwd": "moe_gateup_swiglu_fwd", "sfp8_moe_gemm_down_fwd": "moe_down_fwd",
-            "sfp8_moe_gemm_down_dgrad_swiglu": "moe_down_dgrad_swiglu_bf16",
-            "sfp8_moe_gemm_gateup_dgrad": "moe_gateup_dgrad", "sfp8_moe_topk_sum": "moe_topk_sum"}.get(sym, sym)
+    """Kernel name of a launch: a C-ABI symbol, or an ``ops`` wrapper, and its
+    positional arguments."""
+    if sym == "wgrad_rows":
+        return "wgrad_down" if a[2] == D else "wgrad_gateup"
+    if sym == "weight_quant_experts":
+        return "weight_quant_gu" if a[0].shape[1] == 2 * I else "weight_quant_down"
+    if sym == "moe_wgrad_rows":
+        return "moe_wgrad_down" if a[2] == D else "moe_wgrad_gateup"
+    if sym == "moe_rows_quant":
+        return "moe_gather_quant_x" if a[8] == 0 else "moe_quant_dout"
+    return {"down_dgrad_swiglu": "down_dgrad_swiglu_bf16", "sfp8_update_scales": "update_scales",
+            "block_weight_quant": "post_step_quant", "moe_down_dgrad_swiglu": "moe_down_dgrad_swiglu_bf16"}.get(sym, sym)
 
 
 def rates(work: dict, name: str, ms: float) -> dict:
@@ -442,28 +431,37 @@ def rates(work: dict, name: str, ms: float) -> dict:
 
 def trace_steps(step, steps: int, stream, namer) -> dict:
     """`steps` more steps with HIP events recorded on `stream` around every
-    C-ABI launch: {kernel name: [ms per launch, ...]}."""
+    native wrapper's and every C-ABI launch: {kernel name: [ms per launch, ...]}."""
     import torch
 
-    from spark_gpt_amd import _lib
+    from spark_gpt_amd import _lib, ops
 
     marks = []
+
+    def traced(fn, name=None):
+        def call(*a, **kw):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record(stream)
+            out = fn(*a, **kw)
+            e1.record(stream)
+            marks.append((namer(name, a) if name else namer(a[0], a[1:]), e0, e1))
+            return out
+
+        return call
+
+    plain = {n: getattr(ops, n) for n in ops._NATIVE}
     plain_call = _lib.call
-
-    def traced_call(name, *a):
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        e0.record(stream)
-        plain_call(name, *a)
-        e1.record(stream)
-        marks.append((namer(name, a), e0, e1))
-
-    _lib.call = traced_call
+    _lib.call = traced(plain_call)
+    for n, fn in plain.items():
+        setattr(ops, n, traced(fn, n))
     try:
         for _ in range(steps):
             step()
         torch.cuda.synchronize()
     finally:
         _lib.call = plain_call
+        for n, fn in plain.items():
+            setattr(ops, n, fn)
     per = {}
     for name, e0, e1 in marks:
         per.setdefault(name, []).append(e0.elapsed_time(e1))
@@ -540,12 +538,10 @@ def make_moe(T: int, D: int, I: int, E: int, k: int, seed: int = 4):
 
 
 def bf16_launch_name(sym: str, a) -> str:
-    """Kernel name of a C-ABI launch of the bf16 SwiGLU path."""
-    return {"sfp8_bf16_weight_slabs": "bf16_weight_fold", "sfp8_bf16_rows_prep": "bf16_rows_prep",
-            "sfp8_bf16_gemm_swiglu_fwd": "bf16_gateup_swiglu_fwd", "sfp8_bf16_swiglu_bwd": "bf16_swiglu_bwd_rows",
-            "sfp8_bf16_gemm": "bf16_gateup_dgrad", "sfp8_bf16_norm_dh": "bf16_norm_bwd",
-            "sfp8_bf16_gemm_wgrad": "bf16_wgrad_gateup", "sfp8_bf16_gemm_wgrad_rows": "bf16_wgrad_gateup",
-            "sfp8_bf16_fold_grads": "bf16_fold_grads"}.get(sym, sym)
+    """Kernel name of a launch of the bf16 SwiGLU path."""
+    return {"bf16_weight_slabs": "bf16_weight_fold", "bf16_swiglu_fwd": "bf16_gateup_swiglu_fwd",
+            "bf16_swiglu_bwd": "bf16_swiglu_bwd_rows", "bf16_gemm": "bf16_gateup_dgrad",
+            "bf16_norm_dh": "bf16_norm_bwd", "bf16_wgrad_rows": "bf16_wgrad_gateup"}.get(sym, sym)
 
 
 def time_bf16(T: int, D: int, I: int, steps: int, warmup: int) -> dict:

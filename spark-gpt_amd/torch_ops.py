@@ -199,11 +199,12 @@ def block_bwd_impl(dy: Tensor, h: Tensor, norm_w: Tensor, w_gu: Tensor, w_down: 
     # d_gu8, while part of it is still in the last-level cache (the launch
     # order of train.py:1249-1251 is a9, a10, a11, a12, a13; the results
     # do not depend on it): about 1 % off the backward.
-    dwgu = ops.wgrad_rows(dgu8, x8, 2 * I, D, scale[3:4], scale[0:1])
+    s = scale.split(1)
+    dwgu = ops.wgrad_rows(dgu8, x8, 2 * I, D, s[3], s[0])
     del dgu8
     dh, dnw, dy8t = ops.norm_bwd(h, rstd, dxn, dy, _master(norm_w), scale, amax)
     del dxn
-    dwd = ops.wgrad_rows(dy8t, h8, D, I, scale[4:5], scale[2:3], a_rows=False)
+    dwd = ops.wgrad_rows(dy8t, h8, D, I, s[4], s[2], a_rows=False)
     return dh, dnw, dwgu, dwd
 
 
@@ -273,8 +274,9 @@ def moe_bwd_impl(dout: Tensor, w_gu: Tensor, w_d: Tensor, plan: Tensor, x8: Tens
     dx = ops.moe_gateup_dgrad(dgu8, w8t, plan, scale, wscale[0], R, D)
     # d_gu8, x8 and h8 read as their K-slabs (transposing LDS reads), dout8t
     # token-contiguous, as in the dense block
-    dw_gu = ops.moe_wgrad_rows(dgu8, x8, I2, D, E, plan, scale[3:4], scale[0:1])
-    dw_d = ops.moe_wgrad_rows(dout8t, h8, D, I2 // 2, E, plan, scale[4:5], scale[2:3], a_rows=False)
+    s = scale.split(1)
+    dw_gu = ops.moe_wgrad_rows(dgu8, x8, I2, D, E, plan, s[3], s[0])
+    dw_d = ops.moe_wgrad_rows(dout8t, h8, D, I2 // 2, E, plan, s[4], s[2], a_rows=False)
     dxn = ops.moe_topk_sum(dx, inverse_permutation, T, top_k)
     return dxn, dw_gu, dw_d
 

@@ -112,6 +112,26 @@ def test_ops_reject_host_tensors():
         ops.quant_e4m3_rowcol(h, torch.ones(5), torch.zeros(5))
 
 
+def test_native_wrappers_refuse_host_tensors():
+    """The native wrappers check before they launch: a host tensor raises
+    ValueError, a wrong keyword or a non-tensor TypeError."""
+    b = torch.zeros(4, 128, dtype=torch.bfloat16)
+    f, s = torch.zeros(256, 128), torch.ones(5)
+    x8, g8 = torch.zeros(2, 256, 64).to(ops.E4M3), torch.zeros(2, 256, 64).to(ops.E5M2)
+    for fn, args in ((ops.block_weight_quant, (f, f)), (ops.weight_quant_experts, (f[None], s)),
+                     (ops.gateup_swiglu_fwd, (x8, x8, s, s, s, 4, 128)), (ops.down_fwd, (x8, x8, b, s, s)),
+                     (ops.down_dgrad_swiglu, (b, x8, x8, s, s)), (ops.gateup_dgrad, (g8, x8, s, s, 4, 128)),
+                     (ops.wgrad_rows, (g8, x8, 128, 128, s, s)), (ops.norm_bwd, (b, s, b, b, s, s, s)),
+                     (ops.moe_plan, (torch.ones(2, dtype=torch.int32), 4)), (ops.moe_topk_sum, (b, s, 2, 2)),
+                     (ops.bf16_weight_slabs, (f[None],)), (ops.bf16_norm_dh, (b, b, s))):
+        with pytest.raises(ValueError):
+            fn(*args)
+    with pytest.raises(TypeError):
+        ops.norm_quant(b, s, s, s, 1e-6, rows=True)
+    with pytest.raises(TypeError):
+        ops.down_fwd(None, x8, b, s, s)
+
+
 def test_slab_layout_roundtrip():
     """K-slab copies: element (r, t) at [t // 64, r, t % 64], rows padded to 256."""
     assert ops.slab_rows(1) == 256 and ops.slab_rows(256) == 256 and ops.slab_rows(768) == 768
