@@ -990,8 +990,8 @@ struct TileShape {
   static constexpr int kThreads = SMALL ? 256 : 512;
   static constexpr int kMinWaves = SMALL ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
   static constexpr int kWN = SMALL ? 2 : 4, kTB = SMALL ? 2 : 4;
-  template <bool BF16, int FA, int FB>
-  using Loop = MainLoop<BF16, FA, FB, false, 2, kStages, 0, false, false, kWN, kTB, kM>;
+  template <bool BF16, int FA, int FB, bool TRA = false, bool TRB = false>
+  using Loop = MainLoop<BF16, FA, FB, false, 2, kStages, 0, TRA, TRB, kWN, kTB, kM>;
   static constexpr int kLds = Loop<true, 0, 0>::kLds;
   // the plan's tile of tile row tm, and that tile row's valid rows of it
   static SFP8_DEV int plan_tile(int tm) { return SMALL ? tm >> 1 : tm; }
@@ -1437,9 +1437,9 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // reads (MainLoop TR_A / TR_B); the partials then always go to `out` as the
 // workspace, in the same order (with TRB the columns unpermuted:
 // splitk_reduce_kernel<true>).
-// NW = 4 waves (one per SIMD) of 128 x 128, or 8 (two per SIMD) of 128 x 64,
-// so that one wave's stage waits and barriers are covered by the other's
-// MFMAs; the accumulator order follows the wave shape (acc_order_rc).
+// SMALL: 128 x 128 tiles (4 waves of 64 x 64, two work-groups per CU) instead
+// of 256 x 256 (8 waves of 128 x 64, one per CU); the partials' tiles and
+// accumulator order follow the shape (acc_order_rc), the sums do not.
 // Addressing of a transposed-read operand: row r of block r / 64 (fp8) or
 // r / 32 (bf16) at token t lies at base + block * bs + t * ts, and ext bytes
 // are readable from base (the rest reads as zero).  A row K-slab of [T, L]
@@ -1449,25 +1449,20 @@ struct TrOp {
   int64_t ts, bs, ext;
 };
 
-// Waves per work-group of the weight gradients (FP8 and bf16).
-constexpr int kWgradWaves = 8;
-constexpr int kBf16WgradWaves = 8;
-
-template <bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false, int NW = 4>
-__global__ __launch_bounds__(64 * NW, 1) void wgrad_kernel(
+template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void wgrad_kernel(
     const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldt,
     int64_t kchunk, const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out,
     int tiles_m, int tiles_n, int splits, int partials, TrOp tra, TrOp trb) {
-  static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-  constexpr int NB = NW == 8 ? 2 : 4, WN = NW / 2;  // B blocks of 32 per wave, wave columns
+  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   int tm, tn, sp;
   split_tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, splits, tm, tn, sp);
   if (sp >= splits) return;  // grid padding (work-group uniform)
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-  floatx16 acc[4][NB];
+  floatx16 acc[TS::kTB][2];
   const int64_t kb = (int64_t)sp * kchunk;
   {
     // K-slab operands: slab (kb / 64) of A starts at (kb / 64) * rpa * 64.
@@ -1481,36 +1476,36 @@ __global__ __launch_bounds__(64 * NW, 1) void wgrad_kernel(
     const uint8_t* b0 = TRB ? bt + (n0 / kRows) * trb.bs + t0 * trb.ts : bt + (kb / kStage) * rpb * kStage + n0 * kStage;
     const uint8_t* a_end = TRA ? at + tra.ext : at + ldt * rpa;
     const uint8_t* b_end = TRB ? bt + trb.ext : bt + ldt * rpb;
-    MainLoop<BF16, FMT_A, FMT_B, false, NB, kStages, 0, TRA, TRB, WN>::run(
+    TS::template Loop<BF16, FMT_A, FMT_B, TRA, TRB>::run(
         lds, a0, a_end - a0, [=](int r) { return TRA ? (r / kRows) * abs_ + (r % kRows) * ats : r * kStage; },
         TRA ? kRows * ats : (int)(rpa * kStage), b0, b_end - b0,
-        [=](int r) { return TRB ? (r / kRows) * bbs + (r % kRows) * bts : plain_col_nb<NB>(r) * kStage; },
+        [=](int r) { return TRB ? (r / kRows) * bbs + (r % kRows) * bts : plain_col_nb<2>(r) * kStage; },
         TRB ? kRows * bts : (int)(rpb * kStage), (int)((kchunk < ldt - kb ? kchunk : ldt - kb) / kStage), acc);
   }
   if (BF16 || TRA || TRB || partials) {
     // accumulator order: [split][tile][wave][tb][nb][i][lane][4]
-    float* frag = out + ((int64_t)sp * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (kTile * kTile) +
-                  wave * (kTile * kTile / NW);
+    float* frag = out + ((int64_t)sp * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kM) +
+                  wave * (TS::kM * TS::kM / (TS::kThreads / 64));
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb)
+    for (int tb = 0; tb < TS::kTB; ++tb)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          reinterpret_cast<floatx4*>(frag + (tb * NB + nb) * 1024 + i * 256)[lane] =
+          reinterpret_cast<floatx4*>(frag + (tb * 2 + nb) * 1024 + i * 256)[lane] =
               floatx4{acc[tb][nb][4 * i], acc[tb][nb][4 * i + 1], acc[tb][nb][4 * i + 2], acc[tb][nb][4 * i + 3]};
     return;
   }
   const float deq = 1.0f / (sa[0] * sb[0]);
   float* dst = out;
   const int fr = lane & 31, g = lane >> 5;
-  const int cb = 32 * NB * wn + 16 * NB * g;  // plain_col_nb<NB>
+  const int cb = 64 * wn + 32 * g;  // plain_col_nb<2>
 #pragma unroll
-  for (int tb = 0; tb < 4; ++tb) {
-    const int64_t m = m0 + 128 * wm + 32 * tb + fr;
+  for (int tb = 0; tb < TS::kTB; ++tb) {
+    const int64_t m = m0 + 32 * TS::kTB * wm + 32 * tb + fr;
     if (m >= M) continue;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+    for (int nb = 0; nb < 2; ++nb) {
       const int64_t n = n0 + cb + 16 * nb;
       floatx4* p = reinterpret_cast<floatx4*>(dst + m * N + n);
       // N % 4 == 0: each float4 is wholly inside the row or wholly past it
@@ -1537,13 +1532,12 @@ __global__ __launch_bounds__(64 * NW, 1) void wgrad_kernel(
 // ws[e][sp][tile], summed in split order by splitk_reduce_kernel.
 // BF16: bf16 operands, 2 bytes per padded row (`ldp` counts K bytes), and the
 // partials always go to ws, for bf16_wgrad_reduce_kernel to round.
-template <bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false, int NW = 4>
-__global__ __launch_bounds__(64 * NW, 1) void moe_wgrad_kernel(
+template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void moe_wgrad_kernel(
     const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
     const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out, float* __restrict__ ws,
     const int* __restrict__ plan, int tiles_m, int tiles_n, int splits) {
-  static_assert(NW == 4 || NW == 8, "4 or 8 waves (as wgrad_kernel)");
-  constexpr int NB = NW == 8 ? 2 : 4, WN = NW / 2;
+  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   const MoePlan P{plan};
   const int tiles = tiles_m * tiles_n;
@@ -1551,7 +1545,7 @@ __global__ __launch_bounds__(64 * NW, 1) void moe_wgrad_kernel(
   const int sp = (lid / tiles) % splits, e = lid / (tiles * splits);
   int tm, tn;
   raster(lid % tiles, tiles_m, tiles_n, tm, tn);
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   constexpr int64_t kBpe = BF16 ? 2 : 1;  // K bytes per padded row
@@ -1574,36 +1568,36 @@ __global__ __launch_bounds__(64 * NW, 1) void moe_wgrad_kernel(
   const uint8_t* a_end = TRA ? at + (M / kRows) * ldt_tok * kStage : at + ldp * rpa;
   const uint8_t* b_end = TRB ? bt + (N / kRows) * ldt_tok * kStage : bt + ldp * rpb;
   const int64_t a_bytes = nk > 0 ? a_end - a0 : 0, b_bytes = nk > 0 ? b_end - b0 : 0;
-  floatx16 acc[4][NB];
-  MainLoop<BF16, FMT_A, FMT_B, false, NB, kStages, 0, TRA, TRB, WN>::run(
+  floatx16 acc[TS::kTB][2];
+  TS::template Loop<BF16, FMT_A, FMT_B, TRA, TRB>::run(
       lds, a0, a_bytes, [=](int r) { return TRA ? ((r / kRows) * ltok + (r % kRows)) * kStage : r * kStage; },
       TRA ? kRows * kStage : (int)(rpa * kStage), b0, b_bytes,
-      [=](int r) { return TRB ? ((r / kRows) * ltok + (r % kRows)) * kStage : plain_col_nb<NB>(r) * kStage; },
+      [=](int r) { return TRB ? ((r / kRows) * ltok + (r % kRows)) * kStage : plain_col_nb<2>(r) * kStage; },
       TRB ? kRows * kStage : (int)(rpb * kStage), (int)nk, acc);
   if (BF16 || TRA || TRB || splits > 1) {
     // accumulator order: [expert][split][tile][wave][tb][nb][i][lane][4]
-    float* frag = ws + (((int64_t)e * splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (kTile * kTile) +
-                  wave * (kTile * kTile / NW);
+    float* frag = ws + (((int64_t)e * splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kM) +
+                  wave * (TS::kM * TS::kM / (TS::kThreads / 64));
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb)
+    for (int tb = 0; tb < TS::kTB; ++tb)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          reinterpret_cast<floatx4*>(frag + (tb * NB + nb) * 1024 + i * 256)[lane] =
+          reinterpret_cast<floatx4*>(frag + (tb * 2 + nb) * 1024 + i * 256)[lane] =
               floatx4{acc[tb][nb][4 * i], acc[tb][nb][4 * i + 1], acc[tb][nb][4 * i + 2], acc[tb][nb][4 * i + 3]};
     return;
   }
   const float deq = 1.0f / (sa[0] * sb[0]);
   float* dst = out + (int64_t)e * M * N;
   const int fr = lane & 31, g = lane >> 5;
-  const int cb = 32 * NB * wn + 16 * NB * g;  // plain_col_nb<NB>
+  const int cb = 64 * wn + 32 * g;  // plain_col_nb<2>
 #pragma unroll
-  for (int tb = 0; tb < 4; ++tb) {
-    const int64_t m = m0 + 128 * wm + 32 * tb + fr;
+  for (int tb = 0; tb < TS::kTB; ++tb) {
+    const int64_t m = m0 + 32 * TS::kTB * wm + 32 * tb + fr;
     if (m >= M) continue;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+    for (int nb = 0; nb < 2; ++nb) {
       const int64_t n = n0 + cb + 16 * nb;
       floatx4* p = reinterpret_cast<floatx4*>(dst + m * N + n);
 #pragma unroll
@@ -1621,20 +1615,21 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(float* __restrict__ out,
   if (i < n) *reinterpret_cast<floatx4*>(out + i) = floatx4{0.f, 0.f, 0.f, 0.f};
 }
 
-// Tile row r and column c of the first value of float4 q (< 16384) of one
-// 256 x 256 partial tile of wgrad_kernel<.., NW> in accumulator order
-// [wave][tb][nb][i][lane][4] (NB = 4 or 2 blocks of 32 columns per wave;
-// wave (wm, wn) = (wave & 1, wave >> 1) owns rows 128 wm.. and columns
-// 32 NB wn..): B-tile rows permuted by plain_col_nb<NB> (accumulator v of
-// block nb, lane half g is column 32 NB wn + 16 NB g + 16 nb + v), or with
-// TR_B unpermuted (column 32 NB wn + 32 nb + 8 (v / 4) + 4 g + v % 4).
-template <int NW, bool TR_B>
+// Tile row r and column c of the first value of float4 q of one partial tile
+// of wgrad_kernel<SMALL, ..> in accumulator order [wave][tb][nb][i][lane][4]
+// (kTileQ float4s; wave (wm, wn) = (wave & 1, wave >> 1) owns rows
+// 32 kTB wm.. and columns 64 wn..): B-tile rows permuted by plain_col_nb<2>
+// (accumulator v of block nb, lane half g is column 64 wn + 32 g + 16 nb + v),
+// or with TR_B unpermuted (column 64 wn + 32 nb + 8 (v / 4) + 4 g + v % 4).
+template <bool SMALL>
+constexpr int kTileQLog = SMALL ? 12 : 14;  // log2 of the float4s of a tile
+template <bool SMALL, bool TR_B>
 SFP8_DEV void acc_order_rc(int q, int& r, int& c) {
-  constexpr int NB = NW == 8 ? 2 : 4, NBB = NW == 8 ? 1 : 2;
-  const int lane = q & 63, i = (q >> 6) & 3, nb = (q >> 8) & (NB - 1), tb = (q >> (8 + NBB)) & 3;
-  const int wave = (q >> (10 + NBB)) & (NW - 1), g = lane >> 5;
-  r = 128 * (wave & 1) + 32 * tb + (lane & 31);
-  c = 32 * NB * (wave >> 1) + (TR_B ? 32 * nb + 8 * i + 4 * g : 16 * NB * g + 16 * nb + 4 * i);
+  constexpr int TBB = SMALL ? 1 : 2;  // bits of tb
+  const int lane = q & 63, i = (q >> 6) & 3, nb = (q >> 8) & 1, tb = (q >> 9) & (TileShape<SMALL>::kTB - 1);
+  const int wave = (q >> (9 + TBB)) & (TileShape<SMALL>::kThreads / 64 - 1), g = lane >> 5;
+  r = 32 * TileShape<SMALL>::kTB * (wave & 1) + 32 * tb + (lane & 31);
+  c = 64 * (wave >> 1) + (TR_B ? 32 * nb + 8 * i + 4 * g : 32 * g + 16 * nb + 4 * i);
 }
 
 // Split-K reduction of the accumulator-order partials of wgrad_kernel:
@@ -1642,7 +1637,7 @@ SFP8_DEV void acc_order_rc(int q, int& r, int& c) {
 // q-th float4 of one split's partials; its (m, n) follows from the MFMA
 // accumulator layout (acc_order_rc; TR_B: partials of wgrad_kernel<..,
 // true>).
-template <bool TR_B = false, int NW = 4>
+template <bool SMALL, bool TR_B>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int splits,
                                                             int64_t n4, int tiles_n, int64_t M, int64_t N,
                                                             const float* __restrict__ sa,
@@ -1656,10 +1651,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   floatx4 acc = __builtin_nontemporal_load(w4 + q);
   for (int s = 1; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
   int r, c;
-  acc_order_rc<NW, TR_B>((int)(q & 16383), r, c);
-  const int64_t tile = q >> 14;
+  acc_order_rc<SMALL, TR_B>((int)(q & ((1 << kTileQLog<SMALL>) - 1)), r, c);
+  const int64_t tile = q >> kTileQLog<SMALL>;
   const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
-  const int64_t m = tm * kTile + r, n = tn * kTile + c;
+  const int64_t m = tm * TileShape<SMALL>::kM + r, n = tn * TileShape<SMALL>::kM + c;
   if (m < M && n < N) {
     const float deq = 1.0f / (sa[0] * sb[0]);
     *reinterpret_cast<floatx4*>(out + m * N + n) = acc * deq;
@@ -1829,7 +1824,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // ascending of ws[s]) (the bf16 result of _swiglu_wgrad_kernel,
 // train.py:1983-2026), partials in wgrad_kernel's accumulator order;
 // blockIdx.y = expert of a grouped gradient (out [E, M, N]).
-template <bool TR_B = false, int NW = 4>
+template <bool SMALL, bool TR_B>
 __global__ __launch_bounds__(256) void bf16_wgrad_reduce_kernel(const float* __restrict__ ws, int splits, int64_t n4,
                                                                 int tiles_n, int64_t M, int64_t N,
                                                                 uint16_t* __restrict__ out) {
@@ -1841,10 +1836,10 @@ __global__ __launch_bounds__(256) void bf16_wgrad_reduce_kernel(const float* __r
   floatx4 acc = __builtin_nontemporal_load(w4 + q);
   for (int s = 1; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
   int r, c;
-  acc_order_rc<NW, TR_B>((int)(q & 16383), r, c);
-  const int64_t tile = q >> 14;
+  acc_order_rc<SMALL, TR_B>((int)(q & ((1 << kTileQLog<SMALL>) - 1)), r, c);
+  const int64_t tile = q >> kTileQLog<SMALL>;
   const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
-  const int64_t m = tm * kTile + r, n = tn * kTile + c;
+  const int64_t m = tm * TileShape<SMALL>::kM + r, n = tn * TileShape<SMALL>::kM + c;
   if (m < M && n < N)  // N % 4 == 0: the 4 values are wholly inside or past the row
     *reinterpret_cast<intx2*>(out + m * N + n) = intx2{(int)pack2_bf16(acc[0], acc[1]), (int)pack2_bf16(acc[2], acc[3])};
 }
@@ -1856,8 +1851,8 @@ __global__ __launch_bounds__(256) void bf16_wgrad_reduce_kernel(const float* __r
 // the Newton-Schulz staging matrix ([M, N] bf16, the parameter's layout);
 // grad[m, n] = d when grad is given.  splits == 0: d = 0 (no tokens).  TR_B:
 // the partials' columns are in the transposed-read B order, as for
-// splitk_reduce_kernel<true>; NW: the partials of wgrad_kernel<.., NW>.
-template <bool TR_B = false, int NW = 4>
+// splitk_reduce_kernel<true>; SMALL: the partials of wgrad_kernel<SMALL, ..>.
+template <bool SMALL, bool TR_B>
 __global__ __launch_bounds__(256) void splitk_momentum_kernel(const float* __restrict__ ws, int splits, int64_t n4,
                                                               int tiles_n, int64_t M, int64_t N,
                                                               const float* __restrict__ sa,
@@ -1873,22 +1868,24 @@ __global__ __launch_bounds__(256) void splitk_momentum_kernel(const float* __res
   const floatx4* w4 = reinterpret_cast<const floatx4*>(ws);
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
-  constexpr int NB = NW == 8 ? 2 : 4, NBB = NW == 8 ? 1 : 2;
+  using TS = TileShape<SMALL>;
+  constexpr int TBB = SMALL ? 1 : 2;  // bits of tb
   const int lane = threadIdx.x & 63, i = threadIdx.x >> 6;
   const int64_t b = blockIdx.x;
-  const int nb = (int)(b & (NB - 1)), tb = (int)(b >> NBB) & 3, wave = (int)(b >> (NBB + 2)) & (NW - 1);
-  const int64_t tile = b >> 6;
+  const int nb = (int)(b & 1), tb = (int)(b >> 1) & (TS::kTB - 1);
+  const int wave = (int)(b >> (1 + TBB)) & (TS::kThreads / 64 - 1);
+  const int64_t tile = b >> (kTileQLog<SMALL> - 8);
   const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
   // local column (0..31) of this thread's float4 in the block
   const int c = TR_B ? 8 * i + 4 * (lane >> 5) : 16 * (lane >> 5) + 4 * i;
   blk[lane & 31][c >> 2] = acc * (1.0f / (sa[0] * sb[0]));
   __syncthreads();
   const int r = threadIdx.x >> 3, c2 = 4 * (threadIdx.x & 7);
-  const int64_t m = tm * kTile + 128 * (wave & 1) + 32 * tb + r;
+  const int64_t m = tm * TS::kM + 32 * TS::kTB * (wave & 1) + 32 * tb + r;
   // local column -> output column: TR_B blocks are 32 contiguous columns,
-  // the plain layout's two 16-column halves lie 16 NB columns apart
+  // the plain layout's two 16-column halves lie 32 columns apart
   const int64_t n =
-      tn * kTile + 32 * NB * (wave >> 1) + (TR_B ? 32 * nb + c2 : 16 * nb + (c2 < 16 ? c2 : 16 * NB - 16 + c2));
+      tn * TS::kM + 64 * (wave >> 1) + (TR_B ? 32 * nb + c2 : 16 * nb + (c2 < 16 ? c2 : 16 + c2));
   if (m >= M || n >= N) return;
   const floatx4 d = blk[r][c2 >> 2];
   if (grad) *reinterpret_cast<floatx4*>(grad + m * N + n) = d;
@@ -1976,53 +1973,97 @@ namespace {
 // dgrad 49 -> 26, 50 -> 38, 55 -> 45, 62 -> 71; bf16 dgrad 91 -> 46, 94 -> 73,
 // 99 -> 88, 125 -> 135.  At 320 tiles (a second round of 64) the two differ by
 // less than a tenth either way, and the larger ones stay.
-inline bool use_small_tiles(int64_t M, int64_t N) {
+inline bool use_small_tiles(int64_t M, int64_t N, int64_t parts = 1) {
   constexpr int64_t kCUs = 256;
-  return (int64_t)cdiv(M, kTile) * cdiv(N, kTile) <= kCUs / 2;
+  return (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * parts <= kCUs / 2;
 }
 
-// A GEMM's tile shape over an M x N output, and its launch.
+// A GEMM's tile shape over an M x N output (of each of `parts` K splits times
+// experts), and its launch.
 struct Tiling {
   bool small;
   int m, n, lds;  // tile rows and columns, dynamic LDS
   dim3 grid, block;
 };
-inline Tiling tiling(int64_t M, int64_t N) {
+inline Tiling tiling(int64_t M, int64_t N, int64_t parts = 1) {
   Tiling t;
-  t.small = use_small_tiles(M, N);
+  t.small = use_small_tiles(M, N, parts);
   const int tile = t.small ? TileShape<true>::kM : TileShape<false>::kM;
   t.m = cdiv(M, tile);
   t.n = cdiv(N, tile);
   t.lds = t.small ? TileShape<true>::kLds : TileShape<false>::kLds;
-  t.grid = dim3((unsigned)(t.m * t.n));
+  t.grid = dim3((unsigned)(t.m * t.n * parts));
   t.block = dim3((unsigned)(t.small ? TileShape<true>::kThreads : TileShape<false>::kThreads));
   return t;
 }
 
-// The split partials ws[split][tile] (one 256 x 256 fp32 tile each, in
-// accumulator order of wgrad_kernel<.., kWgradWaves>) of the FP8 weight
-// gradient; TRA / TRB: that operand is the row K-slab of the token-major
-// activation instead of a token-contiguous copy.
-template <bool TRA, bool TRB>
-int wgrad_partials(const void* a, const void* b, int64_t M, int64_t N, int64_t ldt, const float* sa, const float* sb,
-                   float* ws, int splits, hipStream_t st) {
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  const int rc = prep(wgrad_kernel<false, kFmtE5M2, kFmtE4M3, TRA, TRB, kWgradWaves>, kMainLds);
+// wgrad_kernel over one weight gradient's tiles and splits (tl of M x N and
+// `splits` parts): `ldt` and `chunk` K bytes in all and per split.
+template <bool BF16, int FMT_A, int FMT_B, bool TRA, bool TRB>
+int launch_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, int64_t N, int64_t ldt, int64_t chunk,
+                 const float* sa, const float* sb, float* out, int splits, int partials, TrOp tra, TrOp trb,
+                 hipStream_t st) {
+  const auto kern = tl.small ? wgrad_kernel<true, BF16, FMT_A, FMT_B, TRA, TRB>
+                             : wgrad_kernel<false, BF16, FMT_A, FMT_B, TRA, TRB>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  // row K-slabs over ldt tokens
-  const TrOp tra{kStage, ldt * kStage, (M / 64) * ldt * kStage}, trb{kStage, ldt * kStage, (N / 64) * ldt * kStage};
-  hipLaunchKernelGGL((wgrad_kernel<false, kFmtE5M2, kFmtE4M3, TRA, TRB, kWgradWaves>),
-                     dim3((unsigned)wgrad_grid(tiles_m * tiles_n, splits)), dim3(64 * kWgradWaves), kMainLds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldt, wgrad_chunk(ldt, splits), sa,
-                     sb, ws, tiles_m, tiles_n, splits, 1, tra, trb);
+  const dim3 grid = BF16 || tl.small ? tl.grid : dim3((unsigned)wgrad_grid(tl.m * tl.n, splits));
+  hipLaunchKernelGGL(kern, grid, tl.block, tl.lds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldt, chunk, sa, sb,
+                     out, tl.m, tl.n, splits, partials, tra, trb);
   return status();
 }
 
-int wgrad_partials_any(bool a_rows, bool b_rows, const void* a, const void* b, int64_t M, int64_t N, int64_t ldt,
-                       const float* sa, const float* sb, float* ws, int splits, hipStream_t st) {
-  if (a_rows && b_rows) return wgrad_partials<true, true>(a, b, M, N, ldt, sa, sb, ws, splits, st);
-  if (a_rows) return wgrad_partials<true, false>(a, b, M, N, ldt, sa, sb, ws, splits, st);
-  if (b_rows) return wgrad_partials<false, true>(a, b, M, N, ldt, sa, sb, ws, splits, st);
-  return wgrad_partials<false, false>(a, b, M, N, ldt, sa, sb, ws, splits, st);
+// moe_wgrad_kernel over every expert's tiles and splits (tl of M x N and
+// E * splits parts).
+template <bool BF16, int FMT_A, int FMT_B, bool TRA, bool TRB>
+int launch_moe_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, int64_t N, int64_t ldp,
+                     const float* sa, const float* sb, float* out, float* ws, const int* plan, int splits,
+                     hipStream_t st) {
+  const auto kern = tl.small ? moe_wgrad_kernel<true, BF16, FMT_A, FMT_B, TRA, TRB>
+                             : moe_wgrad_kernel<false, BF16, FMT_A, FMT_B, TRA, TRB>;
+  const int rc = prep(kern, tl.lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out,
+                     ws, plan, tl.m, tl.n, splits);
+  return status();
+}
+
+// float4s of one split's partials, and the launches of the reductions over
+// them (E experts; tr_b: the partials of a transposed-read B).
+inline int64_t partial_quads(const Tiling& tl) { return (int64_t)tl.m * tl.n << (tl.small ? 12 : 14); }
+inline dim3 reduce_grid(const Tiling& tl, int64_t E) {
+  return dim3((unsigned)((partial_quads(tl) + 255) / 256), (unsigned)E);
+}
+int launch_reduce(const Tiling& tl, bool tr_b, const float* ws, int splits, int64_t E, int64_t M, int64_t N,
+                  const float* sa, const float* sb, float* out, hipStream_t st) {
+  const auto kern = tl.small ? (tr_b ? splitk_reduce_kernel<true, true> : splitk_reduce_kernel<true, false>)
+                             : (tr_b ? splitk_reduce_kernel<false, true> : splitk_reduce_kernel<false, false>);
+  hipLaunchKernelGGL(kern, reduce_grid(tl, E), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N, sa, sb,
+                     out);
+  return status();
+}
+int launch_bf16_reduce(const Tiling& tl, bool tr_b, const float* ws, int splits, int64_t E, int64_t M, int64_t N,
+                       void* out, hipStream_t st) {
+  const auto kern = tl.small
+                        ? (tr_b ? bf16_wgrad_reduce_kernel<true, true> : bf16_wgrad_reduce_kernel<true, false>)
+                        : (tr_b ? bf16_wgrad_reduce_kernel<false, true> : bf16_wgrad_reduce_kernel<false, false>);
+  hipLaunchKernelGGL(kern, reduce_grid(tl, E), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N,
+                     (uint16_t*)out);
+  return status();
+}
+
+// The split partials ws[split][tile] (one fp32 tile each, in accumulator
+// order) of the FP8 weight gradient; a_rows / b_rows: that operand is the row
+// K-slab of the token-major activation instead of a token-contiguous copy.
+int wgrad_partials(const Tiling& tl, bool a_rows, bool b_rows, const void* a, const void* b, int64_t M, int64_t N,
+                   int64_t ldt, const float* sa, const float* sb, float* ws, int splits, hipStream_t st) {
+  // row K-slabs over ldt tokens
+  const TrOp tra{kStage, ldt * kStage, (M / 64) * ldt * kStage}, trb{kStage, ldt * kStage, (N / 64) * ldt * kStage};
+  const auto launch = a_rows ? (b_rows ? launch_wgrad<false, kFmtE5M2, kFmtE4M3, true, true>
+                                       : launch_wgrad<false, kFmtE5M2, kFmtE4M3, true, false>)
+                             : (b_rows ? launch_wgrad<false, kFmtE5M2, kFmtE4M3, false, true>
+                                       : launch_wgrad<false, kFmtE5M2, kFmtE4M3, false, false>);
+  return launch(tl, a, b, M, N, ldt, wgrad_chunk(ldt, splits), sa, sb, ws, splits, 1, tra, trb, st);
 }
 }  // namespace
 
@@ -2204,19 +2245,12 @@ int sfp8_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_
     hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, out, n);
     return status();
   }
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  int rc = prep(wgrad_kernel<false, kFmtE5M2, kFmtE4M3, false, false, kWgradWaves>, kMainLds);
-  if (rc) return rc;
-  hipLaunchKernelGGL((wgrad_kernel<false, kFmtE5M2, kFmtE4M3, false, false, kWgradWaves>),
-                     dim3((unsigned)wgrad_grid(tiles_m * tiles_n, (int)splits)), dim3(64 * kWgradWaves), kMainLds, st,
-                     (const uint8_t*)at, (const uint8_t*)bt, M, N, ldt, wgrad_chunk(ldt, splits), sa, sb,
-                     splits > 1 ? ws : out, tiles_m, tiles_n, (int)splits, (int)(splits > 1), TrOp{}, TrOp{});
-  rc = status();
+  const Tiling tl = tiling(M, N, splits);
+  const int rc = launch_wgrad<false, kFmtE5M2, kFmtE4M3, false, false>(
+      tl, at, bt, M, N, ldt, wgrad_chunk(ldt, splits), sa, sb, splits > 1 ? ws : out, (int)splits, (int)(splits > 1),
+      TrOp{}, TrOp{}, st);
   if (rc || splits == 1) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  hipLaunchKernelGGL((splitk_reduce_kernel<false, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256), 1), dim3(256), 0,
-                     st, ws, (int)splits, n4, tiles_n, M, N, sa, sb, out);
-  return status();
+  return launch_reduce(tl, false, ws, (int)splits, 1, M, N, sa, sb, out, st);
 }
 
 // ---- grouped (MoE expert) GEMMs over padded expert order (common.h) ----
@@ -2342,19 +2376,11 @@ int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, in
   const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
   if (splits > 1 && (!ws || ws_floats < sfp8_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  int rc = prep(moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, false, false, kWgradWaves>, kMainLds);
-  if (rc) return rc;
-  hipLaunchKernelGGL((moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, false, false, kWgradWaves>),
-                     dim3((unsigned)(tiles_m * tiles_n * splits * E)), dim3(64 * kWgradWaves), kMainLds, st,
-                     (const uint8_t*)at, (const uint8_t*)bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                     (int)splits);
-  rc = status();
+  const Tiling tl = tiling(M, N, E * splits);
+  const int rc = launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, false, false>(tl, at, bt, M, N, ldp, sa, sb, out, ws,
+                                                                           plan, (int)splits, st);
   if (rc || splits == 1) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  hipLaunchKernelGGL((splitk_reduce_kernel<false, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256), (unsigned)E),
-                     dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, sa, sb, out);
-  return status();
+  return launch_reduce(tl, false, ws, (int)splits, E, M, N, sa, sb, out, st);
 }
 
 // ---- the grouped weight gradient with row K-slab operands ----
@@ -2374,42 +2400,13 @@ int sfp8_moe_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b
   const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
   if (ws_floats < sfp8_moe_wgrad_rows_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  const dim3 grid((unsigned)(tiles_m * tiles_n * splits * E));
-  int rc;
-  if (a_rows && b_rows) {
-    rc = prep(moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, true, true, kWgradWaves>, kMainLds);
-    if (!rc)
-      hipLaunchKernelGGL((moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, true, true, kWgradWaves>), grid,
-                         dim3(64 * kWgradWaves), kMainLds, st,
-                         (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                         (int)splits);
-  } else if (a_rows) {
-    rc = prep(moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, true, false, kWgradWaves>, kMainLds);
-    if (!rc)
-      hipLaunchKernelGGL((moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, true, false, kWgradWaves>), grid,
-                         dim3(64 * kWgradWaves), kMainLds, st,
-                         (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                         (int)splits);
-  } else {
-    rc = prep(moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, false, true, kWgradWaves>, kMainLds);
-    if (!rc)
-      hipLaunchKernelGGL((moe_wgrad_kernel<false, kFmtE5M2, kFmtE4M3, false, true, kWgradWaves>), grid,
-                         dim3(64 * kWgradWaves), kMainLds, st,
-                         (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                         (int)splits);
-  }
+  const Tiling tl = tiling(M, N, E * splits);
+  const auto launch = a_rows ? (b_rows ? launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, true, true>
+                                       : launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, true, false>)
+                             : launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, false, true>;
+  const int rc = launch(tl, a, b, M, N, ldp, sa, sb, out, ws, plan, (int)splits, st);
   if (rc) return rc;
-  rc = status();
-  if (rc) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  if (b_rows)
-    hipLaunchKernelGGL((splitk_reduce_kernel<true, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256), (unsigned)E),
-                       dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, sa, sb, out);
-  else
-    hipLaunchKernelGGL((splitk_reduce_kernel<false, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256), (unsigned)E),
-                       dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, sa, sb, out);
-  return status();
+  return launch_reduce(tl, b_rows, ws, (int)splits, E, M, N, sa, sb, out, st);
 }
 
 
@@ -2508,18 +2505,11 @@ int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, i
   }
   const int64_t splits = sfp8_bf16_wgrad_splits(M, N, ldt);
   if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  int rc = prep(wgrad_kernel<true, 0, 0, false, false, kBf16WgradWaves>, kMainLds);
+  const Tiling tl = tiling(M, N, splits);
+  const int rc = launch_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldt, 2 * ldt / splits, nullptr, nullptr,
+                                                        ws, (int)splits, 1, TrOp{}, TrOp{}, st);
   if (rc) return rc;
-  hipLaunchKernelGGL((wgrad_kernel<true, 0, 0, false, false, kBf16WgradWaves>), dim3((unsigned)(tiles_m * tiles_n * splits)),
-                     dim3(64 * kBf16WgradWaves), kMainLds, st, (const uint8_t*)at, (const uint8_t*)bt, M, N, 2 * ldt,
-                     2 * ldt / splits, nullptr, nullptr, ws, tiles_m, tiles_n, (int)splits, 1, TrOp{}, TrOp{});
-  rc = status();
-  if (rc) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  hipLaunchKernelGGL((bf16_wgrad_reduce_kernel<false, kBf16WgradWaves>), dim3((unsigned)((n4 + 255) / 256), 1), dim3(256),
-                     0, st, ws, (int)splits, n4, tiles_n, M, N, (uint16_t*)out);
-  return status();
+  return launch_bf16_reduce(tl, false, ws, (int)splits, 1, M, N, out, st);
 }
 
 int64_t sfp8_bf16_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E) {
@@ -2535,19 +2525,11 @@ int sfp8_bf16_moe_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t 
   const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
   if (!ws || ws_floats < sfp8_bf16_moe_wgrad_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  int rc = prep(moe_wgrad_kernel<true, 0, 0, false, false, kBf16WgradWaves>, kMainLds);
+  const Tiling tl = tiling(M, N, E * splits);
+  const int rc = launch_moe_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldp, nullptr, nullptr, nullptr, ws,
+                                                            plan, (int)splits, st);
   if (rc) return rc;
-  hipLaunchKernelGGL((moe_wgrad_kernel<true, 0, 0, false, false, kBf16WgradWaves>),
-                     dim3((unsigned)(tiles_m * tiles_n * splits * E)), dim3(64 * kBf16WgradWaves), kMainLds, st,
-                     (const uint8_t*)at, (const uint8_t*)bt, M, N, 2 * ldp, nullptr, nullptr, nullptr, ws, plan,
-                     tiles_m, tiles_n, (int)splits);
-  rc = status();
-  if (rc) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  hipLaunchKernelGGL((bf16_wgrad_reduce_kernel<false, kBf16WgradWaves>), dim3((unsigned)((n4 + 255) / 256), (unsigned)E),
-                     dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, (uint16_t*)out);
-  return status();
+  return launch_bf16_reduce(tl, false, ws, (int)splits, E, M, N, out, st);
 }
 
 // ---- the bf16 weight gradients read through transposing LDS reads ----
@@ -2567,37 +2549,16 @@ int sfp8_bf16_gemm_wgrad_rows(const void* a, const void* x, int x_rows, int64_t 
   }
   const int64_t splits = sfp8_bf16_wgrad_splits(M, N, ldt);
   if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
   // a: the bf16 K-slab of [ldt, M] (32 columns per 64-byte row); x (x_rows):
   // row-major [T, N] bf16, tokens T..ldt-1 read as zero through the range
   // check, or else the token-contiguous bf16 K-slab of x^T over ldt tokens
   const TrOp tra{kStage, ldt * kStage, (M / 32) * ldt * kStage}, trb{2 * N, kStage, T * 2 * N};
-  const dim3 grid((unsigned)(tiles_m * tiles_n * splits));
-  int rc;
-  if (x_rows) {
-    rc = prep(wgrad_kernel<true, 0, 0, true, true, kBf16WgradWaves>, kMainLds);
-    if (!rc)
-      hipLaunchKernelGGL((wgrad_kernel<true, 0, 0, true, true, kBf16WgradWaves>), grid, dim3(64 * kBf16WgradWaves),
-                         kMainLds, st, (const uint8_t*)a, (const uint8_t*)x, M, N, 2 * ldt, 2 * ldt / splits, nullptr,
-                         nullptr, ws, tiles_m, tiles_n, (int)splits, 1, tra, trb);
-  } else {
-    rc = prep(wgrad_kernel<true, 0, 0, true, false, kBf16WgradWaves>, kMainLds);
-    if (!rc)
-      hipLaunchKernelGGL((wgrad_kernel<true, 0, 0, true, false, kBf16WgradWaves>), grid, dim3(64 * kBf16WgradWaves),
-                         kMainLds, st, (const uint8_t*)a, (const uint8_t*)x, M, N, 2 * ldt, 2 * ldt / splits, nullptr,
-                         nullptr, ws, tiles_m, tiles_n, (int)splits, 1, tra, TrOp{});
-  }
+  const Tiling tl = tiling(M, N, splits);
+  const auto launch = x_rows ? launch_wgrad<true, 0, 0, true, true> : launch_wgrad<true, 0, 0, true, false>;
+  const int rc = launch(tl, a, x, M, N, 2 * ldt, 2 * ldt / splits, nullptr, nullptr, ws, (int)splits, 1, tra,
+                        x_rows ? trb : TrOp{}, st);
   if (rc) return rc;
-  rc = status();
-  if (rc) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  if (x_rows)
-    hipLaunchKernelGGL((bf16_wgrad_reduce_kernel<true, kBf16WgradWaves>), dim3((unsigned)((n4 + 255) / 256), 1),
-                       dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, (uint16_t*)out);
-  else
-    hipLaunchKernelGGL((bf16_wgrad_reduce_kernel<false, kBf16WgradWaves>), dim3((unsigned)((n4 + 255) / 256), 1),
-                       dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, (uint16_t*)out);
-  return status();
+  return launch_bf16_reduce(tl, x_rows, ws, (int)splits, 1, M, N, out, st);
 }
 
 int sfp8_bf16_moe_gemm_wgrad_rows(const void* a, const void* bt, int64_t M, int64_t N, int64_t E, const int* plan,
@@ -2609,19 +2570,11 @@ int sfp8_bf16_moe_gemm_wgrad_rows(const void* a, const void* bt, int64_t M, int6
   const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
   if (!ws || ws_floats < sfp8_bf16_moe_wgrad_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
-  int rc = prep(moe_wgrad_kernel<true, 0, 0, true, false, kBf16WgradWaves>, kMainLds);
+  const Tiling tl = tiling(M, N, E * splits);
+  const int rc = launch_moe_wgrad<true, 0, 0, true, false>(tl, a, bt, M, N, 2 * ldp, nullptr, nullptr, nullptr, ws,
+                                                           plan, (int)splits, st);
   if (rc) return rc;
-  hipLaunchKernelGGL((moe_wgrad_kernel<true, 0, 0, true, false, kBf16WgradWaves>),
-                     dim3((unsigned)(tiles_m * tiles_n * splits * E)), dim3(64 * kBf16WgradWaves), kMainLds, st,
-                     (const uint8_t*)a, (const uint8_t*)bt, M, N, 2 * ldp, nullptr, nullptr, nullptr, ws, plan,
-                     tiles_m, tiles_n, (int)splits);
-  rc = status();
-  if (rc) return rc;
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  hipLaunchKernelGGL((bf16_wgrad_reduce_kernel<false, kBf16WgradWaves>), dim3((unsigned)((n4 + 255) / 256), (unsigned)E),
-                     dim3(256), 0, st, ws, (int)splits, n4, tiles_n, M, N, (uint16_t*)out);
-  return status();
+  return launch_bf16_reduce(tl, false, ws, (int)splits, E, M, N, out, st);
 }
 
 // ---- the weight gradient with row K-slab operands ----
@@ -2646,17 +2599,10 @@ int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, in
   }
   const int splits = (int)sfp8_wgrad_splits(M, N, ldt);
   if (ws_floats < sfp8_wgrad_rows_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
-  const int rc = wgrad_partials_any(a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, st);
+  const Tiling tl = tiling(M, N, splits);
+  const int rc = wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, st);
   if (rc) return rc;
-  const int tiles_n = cdiv(N, kTile);
-  const int64_t n4 = (int64_t)cdiv(M, kTile) * tiles_n * kTile * kTile / 4;
-  if (b_rows)
-    hipLaunchKernelGGL((splitk_reduce_kernel<true, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256), 1), dim3(256), 0,
-                       st, ws, splits, n4, tiles_n, M, N, sa, sb, out);
-  else
-    hipLaunchKernelGGL((splitk_reduce_kernel<false, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256), 1), dim3(256), 0,
-                       st, ws, splits, n4, tiles_n, M, N, sa, sb, out);
-  return status();
+  return launch_reduce(tl, b_rows, ws, splits, 1, M, N, sa, sb, out, st);
 }
 
 // ---- the weight gradient fused with the optimizer's momentum stage ----
@@ -2674,21 +2620,20 @@ int sfp8_gemm_wgrad_momentum(const void* a, int fmt_a, int a_rows, const void* b
   if (!fits32(slab_rows(M), ldt) || !fits32(slab_rows(N), ldt)) return kErrBadShape;
   if (!al16(a) || !al16(b) || !al16(grad) || !al16(v) || !al16(ws) || (((uintptr_t)u) & 7u)) return kErrBadAlignment;
   hipStream_t st = (hipStream_t)stream;
-  const int tiles_m = cdiv(M, kTile), tiles_n = cdiv(N, kTile);
   int splits = 0;
   if (ldt > 0) {
     splits = (int)sfp8_wgrad_splits(M, N, ldt);
     if (ws_floats < sfp8_wgrad_momentum_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
-    const int rc = wgrad_partials_any(a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, st);
+  }
+  const Tiling tl = tiling(M, N, splits);
+  if (ldt > 0) {
+    const int rc = wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, st);
     if (rc) return rc;
   }
-  const int64_t n4 = (int64_t)tiles_m * tiles_n * kTile * kTile / 4;
-  if (b_rows)
-    hipLaunchKernelGGL((splitk_momentum_kernel<true, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st,
-                       ws, splits, n4, tiles_n, M, N, sa, sb, grad, v, (uint16_t*)u, w_v, 1.0f - w_u);
-  else
-    hipLaunchKernelGGL((splitk_momentum_kernel<false, kWgradWaves>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st,
-                       ws, splits, n4, tiles_n, M, N, sa, sb, grad, v, (uint16_t*)u, w_v, 1.0f - w_u);
+  const auto kern = tl.small ? (b_rows ? splitk_momentum_kernel<true, true> : splitk_momentum_kernel<true, false>)
+                             : (b_rows ? splitk_momentum_kernel<false, true> : splitk_momentum_kernel<false, false>);
+  hipLaunchKernelGGL(kern, reduce_grid(tl, 1), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N, sa, sb,
+                     grad, v, (uint16_t*)u, w_v, 1.0f - w_u);
   return status();
 }
 

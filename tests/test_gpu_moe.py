@@ -352,3 +352,34 @@ def test_moe_weight_cache_refresh(dev, monkeypatch):
     halved = run(True)
     assert not torch.equal(halved[0], cached[0])
     TO.clear_weight_cache()
+
+
+# 128 x 128 tiles up to 128 work-groups of 256 x 256 (tiles x splits x
+# experts), the larger ones from there on: both sides, widths that end inside
+# a tile of either shape, experts without rows and with one.
+@pytest.mark.parametrize("M_,N_,counts", [(320, 192, [300, 0, 513]), (64, 64, [1]), (512, 256, [256, 257] * 4),
+                                          (576, 320, [129, 0, 700, 1] * 3)])
+def test_moe_wgrad_tile_shapes(dev, M_, N_, counts):
+    """Integer operands: every product and partial sum is exact in fp32 (at
+    most 64 * 700 < 2^24), so each expert's gradient is known exactly."""
+    ops = sg.ops
+    E, R = len(counts), sum(counts)
+    g = torch.Generator(device=dev).manual_seed(M_ + N_)
+    plan = ops.moe_plan(torch.cumsum(torch.tensor(counts), 0).to(torch.int32).to(dev), R)
+    ldp = ops.moe_padded_rows(R, E)
+    a = torch.zeros(ldp, M_, device=dev)
+    b = torch.zeros(ldp, N_, device=dev)
+    ref, row = [], 0
+    for c in counts:
+        a[row:row + c] = torch.randint(-8, 9, (c, M_), generator=g, device=dev).float()
+        b[row:row + c] = torch.randint(-8, 9, (c, N_), generator=g, device=dev).float()
+        ref.append(a[row:row + c].t() @ b[row:row + c])
+        row += -(-c // 256) * 256
+    ref = torch.stack(ref)
+    one = torch.ones(1, device=dev)
+    a8, b8 = ops.to_slab(a.to(ops.E5M2)), ops.to_slab(b.to(ops.E4M3))
+    assert torch.equal(ops.moe_wgrad_rows(a8, b8, M_, N_, E, plan, one, one), ref)
+    bt8 = ops.to_slab(b.to(ops.E4M3).t().contiguous())
+    assert torch.equal(ops.moe_wgrad_rows(a8, bt8, M_, N_, E, plan, one, one, b_rows=False), ref)
+    gs, bt = ops.to_slab(a.bfloat16()), ops.to_slab(b.bfloat16().t().contiguous())
+    assert torch.equal(ops.bf16_wgrad_rows(gs, bt, M_, N_, plan=plan, E=E), ref.bfloat16())
