@@ -104,12 +104,11 @@ SFP8_DEV int paired_col8(int r) {
   return 32 * (rl >> 5) + 16 * ((rl >> 2) & 1) + 4 * ((rl >> 3) & 3) + (rl & 3);
 }
 
-// Paired (gate/up) layout: rows 0..127 are gate, 128..255 up; wave column wn
-// owns rows 64*wn.. of each half; column (within the 128-column half)
-// 64*wn + 32*g + 16*nb + v.
-SFP8_DEV int paired_col(int r) {
-  const int rl = r & 63;
-  return (r & 64) + 32 * ((rl >> 2) & 1) + 16 * (rl >> 5) + 4 * ((rl >> 3) & 3) + (rl & 3);
+// B-tile row r of the 128-row paired tile -> (half, column within 64):
+// half = r / 64 (gate, up); column = 32*wn + 16*g + v for the lane layout.
+SFP8_DEV int paired_col64(int r) {
+  const int rl = r & 63, wn = rl >> 5, w = rl & 31;
+  return 32 * wn + 16 * ((w >> 2) & 1) + 4 * (w >> 3) + (w & 3);
 }
 
 // Copy of an LDS tile (nrows rows of 64 * NP bytes, LDS row stride `stride`)
@@ -142,12 +141,33 @@ SFP8_DEV void round16_bf16(const floatx16& a, float s, float (&o)[16]) {
   }
 }
 
+// The two tile shapes of the GEMMs below: 256 x 256 by 8 waves, one
+// work-group per CU, or (SMALL) 128 x 128 by 4 waves, two per CU.  The B
+// rows of both are permuted by plain_col_nb<2>, or with PAIRED (gate rows in
+// the first half of the B tile, up rows in the second) by paired_col8 and
+// paired_col64.
+template <bool SMALL>
+struct TileShape {
+  static constexpr int kM = SMALL ? 128 : 256;
+  static constexpr int kThreads = SMALL ? 256 : 512;
+  static constexpr int kMinWaves = SMALL ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
+  static constexpr int kWN = SMALL ? 2 : 4, kTB = SMALL ? 2 : 4;
+  template <bool BF16, int FA, int FB, bool TRA = false, bool TRB = false, bool PAIRED = false>
+  using Loop = MainLoop<BF16, FA, FB, PAIRED, 2, kStages, 0, TRA, TRB, kWN, kTB, kM>;
+  static constexpr int kLds = Loop<true, 0, 0>::kLds;
+  // the plan's tile of tile row tm, and that tile row's valid rows of it
+  static SFP8_DEV int plan_tile(int tm) { return SMALL ? tm >> 1 : tm; }
+  static SFP8_DEV int plan_skip(int tm) { return SMALL ? 128 * (tm & 1) : 0; }
+};
+
 // ---------------------------------------------------------------------------
 // (a6) gate/up forward + SwiGLU epilogue (spark-gpt train.py:975-1016).
 // Tile: 256 tokens x 128 intermediate columns; the B tile holds gate rows
 // n0..n0+127 then up rows I+n0..I+n0+127 (paired layout), so a lane holds g and
 // u of the same 32 consecutive columns.
-constexpr int kEpiStride = 144;
+// staging row: the tile's 128 (64) bytes of one output, and 16
+template <bool SMALL>
+constexpr int kEpiStride = SMALL ? 80 : 144;
 
 // With a MoE plan (grouped experts): tile row tm of padded expert order,
 // its expert's W8 at w8 + e * w_estride and weight scale wscale[e]; tile
@@ -155,30 +175,38 @@ constexpr int kEpiStride = 144;
 // 8 waves (two per SIMD): wave (wm, wn) owns tile rows 128*wm.. and the gate
 // and up columns 32*wn.. (one 32-column block of each), so the serial
 // epilogue of one wave overlaps the other's on the same SIMD.
-__global__ __launch_bounds__(512, 1) void swiglu_fwd_kernel(
+// SMALL: 128 tokens x 64 columns by 4 waves of 64 rows.
+template <bool SMALL>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void swiglu_fwd_kernel(
     const uint8_t* __restrict__ x8, const uint8_t* __restrict__ w8, int64_t T, int64_t D, int64_t I,
     const float* __restrict__ scale, const float* __restrict__ wscale, float* __restrict__ amax,
     uint8_t* __restrict__ gu8, uint8_t* __restrict__ h8, uint8_t* __restrict__ h8t, int64_t ldt,
     int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t w_estride) {
+  using TS = TileShape<SMALL>;
+  constexpr int kN = TS::kM / 2;  // (gate, up) columns of a tile
+  constexpr int kWaves = TS::kThreads / 64, kEs = kEpiStride<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
   if (plan) {
     const MoePlan P{plan};
-    if (tm >= P.ntiles()) return;  // work-group uniform
-    const int e = P.expert(tm);
+    const int pt = TS::plan_tile(tm);
+    if (pt >= P.ntiles()) return;  // work-group uniform
+    const int e = P.expert(pt);
     w8 += e * w_estride;
     wscale += e;
   }
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * 128;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * kN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-  floatx16 acc[4][2];  // [tb][0] gate, [tb][1] up
+  floatx16 acc[TS::kTB][2];  // [tb][0] gate, [tb][1] up
   // K-slab operands: x8 [D/64][ldt][64], w8 [D/64][2I][64]; one K stage of
-  // the tile is 256 contiguous rows of A and two runs of 128 rows of B
-  MainLoop<false, kFmtE4M3, kFmtE4M3, true, 2, kStages, 0, false, false, 4>::run(
+  // the tile is kM contiguous rows of A and two runs of kN rows of B
+  TS::template Loop<false, kFmtE4M3, kFmtE4M3, false, false, true>::run(
       lds, x8 + m0 * kStage, D * ldt - m0 * kStage, [=](int r) { return r * kStage; }, (int)(ldt * kStage), w8,
-      D * 2 * I, [=](int r) { return ((r >> 7) * (int)I + (int)n0 + paired_col8(r)) * kStage; },
+      D * 2 * I, [=](int r) {
+        return ((r / kN) * (int)I + (int)n0 + (SMALL ? paired_col64(r) : paired_col8(r))) * kStage;
+      },
       (int)(2 * I * kStage), (int)(D / kStage), acc);
   // All scales are powers of two, so the dequantization factor commutes with
   // every rounding step: with gb, ub = bf16(acc) (unscaled),
@@ -192,11 +220,11 @@ __global__ __launch_bounds__(512, 1) void swiglu_fwd_kernel(
   const float m1 = deq * scale[1], m2 = deq * deq * scale[2];
   const float inv1 = 1.0f / m1, inv2 = 1.0f / m2;
   const float bnd1 = kE4M3Max * inv1, bnd2 = kE4M3Max * inv2;
-  // epilogue LDS: the tile's g8, u8 and h8 bytes (256 x 128 each), then the amax slots
+  // epilogue LDS: the tile's g8, u8 and h8 bytes (kM x kN each), then the amax slots
   uint8_t* Gt = lds;
-  uint8_t* Ut = lds + kTile * kEpiStride;
-  uint8_t* Ht = lds + 2 * kTile * kEpiStride;
-  float* red = reinterpret_cast<float*>(lds + 3 * kTile * kEpiStride);
+  uint8_t* Ut = lds + TS::kM * kEs;
+  uint8_t* Ht = lds + 2 * TS::kM * kEs;
+  float* red = reinterpret_cast<float*>(lds + 3 * TS::kM * kEs);
   float m_gu = 0.f, m_h = 0.f;
   const int fr = lane & 31, g = lane >> 5;
   const int cb = 32 * wn + 16 * g;  // first of this lane's 16 columns
@@ -219,8 +247,8 @@ __global__ __launch_bounds__(512, 1) void swiglu_fwd_kernel(
     }
   };
 #pragma unroll
-  for (int tb = 0; tb < 4; ++tb) {
-    const int row = 128 * wm + 32 * tb + fr;  // token within the tile
+  for (int tb = 0; tb < TS::kTB; ++tb) {
+    const int row = 32 * TS::kTB * wm + 32 * tb + fr;  // token within the tile
     uint32_t gw[4], uw[4], hw[4];
     bool bad = false;
     {
@@ -264,9 +292,9 @@ __global__ __launch_bounds__(512, 1) void swiglu_fwd_kernel(
         }
       }
     }
-    store16(Gt + row * kEpiStride + cb, {gw[0], gw[1], gw[2], gw[3]});
-    store16(Ut + row * kEpiStride + cb, {uw[0], uw[1], uw[2], uw[3]});
-    store16(Ht + row * kEpiStride + cb, {hw[0], hw[1], hw[2], hw[3]});
+    store16(Gt + row * kEs + cb, {gw[0], gw[1], gw[2], gw[3]});
+    store16(Ut + row * kEs + cb, {uw[0], uw[1], uw[2], uw[3]});
+    store16(Ht + row * kEs + cb, {hw[0], hw[1], hw[2], hw[3]});
   }
   m_gu *= deq;
   m_h *= deq * deq;
@@ -274,20 +302,27 @@ __global__ __launch_bounds__(512, 1) void swiglu_fwd_kernel(
   // gu8 (gate and up halves) and h8 as 64-column K-slab blocks (every tile
   // row: rows past T are zero padding), then, when asked for, the
   // token-contiguous h8t
-  lds_rows_to_kslab<2, 512>(Gt, kTile, kEpiStride, gu8, ldt, m0, n0);
-  lds_rows_to_kslab<2, 512>(Ut, kTile, kEpiStride, gu8, ldt, m0, I + n0);
-  lds_rows_to_kslab<2, 512>(Ht, kTile, kEpiStride, h8, ldt, m0, n0);
-  if (h8t) lds_tile_store_slab_tr<8, 8>(Ht, kEpiStride, h8t, slab_rows(I), m0, n0);
+  lds_rows_to_kslab<kN / 64, TS::kThreads>(Gt, TS::kM, kEs, gu8, ldt, m0, n0);
+  lds_rows_to_kslab<kN / 64, TS::kThreads>(Ut, TS::kM, kEs, gu8, ldt, m0, I + n0);
+  lds_rows_to_kslab<kN / 64, TS::kThreads>(Ht, TS::kM, kEs, h8, ldt, m0, n0);
+  if (h8t) {
+    if constexpr (SMALL) {
+      lds_rows_store_slab_tr<64, kWaves>(Ht, kN, kEs, h8t, slab_rows(I), m0, n0);
+      lds_rows_store_slab_tr<64, kWaves>(Ht + 64 * kEs, kN, kEs, h8t, slab_rows(I), m0 + 64, n0);
+    } else {
+      lds_tile_store_slab_tr<8, 8>(Ht, kEs, h8t, slab_rows(I), m0, n0);
+    }
+  }
   m_gu = wave_max(m_gu);
   m_h = wave_max(m_h);
-  if (lane == 0) { red[wave] = m_gu; red[8 + wave] = m_h; }
+  if (lane == 0) { red[wave] = m_gu; red[kWaves + wave] = m_h; }
   __syncthreads();
   if (tid == 0) {
-    float a1 = red[0], a2 = red[8];
+    float a1 = red[0], a2 = red[kWaves];
 #pragma unroll
-    for (int w = 1; w < 8; ++w) {
+    for (int w = 1; w < kWaves; ++w) {
       a1 = fmaxf(a1, red[w]);
-      a2 = fmaxf(a2, red[8 + w]);
+      a2 = fmaxf(a2, red[kWaves + w]);
     }
     atomic_max_nonneg(amax + 1, a1);
     atomic_max_nonneg(amax + 2, a2);
@@ -318,13 +353,6 @@ constexpr int kPipeLds = kPipeRing + 2 * kPipeHBytes + 64;
 // the pipe's waves: 8 of 64 x 64 (two row blocks each)
 constexpr int kPipeTB = 2;
 constexpr int kPipeThreads = kPipeTB == 4 ? 256 : 512;
-
-// B-tile row r of the 128-row paired tile -> (half, column within 64):
-// half = r / 64 (gate, up); column = 32*wn + 16*g + v for the lane layout.
-SFP8_DEV int paired_col64(int r) {
-  const int rl = r & 63, wn = rl >> 5, w = rl & 31;
-  return 32 * wn + 16 * ((w >> 2) & 1) + 4 * (w >> 3) + (w & 3);
-}
 
 // The h tile's 256 rows of 64 bytes to 256 consecutive K-slab rows (NT
 // threads, 16 bytes each per pass).
@@ -981,23 +1009,6 @@ SFP8_DEV void write_bf16_small(const uint8_t* lds, int64_t m0, int64_t n0, int64
   }
 }
 
-// The two tile shapes of the GEMMs below: 256 x 256 by 8 waves, one
-// work-group per CU, or (SMALL) 128 x 128 by 4 waves, two per CU.  The B
-// rows of both are permuted by plain_col_nb<2>.
-template <bool SMALL>
-struct TileShape {
-  static constexpr int kM = SMALL ? 128 : 256;
-  static constexpr int kThreads = SMALL ? 256 : 512;
-  static constexpr int kMinWaves = SMALL ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
-  static constexpr int kWN = SMALL ? 2 : 4, kTB = SMALL ? 2 : 4;
-  template <bool BF16, int FA, int FB, bool TRA = false, bool TRB = false>
-  using Loop = MainLoop<BF16, FA, FB, false, 2, kStages, 0, TRA, TRB, kWN, kTB, kM>;
-  static constexpr int kLds = Loop<true, 0, 0>::kLds;
-  // the plan's tile of tile row tm, and that tile row's valid rows of it
-  static SFP8_DEV int plan_tile(int tm) { return SMALL ? tm >> 1 : tm; }
-  static SFP8_DEV int plan_skip(int tm) { return SMALL ? 128 * (tm & 1) : 0; }
-};
-
 // A tile's accumulators times s, as bf16, to out[t, n] (leading dimension N)
 // for rows u0.. below uend and columns n0.. below N.
 template <bool SMALL>
@@ -1144,13 +1155,18 @@ SFP8_DEV void dgrad_swiglu4(const intx4& h0, const intx4& h1, uint32_t gw, uint3
 // rows (its rows urow(tm).. for tile row tm), W_down^T of expert e at
 // wdt + e * w_estride (bytes); the tile count comes from the plan.
 // TCOPY: dgu8t is written too (staged in LDS per pass).
-template <bool TCOPY>
-__global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
+// SMALL: 128 x 128 tiles by 4 waves of 64 x 64, two work-groups per CU, one
+// epilogue pass (not with TCOPY).
+template <bool TCOPY, bool SMALL>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void down_dgrad_swiglu_kernel(
     const uint16_t* __restrict__ dy, const uint16_t* __restrict__ wdt, const uint8_t* __restrict__ gu8,
     int64_t T, int64_t D, int64_t I, const float* __restrict__ scale, float* __restrict__ amax,
     uint8_t* __restrict__ dgu8, uint8_t* __restrict__ dgu8t, int64_t ldt, int tiles_m, int tiles_n,
     const int* __restrict__ plan, int64_t w_estride) {
-  using Loop = MainLoop<true, 0, 0, false, 2, kStages, 0, false, false, 4>;
+  static_assert(!(TCOPY && SMALL), "the copy is staged by the larger tile");
+  using TS = TileShape<SMALL>;
+  using Loop = typename TS::template Loop<true, 0, 0>;
+  constexpr int kWaves = TS::kThreads / 64;
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t ldb = D * 2;  // bytes
@@ -1175,12 +1191,12 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
   //   dgu8 = e5m2(d*q3) = e5m2(d'*(s_gu*q3)),  amax3 = s_gu*max(|dg|,|du|).
   const float m3s = (1.0f / scale[1]) * scale[3];
   const float inv3 = 1.0f / m3s, bnd3 = kE5M2Max * inv3;
-  float* red = reinterpret_cast<float*>(base + 2 * kTile * kEpiStride2);  // 8 floats after the staging tiles
+  float* red = reinterpret_cast<float*>(base + (SMALL ? 128 * kSmallStride : 2 * kTile * kEpiStride2));  // after the staging tiles
   float m3 = 0.f;
   // Persistent: work-group pid runs tiles pid, pid + gridDim.x, ...  (Work-
   // groups started a quarter of a tile apart per XCD, so that the tiles'
   // 256 KiB store bursts would not coincide, measured 2 % slower.)
-  if (plan) tiles_m = MoePlan{plan}.ntiles();
+  if (plan) tiles_m = MoePlan{plan}.ntiles() * (kTile / TS::kM);
   const int ntiles = tiles_m * tiles_n;
   // A = dy row-major (rows past the tile's last read as zero through the
   // range check); B = Wd^T as a bf16 K-slab [2D/64][slab_rows(I)][64] (bytes)
@@ -1196,14 +1212,15 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
     int64_t b_bytes;
   };
   const auto ops_of = [=](int tm, int tn) {
-    const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
+    const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
     int64_t a_row = m0, a_rows = T - m0;
     const uint8_t* wb = reinterpret_cast<const uint8_t*>(wdt);
     if (plan) {
       const MoePlan P{plan};
-      a_row = P.urow(tm);
-      a_rows = P.rows(tm);
-      wb += P.expert(tm) * w_estride;
+      const int pt = TS::plan_tile(tm);
+      a_row = P.urow(pt) + TS::plan_skip(tm);
+      a_rows = P.rows(pt) - TS::plan_skip(tm);  // 0 or less: every row reads as zero
+      wb += P.expert(pt) * w_estride;
     }
     return Ops{reinterpret_cast<const uint8_t*>(dy) + a_row * ldb, a_rows * ldb, wb + n0 * kStage,
                ldb * ip - n0 * kStage};
@@ -1211,19 +1228,24 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
   int tm, tn;
   tile_coords(tile, ntiles, tiles_m, tiles_n, tm, tn);
-  const int64_t m0 = (int64_t)tm * kTile, n0 = (int64_t)tn * kTile;
-  floatx16 acc[4][2];
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  floatx16 acc[TS::kTB][2];
   {
     const Ops o = ops_of(tm, tn);
     Loop::run(base, o.a, o.a_bytes, arow, kStage, o.b, o.b_bytes, brow, (int)(ip * kStage), nk, acc);
   }
-  // Row-order epilogue, in two passes of 128 tile rows (the rows of
-  // stage_bf16_half<P>): dh staged in LDS as bf16, then each thread takes
+  // Row-order epilogue, in two passes (SMALL: one) of 128 tile rows (the rows
+  // of stage_bf16_half<P>): dh staged in LDS as bf16, then each thread takes
   // 16-column chunks of one row, reading gu8 and writing dgu8 as whole K-slab
   // rows; with dgu8t the codes also go to LDS for the token-contiguous copy.
   const __amdgpu_buffer_rsrc_t rgu = make_rsrc(gu8 + m0 * 64, 2 * I * ldt - m0 * 64);
-  const int cols = (int)((I - n0) < kTile ? (I - n0) : kTile);  // 128 or 256
   uint8_t* DH = base;
+  // chunk k of this thread in a pass: 16 columns from chunk_col(k) of staging
+  // row chunk_row(k), tile row tile_row(k, P)
+  constexpr int kSlabs = TS::kM / 64, kDh = SMALL ? kSmallStride : kBf16Stride;
+  const auto chunk_row = [=](int k) { return 16 * ((kWaves * k + wave) / kSlabs) + (lane >> 2); };
+  const auto chunk_col = [=](int k) { return 64 * ((kWaves * k + wave) % kSlabs) + 16 * (lane & 3); };
+  const auto tile_row = [=](int k, int P) { return SMALL ? chunk_row(k) : half_tile_row(chunk_row(k), P); };
   // the staging tiles of the token-contiguous copy (MoE only); their offset
   // goes through an empty asm so that the compiler does not hoist per-lane
   // addresses into them out of the tile loop (a register it had to spill)
@@ -1249,20 +1271,17 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
   const auto gu_loads = [&](int P) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int item = 8 * k + wave, slab = item & 3, lr = 16 * (item >> 2) + (lane >> 2);
-      const int c = 64 * slab + 16 * (lane & 3);
-      const int row = half_tile_row(lr, P);
-      wg[k] = __builtin_amdgcn_raw_buffer_load_b128(rgu, gu_off(c, row), 0, kNT);
-      wu[k] = __builtin_amdgcn_raw_buffer_load_b128(rgu, gu_off(c, row) + (uint32_t)(I * ldt), 0, kNT);
+      const uint32_t o = gu_off(chunk_col(k), tile_row(k, P));
+      wg[k] = __builtin_amdgcn_raw_buffer_load_b128(rgu, o, 0, kNT);
+      wu[k] = __builtin_amdgcn_raw_buffer_load_b128(rgu, o + (uint32_t)(I * ldt), 0, kNT);
     }
   };
-  // the codes of chunk k of pass P (dh from the staged tile, gate and up
+  // the codes of chunk k of the loaded pass (dh from the staged tile, gate and up
   // codes from wg[k], wu[k]); the running amax in m3
-  const auto swiglu_chunk = [&](int P, int k, uint32_t (&pg)[4], uint32_t (&pu)[4]) {
-    const int item = 8 * k + wave, slab = item & 3, lr = 16 * (item >> 2) + (lane >> 2);
-    const int c = 64 * slab + 16 * (lane & 3);
-    const intx4 h0 = *reinterpret_cast<const intx4*>(DH + lr * kBf16Stride + 2 * c);
-    const intx4 h1 = *reinterpret_cast<const intx4*>(DH + lr * kBf16Stride + 2 * c + 16);
+  const auto swiglu_chunk = [&](int k, uint32_t (&pg)[4], uint32_t (&pu)[4]) {
+    const int lr = chunk_row(k), c = chunk_col(k);
+    const intx4 h0 = *reinterpret_cast<const intx4*>(DH + lr * kDh + 2 * c);
+    const intx4 h1 = *reinterpret_cast<const intx4*>(DH + lr * kDh + 2 * c + 16);
     // The 16 values' unclamped codes and their NaN-propagating maximum
     // magnitude (the first maximum3 of each group of four takes the
     // running maximum): when it is inside the e5m2 range (after scaling)
@@ -1307,9 +1326,7 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
   };
   // dgu8 is a K-slab [2I/64][ldt][64]; four lanes write one 64-byte row
   const auto store_chunk = [&](int P, int k, const uint32_t (&pg)[4], const uint32_t (&pu)[4]) {
-    const int item = 8 * k + wave, slab = item & 3, lr = 16 * (item >> 2) + (lane >> 2);
-    const int c = 64 * slab + 16 * (lane & 3);
-    const uint32_t o = gu_off(c, half_tile_row(lr, P));
+    const uint32_t o = gu_off(chunk_col(k), tile_row(k, P));
     __builtin_amdgcn_raw_buffer_store_b128(intx4{(int)pg[0], (int)pg[1], (int)pg[2], (int)pg[3]}, rdg, o, 0, 0);
     __builtin_amdgcn_raw_buffer_store_b128(intx4{(int)pu[0], (int)pu[1], (int)pu[2], (int)pu[3]}, rdg,
                                            o + (uint32_t)(I * ldt), 0, 0);
@@ -1326,13 +1343,14 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         uint32_t pg[4], pu[4];
-        swiglu_chunk(P, k, pg, pu);
+        swiglu_chunk(k, pg, pu);
         store_chunk(P, k, pg, pu);
       }
       __syncthreads();
       // the token-contiguous dgu8t: local rows 0-63 are tile rows 64P.., rows
       // 64-127 tile rows 128 + 64P.. (rows past T hold zero codes)
       const int64_t rp2 = slab_rows(2 * I);
+      const int cols = (int)((I - n0) < kTile ? (I - n0) : kTile);  // 128 or 256
       lds_rows_store_slab_tr<64, 8>(G2, cols, kEpiStride2, dgu8t, rp2, m0 + 64 * P, n0);
       lds_rows_store_slab_tr<64, 8>(G2 + 64 * kEpiStride2, cols, kEpiStride2, dgu8t, rp2, m0 + 128 + 64 * P, n0);
       lds_rows_store_slab_tr<64, 8>(U2, cols, kEpiStride2, dgu8t, rp2, m0 + 64 * P, I + n0);
@@ -1340,6 +1358,17 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
                                     I + n0);
     }
     __syncthreads();  // the next tile's DMA overwrites the staging tiles
+  } else if constexpr (SMALL) {
+    uint32_t pg[4], pu[4];
+    gu_loads(0);
+    stage_bf16_small(DH, acc, 1.0f);  // dh rounded to bf16 (train.py:1082)
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      swiglu_chunk(k, pg, pu);
+      store_chunk(0, k, pg, pu);
+    }
+    __syncthreads();  // the next tile's DMA overwrites the staging tile
   } else {
     // Each chunk is stored as soon as its codes are made, so that the stores
     // drain while the rest is computed.  (Deferring the first pass's stores
@@ -1352,7 +1381,7 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      swiglu_chunk(0, k, pg[k], pu[k]);
+      swiglu_chunk(k, pg[k], pu[k]);
       store_chunk(0, k, pg[k], pu[k]);
     }
     gu_loads(1);
@@ -1361,14 +1390,14 @@ __global__ __launch_bounds__(512, 1) void down_dgrad_swiglu_kernel(
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      swiglu_chunk(1, k, pg[k], pu[k]);
+      swiglu_chunk(k, pg[k], pu[k]);
       store_chunk(1, k, pg[k], pu[k]);
     }
     __syncthreads();  // the next tile's DMA overwrites the staging tile
   }
   }
   m3 *= 1.0f / scale[1];  // s_gu, read again rather than held across the tile loop
-  block_amax_atomic<8>(m3, red, amax + 3);
+  block_amax_atomic<kWaves>(m3, red, amax + 3);
 }
 
 // ---------------------------------------------------------------------------
@@ -1682,60 +1711,71 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // expert-order rows urow(tm) .. + rows(tm); W of expert e at w + e * w_estride
 // (bytes).  Columns from I on (the last tile when I % 128 != 0) are not
 // written.
-constexpr int kGuStride = 272;  // staging row: 128 bf16 columns (256 bytes) + 16
+// staging row: 128 (64) bf16 columns and 16 bytes
+template <bool SMALL>
+constexpr int kGuStride = SMALL ? 144 : 272;
 
 // 8 waves (two per SIMD): wave (wm, wn) owns tile rows 128*wm.. and one
 // 32-column block of gate and one of up, columns 32*wn.. of each half.
-__global__ __launch_bounds__(512, 1) void bf16_swiglu_fwd_kernel(
+// SMALL: 128 rows x 64 columns by 4 waves of 64 rows, staged in one pass.
+template <bool SMALL>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void bf16_swiglu_fwd_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, int64_t T, int64_t D, int64_t I,
     const float* __restrict__ rstd, uint16_t* __restrict__ gu, uint16_t* __restrict__ h, int tiles_m, int tiles_n,
     const int* __restrict__ plan, int64_t w_estride, int64_t ldxs) {
+  using TS = TileShape<SMALL>;
+  constexpr int kN = TS::kM / 2;  // (gate, up) columns of a tile
+  constexpr int kGs = kGuStride<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
-  int64_t r0 = (int64_t)tm * kTile, nrows = T - r0;
+  int64_t r0 = (int64_t)tm * TS::kM, nrows = T - r0;
   if (plan) {
     const MoePlan P{plan};
-    if (tm >= P.ntiles()) return;  // work-group uniform
-    r0 = P.urow(tm);
-    nrows = P.rows(tm);
-    w += P.expert(tm) * w_estride;
+    const int pt = TS::plan_tile(tm);
+    if (pt >= P.ntiles()) return;  // work-group uniform
+    r0 = P.urow(pt) + TS::plan_skip(tm);
+    nrows = P.rows(pt) - TS::plan_skip(tm);
+    if (nrows <= 0) return;  // nothing but padding rows, which have no output
+    w += P.expert(pt) * w_estride;
   }
-  const int64_t n0 = (int64_t)tn * 128;
+  const int64_t n0 = (int64_t)tn * kN;
   const int64_t ldx = D * 2;  // bytes per x row = K bytes
   const int64_t wr = slab_rows(2 * I);
   // the outputs from the tile's first row (gu [rows, 2I], h [rows, I], bf16)
   const __amdgpu_buffer_rsrc_t rgu = make_rsrc(gu + r0 * 2 * I, nrows * 4 * I);
   const __amdgpu_buffer_rsrc_t rho = make_rsrc(h + r0 * I, nrows * 2 * I);
-  floatx16 acc[4][2];  // [tb][0] gate, [tb][1] up
+  floatx16 acc[TS::kTB][2];  // [tb][0] gate, [tb][1] up
   // A: x row-major [T, D] (rows past the tile's last read as zero through
   // the range check), or with ldxs > 0 its row K-slab [2D/64][ldxs][64]
   // (zero padding rows): a K stage of the tile is then one 16 KiB block of
   // whole 128-byte lines instead of 256 half lines 2D bytes apart
   const bool xslab = ldxs > 0;
-  MainLoop<true, 0, 0, true, 2, kStages, 0, false, false, 4>::run(
+  TS::template Loop<true, 0, 0, false, false, true>::run(
       lds, reinterpret_cast<const uint8_t*>(x) + r0 * (xslab ? kStage : ldx),
       xslab ? ldx * ldxs - r0 * kStage : nrows * ldx, [=](int r) { return r * (xslab ? kStage : (int)ldx); },
-      xslab ? (int)(ldxs * kStage) : kStage, w, ldx * wr, [=](int r) { return ((r >> 7) * (int)I + (int)n0 + paired_col8(r)) * kStage; },
+      xslab ? (int)(ldxs * kStage) : kStage, w, ldx * wr, [=](int r) {
+        return ((r / kN) * (int)I + (int)n0 + (SMALL ? paired_col64(r) : paired_col8(r))) * kStage;
+      },
       (int)(wr * kStage), (int)(ldx / kStage), acc);
-  // Epilogue in two passes of 128 tile rows: pass P takes the lanes' row
-  // blocks tb = 2P, 2P+1 (tile row 128 wm + 64 P + 32 (tb & 1) + fr, staging
-  // row 64 wm + 32 (tb & 1) + fr), stages g, u and h as bf16 rows in LDS,
+  // Epilogue in two passes (SMALL: one) of 128 tile rows: pass P takes the
+  // lanes' row blocks tb = 2P, 2P+1 (tile row 32 kTB wm + 64 P + 32 (tb & 1) +
+  // fr, staging row 64 wm + 32 (tb & 1) + fr), stages g, u and h as bf16 rows in LDS,
   // then writes them as whole 256-byte row runs.
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave & 1, wn = wave >> 1, fr = lane & 31, g = lane >> 5;
   const int cb = 32 * wn + 16 * g;  // first of this lane's 16 columns in the tile
   uint8_t* Gs = lds;
-  uint8_t* Us = lds + 128 * kGuStride;
-  uint8_t* Hs = lds + 2 * 128 * kGuStride;
+  uint8_t* Us = lds + 128 * kGs;
+  uint8_t* Hs = lds + 2 * 128 * kGs;
   const float c_exp = -1.4426950408889634f;
 #pragma unroll
-  for (int P = 0; P < 2; ++P) {
+  for (int P = 0; P < TS::kTB / 2; ++P) {
     if (P) __syncthreads();  // the first pass's rows are out of the staging tiles
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const int tb = 2 * P + q;
-      const int lr = 128 * wm + 32 * tb + fr;  // row within the tile
+      const int lr = 32 * TS::kTB * wm + 32 * tb + fr;  // row within the tile
       const float rs = (rstd && lr < nrows) ? rstd[r0 + lr] : 1.0f;
       uint32_t gw[8], uw[8], hw[8];
 #pragma unroll
@@ -1754,30 +1794,30 @@ __global__ __launch_bounds__(512, 1) void bf16_swiglu_fwd_kernel(
       const int sr = 64 * wm + 32 * q + fr;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        store16(Gs + sr * kGuStride + 2 * cb + 16 * j, {gw[4 * j], gw[4 * j + 1], gw[4 * j + 2], gw[4 * j + 3]});
-        store16(Us + sr * kGuStride + 2 * cb + 16 * j, {uw[4 * j], uw[4 * j + 1], uw[4 * j + 2], uw[4 * j + 3]});
-        store16(Hs + sr * kGuStride + 2 * cb + 16 * j, {hw[4 * j], hw[4 * j + 1], hw[4 * j + 2], hw[4 * j + 3]});
+        store16(Gs + sr * kGs + 2 * cb + 16 * j, {gw[4 * j], gw[4 * j + 1], gw[4 * j + 2], gw[4 * j + 3]});
+        store16(Us + sr * kGs + 2 * cb + 16 * j, {uw[4 * j], uw[4 * j + 1], uw[4 * j + 2], uw[4 * j + 3]});
+        store16(Hs + sr * kGs + 2 * cb + 16 * j, {hw[4 * j], hw[4 * j + 1], hw[4 * j + 2], hw[4 * j + 3]});
       }
     }
     __syncthreads();
-    // 128 rows x 16 pieces of 16 bytes per output: sixteen lanes per row;
+    // 128 rows x kN / 8 pieces of 16 bytes per output: kN / 8 lanes per row;
     // buffer stores from the tile's first row, a piece past the valid rows or
     // past I (I % 8 == 0: whole pieces) at offset 2^31 (beyond the range:
     // dropped), so every thread issues the same stores without a branch
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int idx = (int)threadIdx.x + 512 * k;
-      const int sr = idx >> 4, c = idx & 15;
-      const int lr = half_tile_row(sr, P);
+      const int idx = (int)threadIdx.x + TS::kThreads * k;
+      const int sr = idx / (kN / 8), c = idx % (kN / 8);
+      const int lr = SMALL ? sr : half_tile_row(sr, P);
       const int64_t col = n0 + 8 * c;
       const uint32_t in = 0u - (uint32_t)(lr < nrows && col < I);
       const uint32_t og = ((uint32_t)((lr * 2 * I + col) * 2) & in) | (~in & 0x80000000u);
       const uint32_t oh = ((uint32_t)((lr * I + col) * 2) & in) | (~in & 0x80000000u);
-      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Gs + sr * kGuStride + 16 * c), rgu,
+      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Gs + sr * kGs + 16 * c), rgu,
                                              og, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Us + sr * kGuStride + 16 * c), rgu,
+      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Us + sr * kGs + 16 * c), rgu,
                                              og + (uint32_t)(2 * I), 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Hs + sr * kGuStride + 16 * c), rho,
+      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Hs + sr * kGs + 16 * c), rho,
                                              oh, 0, 0);
     }
   }
@@ -1898,10 +1938,12 @@ __global__ __launch_bounds__(256) void splitk_momentum_kernel(const float* __res
 
 }  // namespace sfp8
 
-static_assert(3 * sfp8::kTile * sfp8::kEpiStride + 64 <= sfp8::kMainLds, "swiglu epilogue tiles fit the main loop's LDS");
+static_assert(3 * sfp8::kTile * sfp8::kEpiStride<false> + 64 <= sfp8::kMainLds &&
+                  3 * 128 * sfp8::kEpiStride<true> + 64 <= sfp8::TileShape<true>::kLds, "swiglu epilogue tiles fit the main loop's LDS");
 static_assert(sfp8::kPipeLds <= 160 * 1024, "deferred-epilogue SwiGLU fits the 160 KiB LDS");
 static_assert(128 * sfp8::kBf16Stride <= sfp8::kMainLds, "bf16 epilogue staging fits the main loop's LDS");
-static_assert(3 * 128 * sfp8::kGuStride <= sfp8::kMainLds, "bf16 SwiGLU staging fits the main loop's LDS");
+static_assert(3 * 128 * sfp8::kGuStride<false> <= sfp8::kMainLds &&
+                  3 * 128 * sfp8::kGuStride<true> <= sfp8::TileShape<true>::kLds, "bf16 SwiGLU staging fits the main loop's LDS");
 
 // ============================================================================
 // C ABI
@@ -1962,20 +2004,27 @@ inline int64_t wgrad_chunk(int64_t ldt, int64_t s) {
 }  // namespace
 
 namespace {
-// Whether an M x N output is computed in 128 x 128 tiles (two work-groups per
-// CU) instead of 256 x 256 ones (one per CU): when the larger tiles would
-// leave half of the 256 CUs or more without one.  A CU runs its tile at the
-// same speed however many others are idle, so the quarter tiles, spread over
-// up to four times the CUs, win until they fill the chip; from then on their
-// K loop, with twice the LDS-DMA bytes per FLOP, is the slower one.  Measured
-// (us, 256 -> 128 tiles, at 16, 80, 128 and 192 tiles of 256 x 256, D = 1024,
-// I = 3072): down forward 29 -> 14, 32 -> 24, 36 -> 32, 40 -> 44; gate/up
-// dgrad 49 -> 26, 50 -> 38, 55 -> 45, 62 -> 71; bf16 dgrad 91 -> 46, 94 -> 73,
-// 99 -> 88, 125 -> 135.  At 320 tiles (a second round of 64) the two differ by
-// less than a tenth either way, and the larger ones stay.
-inline bool use_small_tiles(int64_t M, int64_t N, int64_t parts = 1) {
+// Whether an M x N output (of each of `parts` K splits times experts) is
+// computed in 128 x 128 tiles (two work-groups per CU) instead of 256 x 256
+// ones (one per CU): when the larger tiles would leave half of the 256 CUs or
+// more without one.  A CU runs its tile at the same speed however many others
+// are idle, so the quarter tiles, spread over up to four times the CUs, win
+// until they fill the chip; from then on their K loop, with twice the LDS-DMA
+// bytes per FLOP, is the slower one.  Measured (us, 256 -> 128 tiles, at 16,
+// 80, 128 and 192 tiles of 256 x 256, D = 1024, I = 3072): down forward 29 ->
+// 14, 32 -> 24, 36 -> 32, 40 -> 44; gate/up dgrad 49 -> 26, 50 -> 38, 55 ->
+// 45, 62 -> 71; bf16 dgrad 91 -> 46, 94 -> 73, 99 -> 88, 125 -> 135.
+// second: also when the larger tiles would take a second round of 1 to
+// `second` of them, for the kernels whose epilogue is a large part of a tile,
+// which the second work-group of a CU then overlaps: with 128, FP8 SwiGLU
+// forward 32 -> 26 at 272 tiles and 28 -> 26 at 384, bf16 one 49 -> 41 and
+// 42 -> 39, down dgrad 46 -> 41 and 68 -> 66 at 384; with 64, down forward
+// 74 -> 68 and gate/up dgrad 121 -> 113 at 320 (78 -> 79 and 127 -> 131 at
+// 384); none for the bf16 dgrad, nearly all K loop (241 -> 266 at 320).
+inline bool use_small_tiles(int64_t M, int64_t N, int64_t parts, int second) {
   constexpr int64_t kCUs = 256;
-  return (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * parts <= kCUs / 2;
+  const int64_t tiles = (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * parts;
+  return tiles <= kCUs / 2 || (tiles > kCUs && tiles <= kCUs + second);
 }
 
 // A GEMM's tile shape over an M x N output (of each of `parts` K splits times
@@ -1985,9 +2034,9 @@ struct Tiling {
   int m, n, lds;  // tile rows and columns, dynamic LDS
   dim3 grid, block;
 };
-inline Tiling tiling(int64_t M, int64_t N, int64_t parts = 1) {
+inline Tiling tiling_of(bool small, int64_t M, int64_t N, int64_t parts = 1) {
   Tiling t;
-  t.small = use_small_tiles(M, N, parts);
+  t.small = small;
   const int tile = t.small ? TileShape<true>::kM : TileShape<false>::kM;
   t.m = cdiv(M, tile);
   t.n = cdiv(N, tile);
@@ -1995,6 +2044,37 @@ inline Tiling tiling(int64_t M, int64_t N, int64_t parts = 1) {
   t.grid = dim3((unsigned)(t.m * t.n * parts));
   t.block = dim3((unsigned)(t.small ? TileShape<true>::kThreads : TileShape<false>::kThreads));
   return t;
+}
+
+inline Tiling tiling(int64_t M, int64_t N, int64_t parts = 1, int second = 0) {
+  return tiling_of(use_small_tiles(M, N, parts, second), M, N, parts);
+}
+
+// The gate/up forward's: a tile covers half as many (gate, up) columns as rows.
+inline Tiling swiglu_tiling(int64_t M, int64_t I) {
+  return tiling(M, 2 * I, 1, 128);
+}
+
+// The persistent down dgrad over `rows` token rows, the padding that its
+// K-slab output needs among them (with a plan an upper bound: the kernel reads
+// the plan's count), T rows of dy.
+int dgrad_launch(const void* dy, const void* wdt, const void* gu8, int64_t rows, int64_t T, int64_t D, int64_t I,
+                 const float* scale, float* amax, void* dgu8, void* dgu8t, int64_t ldt, const int* plan,
+                 int64_t w_estride, hipStream_t st) {
+  const Tiling tl = dgu8t ? tiling_of(false, rows, I) : tiling(rows, I, 1, 128);
+  const auto kern = dgu8t ? down_dgrad_swiglu_kernel<true, false>
+                          : (tl.small ? down_dgrad_swiglu_kernel<false, true> : down_dgrad_swiglu_kernel<false, false>);
+  int n_cu = 0;
+  int rc = cu_count(&n_cu);
+  if (rc) return rc;
+  const int lds = tl.small ? kDgradLutBytes + TileShape<true>::kLds : kDgradLds;
+  rc = prep(kern, lds);
+  if (rc) return rc;
+  const unsigned wgs = (unsigned)(tl.small ? 2 * n_cu : n_cu);  // resident at once
+  hipLaunchKernelGGL(kern, dim3(tl.grid.x < wgs ? tl.grid.x : wgs), tl.block, lds, st, (const uint16_t*)dy,
+                     (const uint16_t*)wdt, (const uint8_t*)gu8, T, D, I, scale, amax, (uint8_t*)dgu8,
+                     (uint8_t*)dgu8t, ldt, tl.m, tl.n, plan, w_estride);
+  return status();
 }
 
 // wgrad_kernel over one weight gradient's tiles and splits (tl of M x N and
@@ -2097,12 +2177,13 @@ int sfp8_gemm_gateup_swiglu_fwd(const void* x8, const void* w8, int64_t T, int64
                        (int64_t)0);
     return status();
   }
-  const int tiles_m = cdiv(T, kTile), tiles_n = (int)(I / 128);
-  int rc = prep(swiglu_fwd_kernel, kMainLds);
+  const Tiling tl = swiglu_tiling(ldt, I);  // the padding rows' zeros too
+  const auto kern = tl.small ? swiglu_fwd_kernel<true> : swiglu_fwd_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(swiglu_fwd_kernel, dim3(tiles_m * tiles_n), dim3(512), kMainLds, (hipStream_t)stream,
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
                      (const uint8_t*)x8, (const uint8_t*)w8, T, D, I, scale, wscale, amax, (uint8_t*)gu8,
-                     (uint8_t*)h8, (uint8_t*)h8t, ldt, tiles_m, tiles_n, (const int*)nullptr, (int64_t)0);
+                     (uint8_t*)h8, (uint8_t*)h8t, ldt, tl.m, tl.n, (const int*)nullptr, (int64_t)0);
   return status();
 }
 
@@ -2113,7 +2194,7 @@ int sfp8_gemm_down_fwd(const void* h8, const void* wd8, const void* res, int64_t
   if (!fits32(ldt, I) || !fits32(slab_rows(D), I) || !fits32(kTile, 2 * D)) return kErrBadShape;
   if (!al16(h8) || !al16(wd8) || !al16(res) || !al16(y)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const Tiling tl = tiling(T, D);
+  const Tiling tl = tiling(T, D, 1, 64);
   const auto kern = tl.small ? down_fwd_kernel<true> : down_fwd_kernel<false>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
@@ -2132,19 +2213,7 @@ int sfp8_gemm_down_dgrad_swiglu(const void* dy, const void* wdt, const void* gu8
   if (!fits32(kTile, 2 * D) || !fits32(slab_rows(I), 2 * D) || !fits32(ldt, 2 * I)) return kErrBadShape;
   if (!al16(dy) || !al16(wdt) || !al16(gu8) || !al16(dgu8) || !al16(dgu8t)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const int tiles_m = cdiv(T, kTile), tiles_n = cdiv(I, kTile);
-  const int ntiles = tiles_m * tiles_n;
-  int n_cu = 0;
-  int rc = cu_count(&n_cu);
-  if (rc) return rc;
-  const int grid = ntiles < n_cu ? ntiles : n_cu;
-  const auto kern = dgu8t ? down_dgrad_swiglu_kernel<true> : down_dgrad_swiglu_kernel<false>;
-  rc = prep(kern, kDgradLds);
-  if (rc) return rc;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), kDgradLds, (hipStream_t)stream,
-                     (const uint16_t*)dy, (const uint16_t*)wdt, (const uint8_t*)gu8, T, D, I, scale, amax,
-                     (uint8_t*)dgu8, (uint8_t*)dgu8t, ldt, tiles_m, tiles_n, (const int*)nullptr, (int64_t)0);
-  return status();
+  return dgrad_launch(dy, wdt, gu8, ldt, T, D, I, scale, amax, dgu8, dgu8t, ldt, nullptr, 0, (hipStream_t)stream);
 }
 
 int sfp8_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t T, int64_t D, int64_t I,
@@ -2154,7 +2223,7 @@ int sfp8_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t T, int64_t
   if (!fits32(ldt, 2 * I) || !fits32(slab_rows(D), 2 * I) || !fits32(kTile, 2 * D)) return kErrBadShape;
   if (!al16(dgu8) || !al16(w8t) || !al16(dxn)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const Tiling tl = tiling(T, D);
+  const Tiling tl = tiling(T, D, 1, 64);
   const auto kern = tl.small ? gateup_dgrad_kernel<true> : gateup_dgrad_kernel<false>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
@@ -2283,12 +2352,13 @@ int sfp8_moe_gemm_gateup_swiglu_fwd(const void* x8, const void* w8, int64_t E, i
                        D * slab_rows(2 * I));
     return status();
   }
-  const int tiles_m = (int)(ldp / kTile), tiles_n = (int)(I / 128);
-  int rc = prep(swiglu_fwd_kernel, kMainLds);
+  const Tiling tl = swiglu_tiling(ldp, I);
+  const auto kern = tl.small ? swiglu_fwd_kernel<true> : swiglu_fwd_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(swiglu_fwd_kernel, dim3(tiles_m * tiles_n), dim3(512), kMainLds, (hipStream_t)stream,
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
                      (const uint8_t*)x8, (const uint8_t*)w8, ldp, D, I, scale, q_gu, amax, (uint8_t*)gu8,
-                     (uint8_t*)h8, (uint8_t*)h8t, ldp, tiles_m, tiles_n, plan, D * slab_rows(2 * I));
+                     (uint8_t*)h8, (uint8_t*)h8t, ldp, tl.m, tl.n, plan, D * slab_rows(2 * I));
   return status();
 }
 
@@ -2298,7 +2368,7 @@ int sfp8_moe_gemm_down_fwd(const void* h8, const void* wd8, int64_t E, int64_t D
   if (!moe_shape(E, D, I, ldp) || R < 0 || !fits32(ldp, I) || !fits32(slab_rows(D), I) || !fits32(kTile, 2 * D))
     return kErrBadShape;
   if (!al16(h8) || !al16(wd8) || !al16(out)) return kErrBadAlignment;
-  const Tiling tl = tiling(ldp, D);
+  const Tiling tl = tiling(ldp, D, 1, 64);
   const auto kern = tl.small ? down_fwd_kernel<true> : down_fwd_kernel<false>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
@@ -2315,19 +2385,8 @@ int sfp8_moe_gemm_down_dgrad_swiglu(const void* dout, const void* wdt, const voi
   if (!moe_shape(E, D, I, ldp) || R < 0) return kErrBadShape;
   if (!fits32(kTile, 2 * D) || !fits32(slab_rows(I), 2 * D) || !fits32(ldp, 2 * I)) return kErrBadShape;
   if (!al16(dout) || !al16(wdt) || !al16(gu8) || !al16(dgu8) || !al16(dgu8t)) return kErrBadAlignment;
-  int n_cu = 0;
-  int rc = cu_count(&n_cu);
-  if (rc) return rc;
-  const int tiles_m = (int)(ldp / kTile), tiles_n = cdiv(I, kTile);
-  const int ntiles = tiles_m * tiles_n;  // an upper bound: the kernel reads the plan's count
-  const auto kern = dgu8t ? down_dgrad_swiglu_kernel<true> : down_dgrad_swiglu_kernel<false>;
-  rc = prep(kern, kDgradLds);
-  if (rc) return rc;
-  hipLaunchKernelGGL(kern, dim3(ntiles < n_cu ? ntiles : n_cu), dim3(512), kDgradLds,
-                     (hipStream_t)stream, (const uint16_t*)dout, (const uint16_t*)wdt, (const uint8_t*)gu8, R, D, I,
-                     scale, amax, (uint8_t*)dgu8, (uint8_t*)dgu8t, ldp, tiles_m, tiles_n, plan,
-                     2 * D * slab_rows(I));
-  return status();
+  return dgrad_launch(dout, wdt, gu8, ldp, R, D, I, scale, amax, dgu8, dgu8t, ldp, plan, 2 * D * slab_rows(I),
+                      (hipStream_t)stream);
 }
 
 int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int64_t D, int64_t I, const int* plan,
@@ -2337,7 +2396,7 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
       !fits32(kTile, 2 * D))
     return kErrBadShape;
   if (!al16(dgu8) || !al16(w8t) || !al16(dx)) return kErrBadAlignment;
-  const Tiling tl = tiling(ldp, D);
+  const Tiling tl = tiling(ldp, D, 1, 64);
   const auto kern = tl.small ? gateup_dgrad_kernel<true> : gateup_dgrad_kernel<false>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
@@ -2418,14 +2477,14 @@ inline bool bf16_shape(int64_t D, int64_t I) {
 }
 
 int bf16_swiglu_launch(const void* x, const void* w, int64_t T, int64_t D, int64_t I, const float* rstd, void* gu,
-                       void* h, const int* plan, int64_t E, int tiles_m, int64_t ldxs, hipStream_t st) {
-  const int tiles_n = cdiv(I, 128);
-  int rc = prep(bf16_swiglu_fwd_kernel, kMainLds);
+                       void* h, const int* plan, int64_t ldp, int64_t ldxs, hipStream_t st) {
+  const Tiling tl = swiglu_tiling(plan ? ldp : T, I);
+  const auto kern = tl.small ? bf16_swiglu_fwd_kernel<true> : bf16_swiglu_fwd_kernel<false>;
+  const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(bf16_swiglu_fwd_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(512), kMainLds, st,
-                     (const uint16_t*)x, (const uint8_t*)w, T, D, I, rstd, (uint16_t*)gu, (uint16_t*)h, tiles_m,
-                     tiles_n, plan, plan ? 2 * D * slab_rows(2 * I) : 0, ldxs);
-  (void)E;
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st,
+                     (const uint16_t*)x, (const uint8_t*)w, T, D, I, rstd, (uint16_t*)gu, (uint16_t*)h, tl.m,
+                     tl.n, plan, plan ? 2 * D * slab_rows(2 * I) : 0, ldxs);
   return status();
 }
 
@@ -2449,7 +2508,7 @@ int sfp8_bf16_gemm_swiglu_fwd(const void* x, int x_slab, const void* w, int64_t 
   if (x_slab && !fits32(slab_rows(T), 2 * D)) return kErrBadShape;
   if (!al16(x) || !al16(w) || !al16(gu) || !al16(h)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  return bf16_swiglu_launch(x, w, T, D, I, rstd, gu, h, nullptr, 1, cdiv(T, kTile), x_slab ? slab_rows(T) : 0,
+  return bf16_swiglu_launch(x, w, T, D, I, rstd, gu, h, nullptr, 0, x_slab ? slab_rows(T) : 0,
                             (hipStream_t)stream);
 }
 
@@ -2461,7 +2520,7 @@ int sfp8_bf16_moe_gemm_swiglu_fwd(const void* x, const void* w, int64_t E, int64
     return kErrBadShape;
   if (!al16(x) || !al16(w) || !al16(gu) || !al16(h)) return kErrBadAlignment;
   if (ldp == 0) return kOk;
-  return bf16_swiglu_launch(x, w, 0, D, I, nullptr, gu, h, plan, E, (int)(ldp / kTile), 0, (hipStream_t)stream);
+  return bf16_swiglu_launch(x, w, 0, D, I, nullptr, gu, h, plan, ldp, 0, (hipStream_t)stream);
 }
 
 int sfp8_bf16_gemm(const void* a, const void* b, int64_t T, int64_t N, int64_t K, int64_t lda, void* out,

@@ -370,12 +370,13 @@ def test_wgrad_rows_equals_token_contiguous(dev, M, N, T, splits):
     assert torch.equal(ops.wgrad_rows(a_t, b_rows, M, N, sa, sb, a_rows=False), ref)
 
 
-# The bf16-output GEMMs run 128 x 128 tiles up to 128 tiles of 256 x 256 and
-# the larger tiles from 129 on: both sides of that line in rows and in
-# columns, one row past a tile of either shape, widths that end inside one,
+# The bf16-output GEMMs run 128 x 128 tiles up to 128 tiles of 256 x 256, the
+# larger tiles from 129 on and (the FP8 ones) the smaller again from 257 to 320:
+# both sides of those lines in rows and in columns, one row past a tile of either shape, widths that end inside one,
 # the shortest K.
 @pytest.mark.parametrize("T,D,I", [(1, 128, 128), (128, 272, 128), (129, 128, 384), (257, 400, 256),
-                                   (32768, 256, 128), (32769, 256, 128), (8192, 1024, 128), (8193, 1040, 128)])
+                                   (32768, 256, 128), (32769, 256, 128), (8192, 1024, 128), (8193, 1040, 128),
+                                   (65537, 256, 128), (81921, 256, 128)])
 def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
     """Integer operands: every product and sum is exact in fp32 (at most
     64 * 768 < 2^24), so the rounded result of either tile shape is known."""
@@ -399,3 +400,61 @@ def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
     a, b = ints(T, 2 * I, torch.bfloat16), ints(D, 2 * I, torch.bfloat16)
     out = sg.ops.bf16_gemm(padded(a), sg.ops.to_slab(b), T, D, 2 * I)
     assert torch.equal(out, (a.float() @ b.float().t()).bfloat16())
+
+
+# The SwiGLU forwards and the down dgrad run 128-row tiles up to 128 tiles of
+# 256 rows and again from 257 to 384: both sides of each line, with one row in
+# the last tile of either shape (whose padding rows the K-slabs keep as zeros)
+# and columns that end inside one.
+@pytest.mark.parametrize("T,D,I", [(1, 128, 128), (129, 256, 384), (4099, 256, 256), (4097, 128, 1024),
+                                   (16385, 128, 256), (32768, 128, 384), (33025, 128, 384), (12289, 256, 1024)])
+def test_tile_shapes_of_swiglu(dev, T, D, I):
+    """FP8 forward and dgrad against the oracle's formulas on the device:
+    integer operands make gate, up and dh exact; codes of h and of d_gu may
+    differ by one where the sigmoids differ by an ulp."""
+    g = torch.Generator(device=dev).manual_seed(T + D + I)
+    ldt = sg.ops.ldt_of(T)
+
+    def ints(rows, cols, dtype, n=2):
+        return torch.randint(-n, n + 1, (rows, cols), generator=g, device=dev).float().to(dtype)
+
+    def padded(x):
+        return sg.ops.to_slab(torch.cat([x, torch.zeros(ldt - T, x.shape[1], device=dev).to(x.dtype)]))
+
+    def close(got, want, fmt, top):
+        got, ref = sg.ops.unslab(got, ldt), want.clamp(-top, top).to(fmt)
+        assert torch.all(got.view(torch.uint8)[T:] == 0)
+        a, b = (v.contiguous().view(torch.uint8).int() for v in (got[:T], ref))
+        a, b = (torch.where(v >= 128, 128 - v, v) for v in (a, b))
+        assert int((a - b).abs().max()) <= 1 and float((a != b).float().mean()) < 1e-3
+
+    x8, w8 = ints(T, D, E4), ints(2 * I, D, E4)
+    s = torch.tensor([1, 2.0 ** -2, 2.0 ** -4, 1, 1], device=dev)
+    one, amax = torch.ones(2, device=dev), torch.zeros(5, device=dev)
+    gu8, h8, h8t = sg.ops.gateup_swiglu_fwd(padded(x8), sg.ops.to_slab(w8), s, one, amax, T, I)
+    gu = x8.float() @ w8.float().t()  # integers below 2^8 * 4: exact in bf16 up to 256, rounded above
+    gu = gu.bfloat16().float()
+    gate, up = gu.chunk(2, dim=1)
+    close(gu8, gu * s[1], E4, 448.0)
+    close(h8, gate * torch.sigmoid(gate) * up * s[2], E4, 448.0)
+    assert torch.equal(sg.ops.unslab(h8t, I), sg.ops.unslab(h8, ldt).t())
+    assert amax[1].item() == gu.abs().max().item()
+    dy, wdt = ints(T, D, torch.bfloat16), ints(I, D, torch.bfloat16)
+    dgu8, _ = sg.ops.down_dgrad_swiglu(dy, sg.ops.to_slab(wdt), gu8, s, amax, copy=False)
+    dh = (dy.float() @ wdt.float().t()).bfloat16().float()
+    gate, up = (sg.ops.unslab(gu8, T).float() / s[1]).chunk(2, dim=1)
+    sig = torch.sigmoid(gate)
+    close(dgu8, torch.cat([dh * up * (sig * (1 + gate * (1 - sig))), dh * gate * sig], 1),
+          torch.float8_e5m2, 57344.0)
+    # the bf16 forward, from row-major x and from its row K-slab
+    xb, wb = x8.float().bfloat16(), w8.float().bfloat16()
+    ws, _ = sg.ops.bf16_weight_slabs(wb[None], transposed=False)
+    rstd, _, xs = sg.ops.bf16_rows_prep(xb, None, ldt, 1e-6, copy=False, rows=True)
+    ones = torch.ones(T, device=dev)
+    gub, hb = sg.ops.bf16_swiglu_fwd(xb, ws, I)
+    assert torch.equal(gub, gu.bfloat16())
+    gate, up = gu.chunk(2, dim=1)
+    ref = (gate * torch.sigmoid(gate) * up)
+    assert float((hb.float() - ref).norm() / ref.norm().clamp(min=1e-30)) < 2 ** -8  # one bf16 rounding
+    for a, b in zip(sg.ops.bf16_swiglu_fwd(xb, ws, I, rstd=ones, xs=xs), (gub, hb)):
+        assert torch.equal(a, b)
