@@ -141,24 +141,28 @@ SFP8_DEV void round16_bf16(const floatx16& a, float s, float (&o)[16]) {
   }
 }
 
-// The two tile shapes of the GEMMs below: 256 x 256 by 8 waves, one
-// work-group per CU, or (SMALL) 128 x 128 by 4 waves, two per CU.  The B
-// rows of both are permuted by plain_col_nb<2>, or with PAIRED (gate rows in
-// the first half of the B tile, up rows in the second) by paired_col8 and
-// paired_col64.
-template <bool SMALL>
-struct TileShape {
-  static constexpr int kM = SMALL ? 128 : 256;
-  static constexpr int kThreads = SMALL ? 256 : 512;
-  static constexpr int kMinWaves = SMALL ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
-  static constexpr int kWN = SMALL ? 2 : 4, kTB = SMALL ? 2 : 4;
+// Tile shapes of the GEMMs below: 64 TB rows by 64 WN columns, 2 WN waves of
+// 32 TB x 64.  <4, 4> is 256 x 256 by 8 waves, one work-group per CU, <3, 4>
+// the same with 192 rows; <2, 2> is 128 x 128 by 4 waves, two work-groups per
+// CU.  The B rows of each are permuted by plain_col_nb<2>,
+// or with PAIRED (gate rows in the first half of the B tile, up rows in the
+// second) by paired_col8 (WN = 4) and paired_col64 (WN = 2).
+template <int TB, int WN>
+struct Tile {
+  static constexpr int kM = 64 * TB, kN = 64 * WN, kTB = TB, kWN = WN;
+  static constexpr int kThreads = 128 * WN;
+  static constexpr int kMinWaves = WN == 2 ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
   template <bool BF16, int FA, int FB, bool TRA = false, bool TRB = false, bool PAIRED = false>
-  using Loop = MainLoop<BF16, FA, FB, PAIRED, 2, kStages, 0, TRA, TRB, kWN, kTB, kM>;
+  using Loop = MainLoop<BF16, FA, FB, PAIRED, 2, kStages, 0, TRA, TRB, WN, TB, TB == 3 ? 256 : kM>;
   static constexpr int kLds = Loop<true, 0, 0>::kLds;
-  // the plan's tile of tile row tm, and that tile row's valid rows of it
-  static SFP8_DEV int plan_tile(int tm) { return SMALL ? tm >> 1 : tm; }
-  static SFP8_DEV int plan_skip(int tm) { return SMALL ? 128 * (tm & 1) : 0; }
+  static constexpr int kOutStride = 2 * kN + 16;        // a staged bf16 row
+  static constexpr int kPieces = kM * kN / 8 / kThreads;  // 16-byte pieces of it per thread
+  // the plan's tile of tile row tm, and that tile row's first row in it
+  static SFP8_DEV int plan_tile(int tm) { return tm / (256 / kM); }
+  static SFP8_DEV int plan_skip(int tm) { return kM * (tm % (256 / kM)); }
 };
+template <bool SMALL>
+using TileShape = Tile<SMALL ? 2 : 4, SMALL ? 2 : 4>;
 
 // ---------------------------------------------------------------------------
 // (a6) gate/up forward + SwiGLU epilogue (spark-gpt train.py:975-1016).
@@ -888,16 +892,16 @@ SFP8_DEV void stage_bf16_half8(uint8_t* lds, const floatx16 (&acc)[4][2], float 
   }
 }
 
-// The 128 x 128 tile (TileShape<true>): 4 waves of 64 x 64, the whole bf16
-// tile staged at once (stride kSmallStride: consecutive rows shift by 4
-// banks) and written as 256-byte rows.
-constexpr int kSmallStride = 272;
-SFP8_DEV void stage_bf16_small(uint8_t* lds, const floatx16 (&acc)[2][2], float s) {
+// A tile of at most 192 rows staged at once: the bf16 tile of kM rows and kN
+// columns (row stride kOutStride: consecutive rows shift by 4 banks), written
+// as whole tile rows.
+template <class TS>
+SFP8_DEV void stage_bf16_tile(uint8_t* lds, const floatx16 (&acc)[TS::kTB][2], float s) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
   const int fr = lane & 31, g = lane >> 5, cb = 64 * wn + 32 * g;
 #pragma unroll
-  for (int tb = 0; tb < 2; ++tb) {
-    const int lr = 64 * wm + 32 * tb + fr;
+  for (int tb = 0; tb < TS::kTB; ++tb) {
+    const int lr = 32 * TS::kTB * wm + 32 * tb + fr;
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
       uint32_t w0[4], w1[4];
@@ -906,7 +910,7 @@ SFP8_DEV void stage_bf16_small(uint8_t* lds, const floatx16 (&acc)[2][2], float 
         w0[i] = pack2_bf16(acc[tb][nb][2 * i] * s, acc[tb][nb][2 * i + 1] * s);
         w1[i] = pack2_bf16(acc[tb][nb][8 + 2 * i] * s, acc[tb][nb][8 + 2 * i + 1] * s);
       }
-      uint8_t* q = lds + lr * kSmallStride + (cb + 16 * nb) * 2;
+      uint8_t* q = lds + lr * TS::kOutStride + (cb + 16 * nb) * 2;
       store16(q, w0);
       store16(q + 16, w1);
     }
@@ -978,25 +982,27 @@ SFP8_DEV void write_bf16_half_res(const uint8_t* lds, int p, int64_t m0, int64_t
   }
 }
 
-// The staged 128 x 128 tile to out[t, n] (bf16, leading dimension ld), rows
-// m0.. below T, columns below N; with RES the bf16 residual rv (requested by
-// load_res_small) is added first: out = bf16(res + staged).
-SFP8_DEV void load_res_small(__amdgpu_buffer_rsrc_t rres, int64_t n0, int64_t D, intx4 (&rv)[8]) {
+// The tile staged by stage_bf16_tile to out[t, n] (bf16, leading dimension
+// ld), rows m0.. below T, columns below N; with RES the bf16 residual rv
+// (requested by load_res_tile) is added first: out = bf16(res + staged).
+template <class TS>
+SFP8_DEV void load_res_tile(__amdgpu_buffer_rsrc_t rres, int64_t n0, int64_t D, intx4 (&rv)[TS::kPieces]) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = (int)threadIdx.x + 256 * k;
-    rv[k] = __builtin_amdgcn_raw_buffer_load_b128(rres, (uint32_t)(((idx >> 4) * D + n0 + 8 * (idx & 15)) * 2), 0, kNT);
+  for (int k = 0; k < TS::kPieces; ++k) {
+    const int idx = (int)threadIdx.x + TS::kThreads * k;
+    const int lr = idx / (TS::kN / 8), c = idx % (TS::kN / 8);
+    rv[k] = __builtin_amdgcn_raw_buffer_load_b128(rres, (uint32_t)((lr * D + n0 + 8 * c) * 2), 0, kNT);
   }
 }
-template <bool RES>
-SFP8_DEV void write_bf16_small(const uint8_t* lds, int64_t m0, int64_t n0, int64_t T, int64_t N, int64_t ld,
-                               const intx4 (&rv)[8], uint16_t* __restrict__ out) {
+template <class TS, bool RES>
+SFP8_DEV void write_bf16_tile(const uint8_t* lds, int64_t m0, int64_t n0, int64_t T, int64_t N, int64_t ld,
+                              const intx4 (&rv)[TS::kPieces], uint16_t* __restrict__ out) {
   const __amdgpu_buffer_rsrc_t ro = make_rsrc(out + m0 * ld, (T - m0) * ld * 2);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int idx = (int)threadIdx.x + 256 * k;
-    const int lr = idx >> 4, c = idx & 15;
-    intx4 o = *reinterpret_cast<const intx4*>(lds + lr * kSmallStride + c * 16);
+  for (int k = 0; k < TS::kPieces; ++k) {
+    const int idx = (int)threadIdx.x + TS::kThreads * k;
+    const int lr = idx / (TS::kN / 8), c = idx % (TS::kN / 8);
+    intx4 o = *reinterpret_cast<const intx4*>(lds + lr * TS::kOutStride + c * 16);
     if constexpr (RES) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1011,14 +1017,14 @@ SFP8_DEV void write_bf16_small(const uint8_t* lds, int64_t m0, int64_t n0, int64
 
 // A tile's accumulators times s, as bf16, to out[t, n] (leading dimension N)
 // for rows u0.. below uend and columns n0.. below N.
-template <bool SMALL>
-SFP8_DEV void store_bf16_tile(uint8_t* lds, const floatx16 (&acc)[TileShape<SMALL>::kTB][2], float s, int64_t u0,
-                              int64_t n0, int64_t uend, int64_t N, uint16_t* __restrict__ out) {
-  if constexpr (SMALL) {
-    const intx4 none[8] = {};
-    stage_bf16_small(lds, acc, s);
+template <class TS>
+SFP8_DEV void store_bf16_tile(uint8_t* lds, const floatx16 (&acc)[TS::kTB][2], float s, int64_t u0, int64_t n0,
+                              int64_t uend, int64_t N, uint16_t* __restrict__ out) {
+  if constexpr (TS::kTB < 4) {
+    const intx4 none[TS::kPieces] = {};
+    stage_bf16_tile<TS>(lds, acc, s);
     __syncthreads();
-    write_bf16_small<false>(lds, u0, n0, uend, N, N, none, out);
+    write_bf16_tile<TS, false>(lds, u0, n0, uend, N, N, none, out);
   } else {
     stage_bf16_half8<0>(lds, acc, s);
     __syncthreads();
@@ -1037,13 +1043,12 @@ SFP8_DEV void store_bf16_tile(uint8_t* lds, const floatx16 (&acc)[TileShape<SMAL
 // its rows(tm) valid rows to y rows urow(tm).. (expert order, unpadded);
 // W_down8 of expert e at wd8 + e * w_estride, its scale wscale[e] (the dense
 // call passes wscale + 1: [q_gu, q_d]).
-template <bool SMALL>
-__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void down_fwd_kernel(
+template <class TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void down_fwd_kernel(
     const uint8_t* __restrict__ h8, const uint8_t* __restrict__ wd8, const uint16_t* __restrict__ res,
     int64_t T, int64_t D, int64_t I, const float* __restrict__ scale, const float* __restrict__ wscale,
     uint16_t* __restrict__ y, int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan,
     int64_t w_estride) {
-  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
@@ -1059,7 +1064,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     urows = P.rows(pt) - TS::plan_skip(tm);
     if (urows <= 0) return;  // nothing but padding rows, which have no output
   }
-  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
   floatx16 acc[TS::kTB][2];
   // K-slab operands: h8 [I/64][ldt][64], wd8 [I/64][slab_rows(D)][64]
   const int64_t dp = slab_rows(D);
@@ -1068,13 +1073,13 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
       wd8 + n0 * kStage, I * dp - n0 * kStage, [=](int r) { return plain_col_nb<2>(r) * kStage; },
       (int)(dp * kStage), (int)(I / kStage), acc);
   const float deq = 1.0f / (scale[2] * wscale[0]);
-  if constexpr (SMALL) {
-    intx4 rv[8];
-    if (!plan) load_res_small(make_rsrc(res + m0 * D, (T - m0) * D * 2), n0, D, rv);
-    stage_bf16_small(lds, acc, deq);
+  if constexpr (TS::kTB < 4) {
+    intx4 rv[TS::kPieces];
+    if (!plan) load_res_tile<TS>(make_rsrc(res + m0 * D, (T - m0) * D * 2), n0, D, rv);
+    stage_bf16_tile<TS>(lds, acc, deq);
     __syncthreads();
-    if (plan) write_bf16_small<false>(lds, u0, n0, u0 + urows, D, D, rv, y);
-    else write_bf16_small<true>(lds, m0, n0, T, D, D, rv, y);
+    if (plan) write_bf16_tile<TS, false>(lds, u0, n0, u0 + urows, D, D, rv, y);
+    else write_bf16_tile<TS, true>(lds, m0, n0, T, D, D, rv, y);
   } else {
   if (plan) {
     // expert rows, no residual: out rounded to bf16 (train.py:1377-1378 stores acc / (s2 q_d) as bf16)
@@ -1191,7 +1196,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   //   dgu8 = e5m2(d*q3) = e5m2(d'*(s_gu*q3)),  amax3 = s_gu*max(|dg|,|du|).
   const float m3s = (1.0f / scale[1]) * scale[3];
   const float inv3 = 1.0f / m3s, bnd3 = kE5M2Max * inv3;
-  float* red = reinterpret_cast<float*>(base + (SMALL ? 128 * kSmallStride : 2 * kTile * kEpiStride2));  // after the staging tiles
+  float* red = reinterpret_cast<float*>(base + (SMALL ? 128 * TS::kOutStride : 2 * kTile * kEpiStride2));  // after the staging tiles
   float m3 = 0.f;
   // Persistent: work-group pid runs tiles pid, pid + gridDim.x, ...  (Work-
   // groups started a quarter of a tile apart per XCD, so that the tiles'
@@ -1242,7 +1247,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   uint8_t* DH = base;
   // chunk k of this thread in a pass: 16 columns from chunk_col(k) of staging
   // row chunk_row(k), tile row tile_row(k, P)
-  constexpr int kSlabs = TS::kM / 64, kDh = SMALL ? kSmallStride : kBf16Stride;
+  constexpr int kSlabs = TS::kM / 64, kDh = SMALL ? TS::kOutStride : kBf16Stride;
   const auto chunk_row = [=](int k) { return 16 * ((kWaves * k + wave) / kSlabs) + (lane >> 2); };
   const auto chunk_col = [=](int k) { return 64 * ((kWaves * k + wave) % kSlabs) + 16 * (lane & 3); };
   const auto tile_row = [=](int k, int P) { return SMALL ? chunk_row(k) : half_tile_row(chunk_row(k), P); };
@@ -1361,7 +1366,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   } else if constexpr (SMALL) {
     uint32_t pg[4], pu[4];
     gu_loads(0);
-    stage_bf16_small(DH, acc, 1.0f);  // dh rounded to bf16 (train.py:1082)
+    stage_bf16_tile<TS>(DH, acc, 1.0f);  // dh rounded to bf16 (train.py:1082)
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1408,12 +1413,11 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // With a MoE plan: tile row tm of padded expert order writes its rows(tm)
 // valid rows to dxn rows urow(tm).. (expert order, unpadded); W8^T of
 // expert e at w8t + e * w_estride, its scale wscale[e].
-template <bool SMALL>
-__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void gateup_dgrad_kernel(
+template <class TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kernel(
     const uint8_t* __restrict__ dgu8, const uint8_t* __restrict__ w8t, int64_t T, int64_t D, int64_t I,
     const float* __restrict__ scale, const float* __restrict__ wscale, uint16_t* __restrict__ dxn,
     int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t w_estride) {
-  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   const int64_t K = 2 * I;
   const int64_t dp = slab_rows(D);
@@ -1432,7 +1436,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     uend = P.urow(pt) + P.rows(pt);
     if (u0 >= uend) return;  // nothing but padding rows, which have no output
   }
-  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
   floatx16 acc[TS::kTB][2];
   // K-slab operands: dgu8 [2I/64][ldt][64], w8t [2I/64][slab_rows(D)][64]
   TS::template Loop<false, kFmtE5M2, kFmtE4M3>::run(
@@ -1441,7 +1445,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
       (int)(dp * kStage), (int)(K / kStage), acc);
   // the scales are read after the K loop, so that nothing is held across it
   const float sab = (1.0f / scale[3]) * (1.0f / wscale[0]);  // both powers of two
-  store_bf16_tile<SMALL>(lds, acc, sab, u0, n0, uend, D, dxn);
+  store_bf16_tile<TS>(lds, acc, sab, u0, n0, uend, D, dxn);
 }
 
 // ---------------------------------------------------------------------------
@@ -1832,11 +1836,10 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // valid rows to out rows urow(tm).. (expert order); B of expert e at
 // b + e * b_estride (bytes).
 // 8 waves (two per SIMD), each 128 x 64.
-template <bool SMALL>
-__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void bf16_gemm_kernel(
+template <class TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void bf16_gemm_kernel(
     const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int64_t T, int64_t N, int64_t Kb, int64_t lda,
     uint16_t* __restrict__ out, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t b_estride) {
-  using TS = TileShape<SMALL>;
   extern __shared__ __align__(16) uint8_t lds[];
   const int64_t bp = slab_rows(N);
   int tm, tn;
@@ -1851,13 +1854,13 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     uend = P.urow(pt) + P.rows(pt);
     if (u0 >= uend) return;  // nothing but padding rows, which have no output
   }
-  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
   floatx16 acc[TS::kTB][2];
   TS::template Loop<true, 0, 0>::run(
       lds, a + m0 * kStage, Kb * lda - m0 * kStage, [=](int r) { return r * kStage; }, (int)(lda * kStage),
       b + n0 * kStage, Kb * bp - n0 * kStage, [=](int r) { return plain_col_nb<2>(r) * kStage; }, (int)(bp * kStage),
       (int)(Kb / kStage), acc);
-  store_bf16_tile<SMALL>(lds, acc, 1.0f, u0, n0, uend, N, out);
+  store_bf16_tile<TS>(lds, acc, 1.0f, u0, n0, uend, N, out);
 }
 
 // The bf16 weight gradient's reduction: out[m, n] = bf16(sum over s
@@ -2004,51 +2007,75 @@ inline int64_t wgrad_chunk(int64_t ldt, int64_t s) {
 }  // namespace
 
 namespace {
+constexpr int64_t kCUs = 256;
+
 // Whether an M x N output (of each of `parts` K splits times experts) is
 // computed in 128 x 128 tiles (two work-groups per CU) instead of 256 x 256
 // ones (one per CU): when the larger tiles would leave half of the 256 CUs or
 // more without one.  A CU runs its tile at the same speed however many others
 // are idle, so the quarter tiles, spread over up to four times the CUs, win
 // until they fill the chip; from then on their K loop, with twice the LDS-DMA
-// bytes per FLOP, is the slower one.  Measured (us, 256 -> 128 tiles, at 16,
-// 80, 128 and 192 tiles of 256 x 256, D = 1024, I = 3072): down forward 29 ->
-// 14, 32 -> 24, 36 -> 32, 40 -> 44; gate/up dgrad 49 -> 26, 50 -> 38, 55 ->
-// 45, 62 -> 71; bf16 dgrad 91 -> 46, 94 -> 73, 99 -> 88, 125 -> 135.
+// bytes per FLOP, is the slower one.  Measured (us, 256 -> 128 tiles): weight
+// gradient with its reduction 25 -> 15 at 16 work-groups of 256 x 256, 26 ->
+// 17 at 32, 27 -> 25 at 96, 55 -> 52 at 192 but 40 -> 43 at another 192; down
+// dgrad 27 -> 13 at 48 tiles, 17 -> 13 at 128, 39 -> 44 at 240; FP8 SwiGLU
+// forward 11 -> 6 at 32, 12 -> 9 at 128, 15 -> 15 at 256.
 // second: also when the larger tiles would take a second round of 1 to
 // `second` of them, for the kernels whose epilogue is a large part of a tile,
 // which the second work-group of a CU then overlaps: with 128, FP8 SwiGLU
 // forward 32 -> 26 at 272 tiles and 28 -> 26 at 384, bf16 one 49 -> 41 and
-// 42 -> 39, down dgrad 46 -> 41 and 68 -> 66 at 384; with 64, down forward
-// 74 -> 68 and gate/up dgrad 121 -> 113 at 320 (78 -> 79 and 127 -> 131 at
-// 384); none for the bf16 dgrad, nearly all K loop (241 -> 266 at 320).
+// 42 -> 39, down dgrad 46 -> 41 and 68 -> 66 at 384.
 inline bool use_small_tiles(int64_t M, int64_t N, int64_t parts, int second) {
-  constexpr int64_t kCUs = 256;
   const int64_t tiles = (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * parts;
   return tiles <= kCUs / 2 || (tiles > kCUs && tiles <= kCUs + second);
 }
 
-// A GEMM's tile shape over an M x N output (of each of `parts` K splits times
-// experts), and its launch.
+// A GEMM's tile shape Tile<tb, wn> over an M x N output (of each of `parts` K
+// splits times experts), and its launch.
 struct Tiling {
-  bool small;
+  bool small;  // Tile<2, 2>; else of 256 columns
+  int tb;
   int m, n, lds;  // tile rows and columns, dynamic LDS
   dim3 grid, block;
 };
-inline Tiling tiling_of(bool small, int64_t M, int64_t N, int64_t parts = 1) {
+template <int TB, int WN>
+Tiling tiling_of(int64_t M, int64_t N, int64_t parts = 1) {
+  using TS = Tile<TB, WN>;
   Tiling t;
-  t.small = small;
-  const int tile = t.small ? TileShape<true>::kM : TileShape<false>::kM;
-  t.m = cdiv(M, tile);
-  t.n = cdiv(N, tile);
-  t.lds = t.small ? TileShape<true>::kLds : TileShape<false>::kLds;
+  t.small = WN == 2;
+  t.tb = TB;
+  t.m = cdiv(M, TS::kM);
+  t.n = cdiv(N, TS::kN);
+  t.lds = TS::kLds;
   t.grid = dim3((unsigned)(t.m * t.n * parts));
-  t.block = dim3((unsigned)(t.small ? TileShape<true>::kThreads : TileShape<false>::kThreads));
+  t.block = dim3((unsigned)TS::kThreads);
   return t;
 }
-
 inline Tiling tiling(int64_t M, int64_t N, int64_t parts = 1, int second = 0) {
-  return tiling_of(use_small_tiles(M, N, parts, second), M, N, parts);
+  return use_small_tiles(M, N, parts, second) ? tiling_of<2, 2>(M, N, parts) : tiling_of<4, 4>(M, N, parts);
 }
+// The kernels with bf16 outputs have every shape; K: their K bytes.  By the
+// number of 256 x 256 tiles: 128 x 128 ones up to 128; from there on 192 x 256
+// ones where their rounds of 256 work-groups cost less (3 units a round
+// against 4) and the K loop is long enough to outweigh the larger share of
+// prologue and epilogue; else 256 x 256.  Measured (us, D = 1024, I = 3072,
+// gate/up dgrad and bf16 dgrad, 256 x 256 / 192 x 256 / 128 x 128): 16 tiles
+// 48 40 25, 91 75 46; 80 tiles 50 41 37, 93 77 71; 192 tiles 63 62 71, 126 120
+// 136; 256 tiles 77 97 89, 150 194 177; 320 tiles 121 108 113, 245 216 269;
+// 384 tiles 126 119 132, 258 242 312.  At 24 K stages (down forward, I = 1536,
+// 384 tiles) 192 x 256 is the slower one, 50 against 49.  128 x 256 tiles, one
+// per CU, were the faster ones alone at 80 tiles (34 against 37), but the
+// block's step was 3 % slower with them.  Grouped rows come in whole tiles of
+// 256, which 192-row tiles do not divide.
+inline Tiling out_tiling(int64_t M, int64_t N, int64_t K, bool grouped) {
+  const int64_t tiles = (int64_t)cdiv(M, kTile) * cdiv(N, kTile);
+  if (tiles <= kCUs / 2) return tiling_of<2, 2>(M, N);
+  const int64_t rounds = cdiv(tiles, kCUs), rounds192 = cdiv((int64_t)cdiv(M, 192) * cdiv(N, kTile), kCUs);
+  if (!grouped && K >= 48 * kStage && 3 * rounds192 < 4 * rounds) return tiling_of<3, 4>(M, N);
+  return tiling_of<4, 4>(M, N);
+}
+#define OUT_KERNEL(kernel, tl) \
+  ((tl).small ? kernel<Tile<2, 2>> : (tl).tb == 3 ? kernel<Tile<3, 4>> : kernel<Tile<4, 4>>)
 
 // The gate/up forward's: a tile covers half as many (gate, up) columns as rows.
 inline Tiling swiglu_tiling(int64_t M, int64_t I) {
@@ -2061,7 +2088,7 @@ inline Tiling swiglu_tiling(int64_t M, int64_t I) {
 int dgrad_launch(const void* dy, const void* wdt, const void* gu8, int64_t rows, int64_t T, int64_t D, int64_t I,
                  const float* scale, float* amax, void* dgu8, void* dgu8t, int64_t ldt, const int* plan,
                  int64_t w_estride, hipStream_t st) {
-  const Tiling tl = dgu8t ? tiling_of(false, rows, I) : tiling(rows, I, 1, 128);
+  const Tiling tl = dgu8t ? tiling_of<4, 4>(rows, I) : tiling(rows, I, 1, 128);
   const auto kern = dgu8t ? down_dgrad_swiglu_kernel<true, false>
                           : (tl.small ? down_dgrad_swiglu_kernel<false, true> : down_dgrad_swiglu_kernel<false, false>);
   int n_cu = 0;
@@ -2194,8 +2221,8 @@ int sfp8_gemm_down_fwd(const void* h8, const void* wd8, const void* res, int64_t
   if (!fits32(ldt, I) || !fits32(slab_rows(D), I) || !fits32(kTile, 2 * D)) return kErrBadShape;
   if (!al16(h8) || !al16(wd8) || !al16(res) || !al16(y)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const Tiling tl = tiling(T, D, 1, 64);
-  const auto kern = tl.small ? down_fwd_kernel<true> : down_fwd_kernel<false>;
+  const Tiling tl = out_tiling(T, D, I, false);
+  const auto kern = OUT_KERNEL(down_fwd_kernel, tl);
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
   hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
@@ -2223,8 +2250,8 @@ int sfp8_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t T, int64_t
   if (!fits32(ldt, 2 * I) || !fits32(slab_rows(D), 2 * I) || !fits32(kTile, 2 * D)) return kErrBadShape;
   if (!al16(dgu8) || !al16(w8t) || !al16(dxn)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  const Tiling tl = tiling(T, D, 1, 64);
-  const auto kern = tl.small ? gateup_dgrad_kernel<true> : gateup_dgrad_kernel<false>;
+  const Tiling tl = out_tiling(T, D, 2 * I, false);
+  const auto kern = OUT_KERNEL(gateup_dgrad_kernel, tl);
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
   hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
@@ -2368,8 +2395,8 @@ int sfp8_moe_gemm_down_fwd(const void* h8, const void* wd8, int64_t E, int64_t D
   if (!moe_shape(E, D, I, ldp) || R < 0 || !fits32(ldp, I) || !fits32(slab_rows(D), I) || !fits32(kTile, 2 * D))
     return kErrBadShape;
   if (!al16(h8) || !al16(wd8) || !al16(out)) return kErrBadAlignment;
-  const Tiling tl = tiling(ldp, D, 1, 64);
-  const auto kern = tl.small ? down_fwd_kernel<true> : down_fwd_kernel<false>;
+  const Tiling tl = out_tiling(ldp, D, I, true);
+  const auto kern = OUT_KERNEL(down_fwd_kernel, tl);
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
   hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
@@ -2396,8 +2423,8 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
       !fits32(kTile, 2 * D))
     return kErrBadShape;
   if (!al16(dgu8) || !al16(w8t) || !al16(dx)) return kErrBadAlignment;
-  const Tiling tl = tiling(ldp, D, 1, 64);
-  const auto kern = tl.small ? gateup_dgrad_kernel<true> : gateup_dgrad_kernel<false>;
+  const Tiling tl = out_tiling(ldp, D, 2 * I, true);
+  const auto kern = OUT_KERNEL(gateup_dgrad_kernel, tl);
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
   hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, (hipStream_t)stream,
@@ -2490,8 +2517,8 @@ int bf16_swiglu_launch(const void* x, const void* w, int64_t T, int64_t D, int64
 
 int bf16_gemm_launch(const void* a, const void* b, int64_t T, int64_t N, int64_t K, int64_t lda, void* out,
                      const int* plan, hipStream_t st) {
-  const Tiling tl = tiling(plan ? lda : T, N);
-  const auto kern = tl.small ? bf16_gemm_kernel<true> : bf16_gemm_kernel<false>;
+  const Tiling tl = out_tiling(plan ? lda : T, N, 2 * K, plan != nullptr);
+  const auto kern = OUT_KERNEL(bf16_gemm_kernel, tl);
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
   hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st,

@@ -122,13 +122,15 @@ SFP8_DEV void sched_interleave_valu() {
 // transposing read as possibly aliasing any LDS DMA it knows to be in flight
 // and would wait for all of it first; the stage waits and barriers already
 // order every read after its stage's DMA.
-// TB = A blocks of 32 rows per wave: 4 (two wave rows of 128) or 2 (two wave
-// rows of 64 of a TM = 128 tile, or four of a TM = 256 one: then only the
-// fragment, DMA and MFMA pieces, not run()).
+// TB = A blocks of 32 rows per wave: 4 (two wave rows of 128), 3 (two of 96: a
+// 192-row tile in a TM = 256 ring, whose last 64 rows are never read and whose
+// DMA is aimed out of range) or 2 (two wave rows of 64 of a TM = 128 tile, or
+// four of a TM = 256 one: then only the fragment, DMA and MFMA pieces, not
+// run()).
 template <bool BF16, int FMT_A, int FMT_B, bool PAIRED, int NB = 4, int STAGES = kStages, int PRE = 0,
           bool TR_A = false, bool TR_B = false, int WN = 2, int TB = 4, int TM = kTile>
 struct MainLoop {
-  static_assert(TB == 4 || TB == 2, "2 or 4 A blocks per wave");
+  static_assert(TB >= 2 && TB <= 4, "2 to 4 A blocks per wave");
   static constexpr int kWM = TM / (32 * TB);                // wave rows
   static constexpr int kStageA = TM * kStage;               // bytes of A per stage
   static constexpr int kWaves = kWM * WN;
@@ -354,6 +356,31 @@ struct MainLoop {
       __builtin_amdgcn_sched_barrier(0);
       return;
     }
+    if constexpr (TB == 3 && BF16) {
+      // 8 waves of 96 x 64: 12 bf16 MFMAs, five fragments and four DMA issues
+      mfma_then_reads<P + 0, 0, 1>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_then_dma<P + 1, 0, 1>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+      mfma_then_reads<P + 2, 1, 2>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_then_dma<P + 3, 1, 2>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+      mfma_then_reads<P + 4, 2, 3>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_then_dma<P + 5, 2, 4>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+      mfma_then_reads<P + 6, 3, 4>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_then_reads<P + 7, 4, 5>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_range<P + 8, kMfma>(cur, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      return;
+    } else if constexpr (TB == 3) {
+      // the same with 6 fp8 MFMAs
+      mfma_then_reads<P + 0, 0, 2>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_then_reads<P + 1, 2, 4>(lds, cur, nxt, acc, rd_buf, aoff, boff);
+      mfma_range<P + 2, P + 3>(cur, acc);
+      read_frag<4>(lds, rd_buf, aoff, boff, nxt);
+      load_one(0, lds, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+      load_one(1, lds, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma_then_dma<P + 3, 2, 4>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
+      return;
+    } else {
     if constexpr (BF16 && NB == 2) {
       // bf16, 8 waves of 128 x 64: 16 MFMAs of 32 cycles; six fragments and
       // four DMA issues alternate over 10 of them
@@ -424,6 +451,7 @@ struct MainLoop {
     mfma_then_dma<P + H + 2, 4, 6>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
     mfma_range<P + 2 * H, kMfma>(cur, acc);
     __builtin_amdgcn_sched_barrier(0);
+    }
   }
 
   // The stage of a 64 x 64 wave (TB = NB = 2): 4 fp8 MFMAs of 64 cycles or 8
@@ -499,8 +527,11 @@ struct MainLoop {
     const uint32_t chunk_tr =
         BF16 ? (uint32_t)((lane & 3) << 4) : (uint32_t)(((lane & 3) ^ (((lane >> 4) & 1) << 1)) << 4);
 #pragma unroll
-    for (int j = 0; j < kDmaA; ++j)
-      voff_a[j] = (uint32_t)a_rowoff((TM / kWaves) * wave + 16 * j + (lane >> 2)) + (TR_A ? chunk_tr : chunk);
+    for (int j = 0; j < kDmaA; ++j) {
+      const int r = (TM / kWaves) * wave + 16 * j + (lane >> 2);
+      voff_a[j] = (uint32_t)a_rowoff(r) + (TR_A ? chunk_tr : chunk);
+      if constexpr (32 * TB * kWM < TM) voff_a[j] = r < 32 * TB * kWM ? voff_a[j] : 0x80000000u;
+    }
 #pragma unroll
     for (int j = 0; j < kDmaB; ++j)
       voff_b[j] = (uint32_t)b_rowoff((kTileN / kWaves) * wave + 16 * j + (lane >> 2)) + (TR_B ? chunk_tr : chunk);

@@ -370,16 +370,18 @@ def test_wgrad_rows_equals_token_contiguous(dev, M, N, T, splits):
     assert torch.equal(ops.wgrad_rows(a_t, b_rows, M, N, sa, sb, a_rows=False), ref)
 
 
-# The bf16-output GEMMs run 128 x 128 tiles up to 128 tiles of 256 x 256, the
-# larger tiles from 129 on and (the FP8 ones) the smaller again from 257 to 320:
-# both sides of those lines in rows and in columns, one row past a tile of either shape, widths that end inside one,
-# the shortest K.
+# The bf16-output GEMMs run 128 x 128 tiles up to 128 tiles of 256 x 256, then
+# 192 x 256 (K of 48 stages or more, where they take fewer rounds) or 256 x 256
+# ones: both sides of those lines in rows and in columns,
+# one row past a tile of either shape, widths that end inside one, the shortest
+# K.  The FP8 dgrad has 2I bytes of K, the bf16 GEMM 4I, the forward I.
 @pytest.mark.parametrize("T,D,I", [(1, 128, 128), (128, 272, 128), (129, 128, 384), (257, 400, 256),
-                                   (32768, 256, 128), (32769, 256, 128), (8192, 1024, 128), (8193, 1040, 128),
-                                   (65537, 256, 128), (81921, 256, 128)])
+                                   (8192, 1024, 128), (8193, 1040, 128),
+                                   (32768, 256, 128), (32769, 256, 128), (33000, 256, 3072), (9217, 1024, 1536),
+                                   (65537, 256, 768), (66000, 256, 1536)])
 def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
     """Integer operands: every product and sum is exact in fp32 (at most
-    64 * 768 < 2^24), so the rounded result of either tile shape is known."""
+    64 * 6144 < 2^24), so the rounded result of every tile shape is known."""
     g = torch.Generator(device=dev).manual_seed(T + D + I)
     ldt = sg.ops.ldt_of(T)
 
