@@ -338,16 +338,18 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 //
 // Tile 256 tokens x 64 (gate, up) column pairs: B tile = 64 gate rows + 64 up
 // rows (MainLoop NB = 2, paired), so each lane holds g and u of the same 16
-// consecutive columns for each of its 4 row blocks.  One work-group per CU
+// consecutive columns for each of its TB row blocks.  One work-group per CU
 // walks its tiles; after tile i's K loop the lane packs bf16(g), bf16(u) of
-// its 64 pairs into 64 registers (E), and the SwiGLU of tile i runs in 16
-// units of 4 pairs, one per K stage of tile i+1, in the same instruction
+// its 16 TB pairs into registers (E), and the SwiGLU of tile i runs in 4 TB
+// units of 4 pairs over the K stages of tile i+1, in the same instruction
 // stream as its MFMAs (the matrix pipe runs them while the vector ALU does the
-// epilogue): each unit in six pieces, one after each MFMA past the stage's
-// barrier.  The h bytes of a tile also go to one of two LDS
-// tiles; its token-contiguous (K-slab) copy is written at the next tile
-// boundary with LDS transpose reads.  The last tile's epilogue runs alone.
-// NK = D / 64 K stages, fully unrolled so each unit has a fixed stage; the K
+// epilogue): each unit in six pieces, spread evenly after the MFMAs past the
+// stages' barriers (one per MFMA at NK = 16, two at 8, four at 4; there the
+// vector ALU, not the matrix core, sets the pace).  The h bytes of a tile also
+// go to one of two LDS tiles; its token-contiguous (K-slab) copy is written at
+// the next tile boundary with LDS transpose reads.  The last tile's epilogue
+// runs alone.
+// NK = D / 64 K stages, fully unrolled so each piece has a fixed stage; the K
 // stream runs on across tiles (the last three stages of a tile load the next
 // tile's first three), so a tile boundary waits for no DMA.
 constexpr int kPipeHStride = 80;                    // 64 h bytes + 16 per LDS row
@@ -381,11 +383,14 @@ struct SwigluPipe {
   static constexpr int kSt = 4;          // LDS ring stages
   static constexpr int kDma = ML::kDma;
   static constexpr int kPre = TB == 4 ? 2 : 1;  // MFMAs of a stage issued before its wait
-  static constexpr int kSpan = NK / kUnits;     // stages per unit
   static constexpr int kSlots = ML::kMfma - kPre;  // MFMAs past the barrier, one slot each
   static constexpr int kDmaSlots = TB == 4 ? 2 : kSlots;  // slots carrying the DMA
   static_assert(NK >= kSt && NK % kSt == 0, "whole rings of K stages: a tile's stage s sits in slot s % kSt");
-  static_assert(NK % kUnits == 0 && kSpan * kSlots == 6, "each unit's six pieces fill the slots of its stages");
+  // the units' pieces, six each, fill the tile's slots in order
+  static constexpr int kPer = 6 * kUnits / (NK * kSlots);  // pieces per slot
+  static_assert(kPer * NK * kSlots == 6 * kUnits, "whole pieces per slot");
+  // row blocks whose units are complete after stage KT
+  static constexpr int blocks_done(int kt) { return (kt + 1) * kSlots * kPer / 24; }
 
   // A unit's working values between its pieces.
   struct UnitTmp {
@@ -581,9 +586,8 @@ struct SwigluPipe {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kDma * (kSt - 3)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     slots<KT, 0>(c, c.ut, a_ss, b_ss);
-    // the stage that finishes a unit that finishes a row block stores it
-    constexpr int U = KT / kSpan;
-    if constexpr (KT % kSpan == kSpan - 1 && U % 4 == 3) block_store<U / 4>(c);
+    // the stage that finishes a row block's last unit stores it
+    if constexpr (blocks_done(KT) > blocks_done(KT - 1)) block_store<blocks_done(KT) - 1>(c);
   }
   template <int KT, int J>
   static SFP8_DEV void slots(Ctx& c, UnitTmp& t, int a_ss, int b_ss) {
@@ -596,7 +600,7 @@ struct SwigluPipe {
   // Slot J of stage KT: one MFMA past the barrier, then (J < 2) half of the
   // DMA of stage KT+3 (of the next tile past the last stage), one fragment
   // of stage KT+1 (B blocks first: the next stage's first MFMAs use b[0],
-  // b[1] and a[0]) and piece J of the stage's epilogue unit; the scheduling
+  // b[1] and a[0]) and the slot's pieces of the epilogue units; the scheduling
   // barrier keeps the slot's work after its MFMA.
   template <int KT, int J>
   static SFP8_DEV void slot(Ctx& c, UnitTmp& t, int a_ss, int b_ss) {
@@ -626,8 +630,16 @@ struct SwigluPipe {
     } else {
       ML::template read_frag<J == 1 ? 3 : 1>(c.lds, (KT + 1) % kSt, c.aoff, c.boff, c.f[nxt]);
     }
-    unit_piece<KT / kSpan, (KT % kSpan) * kSlots + J>(c, t);
+    pieces<(KT * kSlots + J) * kPer, kPer>(c, t);
     __builtin_amdgcn_sched_barrier(0);
+  }
+  // Pieces P .. P + N - 1 of the tile's units, in order.
+  template <int P, int N>
+  static SFP8_DEV void pieces(Ctx& c, UnitTmp& t) {
+    if constexpr (N > 0) {
+      unit_piece<P / 6, P % 6>(c, t);
+      pieces<P + 1, N - 1>(c, t);
+    }
   }
 
   // Stage LD's byte offset LD * ss, computed where it is used (otherwise
@@ -2082,6 +2094,41 @@ inline Tiling swiglu_tiling(int64_t M, int64_t I) {
   return tiling(M, 2 * I, 1, 128);
 }
 
+// Whether the gate/up forward runs the persistent kernel: at the widths it is
+// built for (4, 8 or 16 K stages), from 640 tiles of 256 x 64 pairs on (2.5 per
+// CU).  Its gain is the epilogue of one tile under the K loop of the next, so
+// it needs several tiles per CU, and the shorter the K loop the larger the
+// epilogue that it hides.  Measured (us, one tile per work-group -> persistent,
+// at 256, 512, 768 and 4096 or more tiles): D = 256 9 -> 11, 15 -> 15, 21 ->
+// 19, 92 -> 74; D = 512 (384, 640, 768, 4608) 16 -> 17, 23 -> 23, 26 -> 24,
+// 149 -> 107; D = 1024 14 -> 15, 23 -> 24, 36 -> 32, 530 -> 423 (640: 31 ->
+// 29).  At D = 2048 the longer K loop prefers the 256-column tile's lower
+// DMA traffic (1.81 against 1.55 ms at T = 65536).
+inline bool use_pipe(int64_t rows, int64_t D, int64_t I) {
+  return (D == 256 || D == 512 || D == 1024) && (int64_t)cdiv(rows, kTile) * (I / 64) >= 5 * kCUs / 2;
+}
+
+// The persistent gate/up forward over `rows` token rows (with a plan an upper
+// bound: the kernel reads the plan's count), one work-group per CU.
+int pipe_launch(const void* x8, const void* w8, int64_t T, int64_t rows, int64_t D, int64_t I, const float* scale,
+                const float* wscale, float* amax, void* gu8, void* h8, void* h8t, int64_t ldt, const int* plan,
+                int64_t w_estride, hipStream_t st) {
+  const auto kern = D == 1024  ? swiglu_pipe_kernel<16, kPipeTB>
+                    : D == 512 ? swiglu_pipe_kernel<8, kPipeTB>
+                               : swiglu_pipe_kernel<4, kPipeTB>;
+  const int tiles_m = cdiv(rows, kTile), tiles_n = (int)(I / 64);
+  const int ntiles = tiles_m * tiles_n;
+  int n_cu = 0;
+  int rc = cu_count(&n_cu);
+  if (rc) return rc;
+  rc = prep(kern, kPipeLds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, dim3(ntiles < n_cu ? ntiles : n_cu), dim3(kPipeThreads), kPipeLds, st, (const uint8_t*)x8,
+                     (const uint8_t*)w8, T, D, I, scale, wscale, amax, (uint8_t*)gu8, (uint8_t*)h8, (uint8_t*)h8t,
+                     ldt, tiles_m, tiles_n, plan, w_estride);
+  return status();
+}
+
 // The persistent down dgrad over `rows` token rows, the padding that its
 // K-slab output needs among them (with a plan an upper bound: the kernel reads
 // the plan's count), T rows of dy.
@@ -2188,22 +2235,8 @@ int sfp8_gemm_gateup_swiglu_fwd(const void* x8, const void* w8, int64_t T, int64
   if (!fits32(ldt, D) || !fits32(2 * I, D) || !fits32(ldt, I) || !fits32(ldt, 2 * I)) return kErrBadShape;
   if (!al16(x8) || !al16(w8) || !al16(gu8) || !al16(h8) || !al16(h8t)) return kErrBadAlignment;
   if (T == 0) return kOk;
-  if (D == 1024) {
-    // persistent, one work-group per CU, SwiGLU of each tile overlapped with
-    // the next tile's K loop
-    const int tiles_m = cdiv(T, kTile), tiles_n = (int)(I / 64);
-    const int ntiles = tiles_m * tiles_n;
-    int n_cu = 0;
-    int rc = cu_count(&n_cu);
-    if (rc) return rc;
-    rc = prep(swiglu_pipe_kernel<16, kPipeTB>, kPipeLds);
-    if (rc) return rc;
-    hipLaunchKernelGGL((swiglu_pipe_kernel<16, kPipeTB>), dim3(ntiles < n_cu ? ntiles : n_cu), dim3(kPipeThreads), kPipeLds,
-                       (hipStream_t)stream, (const uint8_t*)x8, (const uint8_t*)w8, T, D, I, scale, wscale, amax,
-                       (uint8_t*)gu8, (uint8_t*)h8, (uint8_t*)h8t, ldt, tiles_m, tiles_n, (const int*)nullptr,
-                       (int64_t)0);
-    return status();
-  }
+  if (use_pipe(ldt, D, I))
+    return pipe_launch(x8, w8, T, ldt, D, I, scale, wscale, amax, gu8, h8, h8t, ldt, nullptr, 0, (hipStream_t)stream);
   const Tiling tl = swiglu_tiling(ldt, I);  // the padding rows' zeros too
   const auto kern = tl.small ? swiglu_fwd_kernel<true> : swiglu_fwd_kernel<false>;
   const int rc = prep(kern, tl.lds);
@@ -2363,22 +2396,9 @@ int sfp8_moe_gemm_gateup_swiglu_fwd(const void* x8, const void* w8, int64_t E, i
   if (!x8 || !w8 || !plan || !scale || !q_gu || !amax || !gu8 || !h8) return kErrNullPointer;
   if (!moe_shape(E, D, I, ldp) || !fits32(ldp, D) || !fits32(2 * I, D) || !fits32(ldp, 2 * I)) return kErrBadShape;
   if (!al16(x8) || !al16(w8) || !al16(gu8) || !al16(h8) || !al16(h8t)) return kErrBadAlignment;
-  if (D == 1024) {
-    // the persistent kernel walks the plan's tiles (its count read on the
-    // device); the grid is sized for the worst case
-    const int tiles_m = (int)(ldp / kTile), tiles_n = (int)(I / 64);
-    const int ntiles = tiles_m * tiles_n;
-    int n_cu = 0;
-    int rc = cu_count(&n_cu);
-    if (rc) return rc;
-    rc = prep(swiglu_pipe_kernel<16, kPipeTB>, kPipeLds);
-    if (rc) return rc;
-    hipLaunchKernelGGL((swiglu_pipe_kernel<16, kPipeTB>), dim3(ntiles < n_cu ? ntiles : n_cu), dim3(kPipeThreads), kPipeLds,
-                       (hipStream_t)stream, (const uint8_t*)x8, (const uint8_t*)w8, ldp, D, I, scale, q_gu, amax,
-                       (uint8_t*)gu8, (uint8_t*)h8, (uint8_t*)h8t, ldp, tiles_m, tiles_n, plan,
-                       D * slab_rows(2 * I));
-    return status();
-  }
+  if (use_pipe(ldp, D, I))
+    return pipe_launch(x8, w8, ldp, ldp, D, I, scale, q_gu, amax, gu8, h8, h8t, ldp, plan, D * slab_rows(2 * I),
+                       (hipStream_t)stream);
   const Tiling tl = swiglu_tiling(ldp, I);
   const auto kern = tl.small ? swiglu_fwd_kernel<true> : swiglu_fwd_kernel<false>;
   const int rc = prep(kern, tl.lds);

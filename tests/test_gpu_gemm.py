@@ -405,11 +405,13 @@ def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
 
 
 # The SwiGLU forwards and the down dgrad run 128-row tiles up to 128 tiles of
-# 256 rows and again from 257 to 384: both sides of each line, with one row in
+# 256 rows and again from 257 to 384, the FP8 forward at D = 256, 512 and 1024
+# the persistent kernel from 640 tiles of 64 column pairs: both sides of each line, with one row in
 # the last tile of either shape (whose padding rows the K-slabs keep as zeros)
 # and columns that end inside one.
 @pytest.mark.parametrize("T,D,I", [(1, 128, 128), (129, 256, 384), (4099, 256, 256), (4097, 128, 1024),
-                                   (16385, 128, 256), (32768, 128, 384), (33025, 128, 384), (12289, 256, 1024)])
+                                   (16385, 128, 256), (32768, 128, 384), (33025, 128, 384), (12289, 256, 1024),
+                                   (9984, 256, 1024), (9985, 256, 1024), (5121, 512, 1920), (4097, 1024, 2560)])
 def test_tile_shapes_of_swiglu(dev, T, D, I):
     """FP8 forward and dgrad against the oracle's formulas on the device:
     integer operands make gate, up and dh exact; codes of h and of d_gu may
@@ -460,3 +462,34 @@ def test_tile_shapes_of_swiglu(dev, T, D, I):
     assert float((hb.float() - ref).norm() / ref.norm().clamp(min=1e-30)) < 2 ** -8  # one bf16 rounding
     for a, b in zip(sg.ops.bf16_swiglu_fwd(xb, ws, I, rstd=ones, xs=xs), (gub, hb)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,D,I", [(16384, 256, 1024), (10241, 512, 1152), (4099, 1024, 2688)])
+def test_persistent_swiglu_exact_path(dev, T, D, I):
+    """Rows are independent: NaN, saturating and ordinary rows through the
+    persistent kernel (several tiles per work-group) have the bytes that the
+    one-tile kernel gives each of them in a batch of a few hundred rows, and
+    the maxima are the larger of the batches'."""
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    x8 = torch.randint(-8, 9, (T, D), generator=g, device=dev).float().to(E4)
+    x8.view(torch.uint8)[::97, 3] = 0x7F          # NaN rows
+    x8[5::89] = (x8[5::89].float() * 32).to(E4)   # rows beyond the e4m3 range of gu and h
+    w8 = torch.randint(-8, 9, (2 * I, D), generator=g, device=dev).float().to(E4)
+    s = torch.tensor([1.0, 2.0 ** -4, 2.0 ** -8, 1, 1], device=dev)
+    ws, ws8 = torch.ones(2, device=dev), sg.ops.to_slab(w8)
+
+    def run(x):
+        n = x.shape[0]
+        ldt = sg.ops.ldt_of(n)
+        amax = torch.zeros(5, device=dev)
+        pad = torch.zeros(ldt - n, D, device=dev).to(E4)
+        gu8, h8, _ = sg.ops.gateup_swiglu_fwd(sg.ops.to_slab(torch.cat([x, pad])), ws8, s, ws, amax, n, I, copy=False)
+        return u8(sg.ops.unslab(gu8, n)), u8(sg.ops.unslab(h8, n)), amax
+
+    gu, h, amax = run(x8)
+    most = torch.zeros(5, device=dev)
+    for i in range(0, T, 512):
+        a, b, m = run(x8[i:i + 512])
+        assert torch.equal(a, gu[i:i + 512]) and torch.equal(b, h[i:i + 512])
+        most = torch.maximum(most, m)
+    assert torch.equal(most, amax) and amax[1] > 0 and amax[2] > 0
