@@ -1839,6 +1839,375 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   }
 }
 
+// The bf16 gate/up forward, persistent, with the SwiGLU of each tile under the
+// K loop of the next, after swiglu_pipe_kernel: tiles of 256 rows x 64 (gate,
+// up) column pairs, 8 waves of 64 x 64, one work-group per CU.  At K = 16
+// stages (D = 512) the one-tile kernel spends as long writing its 6 bytes per
+// pair as in its K loop, each with the other idle.
+//
+// At a tile's end a lane packs bf16(g * rs), bf16(u * rs) of its 32 pairs into
+// 32 registers (rs = rstd of the row, brought to LDS by DMA with the tile's
+// first stages); the next tile's first KE stages run the 8 units of 4 pairs in
+// six pieces each.  A unit leaves its gate and up words in place of the pairs
+// and two h words; a finished row block goes to LDS and, in the next stage,
+// out as whole 128-byte rows.  (Stored from the registers, 32 contiguous bytes
+// of each row per instruction, the stores took as long as the rest: 224
+// against 149 us without them.)  Stages past KE have a plain loop of four, so
+// D is any multiple of 128 from 32 KE on.  Operands, plan and rounding as
+// bf16_swiglu_fwd_kernel.
+template <int KE, bool EXACT>
+struct Bf16Pipe {
+  using ML = MainLoop<true, 0, 0, true, 2, kStages, 0, false, false, 2, 2>;
+  static constexpr int kUnits = 8, kPre = 2, kSlots = ML::kMfma - kPre;
+  // the pieces fill the slots of stages 0 .. KE - 2; a row block staged at the
+  // end of a stage is written in the next
+  static constexpr int kAllSlots = (KE - 1) * kSlots, kPieces = 6 * kUnits;
+  static constexpr int first_piece(int slot) { return slot < kAllSlots ? slot * kPieces / kAllSlots : kPieces; }
+  static constexpr int blocks_done(int kt) { return first_piece((kt + 1) * kSlots) / 24; }
+  static constexpr int kRow = 144, kOut = 128 * kRow;  // staging: row stride, bytes per output
+  static constexpr int kWrites = 6;  // stores per thread of a row block: 128 rows x 8 pieces x 3 outputs
+  // the row block written in stage kt, or -1
+  static constexpr int written(int kt) { return kt > 0 && blocks_done(kt - 1) > blocks_done(kt - 2) ? blocks_done(kt - 1) - 1 : -1; }
+
+  struct Ctx {
+    uint8_t* lds;
+    uint8_t* stg;  // staging rows
+    intx4 rv;      // the piece read last
+    __amdgpu_buffer_rsrc_t ra, rb, nra, nrb;  // this tile's operands and the next's (no records: none)
+    uint32_t voff_a[4], voff_b[2], aoff[8], boff[8];
+    int nk, a_ss, b_ss, wave;
+    typename ML::Frag f[2];
+    floatx16 acc[2][2];
+    // the previous tile's epilogue
+    uint32_t E[2][16], hw[8];
+    float gb[4], ub[4], hb[4], ex[4], sg[4];
+    __amdgpu_buffer_rsrc_t rgu, rh;  // its outputs from its first row (no records: no previous tile)
+    int so_g, so_u, so_h;            // its first column's byte offsets
+    int ld_gu, ld_h;                 // bytes per output row
+  };
+
+  template <int RB, int Q, int I>
+  static SFP8_DEV void unpack(Ctx& c) {
+    uint32_t p = c.E[RB][4 * Q + I];
+    asm volatile("" : "+v"(p));
+    c.gb[I] = __uint_as_float(p << 16);
+    c.ub[I] = __uint_as_float(p & 0xffff0000u);
+    c.ex[I] = __builtin_amdgcn_exp2f(c.gb[I] * -1.4426950408889634f);
+  }
+  // Piece P of unit U, kept in its slot by empty asm statements as in
+  // SwigluPipe::unit_piece.
+  template <int U, int P>
+  static SFP8_DEV void unit_piece(Ctx& c) {
+    constexpr int RB = U / 4, Q = U % 4;
+    if constexpr (P == 0) {
+      unpack<RB, Q, 0>(c);
+      unpack<RB, Q, 1>(c);
+      asm volatile("" ::"v"(c.ex[0]), "v"(c.ex[1]));
+    } else if constexpr (P == 1) {
+      c.sg[0] = __builtin_amdgcn_rcpf(1.0f + c.ex[0]);
+      c.sg[1] = __builtin_amdgcn_rcpf(1.0f + c.ex[1]);
+      unpack<RB, Q, 2>(c);
+      asm volatile("" ::"v"(c.sg[0]), "v"(c.sg[1]), "v"(c.ex[2]));
+    } else if constexpr (P == 2) {
+      unpack<RB, Q, 3>(c);
+      c.sg[2] = __builtin_amdgcn_rcpf(1.0f + c.ex[2]);
+      c.hb[0] = c.gb[0] * c.sg[0] * c.ub[0];
+      c.hb[1] = c.gb[1] * c.sg[1] * c.ub[1];
+      asm volatile("" ::"v"(c.ex[3]), "v"(c.sg[2]), "v"(c.hb[0]), "v"(c.hb[1]));
+    } else if constexpr (P == 3) {
+      c.sg[3] = __builtin_amdgcn_rcpf(1.0f + c.ex[3]);
+      c.hb[2] = c.gb[2] * c.sg[2] * c.ub[2];
+      c.hw[2 * Q] = pack2_bf16(c.hb[0], c.hb[1]);
+      asm volatile("" ::"v"(c.sg[3]), "v"(c.hb[2]), "v"(c.hw[2 * Q]));
+    } else if constexpr (P == 4) {
+      c.hb[3] = c.gb[3] * c.sg[3] * c.ub[3];
+      c.hw[2 * Q + 1] = pack2_bf16(c.hb[2], c.hb[3]);
+      asm volatile("" ::"v"(c.hw[2 * Q + 1]));
+    } else {
+      // four pairs -> two gate words, two up words
+      const uint32_t e0 = c.E[RB][4 * Q], e1 = c.E[RB][4 * Q + 1], e2 = c.E[RB][4 * Q + 2], e3 = c.E[RB][4 * Q + 3];
+      c.E[RB][4 * Q] = __builtin_amdgcn_perm(e1, e0, 0x05040100u);
+      c.E[RB][4 * Q + 1] = __builtin_amdgcn_perm(e3, e2, 0x05040100u);
+      c.E[RB][4 * Q + 2] = __builtin_amdgcn_perm(e1, e0, 0x07060302u);
+      c.E[RB][4 * Q + 3] = __builtin_amdgcn_perm(e3, e2, 0x07060302u);
+      asm volatile("" ::"v"(c.E[RB][4 * Q]), "v"(c.E[RB][4 * Q + 1]), "v"(c.E[RB][4 * Q + 2]),
+                   "v"(c.E[RB][4 * Q + 3]));
+    }
+  }
+  template <int P, int END>
+  static SFP8_DEV void pieces(Ctx& c) {
+    if constexpr (P < END) {
+      unit_piece<P / 6, P % 6>(c);
+      pieces<P + 1, END>(c);
+    }
+  }
+
+  // Row block RB of the previous tile (128 rows: 32 of each wave row) into the
+  // staging rows: gate, up, h, each 64 columns.
+  template <int RB>
+  static SFP8_DEV void block_stage(Ctx& c) {
+    const int lane = threadIdx.x & 63, wm = c.wave % ML::kWM, wn = c.wave / ML::kWM;
+    uint8_t* p = c.stg + (32 * wm + (lane & 31)) * kRow + 64 * wn + 32 * (lane >> 5);
+    uint32_t(&E)[16] = c.E[RB];
+    store16(p, {E[0], E[1], E[4], E[5]});
+    store16(p + 16, {E[8], E[9], E[12], E[13]});
+    store16(p + kOut, {E[2], E[3], E[6], E[7]});
+    store16(p + kOut + 16, {E[10], E[11], E[14], E[15]});
+    store16(p + 2 * kOut, {c.hw[0], c.hw[1], c.hw[2], c.hw[3]});
+    store16(p + 2 * kOut + 16, {c.hw[4], c.hw[5], c.hw[6], c.hw[7]});
+  }
+  // Piece K of this thread of the staged row block RB: read, and stored as part
+  // of a whole 128-byte row.  Rows past the tile's last lie past the
+  // descriptors' records and are dropped (so are all when there is no previous
+  // tile).
+  template <int K>
+  static SFP8_DEV intx4 row_read(const Ctx& c) {
+    const int tid = threadIdx.x;
+    return *reinterpret_cast<const intx4*>(c.stg + (K / 2) * kOut + ((tid >> 3) + 64 * (K & 1)) * kRow + 16 * (tid & 7));
+  }
+  template <int RB, int K>
+  static SFP8_DEV void row_write(const Ctx& c, const intx4& v) {
+    const int tid = threadIdx.x, sr = (tid >> 3) + 64 * (K & 1);
+    const int row = 64 * (sr >> 5) + 32 * RB + (sr & 31);
+    // the column goes in the vector offset: with a scalar register there the
+    // compiler sees no hazard in a vector instruction that overwrites the data
+    // right after the store, and such stores wrote that instruction's result
+    const uint32_t vo = (uint32_t)(row * (K < 4 ? c.ld_gu : c.ld_h) + 16 * (tid & 7)) +
+                        (uint32_t)(K < 2 ? c.so_g : K < 4 ? c.so_u : c.so_h);
+    __builtin_amdgcn_raw_buffer_store_b128(v, K < 4 ? c.rgu : c.rh, vo, 0, 0);
+  }
+
+  // One stage: kPre MFMAs, the wait for the next stage's DMA and the barrier,
+  // then a slot per MFMA with the DMA (instruction j of stage kt + 3, or of
+  // stage NEXT of the next tile), the fragment reads (those the next stage
+  // starts with first) and, in the first KE stages, the pieces.
+  // PH = stage % 4; KT = the stage, or -1 past KE; PREV = the stage before, if
+  // it may be one that writes
+  template <int PH, int KT, int NEXT, int PREV = KT - 1>
+  static SFP8_DEV void stage(Ctx& c, int kt) {
+    static_assert(kSlots == kWrites, "a piece per slot");
+    ML::template mfma_range<0, kPre>(c.f[PH & 1], c.acc);
+    __builtin_amdgcn_sched_barrier(0);
+    // what the stage before issued may still fly: its DMA and, after a write
+    // stage, its stores; block_stage's LDS writes must have landed
+    constexpr int kFly = ML::kDma + (PREV >= 0 && written(PREV) >= 0 ? kWrites : 0);
+    if constexpr (KT >= 0 && written(KT) >= 0)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFly) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kFly) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    slots<PH, KT, NEXT, 0>(c, kt);
+    if constexpr (KT >= 0) {
+      if constexpr (written(KT) >= 0) row_write<written(KT), kSlots - 1>(c, c.rv);
+      if constexpr (blocks_done(KT) > blocks_done(KT - 1)) block_stage<blocks_done(KT) - 1>(c);
+    }
+  }
+  template <int PH, int KT, int NEXT, int J>
+  static SFP8_DEV void slots(Ctx& c, int kt) {
+    if constexpr (J < kSlots) {
+      ML::template mfma_range<kPre + J, kPre + J + 1>(c.f[PH & 1], c.acc);
+#pragma unroll
+      for (int j = J * ML::kDma / kSlots; j < (J + 1) * ML::kDma / kSlots; ++j) {
+        const int s = NEXT >= 0 ? NEXT : kt + kStages - 1;
+        int ass = c.a_ss, bss = c.b_ss;
+        asm volatile("" : "+s"(ass), "+s"(bss));  // the products are made here, not kept for every stage
+        ML::load_one(j, c.lds, (PH + 3) % kStages, NEXT >= 0 ? c.nra : c.ra, NEXT >= 0 ? c.nrb : c.rb, c.voff_a,
+                     c.voff_b, s * ass, s * bss, c.wave);
+      }
+      if constexpr (J == 0) {
+        ML::template read_frag<0>(c.lds, (PH + 1) % kStages, c.aoff, c.boff, c.f[(PH & 1) ^ 1]);
+        ML::template read_frag<2>(c.lds, (PH + 1) % kStages, c.aoff, c.boff, c.f[(PH & 1) ^ 1]);
+      } else if constexpr (J < 3) {
+        ML::template read_frag<J == 1 ? 3 : 1>(c.lds, (PH + 1) % kStages, c.aoff, c.boff, c.f[(PH & 1) ^ 1]);
+      }
+      if constexpr (KT >= 0) {
+        if constexpr (written(KT) >= 0) {  // each piece stored a slot after it is read
+          if constexpr (J > 0) row_write<written(KT), J - 1>(c, c.rv);
+          c.rv = row_read<J>(c);
+        }
+        pieces<first_piece(KT * kSlots + J), first_piece(KT * kSlots + J + 1)>(c);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      slots<PH, KT, NEXT, J + 1>(c, kt);
+    }
+  }
+  // Stages KT .. KE - 1; EXACT: the tile has no others, so the last three
+  // load the next tile's first.
+  template <int KT>
+  static SFP8_DEV void stages(Ctx& c) {
+    if constexpr (KT < KE) {
+      stage<KT % kStages, KT, (EXACT ? KT + kStages - 1 - KE : -1)>(c, KT);
+      stages<KT + 1>(c);
+    }
+  }
+  static SFP8_DEV void rest(Ctx& c) {
+    int kt = KE;
+    // (the first of these follows a write stage; waiting for the stores there
+    // too keeps one loop body)
+    for (; kt < c.nk - 4; kt += 4) {
+      stage<0, -1, -1>(c, kt);
+      stage<1, -1, -1>(c, kt + 1);
+      stage<2, -1, -1>(c, kt + 2);
+      stage<3, -1, -1>(c, kt + 3);
+    }
+    stage<0, -1, -1>(c, kt);
+    stage<1, -1, 0>(c, kt + 1);
+    stage<2, -1, 1>(c, kt + 2);
+    stage<3, -1, 2>(c, kt + 3);
+  }
+  template <int RB, int K = 0>
+  static SFP8_DEV void write_all(Ctx& c) {
+    if constexpr (K < kWrites) {
+      row_write<RB, K>(c, row_read<K>(c));
+      write_all<RB, K + 1>(c);
+    }
+  }
+  static SFP8_DEV void tail(Ctx& c) {
+    pieces<0, kPieces / 2>(c);
+    block_stage<0>(c);
+    __syncthreads();
+    write_all<0>(c);
+    pieces<kPieces / 2, kPieces>(c);
+    __syncthreads();
+    block_stage<1>(c);
+    __syncthreads();
+    write_all<1>(c);
+  }
+};
+// the ring, three slots of rstd, the staging rows
+constexpr int kBf16PipeRing = Bf16Pipe<8, true>::ML::kLds;
+constexpr int kBf16PipeStg = kBf16PipeRing + 3 * kTile * 4;
+constexpr int kBf16PipeLds = kBf16PipeStg + 3 * Bf16Pipe<8, true>::kOut;
+static_assert(kBf16PipeLds <= 160 * 1024, "fits the LDS");
+
+template <int KE, bool EXACT>
+__global__ __launch_bounds__(512, 1) void bf16_swiglu_pipe_kernel(
+    const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, int64_t T, int64_t D, int64_t I,
+    const float* __restrict__ rstd, uint16_t* __restrict__ gu, uint16_t* __restrict__ h, int tiles_m, int tiles_n,
+    const int* __restrict__ plan, int64_t w_estride, int64_t ldxs) {
+  using P = Bf16Pipe<KE, EXACT>;
+  using ML = typename P::ML;
+  extern __shared__ __align__(16) uint8_t lds[];
+  typename P::Ctx c;
+  c.lds = lds;
+  c.stg = lds + kBf16PipeStg;
+  c.wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wm = c.wave % ML::kWM, wn = c.wave / ML::kWM;
+  const int fr = lane & 31, g = lane >> 5;
+  const uint32_t chunk = (uint32_t)(((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  const int sw = (fr >> 2) & 3;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    c.aoff[k] = (uint32_t)((64 * wm + fr) * kStage + (((2 * g + k) ^ sw) << 4));
+    c.boff[k] = (uint32_t)(ML::kLdsB + (BLayout<true, 2>::kWaveStride * wn + fr) * kStage + (((2 * g + k) ^ sw) << 4));
+  }
+  const bool xslab = ldxs > 0;
+  const int64_t ldx = D * 2, wr = slab_rows(2 * I);
+  c.nk = (int)(ldx / kStage);
+  c.a_ss = xslab ? (int)(ldxs * kStage) : kStage;
+  c.b_ss = (int)(wr * kStage);
+  c.ld_gu = (int)(4 * I);
+  c.ld_h = (int)(2 * I);
+#pragma unroll
+  for (int j = 0; j < ML::kDmaA; ++j) {
+    const int r = (kTile / ML::kWaves) * c.wave + 16 * j + (lane >> 2);
+    c.voff_a[j] = (uint32_t)(r * (xslab ? kStage : (int)ldx)) + chunk;
+  }
+#pragma unroll
+  for (int j = 0; j < ML::kDmaB; ++j) {
+    const int r = (128 / ML::kWaves) * c.wave + 16 * j + (lane >> 2);
+    c.voff_b[j] = (uint32_t)(((r >> 6) * (int)I + paired_col64(r)) * kStage) + chunk;
+  }
+  if (plan) tiles_m = MoePlan{plan}.ntiles();
+  const int ntiles = tiles_m * tiles_n;
+  // tile -> its first row, rows and first column, and its operands
+  auto tile_of = [&](int tile, int64_t& r0, int64_t& nrows, int64_t& n0, __amdgpu_buffer_rsrc_t& ra,
+                     __amdgpu_buffer_rsrc_t& rb) {
+    int tm, tn;
+    tile_coords(tile, ntiles, tiles_m, tiles_n, tm, tn);
+    r0 = (int64_t)tm * kTile;
+    nrows = T - r0;
+    const uint8_t* wb = w;
+    if (plan) {
+      const MoePlan M{plan};
+      r0 = M.urow(tm);
+      nrows = M.rows(tm);
+      wb += M.expert(tm) * w_estride;
+    }
+    n0 = (int64_t)tn * 64;
+    ra = make_rsrc(reinterpret_cast<const uint8_t*>(x) + r0 * (xslab ? kStage : ldx),
+                   xslab ? ldx * ldxs - r0 * kStage : nrows * ldx);
+    rb = make_rsrc(wb + n0 * kStage, ldx * wr - n0 * kStage);
+  };
+  // rstd of the 256 rows from r0 into LDS slot `slot` (rows past T read as
+  // zero; every wave brings the same 1 KiB, so that its waits count it).  Three
+  // slots: while a wave requests the next tile's, another may still read the
+  // previous tile's.
+  auto load_rstd = [&](int64_t r0, int slot) {
+    if (rstd)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(rstd + r0, (T - r0) * 4),
+                                               (lds_ptr_t)(lds + kBf16PipeRing + slot * kTile * 4), 16,
+                                               (uint32_t)(lane * 16), 0, 0, 0);
+  };
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) c.E[tb][v] = 0u;
+  c.rgu = make_rsrc(gu, 0);  // no previous tile: its stores are dropped
+  c.rh = make_rsrc(h, 0);
+  c.so_g = c.so_u = c.so_h = 0;
+  int64_t r0 = 0, nrows = 0, n0 = 0;
+  int it = 0;
+  if ((int)blockIdx.x < ntiles) {
+    tile_of(blockIdx.x, r0, nrows, n0, c.ra, c.rb);
+    load_rstd(r0, 0);
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      ML::load_stage(lds, s, c.ra, c.rb, c.voff_a, c.voff_b, s * c.a_ss, s * c.b_ss, c.wave);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * ML::kDma) : "memory");
+    ML::read_frags(lds, 0, c.aoff, c.boff, c.f[0]);
+  }
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x, ++it) {
+    int64_t nr0 = 0, nnrows = 0, nn0 = 0;
+    const bool has_next = tile + (int)gridDim.x < ntiles;
+    if (has_next) {
+      tile_of(tile + (int)gridDim.x, nr0, nnrows, nn0, c.nra, c.nrb);
+      load_rstd(nr0, (it + 1) % 3);
+    } else {  // no records: the stages past the last read nothing
+      c.nra = make_rsrc(x, 0);
+      c.nrb = make_rsrc(w, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) c.acc[i][j] = floatx16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                                                          0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    P::template stages<0>(c);
+    if constexpr (!EXACT) P::rest(c);
+    // this tile's g, u times rstd (bf16) become the next epilogue's input; its
+    // rstd landed with its first stages, many barriers ago
+    const float* rs = reinterpret_cast<const float*>(lds + kBf16PipeRing + (it % 3) * kTile * 4);
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+      const float s = rstd ? rs[64 * wm + 32 * tb + fr] : 1.0f;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) c.E[tb][v] = pack2_bf16(c.acc[tb][0][v] * s, c.acc[tb][1][v] * s);
+    }
+    c.rgu = make_rsrc(gu + r0 * 2 * I, nrows * 4 * I);
+    c.rh = make_rsrc(h + r0 * I, nrows * 2 * I);
+    c.so_g = (int)(n0 * 2);
+    c.so_u = (int)((I + n0) * 2);
+    c.so_h = (int)(n0 * 2);
+    r0 = nr0;
+    nrows = nnrows;
+    n0 = nn0;
+    c.ra = c.nra;
+    c.rb = c.nrb;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (it) P::tail(c);
+}
+
 // out[u, n] = bf16(sum_k A[m, k] * B[n, k]) with A a bf16 K-slab over lda
 // rows (Kb bytes of K) and B a bf16 K-slab [Kb/64][slab_rows(N)][64]: the
 // dgrad of the SwiGLU path (_swiglu_dgrad_kernel, train.py:1907-1980, its
@@ -2523,8 +2892,38 @@ inline bool bf16_shape(int64_t D, int64_t I) {
   return D > 0 && I > 0 && D % 64 == 0 && I % 64 == 0 && fits32(kTile, 4 * I);
 }
 
+// Whether the bf16 gate/up forward runs the persistent kernel: from 640 tiles
+// of 64 column pairs on (2.5 per CU) and up to the width where its K loop,
+// which reads a third more LDS per FLOP than 256 x 256 tiles, loses more than
+// the hidden epilogue gains.  Measured (us, one tile per work-group ->
+// persistent, reading the row K-slab): D = 256 39 -> 33 at 1024 tiles (21 ->
+// 21 at 512), 155 -> 128 at 4096; D = 512 40 -> 35 at 768, 225 -> 190 at 4608;
+// D = 640 98 -> 82 at 1728; D = 768 42 -> 41 at 544, 362 -> 337 at 6144; D =
+// 1024 201 -> 225 at 3072.  Reading row-major rows (half lines per K stage):
+// D = 640 99 -> 86, D = 768 117 -> 120.  Widths of whole 4-stage rings only.
+inline bool use_bf16_pipe(int64_t rows, int64_t D, int64_t I, bool slab) {
+  return D % 128 == 0 && D >= 256 && D <= (slab ? 768 : 640) &&
+         (int64_t)cdiv(rows, kTile) * (I / 64) >= 5 * kCUs / 2;
+}
+
 int bf16_swiglu_launch(const void* x, const void* w, int64_t T, int64_t D, int64_t I, const float* rstd, void* gu,
                        void* h, const int* plan, int64_t ldp, int64_t ldxs, hipStream_t st) {
+  if (use_bf16_pipe(plan ? ldp : T, D, I, ldxs > 0)) {
+    const auto kern = D == 256   ? bf16_swiglu_pipe_kernel<8, true>
+                      : D == 384 ? bf16_swiglu_pipe_kernel<8, false>
+                      : D == 512 ? bf16_swiglu_pipe_kernel<16, true>
+                                 : bf16_swiglu_pipe_kernel<16, false>;
+    const int tiles_m = cdiv(plan ? ldp : T, kTile), tiles_n = (int)(I / 64), ntiles = tiles_m * tiles_n;
+    int n_cu = 0;
+    int rc = cu_count(&n_cu);
+    if (rc) return rc;
+    rc = prep(kern, kBf16PipeLds);
+    if (rc) return rc;
+    hipLaunchKernelGGL(kern, dim3(ntiles < n_cu ? ntiles : n_cu), dim3(512), kBf16PipeLds, st, (const uint16_t*)x,
+                       (const uint8_t*)w, T, D, I, rstd, (uint16_t*)gu, (uint16_t*)h, tiles_m, tiles_n, plan,
+                       plan ? 2 * D * slab_rows(2 * I) : 0, ldxs);
+    return status();
+  }
   const Tiling tl = swiglu_tiling(plan ? ldp : T, I);
   const auto kern = tl.small ? bf16_swiglu_fwd_kernel<true> : bf16_swiglu_fwd_kernel<false>;
   const int rc = prep(kern, tl.lds);

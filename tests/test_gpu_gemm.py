@@ -405,13 +405,14 @@ def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
 
 
 # The SwiGLU forwards and the down dgrad run 128-row tiles up to 128 tiles of
-# 256 rows and again from 257 to 384, the FP8 forward at D = 256, 512 and 1024
-# the persistent kernel from 640 tiles of 64 column pairs: both sides of each line, with one row in
+# 256 rows and again from 257 to 384, the forwards at some widths
+# persistent kernels from 640 tiles of 64 column pairs: both sides of each line, with one row in
 # the last tile of either shape (whose padding rows the K-slabs keep as zeros)
 # and columns that end inside one.
 @pytest.mark.parametrize("T,D,I", [(1, 128, 128), (129, 256, 384), (4099, 256, 256), (4097, 128, 1024),
                                    (16385, 128, 256), (32768, 128, 384), (33025, 128, 384), (12289, 256, 1024),
-                                   (9984, 256, 1024), (9985, 256, 1024), (5121, 512, 1920), (4097, 1024, 2560)])
+                                   (9984, 256, 1024), (9985, 256, 1024), (5121, 512, 1920), (5121, 512, 2048),
+                                   (5121, 384, 2048), (5121, 640, 2048), (5121, 768, 2048), (4097, 1024, 2560)])
 def test_tile_shapes_of_swiglu(dev, T, D, I):
     """FP8 forward and dgrad against the oracle's formulas on the device:
     integer operands make gate, up and dh exact; codes of h and of d_gu may
@@ -462,6 +463,33 @@ def test_tile_shapes_of_swiglu(dev, T, D, I):
     assert float((hb.float() - ref).norm() / ref.norm().clamp(min=1e-30)) < 2 ** -8  # one bf16 rounding
     for a, b in zip(sg.ops.bf16_swiglu_fwd(xb, ws, I, rstd=ones, xs=xs), (gub, hb)):
         assert torch.equal(a, b)
+    pow2 = 2.0 ** torch.randint(-3, 4, (T,), generator=g, device=dev).float()  # rows scaled exactly
+    gub, hb = sg.ops.bf16_swiglu_fwd(xb, ws, I, rstd=pow2, xs=xs)
+    assert torch.equal(gub.float(), gu * pow2[:, None])
+    gate, up = gub.float().chunk(2, dim=1)
+    ref = gate * torch.sigmoid(gate) * up
+    assert float((hb.float() - ref).norm() / ref.norm().clamp(min=1e-30)) < 2 ** -8
+
+
+@pytest.mark.parametrize("D", [256, 512, 640])
+def test_persistent_bf16_swiglu_grouped(dev, D):
+    """The grouped bf16 forward on the persistent kernel has, for each
+    expert's rows, the bytes of the dense forward of those rows alone (the
+    one-tile kernel): ragged, full-tile, single-row and empty experts."""
+    counts, I = [3000, 0, 1, 2049, 256, 700], 1536
+    E, R = len(counts), sum(counts)
+    g = torch.Generator(device=dev).manual_seed(D)
+    x = torch.randn(R, D, generator=g, device=dev).bfloat16()
+    w = (torch.randn(E, 2 * I, D, generator=g, device=dev) * D ** -0.5).bfloat16()
+    plan = sg.ops.moe_plan(torch.cumsum(torch.tensor(counts), 0).to(torch.int32).to(dev), R)
+    ws, _ = sg.ops.bf16_weight_slabs(w, transposed=False)
+    gu, h = sg.ops.bf16_swiglu_fwd(x, ws, I, plan=plan, ldp=sg.ops.moe_padded_rows(R, E))
+    row = 0
+    for e, c in enumerate(counts):
+        if c:
+            a, b = sg.ops.bf16_swiglu_fwd(x[row:row + c].contiguous(), ws[e:e + 1], I)
+            assert torch.equal(gu[row:row + c], a) and torch.equal(h[row:row + c], b)
+        row += c
 
 
 @pytest.mark.parametrize("T,D,I", [(16384, 256, 1024), (10241, 512, 1152), (4099, 1024, 2688)])
