@@ -381,6 +381,12 @@ int sfp8_bf16_rows_prep(const void* x, int64_t nsrc, int64_t D, const int* plan,
 int sfp8_bf16_gemm_swiglu_fwd(const void* x, int x_slab, const void* w, int64_t T, int64_t D, int64_t I,
                               const float* rstd, void* gu, void* h, void* stream);
 
+/* The dense gate/up forward for evaluation, when no gradient will be taken:
+ * h [T, I] = bf16(g * sigmoid(g) * u), g, u = bf16(x W^T) with x [T, D] and
+ * W [2I, D] (gate rows first) both row-major bf16 as the caller has them;
+ * nothing else is written. */
+int sfp8_bf16_swiglu_eval(const void* x, const void* w, int64_t T, int64_t D, int64_t I, void* h, void* stream);
+
 /* The same grouped (E experts, _FusedSwiGLU with several groups): x, gu, h
  * in expert order, w the stacked per-expert K-slabs. */
 int sfp8_bf16_moe_gemm_swiglu_fwd(const void* x, const void* w, int64_t E, int64_t D, int64_t I, const int* plan,

@@ -59,6 +59,7 @@ SIGNATURES = {
     "sfp8_bf16_weight_slabs": (_INT, [_P, _INT, _P, _I64, _I64, _I64, _P, _P, _P]),
     "sfp8_bf16_rows_prep": (_INT, [_P, _I64, _I64, _P, _I64, _F32, _P, _P, _P, _P]),
     "sfp8_bf16_gemm_swiglu_fwd": (_INT, [_P, _INT, _P, _I64, _I64, _I64, _P, _P, _P, _P]),
+    "sfp8_bf16_swiglu_eval": (_INT, [_P, _P, _I64, _I64, _I64, _P, _P]),
     "sfp8_bf16_moe_gemm_swiglu_fwd": (_INT, [_P, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P]),
     "sfp8_bf16_swiglu_bwd": (_INT, [_P, _P, _I64, _I64, _P, _P, _I64, _P, _P, _P]),
     "sfp8_bf16_gemm": (_INT, [_P, _P, _I64, _I64, _I64, _I64, _P, _P]),

@@ -1734,11 +1734,13 @@ constexpr int kGuStride = SMALL ? 144 : 272;
 // 8 waves (two per SIMD): wave (wm, wn) owns tile rows 128*wm.. and one
 // 32-column block of gate and one of up, columns 32*wn.. of each half.
 // SMALL: 128 rows x 64 columns by 4 waves of 64 rows, staged in one pass.
+// w_rows: W is row-major [2I, D] bf16 as the caller has it instead of its
+// K-slab; gu may be null (evaluation: nothing is saved).
 template <bool SMALL>
 __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void bf16_swiglu_fwd_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w, int64_t T, int64_t D, int64_t I,
     const float* __restrict__ rstd, uint16_t* __restrict__ gu, uint16_t* __restrict__ h, int tiles_m, int tiles_n,
-    const int* __restrict__ plan, int64_t w_estride, int64_t ldxs) {
+    const int* __restrict__ plan, int64_t w_estride, int64_t ldxs, int w_rows) {
   using TS = TileShape<SMALL>;
   constexpr int kN = TS::kM / 2;  // (gate, up) columns of a tile
   constexpr int kGs = kGuStride<SMALL>;
@@ -1759,7 +1761,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   const int64_t ldx = D * 2;  // bytes per x row = K bytes
   const int64_t wr = slab_rows(2 * I);
   // the outputs from the tile's first row (gu [rows, 2I], h [rows, I], bf16)
-  const __amdgpu_buffer_rsrc_t rgu = make_rsrc(gu + r0 * 2 * I, nrows * 4 * I);
+  const __amdgpu_buffer_rsrc_t rgu = make_rsrc(gu + r0 * 2 * I, gu ? nrows * 4 * I : 0);
   const __amdgpu_buffer_rsrc_t rho = make_rsrc(h + r0 * I, nrows * 2 * I);
   floatx16 acc[TS::kTB][2];  // [tb][0] gate, [tb][1] up
   // A: x row-major [T, D] (rows past the tile's last read as zero through
@@ -1770,10 +1772,10 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   TS::template Loop<true, 0, 0, false, false, true>::run(
       lds, reinterpret_cast<const uint8_t*>(x) + r0 * (xslab ? kStage : ldx),
       xslab ? ldx * ldxs - r0 * kStage : nrows * ldx, [=](int r) { return r * (xslab ? kStage : (int)ldx); },
-      xslab ? (int)(ldxs * kStage) : kStage, w, ldx * wr, [=](int r) {
-        return ((r / kN) * (int)I + (int)n0 + (SMALL ? paired_col64(r) : paired_col8(r))) * kStage;
+      xslab ? (int)(ldxs * kStage) : kStage, w, ldx * (w_rows ? 2 * I : wr), [=](int r) {
+        return ((r / kN) * (int)I + (int)n0 + (SMALL ? paired_col64(r) : paired_col8(r))) * (w_rows ? (int)ldx : kStage);
       },
-      (int)(wr * kStage), (int)(ldx / kStage), acc);
+      w_rows ? kStage : (int)(wr * kStage), (int)(ldx / kStage), acc);
   // Epilogue in two passes (SMALL: one) of 128 tile rows: pass P takes the
   // lanes' row blocks tb = 2P, 2P+1 (tile row 32 kTB wm + 64 P + 32 (tb & 1) +
   // fr, staging row 64 wm + 32 (tb & 1) + fr), stages g, u and h as bf16 rows in LDS,
@@ -1829,14 +1831,102 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
       const uint32_t in = 0u - (uint32_t)(lr < nrows && col < I);
       const uint32_t og = ((uint32_t)((lr * 2 * I + col) * 2) & in) | (~in & 0x80000000u);
       const uint32_t oh = ((uint32_t)((lr * I + col) * 2) & in) | (~in & 0x80000000u);
-      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Gs + sr * kGs + 16 * c), rgu,
-                                             og, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Us + sr * kGs + 16 * c), rgu,
-                                             og + (uint32_t)(2 * I), 0, 0);
+      if (gu) {  // uniform
+        __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Gs + sr * kGs + 16 * c), rgu,
+                                               og, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Us + sr * kGs + 16 * c), rgu,
+                                               og + (uint32_t)(2 * I), 0, 0);
+      }
       __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const intx4*>(Hs + sr * kGs + 16 * c), rho,
                                              oh, 0, 0);
     }
   }
+}
+
+// Evaluation of a few rows (generation): h = bf16(g * sigmoid(g) * u), g, u =
+// bf16(x W^T), for up to 64 rows of x and W row-major [2I, D] bf16 as the
+// caller has it.  The call reads W once and little else, so it is bound by the
+// memory's bandwidth and latency: a work-group of 8 waves takes 16 gate and
+// the 16 up rows of W, the waves share K (wave w the 32-wide K steps w, w + 8,
+// ...), and each requests several steps' rows before it uses any.  The MFMA's
+// A operand is W (16 rows), its B operand 16 rows of x, so a lane ends with
+// four consecutive columns of one row of x; the waves' sums are added through
+// LDS in wave order.  NT = 16-row tiles of x; rows past T repeat the last and
+// are not written.  Measured (us, laying W out as K-slabs and the tiled kernel
+// -> this one): D = 1024, I = 3072, 8 rows 19 -> 4.4 (2.9 TB/s), 64 rows 19 ->
+// 7.8; D = 2048, I = 8192, 8 rows 41 -> 12.6 (5.3 TB/s).  From 65 rows on the
+// tiled kernel with row-major W takes over: 10.3 at 65, D = 1024 (and no slower
+// than on K-slabs: 29 against 32 at 2017 rows).
+constexpr int kEvalRows = 64;  // most rows of x
+template <int NT>
+__global__ __launch_bounds__(512) void bf16_swiglu_eval_kernel(const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ w, int T, int D, int I,
+                                                               uint16_t* __restrict__ h) {
+  constexpr int kU = NT == 1 ? 4 : 2;  // K steps requested at once
+  __shared__ floatx4 part[8][NT][2][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+  const int64_t n0 = (int64_t)blockIdx.x * 16;
+  const int steps = D / 32;
+  const uint16_t* wg = w + (n0 + r) * D + 8 * q;
+  const uint16_t* wu = w + (I + n0 + r) * D + 8 * q;
+  const uint16_t* xr[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) xr[t] = x + (int64_t)(16 * t + r < T ? 16 * t + r : T - 1) * D + 8 * q;
+  floatx4 ag[NT], au[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) ag[t] = au[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const auto at = [](const uint16_t* p, int s) { return *reinterpret_cast<const bf16x8*>(p + 32 * s); };
+  int s = wave;
+  for (; s + 8 * (kU - 1) < steps; s += 8 * kU) {
+    bf16x8 g[kU], u[kU], v[kU][NT];
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      g[k] = at(wg, s + 8 * k);
+      u[k] = at(wu, s + 8 * k);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) v[k][t] = at(xr[t], s + 8 * k);
+    }
+#pragma unroll
+    for (int k = 0; k < kU; ++k)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        ag[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[k], v[k][t], ag[t], 0, 0, 0);
+        au[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u[k], v[k][t], au[t], 0, 0, 0);
+      }
+  }
+  for (; s < steps; s += 8) {
+    const bf16x8 g = at(wg, s), u = at(wu, s);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const bf16x8 v = at(xr[t], s);
+      ag[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g, v, ag[t], 0, 0, 0);
+      au[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u, v, au[t], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    part[wave][t][0][lane] = ag[t];
+    part[wave][t][1][lane] = au[t];
+  }
+  __syncthreads();
+  if (wave >= NT) return;
+  floatx4 g = part[0][wave][0][lane], u = part[0][wave][1][lane];
+#pragma unroll
+  for (int k = 1; k < 8; ++k) {
+    g += part[k][wave][0][lane];
+    u += part[k][wave][1][lane];
+  }
+  const int row = 16 * wave + r;
+  if (row >= T) return;
+  uint32_t o[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float g0 = g[2 * i], g1 = g[2 * i + 1], u0 = u[2 * i], u1 = u[2 * i + 1];
+    round2_bf16(g0, g1);
+    round2_bf16(u0, u1);
+    o[i] = pack2_bf16(g0 * sigmoid_fast(g0) * u0, g1 * sigmoid_fast(g1) * u1);
+  }
+  *reinterpret_cast<intx2*>(h + (int64_t)row * I + n0 + 4 * q) = intx2{(int)o[0], (int)o[1]};
 }
 
 // The bf16 gate/up forward, persistent, with the SwiGLU of each tile under the
@@ -2930,7 +3020,7 @@ int bf16_swiglu_launch(const void* x, const void* w, int64_t T, int64_t D, int64
   if (rc) return rc;
   hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st,
                      (const uint16_t*)x, (const uint8_t*)w, T, D, I, rstd, (uint16_t*)gu, (uint16_t*)h, tl.m,
-                     tl.n, plan, plan ? 2 * D * slab_rows(2 * I) : 0, ldxs);
+                     tl.n, plan, plan ? 2 * D * slab_rows(2 * I) : 0, ldxs, 0);
   return status();
 }
 
@@ -2956,6 +3046,31 @@ int sfp8_bf16_gemm_swiglu_fwd(const void* x, int x_slab, const void* w, int64_t 
   if (T == 0) return kOk;
   return bf16_swiglu_launch(x, w, T, D, I, rstd, gu, h, nullptr, 0, x_slab ? slab_rows(T) : 0,
                             (hipStream_t)stream);
+}
+
+int sfp8_bf16_swiglu_eval(const void* x, const void* w, int64_t T, int64_t D, int64_t I, void* h, void* stream) {
+  if (!w || (T > 0 && (!x || !h))) return kErrNullPointer;
+  if (T < 0 || !bf16_shape(D, I) || !fits32(kTile, 2 * D) || !fits32(2 * I, 2 * D)) return kErrBadShape;
+  if (!al16(x) || !al16(w) || !al16(h)) return kErrBadAlignment;
+  if (T == 0) return kOk;
+  hipStream_t st = (hipStream_t)stream;
+  if (T <= kEvalRows) {
+    const auto kern = T <= 16   ? bf16_swiglu_eval_kernel<1>
+                      : T <= 32 ? bf16_swiglu_eval_kernel<2>
+                      : T <= 48 ? bf16_swiglu_eval_kernel<3>
+                                : bf16_swiglu_eval_kernel<4>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(I / 16)), dim3(512), 0, st, (const uint16_t*)x, (const uint16_t*)w, (int)T,
+                       (int)D, (int)I, (uint16_t*)h);
+    return status();
+  }
+  const Tiling tl = swiglu_tiling(T, I);
+  const auto kern = tl.small ? bf16_swiglu_fwd_kernel<true> : bf16_swiglu_fwd_kernel<false>;
+  const int rc = prep(kern, tl.lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st, (const uint16_t*)x, (const uint8_t*)w, T, D, I,
+                     (const float*)nullptr, (uint16_t*)nullptr, (uint16_t*)h, tl.m, tl.n, (const int*)nullptr,
+                     (int64_t)0, (int64_t)0, 1);
+  return status();
 }
 
 int sfp8_bf16_moe_gemm_swiglu_fwd(const void* x, const void* w, int64_t E, int64_t D, int64_t I, const int* plan,

@@ -416,6 +416,17 @@ std::tuple<Tensor, Tensor> bf16_swiglu_fwd(const Tensor& x, const Tensor& ws, in
   return {gu, h};
 }
 
+Tensor bf16_swiglu_eval(const Tensor& x, const Tensor& w) {
+  contig("x", x, kBF16, 2);
+  contig("w", w, kBF16, 2);
+  const int64_t T = x.size(0), D = x.size(1), I = w.size(0) / 2;
+  need(w.size(0) % 2 == 0 && w.size(1) == D, "w must be [2I, D]");
+  need(w.device() == x.device(), "x and w on one device");
+  Tensor h = empty({T, I}, kBF16, x);
+  CALL(sfp8_bf16_swiglu_eval, ptr(x), ptr(w), T, D, I, ptr(h), stream_of(x));
+  return h;
+}
+
 std::tuple<Tensor, OptTensor> bf16_swiglu_bwd(const Tensor& gu, const Tensor& dout, const OptTensor& rstd,
                                               const OptTensor& plan, int64_t ldp, bool copy) {
   contig("gu", gu, kBF16, 2);
@@ -570,6 +581,9 @@ PYBIND11_MODULE(_native, m) {
         "(gu [rows, 2I], h [rows, I]) bf16: the gate/up GEMM with the SwiGLU epilogue, rows scaled by rstd when given "
         "(dense) or grouped by a plan.  Dense: xs, the row K-slab of x from bf16_rows_prep(rows=True), when given is "
         "read instead of x (the same result, a faster read).");
+  m.def("bf16_swiglu_eval", &bf16_swiglu_eval, arg("x"), arg("w"),
+        "h [T, I] bf16 = silu(x Wg^T) * (x Wu^T) for x [T, D] and W [2I, D] bf16 row-major, when no gradient will be "
+        "taken: nothing is saved, W is read as it is.");
   m.def("bf16_swiglu_bwd", &bf16_swiglu_bwd, arg("gu"), arg("dout"), arg("rstd"), arg("plan"), arg("ldp"), kw,
         arg("copy") = true,
         "(gs, gt): G' = bf16 SwiGLU gradient of the rows (times rstd when given) as the K-slab over ldp padded rows "

@@ -106,8 +106,9 @@ def _dense_weights(m: nn.Module):
 
 class MLP(nn.Module):
     """Same parameters, buffers and forward as the reference MLP
-    (train.py:247-262): the fused bf16 SwiGLU (``_FusedSwiGLU``) when
-    ``_use_fused_swiglu(x)``, else gate/up -> silu * up -> down in torch."""
+    (train.py:247-262): the fused bf16 SwiGLU (``_FusedSwiGLU``, or
+    ``_EvalSwiGLU`` while gradients are off) when ``_use_fused_swiglu(x)``, else
+    gate/up -> silu * up -> down in torch."""
 
     def __init__(self, dim: int, hidden_dim: int):
         super().__init__()
@@ -119,9 +120,11 @@ class MLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if _swiglu._use_fused_swiglu(x):
-            weight = self.gate_up_proj.weight.to(dtype=x.dtype).unsqueeze(0)
+            weight = self.gate_up_proj.weight.to(dtype=x.dtype)
+            if _swiglu._eval_swiglu(weight):
+                return self.down_proj(_swiglu._EvalSwiGLU.apply(x, weight))
             offs = torch.full((1,), x.shape[0], device=x.device, dtype=torch.int32)
-            return self.down_proj(_swiglu._FusedSwiGLU.apply(x, weight, offs))
+            return self.down_proj(_swiglu._FusedSwiGLU.apply(x, weight.unsqueeze(0), offs))
         gate, up = self.gate_up_proj(x).chunk(2, dim=-1)
         return self.down_proj(F.silu(gate) * up)
 

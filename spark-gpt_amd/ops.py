@@ -20,8 +20,8 @@ from . import _lib
 _NATIVE = ("norm_quant", "block_weight_quant", "weight_quant_experts", "gateup_swiglu_fwd", "down_fwd",
            "down_dgrad_swiglu", "gateup_dgrad", "wgrad_rows", "norm_bwd", "moe_plan", "moe_rows_quant",
            "moe_gateup_swiglu_fwd", "moe_down_fwd", "moe_down_dgrad_swiglu", "moe_gateup_dgrad", "moe_wgrad_rows",
-           "moe_topk_sum", "bf16_weight_slabs", "bf16_rows_prep", "bf16_swiglu_fwd", "bf16_swiglu_bwd", "bf16_gemm",
-           "bf16_norm_dh", "bf16_wgrad_rows", "bf16_fold_grads")
+           "moe_topk_sum", "bf16_weight_slabs", "bf16_rows_prep", "bf16_swiglu_fwd", "bf16_swiglu_eval",
+           "bf16_swiglu_bwd", "bf16_gemm", "bf16_norm_dh", "bf16_wgrad_rows", "bf16_fold_grads")
 
 
 def _missing(name: str, why: str):

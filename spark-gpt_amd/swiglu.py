@@ -150,6 +150,27 @@ class _FusedSwiGLU(torch.autograd.Function):
         return dx, dw, None
 
 
+class _EvalSwiGLU(torch.autograd.Function):
+    """h = silu(x W_gate^T) * (x W_up^T) of a dense MLP while gradients are off
+    (generation, evaluation): x [T, D], weight [2I, D] bf16.  W is read as it
+    is and only h is written, where ``_FusedSwiGLU`` lays W out, plans the rows
+    and saves gu for a backward.  A Function so that whatever it cannot
+    follow (forward-mode, vmap) is refused as ``_FusedSwiGLU`` refuses it."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        return torch_ops.op("swiglu_eval")(x, weight)
+
+    @staticmethod
+    def backward(ctx, dh):
+        raise RuntimeError("_EvalSwiGLU saves nothing for a backward")
+
+
+def _eval_swiglu(weight) -> bool:
+    """Whether ``MLP.forward`` runs ``_EvalSwiGLU``: gradients off and a width the kernels take."""
+    return not torch.is_grad_enabled() and weight.shape[0] % 2 == 0 and _kernel_shape(weight.shape[1], weight.shape[0] // 2)
+
+
 class _NormSwiGLU(torch.autograd.Function):
     """SwiGLU(gate_up(rmsnorm(h))) of a dense MLP (train.py:2101-2131), the
     norm weight folded into the gate/up weight (W' = bf16(w_gu * norm_w)) and

@@ -398,6 +398,20 @@ def _swiglu_fwd_fake(x, weight, offs):
             x.new_empty((_plan_ints(R, E),), dtype=torch.int32))
 
 
+def swiglu_eval_impl(x: Tensor, weight: Tensor) -> Tensor:
+    """The forward of a dense MLP's gate/up and SwiGLU while gradients are off:
+    h [T, I] bf16 from x [T, D] and weight [2I, D] bf16, nothing saved."""
+    return ops.bf16_swiglu_eval(x.contiguous(), weight.contiguous())
+
+
+swiglu_eval = torch.library.custom_op("sparkfp8::swiglu_eval", swiglu_eval_impl, mutates_args=())
+
+
+@swiglu_eval.register_fake
+def _swiglu_eval_fake(x, weight):
+    return x.new_empty((x.shape[0], weight.shape[0] // 2), dtype=BF16)
+
+
 def swiglu_bwd_impl(dh: Tensor, x: Tensor, weight: Tensor, gu: Tensor, plan: Tensor) -> Tuple[Tensor, Tensor]:
     """_FusedSwiGLU.backward (train.py:2083-2090): (dx [R, D] bf16, dW [E, 2I, D]
     bf16), the SwiGLU gradient G' (bf16) computed once for both GEMMs."""

@@ -420,3 +420,29 @@ def test_bf16_moe_wgrad_rows_equals_token_contiguous(dev, counts):
     # the SwiGLU gradient without its token-contiguous copy: the same K-slab
     gs2, none = ops.bf16_swiglu_bwd(gu, dout, None, plan, ldp, copy=False)
     assert none is None and torch.equal(gs2, gs)
+
+
+# generation kernel up to 64 rows (16-row tiles, 8 K steps at a time and the
+# rest singly), tiled kernel from 65 on
+@pytest.mark.parametrize("T,D,I", [(1, 64, 64), (7, 320, 192), (16, 1024, 128), (17, 576, 64), (48, 2048, 64),
+                                   (64, 256, 320), (65, 320, 192), (300, 1024, 704), (2017, 256, 1984)])
+def test_eval_mlp(dev, T, D, I):
+    """MLP.forward while gradients are off against the training path of the
+    same module: gate and up are sums of at most 2048 fp32 products in another
+    order (relative 1e-6), which moves a bf16 rounding only now and then, so h
+    agrees to a bf16 step (2^-8) and mostly exactly; nothing requires grad."""
+    torch.manual_seed(T + D)
+    mlp = sg.MLP(D, I).to(dev).to(torch.bfloat16)
+    x = torch.randn(T, D, device=dev).bfloat16()
+    w = mlp.gate_up_proj.weight
+    offs = torch.full((1,), T, device=dev, dtype=torch.int32)
+    ref = sg._FusedSwiGLU.apply(x, w.unsqueeze(0), offs)
+    with torch.no_grad():
+        h = sg.swiglu._EvalSwiGLU.apply(x, w)
+        y = mlp(x)
+    assert h.shape == (T, I) and not y.requires_grad
+    a, b = h.float(), ref.detach().float()
+    # g and u may each round the other way, and h once more: three bf16 steps
+    assert torch.all((a - b).abs() <= 3 * 2 ** -8 * b.abs().clamp(min=1e-4))
+    assert float((a != b).float().mean()) < 0.02
+    assert O.rel_l2(y.float().cpu(), mlp(x).detach().float().cpu()) < 1e-2
