@@ -2764,35 +2764,25 @@ static bool wgrad_split_ok(int64_t s, int64_t ldt) {
   return c >= 2048 && ldt - (s - 1) * c > 0;
 }
 
-// bf16 operands (ldt counts K bytes): splits double while the grid has fewer
-// than 512 work-groups, stopping at 8 once it has 384; every split equal.
-static int64_t wgrad_splits_doubling(int64_t M, int64_t N, int64_t ldt) {
-  const int64_t tiles = (int64_t)cdiv(M, kTile) * cdiv(N, kTile);
-  int64_t s = 1;
-  while (tiles * s < 512 && !(s >= 8 && tiles * s >= 384) && ldt % (2 * s) == 0 &&
-         (ldt / (2 * s)) % (2 * kStage) == 0 && ldt / (2 * s) >= 2048)
-    s *= 2;
-  return s;
-}
-
-int64_t sfp8_wgrad_splits(int64_t M, int64_t N, int64_t ldt) {
+static int64_t wgrad_splits(int64_t M, int64_t N, int64_t kbytes) {
   // The count (any, not only a power of two) that minimises the modelled
   // time: the rounds of work-groups the 256 CUs run, times the longest
-  // split's 64-token K stages, plus the split partials' traffic (4 bytes
+  // split's 64-byte K stages, plus the split partials' traffic (4 bytes
   // written and read per output and split, at about 5 TB/s: M * N * 8 /
   // 3.5e6 stage times of 0.7 us).  At T = 65536 this gives 5 splits for both
   // the down gradient (48 tiles: 240 work-groups in one round, where 4
   // splits leave 64 CUs idle) and the gate/up one (96 tiles: 480 work-groups
   // in two rounds, against three rounds of 256 with 8).  Ties go to fewer
-  // splits.
-  constexpr int64_t kCUs = 256;
+  // splits.  A bf16 stage holds half the tokens in the same bytes and takes as
+  // long: at T = 49152, M = 3072, N = 512 (24 tiles) it gives 10 splits in one
+  // round, 150 us with the reduction against 186 for 16 (a round and a half).
   const int64_t tiles = (int64_t)cdiv(M, kTile) * cdiv(N, kTile);
   const double part = (double)M * (double)N * 8.0 / 3.5e6;
   int64_t best = 1;
   double best_cost = 0.0;
   for (int64_t s = 1; s <= 64 && tiles * s <= 2048; ++s) {
-    if (!wgrad_split_ok(s, ldt)) continue;
-    const double stages = (double)wgrad_chunk(ldt, s) / kStage;
+    if (!wgrad_split_ok(s, kbytes)) continue;
+    const double stages = (double)wgrad_chunk(kbytes, s) / kStage;
     const double cost = (double)((tiles * s + kCUs - 1) / kCUs) * stages + (s > 1 ? s * part : 0.0);
     if (s == 1 || cost < best_cost - 1e-9) {
       best = s;
@@ -2801,6 +2791,8 @@ int64_t sfp8_wgrad_splits(int64_t M, int64_t N, int64_t ldt) {
   }
   return best;
 }
+
+int64_t sfp8_wgrad_splits(int64_t M, int64_t N, int64_t ldt) { return wgrad_splits(M, N, ldt); }
 
 int64_t sfp8_slab_bytes(int64_t rows, int64_t k) {
   if (rows < 0 || k < 0 || k % kStage) return -1;
@@ -2915,13 +2907,15 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
 // K splits of a grouped weight gradient: enough work-groups to fill the GPU
 // (about 512) when there are few experts and tiles.
 int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E) {
-  // at least 2 splits, then doubling until the grid has 384 work-groups (8 at
-  // most): at the MoE headline shape (8 experts, D=1024, I=1536) the down
-  // gradient takes 0.234 ms with 2 splits against 0.245 with 4, the gate/up
-  // one 0.397 with 2 against 0.413 with 1
+  // at least 2 splits, then doubling until the grid has 192 work-groups (8 at
+  // most): at 8 experts, D=1024, I=1536 the down gradient takes 0.234 ms with
+  // 2 splits against 0.245 with 4, the gate/up one 0.397 with 2 against 0.413
+  // with 1; at 8 experts, D=512, I=768 and 16384 rows the bf16 gate/up one 53
+  // us with its reduction with 2 (192 work-groups, one round) against 66 with 4
+  // (a round and a half, and twice the partials)
   const int64_t wgs = (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * E;
   int64_t s = 1;
-  while (s < 8 && (s < 2 || wgs * s < 384)) s *= 2;
+  while (s < 8 && (s < 2 || wgs * s < 192)) s *= 2;
   return s;
 }
 
@@ -3104,7 +3098,7 @@ int sfp8_bf16_moe_gemm(const void* a, const void* b, int64_t E, int64_t N, int64
   return bf16_gemm_launch(a, b, 0, N, K, ldp, out, plan, (hipStream_t)stream);
 }
 
-int64_t sfp8_bf16_wgrad_splits(int64_t M, int64_t N, int64_t ldt) { return wgrad_splits_doubling(M, N, 2 * ldt); }
+int64_t sfp8_bf16_wgrad_splits(int64_t M, int64_t N, int64_t ldt) { return wgrad_splits(M, N, 2 * ldt); }
 
 int64_t sfp8_bf16_wgrad_workspace_floats(int64_t M, int64_t N, int64_t ldt) {
   return sfp8_bf16_wgrad_splits(M, N, ldt) * (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * kTile * kTile;
@@ -3126,7 +3120,7 @@ int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, i
   const int64_t splits = sfp8_bf16_wgrad_splits(M, N, ldt);
   if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   const Tiling tl = tiling(M, N, splits);
-  const int rc = launch_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldt, 2 * ldt / splits, nullptr, nullptr,
+  const int rc = launch_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr,
                                                         ws, (int)splits, 1, TrOp{}, TrOp{}, st);
   if (rc) return rc;
   return launch_bf16_reduce(tl, false, ws, (int)splits, 1, M, N, out, st);
@@ -3175,7 +3169,7 @@ int sfp8_bf16_gemm_wgrad_rows(const void* a, const void* x, int x_rows, int64_t 
   const TrOp tra{kStage, ldt * kStage, (M / 32) * ldt * kStage}, trb{2 * N, kStage, T * 2 * N};
   const Tiling tl = tiling(M, N, splits);
   const auto launch = x_rows ? launch_wgrad<true, 0, 0, true, true> : launch_wgrad<true, 0, 0, true, false>;
-  const int rc = launch(tl, a, x, M, N, 2 * ldt, 2 * ldt / splits, nullptr, nullptr, ws, (int)splits, 1, tra,
+  const int rc = launch(tl, a, x, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr, ws, (int)splits, 1, tra,
                         x_rows ? trb : TrOp{}, st);
   if (rc) return rc;
   return launch_bf16_reduce(tl, x_rows, ws, (int)splits, 1, M, N, out, st);
