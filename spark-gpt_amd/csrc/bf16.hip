@@ -131,11 +131,14 @@ __global__ __launch_bounds__(256) void bf16_weight_slabs_kernel(const void* __re
 // for p < nsrc (the row scale of _swiglu_gemm_kernel's NORM mode,
 // train.py:1689-1700; the sum of squares is exact, in fp64).  A work-group
 // takes 64 padded rows, the columns in 64-wide chunks through an LDS
-// transpose.  D % 64 == 0.
+// transpose: all of them when rstd needs whole rows, else `cols` of them from
+// cols * blockIdx.y (a chunk's load, transpose and store are one dependent
+// chain, so the chunks of a row block run as work-groups of their own: at
+// T = 8192 top-2, D = 512, 16.9 -> 9.9 us).  D % 64 == 0.
 __global__ __launch_bounds__(256) void bf16_rows_prep_kernel(const uint16_t* __restrict__ x, int64_t nsrc, int64_t D,
                                                              const int* __restrict__ plan, float eps,
                                                              float* __restrict__ rstd, uint8_t* __restrict__ xt,
-                                                             uint8_t* __restrict__ xs) {
+                                                             uint8_t* __restrict__ xs, int64_t cols) {
   __shared__ __align__(16) uint8_t tile[64 * kTrStride];
   __shared__ int64_t rsrc[64];
   const int64_t p0 = (int64_t)blockIdx.x * 64;
@@ -143,7 +146,8 @@ __global__ __launch_bounds__(256) void bf16_rows_prep_kernel(const uint16_t* __r
   __syncthreads();
   const int64_t dp = slab_rows(D);
   double ss[2] = {0.0, 0.0};
-  for (int64_t c0 = 0; c0 < D; c0 += 64) {
+  const int64_t cb = cols * blockIdx.y, ce = cb + cols < D ? cb + cols : D;
+  for (int64_t c0 = cb; c0 < ce; c0 += 64) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int u = threadIdx.x + 256 * k;
@@ -186,6 +190,47 @@ __global__ __launch_bounds__(256) void bf16_rows_prep_kernel(const uint16_t* __r
       const float var = (float)t / (float)D + eps;
       rstd[p] = (float)(1.0 / __builtin_sqrt((double)var));
     }
+  }
+}
+
+// rstd and / or the row K-slab of dense x (no plan, no transposed copy), the
+// same values: eight lanes a row, 16 rows per work-group of two waves, and
+// each lane requests six 64-column chunks before it uses any (the loop above
+// keeps one in flight: T = 4099, D = 768
+// 14.8 -> 6.4 us, T = 49152, D = 512 23.0 -> 20.2).
+__global__ __launch_bounds__(128) void bf16_rows_slab_kernel(const uint16_t* __restrict__ x, int64_t T, int64_t D,
+                                                             float eps, float* __restrict__ rstd,
+                                                             uint8_t* __restrict__ xs, int64_t ldp) {
+  constexpr int kU = 6;
+  const int c8 = threadIdx.x & 7;
+  const int64_t p = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 3);
+  const bool live = p < T;
+  const uint16_t* row = x + p * D + 8 * c8;
+  // columns c0 + 8 c8 .. are 16 bytes of slab (c0 + 8 c8) / 32
+  uint8_t* out = xs + (int64_t)(c8 >> 2) * ldp * 64 + p * 64 + 16 * (c8 & 3);
+  double ss = 0.0;
+  for (int64_t c0 = 0; c0 < D; c0 += 64 * kU) {
+    intx4 v[kU];
+#pragma unroll
+    for (int k = 0; k < kU; ++k)
+      v[k] = live && c0 + 64 * k < D ? __builtin_nontemporal_load(reinterpret_cast<const intx4*>(row + c0 + 64 * k))
+                                     : intx4{0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      if (xs && c0 + 64 * k < D) *reinterpret_cast<intx4*>(out + ((c0 + 64 * k) >> 5) * ldp * 64) = v[k];
+      float f[8];
+      unpack8_bf16(v[k], f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = __builtin_fma((double)f[j], (double)f[j], ss);  // exact
+    }
+  }
+  if (!rstd) return;
+  ss += __shfl_xor(ss, 1, 64);  // the 8 lanes of a row are consecutive
+  ss += __shfl_xor(ss, 2, 64);
+  ss += __shfl_xor(ss, 4, 64);
+  if (c8 == 0 && live) {
+    const float var = (float)ss / (float)D + eps;
+    rstd[p] = (float)(1.0 / __builtin_sqrt((double)var));
   }
 }
 
@@ -386,8 +431,15 @@ int sfp8_bf16_rows_prep(const void* x, int64_t nsrc, int64_t D, const int* plan,
   if (nsrc < 0 || D <= 0 || D % 64 || ldp < 0 || ldp % 256 || (!plan && ldp < nsrc)) return kErrBadShape;
   if (!bf_al16(x) || !bf_al16(xt) || !bf_al16(xs)) return kErrBadAlignment;
   if (ldp == 0) return kOk;
-  hipLaunchKernelGGL(bf16_rows_prep_kernel, dim3((unsigned)(ldp / 64)), dim3(256), 0, (hipStream_t)stream,
-                     (const uint16_t*)x, nsrc, D, plan, eps, rstd, (uint8_t*)xt, (uint8_t*)xs);
+  if (!xt && !plan) {
+    hipLaunchKernelGGL(bf16_rows_slab_kernel, dim3((unsigned)(ldp / 16)), dim3(128), 0, (hipStream_t)stream,
+                       (const uint16_t*)x, nsrc, D, eps, rstd, (uint8_t*)xs, ldp);
+    return bf_status();
+  }
+  const int64_t cols = rstd ? D : 64;
+  hipLaunchKernelGGL(bf16_rows_prep_kernel, dim3((unsigned)(ldp / 64), (unsigned)((D + cols - 1) / cols)), dim3(256), 0,
+                     (hipStream_t)stream, (const uint16_t*)x, nsrc, D, plan, eps, rstd, (uint8_t*)xt, (uint8_t*)xs,
+                     cols);
   return bf_status();
 }
 

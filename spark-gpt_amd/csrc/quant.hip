@@ -161,12 +161,14 @@ __global__ __launch_bounds__(256) void quant_rowcol_kernel(
 // operands.
 // Each work-group owns RT rows; a row is split over LPR lanes holding CPL
 // 8-element chunks each.
-template <int D>
+// FEW: 16 rows, for batches whose larger row blocks would leave CUs without
+// one (few_rows below).
+template <int D, bool FEW = false>
 struct NormCfg {
   static constexpr int LPR = (D / 8) < 64 ? (D / 8) : 64;  // lanes per row
   static constexpr int RPW = 64 / LPR;                       // rows per wave pass
   static constexpr int CPL = D / (8 * LPR);                  // chunks per lane
-  static constexpr int RT = (65536 / D) < 64 ? (65536 / D) : 64;  // rows per WG
+  static constexpr int RT = FEW ? 16 : (65536 / D) < 64 ? (65536 / D) : 64;  // rows per WG
   // LDS row stride: D + 16 bytes puts the 8 rows of a transposing read on
   // distinct bank pairs
   static constexpr int STRIDE = D + 16;
@@ -196,13 +198,13 @@ struct NormCfg {
   static_assert(QPASSES % PB == 0 && PASSES % PB_BWD == 0, "whole load batches");
 };
 
-template <int D>
+template <int D, bool FEW>
 __global__ __launch_bounds__(64 * NormCfg<D>::QW) __attribute__((amdgpu_waves_per_eu(NormCfg<D>::QW / 2)))
 void norm_quant_kernel(
     const uint16_t* __restrict__ h, const float* __restrict__ nw, int64_t T, float eps,
     const float* __restrict__ scale, float* __restrict__ amax, uint8_t* __restrict__ x8,
     uint8_t* __restrict__ x8t, int64_t ldt, float* __restrict__ rstd) {
-  using Cfg = NormCfg<D>;
+  using Cfg = NormCfg<D, FEW>;
   extern __shared__ __align__(16) uint8_t smem[];
   __shared__ float red[Cfg::QW];
   uint8_t* tile = smem;
@@ -652,21 +654,20 @@ __global__ void update_scales_kernel(float* __restrict__ scale, float* __restric
 // [D/64][ldt][64] and/or the token-contiguous K-slab copy dy8t (each
 // optional; zeros for tokens T..ldt-1), and amax slot 4 = max|dy|
 // (recorded at train.py:1074-1081).
-template <int D>
+template <int D, bool FEW>
 __global__ __launch_bounds__(64 * NormCfg<D>::BW) __attribute__((amdgpu_waves_per_eu(NormCfg<D>::BW == 8 ? 4 : 1)))
 void norm_bwd_kernel(
     const uint16_t* __restrict__ h, const float* __restrict__ rstd, const uint16_t* __restrict__ dxn,
     const uint16_t* __restrict__ dy, const float* __restrict__ nw, int64_t T,
     const float* __restrict__ scale, float* __restrict__ amax, uint16_t* __restrict__ dh,
     float* __restrict__ dnw_part, uint8_t* __restrict__ dy8, uint8_t* __restrict__ dy8t, int64_t ldt) {
-  using Cfg = NormCfg<D>;
+  using Cfg = NormCfg<D, FEW>;
   extern __shared__ __align__(16) uint8_t smem[];
   __shared__ float red[Cfg::BW];
   uint8_t* tile = smem;
   // [BW waves][D] floats, in the tile's LDS after the dy8 / dy8t stores have
   // read it (the only LDS when there is neither)
   float* dnw_red = reinterpret_cast<float*>(smem);
-  static_assert(Cfg::BW * D * sizeof(float) <= Cfg::RT * Cfg::STRIDE, "dnw reduction fits in the tile");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int sr = lane / Cfg::LPR, li = lane % Cfg::LPR;
   const int blk = xcd_row_block(blockIdx.x, gridDim.x);
@@ -1077,30 +1078,48 @@ static int allow_lds(K kernel, size_t bytes) {
   return e == hipSuccess ? kOk : (int)e;
 }
 
+// Whether the norm kernels take 16 rows per work-group: at D = 1024 and 2048
+// when their usual row blocks are fewer than the 256 CUs.  At T = 5003, D =
+// 1024 (80 blocks of 64 rows) norm_quant 12.2 -> 8.7 us and norm_bwd 18.7 ->
+// 16.0.  Narrower rows leave each work-group too little: T = 8192, D = 256 (128
+// blocks) 7.0 -> 8.5 and 11.2 -> 11.9.  (At D = 4096 a block is 16 rows anyway.)
 template <int D>
+static bool few_rows(int64_t ldt) {
+  return (D == 1024 || D == 2048) && ldt / NormCfg<D>::RT < 256;
+}
+
+template <int D, bool FEW>
 static int launch_norm_quant(const void* h, const float* nw, int64_t T, float eps, const float* scale,
                              float* amax, void* x8, void* x8t, int64_t ldt, float* rstd, hipStream_t st) {
-  using Cfg = NormCfg<D>;
+  if constexpr (!FEW && (D == 1024 || D == 2048))
+    if (few_rows<D>(ldt)) return launch_norm_quant<D, true>(h, nw, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+  using Cfg = NormCfg<D, FEW>;
   const size_t lds = x8t ? (size_t)Cfg::RT * Cfg::STRIDE : 0;  // the transposing tile
   const unsigned nblk = (unsigned)(ldt / Cfg::RT);
-  const int rc = allow_lds(norm_quant_kernel<D>, lds);
+  const auto kern = norm_quant_kernel<D, FEW>;
+  const int rc = allow_lds(kern, lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(norm_quant_kernel<D>, dim3(nblk), dim3(64 * Cfg::QW), lds, st, (const uint16_t*)h, nw, T,
+  hipLaunchKernelGGL(kern, dim3(nblk), dim3(64 * Cfg::QW), lds, st, (const uint16_t*)h, nw, T,
                      eps, scale, amax, (uint8_t*)x8, (uint8_t*)x8t, ldt, rstd);
   return launch_status();
 }
 
-template <int D>
+template <int D, bool FEW>
 static int launch_norm_bwd(const void* h, const float* rstd, const void* dxn, const void* dy,
                            const float* nw, int64_t T, const float* scale, float* amax, void* dh,
                            float* dnw, float* part, void* dy8, void* dy8t, int64_t ldt, hipStream_t st) {
-  using Cfg = NormCfg<D>;
-  // the transposing tile, or only the dnw reduction rows
-  const size_t lds = (dy8 || dy8t) ? (size_t)Cfg::RT * Cfg::STRIDE : (size_t)Cfg::BW * D * sizeof(float);
+  if constexpr (!FEW && (D == 1024 || D == 2048))
+    if (few_rows<D>(ldt))
+      return launch_norm_bwd<D, true>(h, rstd, dxn, dy, nw, T, scale, amax, dh, dnw, part, dy8, dy8t, ldt, st);
+  using Cfg = NormCfg<D, FEW>;
+  // the transposing tile (if a copy is written), then the dnw reduction rows
+  const size_t tile = (dy8 || dy8t) ? (size_t)Cfg::RT * Cfg::STRIDE : 0, rows = (size_t)Cfg::BW * D * sizeof(float);
+  const size_t lds = tile > rows ? tile : rows;
   const unsigned nblk = (unsigned)(ldt / Cfg::RT);
-  const int rc = allow_lds(norm_bwd_kernel<D>, lds);
+  const auto kern = norm_bwd_kernel<D, FEW>;
+  const int rc = allow_lds(kern, lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(norm_bwd_kernel<D>, dim3(nblk), dim3(64 * Cfg::BW), lds, st, (const uint16_t*)h, rstd,
+  hipLaunchKernelGGL(kern, dim3(nblk), dim3(64 * Cfg::BW), lds, st, (const uint16_t*)h, rstd,
                      (const uint16_t*)dxn, (const uint16_t*)dy, nw, T, scale, amax, (uint16_t*)dh, part,
                      (uint8_t*)dy8, (uint8_t*)dy8t, ldt);
   const int rc2 = launch_status();
@@ -1170,12 +1189,12 @@ int sfp8_norm_quant(const void* h, const float* norm_w, int64_t T, int64_t D, fl
   if (ldt == 0) return kOk;
   hipStream_t st = (hipStream_t)stream;
   switch (D) {
-    case 128: return launch_norm_quant<128>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
-    case 256: return launch_norm_quant<256>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
-    case 512: return launch_norm_quant<512>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
-    case 1024: return launch_norm_quant<1024>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
-    case 2048: return launch_norm_quant<2048>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
-    case 4096: return launch_norm_quant<4096>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+    case 128: return launch_norm_quant<128, false>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+    case 256: return launch_norm_quant<256, false>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+    case 512: return launch_norm_quant<512, false>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+    case 1024: return launch_norm_quant<1024, false>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+    case 2048: return launch_norm_quant<2048, false>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
+    case 4096: return launch_norm_quant<4096, false>(h, norm_w, T, eps, scale, amax, x8, x8t, ldt, rstd, st);
     default:
       if (wide_hidden(D)) return launch_norm_quant_wide(h, norm_w, T, D, eps, scale, amax, x8, x8t, ldt, rstd, st);
       return kErrBadShape;
@@ -1265,12 +1284,12 @@ int sfp8_update_scales(float* scale, float* amax, int64_t nsets, void* stream) {
 
 static int64_t norm_bwd_blocks(int64_t D, int64_t ldt) {
   switch (D) {
-    case 128: return ldt / NormCfg<128>::RT;
-    case 256: return ldt / NormCfg<256>::RT;
-    case 512: return ldt / NormCfg<512>::RT;
-    case 1024: return ldt / NormCfg<1024>::RT;
-    case 2048: return ldt / NormCfg<2048>::RT;
-    case 4096: return ldt / NormCfg<4096>::RT;
+    case 128: return ldt / (few_rows<128>(ldt) ? 16 : NormCfg<128>::RT);
+    case 256: return ldt / (few_rows<256>(ldt) ? 16 : NormCfg<256>::RT);
+    case 512: return ldt / (few_rows<512>(ldt) ? 16 : NormCfg<512>::RT);
+    case 1024: return ldt / (few_rows<1024>(ldt) ? 16 : NormCfg<1024>::RT);
+    case 2048: return ldt / (few_rows<2048>(ldt) ? 16 : NormCfg<2048>::RT);
+    case 4096: return ldt / (few_rows<4096>(ldt) ? 16 : NormCfg<4096>::RT);
     default: return wide_hidden(D) ? ldt / kWideRows : -1;
   }
 }
@@ -1291,12 +1310,12 @@ static int norm_bwd_launch(const void* h, const float* rstd, const void* dxn, co
     return launch_status();
   }
   switch (D) {
-    case 128: return launch_norm_bwd<128>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
-    case 256: return launch_norm_bwd<256>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
-    case 512: return launch_norm_bwd<512>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
-    case 1024: return launch_norm_bwd<1024>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
-    case 2048: return launch_norm_bwd<2048>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
-    case 4096: return launch_norm_bwd<4096>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
+    case 128: return launch_norm_bwd<128, false>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
+    case 256: return launch_norm_bwd<256, false>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
+    case 512: return launch_norm_bwd<512, false>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
+    case 1024: return launch_norm_bwd<1024, false>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
+    case 2048: return launch_norm_bwd<2048, false>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
+    case 4096: return launch_norm_bwd<4096, false>(h, rstd, dxn, dy, norm_w, T, scale, amax, dh, dnw, partials, dy8, dy8t, ldt, st);
     default:
       if (wide_hidden(D)) return launch_norm_bwd_wide(h, rstd, dxn, dy, norm_w, T, D, scale, amax, dh, dnw, partials,
                                                      dy8, dy8t, ldt, st);

@@ -93,3 +93,59 @@ def test_norm_bwd(dev, T, D):
     y8 = u8(sg.ops.unslab(dy8, ldt))
     assert torch.equal(y8[:T], u8(ref8))
     assert torch.all(y8[T:] == 0)
+
+
+@pytest.mark.parametrize("T,D", [(16385, 1024), (8192, 2048)])
+def test_row_block_sizes_agree(dev, T, D):
+    """At these widths the norm kernels take 64 (32 at D = 2048) rows a
+    work-group from 256 row blocks on, below 16: a row's bytes do not depend on it, nor the maxima;
+    the norm weight's gradient is an fp32 sum of T rows in another order
+    (relative error of a pairwise-like sum over 16 to 64 rows a block: 1e-5)."""
+    from spark_gpt_amd import _lib
+
+    ops = sg.ops
+    ldt, few = ops.ldt_of(T), ops.ldt_of(T) // 2 // 256 * 256
+    blocks = lambda n: _lib.query("sfp8_norm_bwd_partials", D, n) - 32
+    assert blocks(ldt) == ldt // (64 if D < 2048 else 32) and blocks(few) == few // 16
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    h, dxn = (torch.randn(T, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    dy = (torch.randn(T, D, generator=g, device=dev) * 1e-3).bfloat16()
+    nw = torch.rand(D, generator=g, device=dev) + 0.5
+    scale = torch.tensor([32.0, 1, 1, 1, 2.0 ** 20], device=dev)
+
+    def run(a, b):
+        amax = torch.zeros(5, device=dev)
+        n = b - a
+        x8, x8t, rstd = ops.norm_quant(h[a:b], nw, scale, amax, 1e-6)
+        dh, dnw, dy8t = ops.norm_bwd(h[a:b], rstd, dxn[a:b], dy[a:b], nw, scale, amax)
+        assert torch.equal(ops.unslab(x8t, D).view(torch.uint8)[:, :n], ops.unslab(x8, n).view(torch.uint8).t())
+        return (ops.unslab(x8, n).view(torch.uint8), rstd, dh, ops.unslab(dy8t, D).view(torch.uint8)[:, :n].t()), dnw, amax
+
+    whole, dnw, amax = run(0, T)
+    parts = [run(a, min(T, a + few)) for a in range(0, T, few)]
+    for i, w in enumerate(whole):
+        assert torch.equal(torch.cat([p[0][i] for p in parts]), w)
+    assert torch.equal(torch.stack([p[2] for p in parts]).amax(0), amax)
+    exact = (dxn.double() * h.double() * whole[1].double()[:, None]).sum(0)
+    for got in (dnw.double(), sum(p[1].double() for p in parts)):
+        assert float((got - exact).norm() / exact.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("T,D", [(1, 64), (17, 320), (4099, 768), (300, 1024)])
+def test_bf16_rows_slab(dev, T, D):
+    """rstd and the row K-slab of dense rows without the transposed copy: the
+    slab is x's bytes with zero padding rows, rstd the fp32 rounding of the
+    exact sum of squares (one more rounding each for the mean and the root)."""
+    ops = sg.ops
+    x = torch.randn(T, D, device=dev).bfloat16()
+    ldt = ops.ldt_of(T)
+    rstd, none, xs = ops.bf16_rows_prep(x, None, ldt, 1e-6, copy=False, rows=True)
+    assert none is None
+    ref = torch.cat([x, torch.zeros(ldt - T, D, device=dev, dtype=x.dtype)])
+    assert torch.equal(ops.unslab(xs, ldt).view(torch.uint8), ref.view(torch.uint8).view(ldt, 2 * D))
+    want = torch.rsqrt(x.double().square().mean(1) + 1e-6)
+    assert float(((rstd.double() - want) / want).abs().max()) < 2 ** -22
+    only, _, _ = ops.bf16_rows_prep(x, None, ldt, 1e-6, copy=False)
+    both, xt, xs2 = ops.bf16_rows_prep(x, None, ldt, 1e-6, rows=True)
+    assert torch.equal(only, rstd) and torch.equal(both, rstd) and torch.equal(xs2, xs)
+    assert torch.equal(ops.unslab(xt, D).view(torch.int16), ref.t().contiguous().view(torch.int16))
