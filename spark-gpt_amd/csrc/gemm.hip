@@ -164,6 +164,34 @@ struct Tile {
 template <bool SMALL>
 using TileShape = Tile<SMALL ? 2 : 4, SMALL ? 2 : 4>;
 
+// The last round of a kernel of 256 x 256 tiles, one per CU, in halves: when
+// the remainder r of a round of nwg work-groups is at most half of it, these
+// tiles are split into 128-row halves (half: tm counts rows of 128), a
+// work-group each, so that the last round takes half as long.  False: no work
+// for this index.  Measured (us): gate/up dgrad, D = 1024, I = 3072, 121 -> 106
+// at 320 tiles, 369 -> 341 at 1040; down dgrad 102 -> 94 at 576 tiles, 457 ->
+// 447 at 3084; a block's step, T = 20000, D = 1024, I = 2048, 563 -> 549;
+// unchanged where the rounds are full.
+SFP8_DEV int tail_full(int ntiles, int nwg) {
+  const int r = ntiles % nwg;
+  return 2 * r <= nwg ? ntiles - r : ntiles;
+}
+SFP8_DEV bool tail_half(int h, int full, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int tile = full + (h >> 1);
+  if (tile >= tiles_m * tiles_n) return false;
+  raster(tile, tiles_m, tiles_n, tm, tn);
+  tm = 2 * tm + (h & 1);
+  return true;
+}
+constexpr int kRound = 256;  // work-groups of a round: one per CU
+SFP8_DEV bool tail_tile(int tiles_m, int tiles_n, int& tm, int& tn, bool& half, bool rev = false) {
+  const int full = tail_full(tiles_m * tiles_n, kRound), pid = blockIdx.x;
+  half = pid >= full;
+  if (half) return tail_half(pid - full, full, tiles_m, tiles_n, tm, tn);
+  tile_coords(pid, full, tiles_m, tiles_n, tm, tn, rev);
+  return true;
+}
+
 // ---------------------------------------------------------------------------
 // (a6) gate/up forward + SwiGLU epilogue (spark-gpt train.py:975-1016).
 // Tile: 256 tokens x 128 intermediate columns; the B tile holds gate rows
@@ -1056,14 +1084,11 @@ SFP8_DEV void store_bf16_tile(uint8_t* lds, const floatx16 (&acc)[TS::kTB][2], f
 // W_down8 of expert e at wd8 + e * w_estride, its scale wscale[e] (the dense
 // call passes wscale + 1: [q_gu, q_d]).
 template <class TS>
-__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void down_fwd_kernel(
-    const uint8_t* __restrict__ h8, const uint8_t* __restrict__ wd8, const uint16_t* __restrict__ res,
-    int64_t T, int64_t D, int64_t I, const float* __restrict__ scale, const float* __restrict__ wscale,
-    uint16_t* __restrict__ y, int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan,
+SFP8_DEV void down_fwd_tile(
+    uint8_t* lds, int tm, int tn, const uint8_t* __restrict__ h8, const uint8_t* __restrict__ wd8,
+    const uint16_t* __restrict__ res, int64_t T, int64_t D, int64_t I, const float* __restrict__ scale,
+    const float* __restrict__ wscale, uint16_t* __restrict__ y, int64_t ldt, const int* __restrict__ plan,
     int64_t w_estride) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  int tm, tn;
-  tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
   int64_t u0 = 0, urows = 0;
   if (plan) {
     const MoePlan P{plan};
@@ -1077,6 +1102,7 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void down_fwd_kernel(
     if (urows <= 0) return;  // nothing but padding rows, which have no output
   }
   const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
+  if (!plan && m0 >= T) return;  // the second half of the last tile, past the last row
   floatx16 acc[TS::kTB][2];
   // K-slab operands: h8 [I/64][ldt][64], wd8 [I/64][slab_rows(D)][64]
   const int64_t dp = slab_rows(D);
@@ -1121,6 +1147,26 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void down_fwd_kernel(
   __syncthreads();
   write_bf16_half_res<512>(lds, 1, m0, n0, T, D, rv1, y);
   }
+}
+template <class TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void down_fwd_kernel(
+    const uint8_t* __restrict__ h8, const uint8_t* __restrict__ wd8, const uint16_t* __restrict__ res,
+    int64_t T, int64_t D, int64_t I, const float* __restrict__ scale, const float* __restrict__ wscale,
+    uint16_t* __restrict__ y, int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan,
+    int64_t w_estride) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  int tm, tn;
+  if constexpr (TS::kTB == 4) {
+    bool half;
+    if (!tail_tile(plan ? MoePlan{plan}.ntiles() : tiles_m, tiles_n, tm, tn, half)) return;
+    if (half) {
+      down_fwd_tile<Tile<2, 4>>(lds, tm, tn, h8, wd8, res, T, D, I, scale, wscale, y, ldt, plan, w_estride);
+      return;
+    }
+  } else {
+    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+  }
+  down_fwd_tile<TS>(lds, tm, tn, h8, wd8, res, T, D, I, scale, wscale, y, ldt, plan, w_estride);
 }
 
 // ---------------------------------------------------------------------------
@@ -1181,9 +1227,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     uint8_t* __restrict__ dgu8, uint8_t* __restrict__ dgu8t, int64_t ldt, int tiles_m, int tiles_n,
     const int* __restrict__ plan, int64_t w_estride) {
   static_assert(!(TCOPY && SMALL), "the copy is staged by the larger tile");
-  using TS = TileShape<SMALL>;
-  using Loop = typename TS::template Loop<true, 0, 0>;
-  constexpr int kWaves = TS::kThreads / 64;
+  constexpr int kWaves = TileShape<SMALL>::kThreads / 64;
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t ldb = D * 2;  // bytes
@@ -1208,12 +1252,12 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   //   dgu8 = e5m2(d*q3) = e5m2(d'*(s_gu*q3)),  amax3 = s_gu*max(|dg|,|du|).
   const float m3s = (1.0f / scale[1]) * scale[3];
   const float inv3 = 1.0f / m3s, bnd3 = kE5M2Max * inv3;
-  float* red = reinterpret_cast<float*>(base + (SMALL ? 128 * TS::kOutStride : 2 * kTile * kEpiStride2));  // after the staging tiles
+  float* red = reinterpret_cast<float*>(base + (SMALL ? 128 * TileShape<SMALL>::kOutStride : 2 * kTile * kEpiStride2));  // after the staging tiles
   float m3 = 0.f;
   // Persistent: work-group pid runs tiles pid, pid + gridDim.x, ...  (Work-
   // groups started a quarter of a tile apart per XCD, so that the tiles'
   // 256 KiB store bursts would not coincide, measured 2 % slower.)
-  if (plan) tiles_m = MoePlan{plan}.ntiles() * (kTile / TS::kM);
+  if (plan) tiles_m = MoePlan{plan}.ntiles() * (kTile / TileShape<SMALL>::kM);
   const int ntiles = tiles_m * tiles_n;
   // A = dy row-major (rows past the tile's last read as zero through the
   // range check); B = Wd^T as a bf16 K-slab [2D/64][slab_rows(I)][64] (bytes)
@@ -1228,8 +1272,9 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     const uint8_t* b;
     int64_t b_bytes;
   };
-  const auto ops_of = [=](int tm, int tn) {
-    const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  const auto ops_of = [=](auto shape, int tm, int tn) {
+    using TS = decltype(shape);
+    const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
     int64_t a_row = m0, a_rows = T - m0;
     const uint8_t* wb = reinterpret_cast<const uint8_t*>(wdt);
     if (plan) {
@@ -1242,16 +1287,16 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     return Ops{reinterpret_cast<const uint8_t*>(dy) + a_row * ldb, a_rows * ldb, wb + n0 * kStage,
                ldb * ip - n0 * kStage};
   };
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-  int tm, tn;
-  tile_coords(tile, ntiles, tiles_m, tiles_n, tm, tn);
-  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  const auto run_tile = [&](auto shape, int tm, int tn) {
+  using TS = decltype(shape);
+  using Loop = typename TS::template Loop<true, 0, 0>;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
   floatx16 acc[TS::kTB][2];
   {
-    const Ops o = ops_of(tm, tn);
+    const Ops o = ops_of(shape, tm, tn);
     Loop::run(base, o.a, o.a_bytes, arow, kStage, o.b, o.b_bytes, brow, (int)(ip * kStage), nk, acc);
   }
-  // Row-order epilogue, in two passes (SMALL: one) of 128 tile rows (the rows
+  // Row-order epilogue, in two passes (128-row tiles: one) of 128 tile rows (the rows
   // of stage_bf16_half<P>): dh staged in LDS as bf16, then each thread takes
   // 16-column chunks of one row, reading gu8 and writing dgu8 as whole K-slab
   // rows; with dgu8t the codes also go to LDS for the token-contiguous copy.
@@ -1259,10 +1304,12 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   uint8_t* DH = base;
   // chunk k of this thread in a pass: 16 columns from chunk_col(k) of staging
   // row chunk_row(k), tile row tile_row(k, P)
-  constexpr int kSlabs = TS::kM / 64, kDh = SMALL ? TS::kOutStride : kBf16Stride;
+  constexpr int kSlabs = TS::kN / 64, kDh = TS::kOutStride;
+  constexpr bool kOne = TS::kTB == 2;  // one pass
+  static_assert(kDh == (SMALL ? kDh : kBf16Stride), "the staging rows of stage_bf16_half8");
   const auto chunk_row = [=](int k) { return 16 * ((kWaves * k + wave) / kSlabs) + (lane >> 2); };
   const auto chunk_col = [=](int k) { return 64 * ((kWaves * k + wave) % kSlabs) + 16 * (lane & 3); };
-  const auto tile_row = [=](int k, int P) { return SMALL ? chunk_row(k) : half_tile_row(chunk_row(k), P); };
+  const auto tile_row = [=](int k, int P) { return kOne ? chunk_row(k) : half_tile_row(chunk_row(k), P); };
   // the staging tiles of the token-contiguous copy (MoE only); their offset
   // goes through an empty asm so that the compiler does not hoist per-lane
   // addresses into them out of the tile loop (a register it had to spill)
@@ -1375,7 +1422,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
                                     I + n0);
     }
     __syncthreads();  // the next tile's DMA overwrites the staging tiles
-  } else if constexpr (SMALL) {
+  } else if constexpr (kOne) {
     uint32_t pg[4], pu[4];
     gu_loads(0);
     stage_bf16_tile<TS>(DH, acc, 1.0f);  // dh rounded to bf16 (train.py:1082)
@@ -1412,6 +1459,17 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     }
     __syncthreads();  // the next tile's DMA overwrites the staging tile
   }
+  };
+  // the last round in halves (tail_full), except with the copy and the small
+  // tiles
+  const int nwg = gridDim.x, full = TCOPY || SMALL ? ntiles : tail_full(ntiles, nwg);
+  int tm, tn;
+  for (int tile = blockIdx.x; tile < full; tile += nwg) {
+    tile_coords(tile, full, tiles_m, tiles_n, tm, tn);
+    run_tile(TileShape<SMALL>{}, tm, tn);
+  }
+  if constexpr (!TCOPY && !SMALL) {
+    if (tail_half(blockIdx.x, full, tiles_m, tiles_n, tm, tn)) run_tile(Tile<2, 4>{}, tm, tn);
   }
   m3 *= 1.0f / scale[1];  // s_gu, read again rather than held across the tile loop
   block_amax_atomic<kWaves>(m3, red, amax + 3);
@@ -1426,16 +1484,12 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // valid rows to dxn rows urow(tm).. (expert order, unpadded); W8^T of
 // expert e at w8t + e * w_estride, its scale wscale[e].
 template <class TS>
-__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kernel(
-    const uint8_t* __restrict__ dgu8, const uint8_t* __restrict__ w8t, int64_t T, int64_t D, int64_t I,
-    const float* __restrict__ scale, const float* __restrict__ wscale, uint16_t* __restrict__ dxn,
-    int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t w_estride) {
-  extern __shared__ __align__(16) uint8_t lds[];
+SFP8_DEV void gateup_dgrad_tile(
+    uint8_t* lds, int tm, int tn, const uint8_t* __restrict__ dgu8, const uint8_t* __restrict__ w8t, int64_t T,
+    int64_t D, int64_t I, const float* __restrict__ scale, const float* __restrict__ wscale,
+    uint16_t* __restrict__ dxn, int64_t ldt, const int* __restrict__ plan, int64_t w_estride) {
   const int64_t K = 2 * I;
   const int64_t dp = slab_rows(D);
-  int tm, tn;
-  // backwards: the dgrad wrote d_gu8 in forward order (0.304 -> 0.302 ms)
-  tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn, true);
   int64_t u0 = (int64_t)tm * TS::kM, uend = T;  // output rows of this tile
   if (plan) {
     const MoePlan P{plan};
@@ -1449,6 +1503,7 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kern
     if (u0 >= uend) return;  // nothing but padding rows, which have no output
   }
   const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
+  if (!plan && m0 >= T) return;  // the second half of the last tile, past the last row
   floatx16 acc[TS::kTB][2];
   // K-slab operands: dgu8 [2I/64][ldt][64], w8t [2I/64][slab_rows(D)][64]
   TS::template Loop<false, kFmtE5M2, kFmtE4M3>::run(
@@ -1458,6 +1513,26 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kern
   // the scales are read after the K loop, so that nothing is held across it
   const float sab = (1.0f / scale[3]) * (1.0f / wscale[0]);  // both powers of two
   store_bf16_tile<TS>(lds, acc, sab, u0, n0, uend, D, dxn);
+}
+template <class TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kernel(
+    const uint8_t* __restrict__ dgu8, const uint8_t* __restrict__ w8t, int64_t T, int64_t D, int64_t I,
+    const float* __restrict__ scale, const float* __restrict__ wscale, uint16_t* __restrict__ dxn,
+    int64_t ldt, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t w_estride) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  int tm, tn;
+  // backwards: the dgrad wrote d_gu8 in forward order (0.304 -> 0.302 ms)
+  if constexpr (TS::kTB == 4) {
+    bool half;
+    if (!tail_tile(plan ? MoePlan{plan}.ntiles() : tiles_m, tiles_n, tm, tn, half, true)) return;
+    if (half) {
+      gateup_dgrad_tile<Tile<2, 4>>(lds, tm, tn, dgu8, w8t, T, D, I, scale, wscale, dxn, ldt, plan, w_estride);
+      return;
+    }
+  } else {
+    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn, true);
+  }
+  gateup_dgrad_tile<TS>(lds, tm, tn, dgu8, w8t, T, D, I, scale, wscale, dxn, ldt, plan, w_estride);
 }
 
 // ---------------------------------------------------------------------------
@@ -2308,13 +2383,11 @@ __global__ __launch_bounds__(512, 1) void bf16_swiglu_pipe_kernel(
 // b + e * b_estride (bytes).
 // 8 waves (two per SIMD), each 128 x 64.
 template <class TS>
-__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void bf16_gemm_kernel(
-    const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int64_t T, int64_t N, int64_t Kb, int64_t lda,
-    uint16_t* __restrict__ out, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t b_estride) {
-  extern __shared__ __align__(16) uint8_t lds[];
+SFP8_DEV void bf16_gemm_tile(
+    uint8_t* lds, int tm, int tn, const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int64_t T,
+    int64_t N, int64_t Kb, int64_t lda, uint16_t* __restrict__ out, const int* __restrict__ plan,
+    int64_t b_estride) {
   const int64_t bp = slab_rows(N);
-  int tm, tn;
-  tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
   int64_t u0 = (int64_t)tm * TS::kM, uend = T;  // output rows of this tile
   if (plan) {
     const MoePlan P{plan};
@@ -2326,12 +2399,31 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void bf16_gemm_kernel(
     if (u0 >= uend) return;  // nothing but padding rows, which have no output
   }
   const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
+  if (!plan && m0 >= T) return;  // the second half of the last tile, past the last row
   floatx16 acc[TS::kTB][2];
   TS::template Loop<true, 0, 0>::run(
       lds, a + m0 * kStage, Kb * lda - m0 * kStage, [=](int r) { return r * kStage; }, (int)(lda * kStage),
       b + n0 * kStage, Kb * bp - n0 * kStage, [=](int r) { return plain_col_nb<2>(r) * kStage; }, (int)(bp * kStage),
       (int)(Kb / kStage), acc);
   store_bf16_tile<TS>(lds, acc, 1.0f, u0, n0, uend, N, out);
+}
+template <class TS>
+__global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void bf16_gemm_kernel(
+    const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, int64_t T, int64_t N, int64_t Kb, int64_t lda,
+    uint16_t* __restrict__ out, int tiles_m, int tiles_n, const int* __restrict__ plan, int64_t b_estride) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  int tm, tn;
+  if constexpr (TS::kTB == 4) {
+    bool half;
+    if (!tail_tile(plan ? MoePlan{plan}.ntiles() : tiles_m, tiles_n, tm, tn, half)) return;
+    if (half) {
+      bf16_gemm_tile<Tile<2, 4>>(lds, tm, tn, a, b, T, N, Kb, lda, out, plan, b_estride);
+      return;
+    }
+  } else {
+    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+  }
+  bf16_gemm_tile<TS>(lds, tm, tn, a, b, T, N, Kb, lda, out, plan, b_estride);
 }
 
 // The bf16 weight gradient's reduction: out[m, n] = bf16(sum over s
@@ -2527,23 +2619,35 @@ inline Tiling tiling(int64_t M, int64_t N, int64_t parts = 1, int second = 0) {
 }
 // The kernels with bf16 outputs have every shape; K: their K bytes.  By the
 // number of 256 x 256 tiles: 128 x 128 ones up to 128; from there on 192 x 256
-// ones where their rounds of 256 work-groups cost less (3 units a round
-// against 4) and the K loop is long enough to outweigh the larger share of
-// prologue and epilogue; else 256 x 256.  Measured (us, D = 1024, I = 3072,
-// gate/up dgrad and bf16 dgrad, 256 x 256 / 192 x 256 / 128 x 128): 16 tiles
-// 48 40 25, 91 75 46; 80 tiles 50 41 37, 93 77 71; 192 tiles 63 62 71, 126 120
-// 136; 256 tiles 77 97 89, 150 194 177; 320 tiles 121 108 113, 245 216 269;
-// 384 tiles 126 119 132, 258 242 312.  At 24 K stages (down forward, I = 1536,
-// 384 tiles) 192 x 256 is the slower one, 50 against 49.  128 x 256 tiles, one
-// per CU, were the faster ones alone at 80 tiles (34 against 37), but the
-// block's step was 3 % slower with them.  Grouped rows come in whole tiles of
-// 256, which 192-row tiles do not divide.
-inline Tiling out_tiling(int64_t M, int64_t N, int64_t K, bool grouped) {
+// ones where their rounds of 256 work-groups cost less (15 units a round
+// against 20, or 12 for a last one in halves) and the K loop is long enough to
+// outweigh the larger share of prologue and epilogue; else 256 x 256.
+// Measured (us, D = 1024, I = 3072, gate/up dgrad and bf16 dgrad, 256 x 256 /
+// 192 x 256 / 128 x 128): 16 tiles 48 40 25, 91 75 46; 80 tiles 50 41 37, 93 77
+// 71; 192 tiles 63 62 71, 126 120 136; 256 tiles 77 97 89, 150 194 177; with
+// the halves 320 tiles 106 108, 234 218; 448 tiles 138 161, 303 334; 544 tiles
+// 191 179, 381 367; 640 tiles 210 229, 407 460.  At 24 K stages (down forward,
+// I = 1536, 384 tiles) 192 x 256 is no faster.  128 x 256 tiles, one per CU,
+// were the faster ones alone at 80 tiles (34 against 37), but the block's step
+// was 3 % slower with them.  Grouped rows come in whole tiles of 256, which
+// 192-row tiles do not divide.
+inline Tiling out_shape(int64_t M, int64_t N, int64_t K, bool grouped) {
   const int64_t tiles = (int64_t)cdiv(M, kTile) * cdiv(N, kTile);
   if (tiles <= kCUs / 2) return tiling_of<2, 2>(M, N);
-  const int64_t rounds = cdiv(tiles, kCUs), rounds192 = cdiv((int64_t)cdiv(M, 192) * cdiv(N, kTile), kCUs);
-  if (!grouped && K >= 48 * kStage && 3 * rounds192 < 4 * rounds) return tiling_of<3, 4>(M, N);
+  const int64_t r = tiles % kCUs, cost = 20 * (tiles / kCUs) + (r == 0 ? 0 : 2 * r <= kCUs ? 12 : 20);
+  const int64_t cost192 = 15 * cdiv((int64_t)cdiv(M, 192) * cdiv(N, kTile), kCUs);
+  if (!grouped && K >= 48 * kStage && cost192 < cost) return tiling_of<3, 4>(M, N);
   return tiling_of<4, 4>(M, N);
+}
+// The grid of the 256 x 256 tiles and their halves (tail_tile); grouped: an
+// upper bound, the kernel reads the plan's count.
+inline Tiling with_tail(Tiling tl, bool grouped) {
+  const int n = tl.m * tl.n, r = n % kRound;
+  if (!tl.small && tl.tb == 4) tl.grid.x = (unsigned)(grouped ? n + kRound / 2 : 2 * r <= kRound ? n + r : n);
+  return tl;
+}
+inline Tiling out_tiling(int64_t M, int64_t N, int64_t K, bool grouped) {
+  return with_tail(out_shape(M, N, K, grouped), grouped);
 }
 #define OUT_KERNEL(kernel, tl) \
   ((tl).small ? kernel<Tile<2, 2>> : (tl).tb == 3 ? kernel<Tile<3, 4>> : kernel<Tile<4, 4>>)

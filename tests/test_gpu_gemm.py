@@ -372,13 +372,14 @@ def test_wgrad_rows_equals_token_contiguous(dev, M, N, T, splits):
 
 # The bf16-output GEMMs run 128 x 128 tiles up to 128 tiles of 256 x 256, then
 # 192 x 256 (K of 48 stages or more, where they take fewer rounds) or 256 x 256
-# ones: both sides of those lines in rows and in columns,
+# ones, a last round of up to 128 of these in halves: both sides of those lines in rows and in columns,
 # one row past a tile of either shape, widths that end inside one, the shortest
 # K.  The FP8 dgrad has 2I bytes of K, the bf16 GEMM 4I, the forward I.
 @pytest.mark.parametrize("T,D,I", [(1, 128, 128), (128, 272, 128), (129, 128, 384), (257, 400, 256),
                                    (8192, 1024, 128), (8193, 1040, 128),
                                    (32768, 256, 128), (32769, 256, 128), (33000, 256, 3072), (9217, 1024, 1536),
-                                   (65537, 256, 768), (66000, 256, 1536)])
+                                   (65537, 256, 768), (66000, 256, 1536),
+                                   (16641, 1024, 128), (24321, 1040, 128)])
 def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
     """Integer operands: every product and sum is exact in fp32 (at most
     64 * 6144 < 2^24), so the rounded result of every tile shape is known."""
@@ -406,11 +407,12 @@ def test_tile_shapes_of_bf16_outputs(dev, T, D, I):
 
 # The SwiGLU forwards and the down dgrad run 128-row tiles up to 128 tiles of
 # 256 rows and again from 257 to 384, the forwards at some widths
-# persistent kernels from 640 tiles of 64 column pairs: both sides of each line, with one row in
+# persistent kernels from 640 tiles of 64 column pairs, the dgrad a last round of
+# up to 128 tiles in halves: both sides of each line, with one row in
 # the last tile of either shape (whose padding rows the K-slabs keep as zeros)
 # and columns that end inside one.
 @pytest.mark.parametrize("T,D,I", [(1, 128, 128), (129, 256, 384), (4099, 256, 256), (4097, 128, 1024),
-                                   (16385, 128, 256), (32768, 128, 384), (33025, 128, 384), (12289, 256, 1024),
+                                   (16385, 128, 256), (32768, 128, 384), (33025, 128, 384), (12289, 256, 1024), (16641, 128, 1024), (25089, 128, 1408),
                                    (9984, 256, 1024), (9985, 256, 1024), (5121, 512, 1920), (5121, 512, 2048),
                                    (5121, 384, 2048), (5121, 640, 2048), (5121, 768, 2048), (4097, 1024, 2560)])
 def test_tile_shapes_of_swiglu(dev, T, D, I):
