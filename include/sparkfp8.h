@@ -313,7 +313,9 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
  * replaced by split partials summed in order: deterministic):
  * out[e] = sum over expert e's rows of at[:, t] bt[:, t]^T / (sa * sb),
  * fp32 [E, M, N]; experts without rows get zeros.  ws: fp32 workspace of
- * sfp8_moe_wgrad_workspace_floats(M, N, E) floats (may be NULL when 0). */
+ * sfp8_moe_wgrad_workspace_floats(M, N, E) floats (may be NULL when 0), room
+ * for the most splits that a call takes (sfp8_moe_wgrad_splits): with few rows
+ * it takes fewer. */
 int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E);
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E);
 int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_t M, int64_t N, int64_t E,

@@ -1547,16 +1547,16 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kern
 // (frag_offset below: each wave store instruction is one contiguous 1 KiB
 // run) and splitk_reduce_kernel sums them in split order (deterministic) and
 // scatters them to [M, N].
-// With `partials` (and always with BF16) the raw partials go to `out` as the
-// workspace, also for one split (the reductions that round to bf16 or apply
-// the optimizer's momentum stage).  BF16: bf16 operands (2 bytes per token:
-// `ldt` and `kchunk` count K bytes).
+// With `partials` the raw partials go to `out` as the workspace, also for one
+// split (the reduction that applies the optimizer's momentum stage); without,
+// there is one split and the gradient itself goes to `out` (store_grad_tile).
+// BF16: bf16 operands (2 bytes per token: `ldt` and `kchunk` count K bytes)
+// and a bf16 gradient.
 // TRA / TRB: that operand is instead a row K-slab of the token-major
 // activation ([M/64][ldt][64] or [N/64][ldt][64]: h8 and dgu8 as their
 // producers write them for the forward GEMMs), read through transposing LDS
-// reads (MainLoop TR_A / TR_B); the partials then always go to `out` as the
-// workspace, in the same order (with TRB the columns unpermuted:
-// splitk_reduce_kernel<true>).
+// reads (MainLoop TR_A / TR_B); with TRB the accumulator columns are
+// unpermuted (splitk_reduce_kernel<true>).
 // SMALL: 128 x 128 tiles (4 waves of 64 x 64, two work-groups per CU) instead
 // of 256 x 256 (8 waves of 128 x 64, one per CU); the partials' tiles and
 // accumulator order follow the shape (acc_order_rc), the sums do not.
@@ -1568,6 +1568,49 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kern
 struct TrOp {
   int64_t ts, bs, ext;
 };
+
+// One split's gradient tile, in place of its partials: the accumulators times
+// s to out[m, n] (fp32, or rounded to bf16) for m below M, n below N, through
+// LDS in passes of 64 tile rows (32 of each wave row; rows of 4 kN + 16 bytes,
+// which shift by 4 banks), so that whole tile rows are written: a lane holds
+// four consecutive columns of 32 rows.  The values are the reductions' with one
+// split.  A write, a read and a launch less: gate/up and down gradient with one
+// split (us), D = 1024, I = 3072, 1024 tokens 26 -> 15 and 18 -> 11; D = 2048, I =
+// 6144, 3000 tokens 102 -> 77 and 54 -> 38 (bf16 gate/up 161 -> 134).
+template <class TS, bool BF16, bool TRB>
+SFP8_DEV void store_grad_tile(uint8_t* lds, const floatx16 (&acc)[TS::kTB][2], float s, int64_t m0, int64_t n0,
+                              int64_t M, int64_t N, float* __restrict__ out) {
+  constexpr int kRow = 4 * TS::kN + 16, kQuads = TS::kN / 4;  // bytes of a staged row, float4s in it
+  static_assert(64 * kRow <= TS::kLds, "a pass fits the ring");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
+  const int fr = lane & 31, g = lane >> 5;
+#pragma unroll
+  for (int tb = 0; tb < TS::kTB; ++tb) {
+    if (tb) __syncthreads();  // the pass before has been read
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = 64 * wn + (TRB ? 32 * nb + 8 * i + 4 * g : 32 * g + 16 * nb + 4 * i);  // acc_order_rc
+        *reinterpret_cast<floatx4*>(lds + (32 * wm + fr) * kRow + 4 * c) =
+            floatx4{acc[tb][nb][4 * i] * s, acc[tb][nb][4 * i + 1] * s, acc[tb][nb][4 * i + 2] * s,
+                    acc[tb][nb][4 * i + 3] * s};
+      }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 64 * kQuads / TS::kThreads; ++k) {
+      const int idx = (int)threadIdx.x + TS::kThreads * k, lr = idx / kQuads, q = idx % kQuads;
+      const int64_t m = m0 + 32 * TS::kTB * (lr >> 5) + 32 * tb + (lr & 31), n = n0 + 4 * q;
+      const floatx4 v = *reinterpret_cast<const floatx4*>(lds + lr * kRow + 16 * q);
+      if (m >= M || n >= N) continue;  // N % 4 == 0: the 4 values are wholly inside or past the row
+      if constexpr (BF16)
+        *reinterpret_cast<intx2*>(reinterpret_cast<uint16_t*>(out) + m * N + n) =
+            intx2{(int)pack2_bf16(v[0], v[1]), (int)pack2_bf16(v[2], v[3])};
+      else
+        *reinterpret_cast<floatx4*>(out + m * N + n) = v;
+    }
+  }
+}
 
 template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
 __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void wgrad_kernel(
@@ -1602,7 +1645,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
         [=](int r) { return TRB ? (r / kRows) * bbs + (r % kRows) * bts : plain_col_nb<2>(r) * kStage; },
         TRB ? kRows * bts : (int)(rpb * kStage), (int)((kchunk < ldt - kb ? kchunk : ldt - kb) / kStage), acc);
   }
-  if (BF16 || TRA || TRB || partials) {
+  if (partials) {
     // accumulator order: [split][tile][wave][tb][nb][i][lane][4]
     float* frag = out + ((int64_t)sp * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kM) +
                   wave * (TS::kM * TS::kM / (TS::kThreads / 64));
@@ -1616,26 +1659,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
               floatx4{acc[tb][nb][4 * i], acc[tb][nb][4 * i + 1], acc[tb][nb][4 * i + 2], acc[tb][nb][4 * i + 3]};
     return;
   }
-  const float deq = 1.0f / (sa[0] * sb[0]);
-  float* dst = out;
-  const int fr = lane & 31, g = lane >> 5;
-  const int cb = 64 * wn + 32 * g;  // plain_col_nb<2>
-#pragma unroll
-  for (int tb = 0; tb < TS::kTB; ++tb) {
-    const int64_t m = m0 + 32 * TS::kTB * wm + 32 * tb + fr;
-    if (m >= M) continue;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-      const int64_t n = n0 + cb + 16 * nb;
-      floatx4* p = reinterpret_cast<floatx4*>(dst + m * N + n);
-      // N % 4 == 0: each float4 is wholly inside the row or wholly past it
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n + 4 * i < N)
-          p[i] = floatx4{acc[tb][nb][4 * i] * deq, acc[tb][nb][4 * i + 1] * deq, acc[tb][nb][4 * i + 2] * deq,
-                         acc[tb][nb][4 * i + 3] * deq};
-    }
-  }
+  store_grad_tile<TS, BF16, TRB>(lds, acc, BF16 ? 1.0f : 1.0f / (sa[0] * sb[0]), m0, n0, M, N, out);
 }
 
 // Grouped (MoE) weight gradient: out[e, m, n] = sum over expert e's padded
@@ -1650,8 +1674,8 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // 3.9x the algorithmic bytes at the MoE workload).  With one split it
 // writes out[e] itself; otherwise its raw partial in accumulator order to
 // ws[e][sp][tile], summed in split order by splitk_reduce_kernel.
-// BF16: bf16 operands, 2 bytes per padded row (`ldp` counts K bytes), and the
-// partials always go to ws, for bf16_wgrad_reduce_kernel to round.
+// BF16: bf16 operands, 2 bytes per padded row (`ldp` counts K bytes), and a
+// bf16 gradient (bf16_wgrad_reduce_kernel).
 template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
 __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void moe_wgrad_kernel(
     const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
@@ -1694,7 +1718,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
       TRA ? kRows * kStage : (int)(rpa * kStage), b0, b_bytes,
       [=](int r) { return TRB ? ((r / kRows) * ltok + (r % kRows)) * kStage : plain_col_nb<2>(r) * kStage; },
       TRB ? kRows * kStage : (int)(rpb * kStage), (int)nk, acc);
-  if (BF16 || TRA || TRB || splits > 1) {
+  if (splits > 1) {
     // accumulator order: [expert][split][tile][wave][tb][nb][i][lane][4]
     float* frag = ws + (((int64_t)e * splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kM) +
                   wave * (TS::kM * TS::kM / (TS::kThreads / 64));
@@ -1708,25 +1732,9 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
               floatx4{acc[tb][nb][4 * i], acc[tb][nb][4 * i + 1], acc[tb][nb][4 * i + 2], acc[tb][nb][4 * i + 3]};
     return;
   }
-  const float deq = 1.0f / (sa[0] * sb[0]);
-  float* dst = out + (int64_t)e * M * N;
-  const int fr = lane & 31, g = lane >> 5;
-  const int cb = 64 * wn + 32 * g;  // plain_col_nb<2>
-#pragma unroll
-  for (int tb = 0; tb < TS::kTB; ++tb) {
-    const int64_t m = m0 + 32 * TS::kTB * wm + 32 * tb + fr;
-    if (m >= M) continue;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-      const int64_t n = n0 + cb + 16 * nb;
-      floatx4* p = reinterpret_cast<floatx4*>(dst + m * N + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n + 4 * i < N)
-          p[i] = floatx4{acc[tb][nb][4 * i] * deq, acc[tb][nb][4 * i + 1] * deq, acc[tb][nb][4 * i + 2] * deq,
-                         acc[tb][nb][4 * i + 3] * deq};
-    }
-  }
+  const int64_t skip = (int64_t)e * M * N;
+  store_grad_tile<TS, BF16, TRB>(lds, acc, BF16 ? 1.0f : 1.0f / (sa[0] * sb[0]), m0, n0, M, N,
+                                 BF16 ? reinterpret_cast<float*>(reinterpret_cast<uint16_t*>(out) + skip) : out + skip);
 }
 
 // out[0, n) = 0: four floats per thread (n % 4 == 0, out 16-byte aligned).
@@ -2772,15 +2780,17 @@ int launch_bf16_reduce(const Tiling& tl, bool tr_b, const float* ws, int splits,
 // The split partials ws[split][tile] (one fp32 tile each, in accumulator
 // order) of the FP8 weight gradient; a_rows / b_rows: that operand is the row
 // K-slab of the token-major activation instead of a token-contiguous copy.
+// partials 0: one split, whose gradient goes to `out`.
 int wgrad_partials(const Tiling& tl, bool a_rows, bool b_rows, const void* a, const void* b, int64_t M, int64_t N,
-                   int64_t ldt, const float* sa, const float* sb, float* ws, int splits, hipStream_t st) {
+                   int64_t ldt, const float* sa, const float* sb, float* out, int splits, int partials,
+                   hipStream_t st) {
   // row K-slabs over ldt tokens
   const TrOp tra{kStage, ldt * kStage, (M / 64) * ldt * kStage}, trb{kStage, ldt * kStage, (N / 64) * ldt * kStage};
   const auto launch = a_rows ? (b_rows ? launch_wgrad<false, kFmtE5M2, kFmtE4M3, true, true>
                                        : launch_wgrad<false, kFmtE5M2, kFmtE4M3, true, false>)
                              : (b_rows ? launch_wgrad<false, kFmtE5M2, kFmtE4M3, false, true>
                                        : launch_wgrad<false, kFmtE5M2, kFmtE4M3, false, false>);
-  return launch(tl, a, b, M, N, ldt, wgrad_chunk(ldt, splits), sa, sb, ws, splits, 1, tra, trb, st);
+  return launch(tl, a, b, M, N, ldt, wgrad_chunk(ldt, splits), sa, sb, out, splits, partials, tra, trb, st);
 }
 }  // namespace
 
@@ -2940,6 +2950,50 @@ int sfp8_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_
 // ---- grouped (MoE expert) GEMMs over padded expert order (common.h) ----
 // ldp = padded rows (256 * sfp8_moe_padded_rows); plan from sfp8_moe_plan.
 namespace {
+// The modelled time (us) of `parts` M x N gradients (the experts') over
+// `stages` 64-byte K stages each, in s splits.  A stage of a 256 x 256 tile
+// takes 0.4 us, and up to 0.35 more the fuller the rounds are (the clock
+// falls); one of a 128 x 128 tile 0.3 us alone on its CU and 0.4 (bf16: 0.48)
+// beside another.  With one split the gradient is written by its own
+// work-group; several write and read 8 bytes per output each, at about 5
+// TB/s, and launch the reduction.  Measured against it (us, gradient and
+// reduction, 1 / 2 / 4 splits; the model's choice is marked): 8 experts, M =
+// 3072, N = 1024, 131072 rows 332* 362 410, 16384 rows 57* 124 181; M = 1536, N
+// = 512, 65536 rows fp8 52* 59 75, bf16 130 107* 128; 4 experts, M = 1024, N =
+// 512, 16384 rows bf16 38 31* 32; 16 experts, M = 512, N = 256 10* 19 25.
+inline double wgrad_us(int64_t M, int64_t N, int64_t parts, double stages, int64_t s, bool bf16) {
+  const Tiling tl = tiling(M, N, parts * s);
+  const int64_t n = (int64_t)tl.m * tl.n * parts * s;
+  const int64_t rounds = cdiv(n, tl.small ? 2 * kCUs : kCUs);
+  const double us = !tl.small ? 0.4 + 0.35 * (double)n / (double)(rounds * kCUs) : n <= kCUs ? 0.3 : bf16 ? 0.48 : 0.4;
+  return (double)rounds * us * stages / (double)s +
+         (s > 1 ? 2.5 + (double)s * (double)parts * (double)M * (double)N * 8.0 / 5e6 : 0.0);
+}
+// Most K splits of a grouped gradient, by which its workspace is sized before
+// its rows are known: at least 2, then doubling until the grid has 192
+// work-groups (8 at most).
+inline int64_t moe_splits_most(int64_t M, int64_t N, int64_t E) {
+  const int64_t wgs = (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * E;
+  int64_t s = 2;
+  while (s < 8 && wgs * s < 192) s *= 2;
+  return s;
+}
+// Its K splits (1, 2, 4 or 8) over ldp padded rows: more only where the model
+// gains a tenth.
+inline int64_t moe_wgrad_splits(int64_t M, int64_t N, int64_t E, int64_t ldp, bool bf16) {
+  const double stages = (double)ldp * (bf16 ? 2 : 1) / (double)kStage / (double)E;
+  const int64_t most = moe_splits_most(M, N, E);
+  int64_t best = 1;
+  double best_us = wgrad_us(M, N, E, stages, 1, bf16);
+  for (int64_t s = 2; s <= most; s *= 2) {
+    const double us = wgrad_us(M, N, E, stages, s, bf16);
+    if (us < 0.9 * best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
 inline bool moe_shape(int64_t E, int64_t D, int64_t I, int64_t ldp) {
   return E > 0 && D > 0 && I > 0 && D % 128 == 0 && I % 128 == 0 && ldp > 0 && ldp % kTile == 0;
 }
@@ -3008,20 +3062,7 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
   return status();
 }
 
-// K splits of a grouped weight gradient: enough work-groups to fill the GPU
-// (about 512) when there are few experts and tiles.
-int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E) {
-  // at least 2 splits, then doubling until the grid has 192 work-groups (8 at
-  // most): at 8 experts, D=1024, I=1536 the down gradient takes 0.234 ms with
-  // 2 splits against 0.245 with 4, the gate/up one 0.397 with 2 against 0.413
-  // with 1; at 8 experts, D=512, I=768 and 16384 rows the bf16 gate/up one 53
-  // us with its reduction with 2 (192 work-groups, one round) against 66 with 4
-  // (a round and a half, and twice the partials)
-  const int64_t wgs = (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * E;
-  int64_t s = 1;
-  while (s < 8 && (s < 2 || wgs * s < 192)) s *= 2;
-  return s;
-}
+int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E) { return moe_splits_most(M, N, E); }
 
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E) {
   const int64_t s = sfp8_moe_wgrad_splits(M, N, E);
@@ -3036,7 +3077,7 @@ int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, in
   if (fmt_a != kFmtE5M2 || fmt_b != kFmtE4M3) return kErrBadShape;
   if (!fits32(slab_rows(M), ldp) || !fits32(slab_rows(N), ldp)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
+  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, false);
   if (splits > 1 && (!ws || ws_floats < sfp8_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
@@ -3048,7 +3089,7 @@ int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, in
 
 // ---- the grouped weight gradient with row K-slab operands ----
 int64_t sfp8_moe_wgrad_rows_workspace_floats(int64_t M, int64_t N, int64_t E) {
-  return E * sfp8_moe_wgrad_splits(M, N, E) * (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * kTile * kTile;
+  return sfp8_moe_wgrad_workspace_floats(M, N, E);
 }
 
 int sfp8_moe_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, int fmt_b, int b_rows, int64_t M,
@@ -3060,7 +3101,7 @@ int sfp8_moe_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b
   if (fmt_a != kFmtE5M2 || fmt_b != kFmtE4M3) return kErrBadShape;
   if (!fits32(slab_rows(M), ldp) || !fits32(slab_rows(N), ldp)) return kErrBadShape;
   if (!al16(a) || !al16(b) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
+  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, false);
   if (ws_floats < sfp8_moe_wgrad_rows_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
@@ -3068,7 +3109,7 @@ int sfp8_moe_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b
                                        : launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, true, false>)
                              : launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, false, true>;
   const int rc = launch(tl, a, b, M, N, ldp, sa, sb, out, ws, plan, (int)splits, st);
-  if (rc) return rc;
+  if (rc || splits == 1) return rc;
   return launch_reduce(tl, b_rows, ws, (int)splits, E, M, N, sa, sb, out, st);
 }
 
@@ -3205,7 +3246,8 @@ int sfp8_bf16_moe_gemm(const void* a, const void* b, int64_t E, int64_t N, int64
 int64_t sfp8_bf16_wgrad_splits(int64_t M, int64_t N, int64_t ldt) { return wgrad_splits(M, N, 2 * ldt); }
 
 int64_t sfp8_bf16_wgrad_workspace_floats(int64_t M, int64_t N, int64_t ldt) {
-  return sfp8_bf16_wgrad_splits(M, N, ldt) * (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * kTile * kTile;
+  const int64_t s = sfp8_bf16_wgrad_splits(M, N, ldt);
+  return s > 1 ? s * (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * kTile * kTile : 0;
 }
 
 int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, int64_t ldt, void* out, float* ws,
@@ -3225,13 +3267,14 @@ int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, i
   if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   const Tiling tl = tiling(M, N, splits);
   const int rc = launch_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr,
-                                                        ws, (int)splits, 1, TrOp{}, TrOp{}, st);
-  if (rc) return rc;
+                                                        splits > 1 ? ws : (float*)out, (int)splits, splits > 1, TrOp{},
+                                                        TrOp{}, st);
+  if (rc || splits == 1) return rc;
   return launch_bf16_reduce(tl, false, ws, (int)splits, 1, M, N, out, st);
 }
 
 int64_t sfp8_bf16_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E) {
-  return E * sfp8_moe_wgrad_splits(M, N, E) * (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * kTile * kTile;
+  return sfp8_moe_wgrad_workspace_floats(M, N, E);
 }
 
 int sfp8_bf16_moe_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, int64_t E, const int* plan,
@@ -3240,13 +3283,13 @@ int sfp8_bf16_moe_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t 
   if (M <= 0 || N <= 0 || E <= 0 || N % 4 || ldp <= 0 || ldp % kTile) return kErrBadShape;
   if (!fits32(slab_rows(M), 2 * ldp) || !fits32(slab_rows(N), 2 * ldp)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
+  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, true);
   if (!ws || ws_floats < sfp8_bf16_moe_wgrad_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
-  const int rc = launch_moe_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldp, nullptr, nullptr, nullptr, ws,
-                                                            plan, (int)splits, st);
-  if (rc) return rc;
+  const int rc = launch_moe_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldp, nullptr, nullptr, (float*)out,
+                                                           ws, plan, (int)splits, st);
+  if (rc || splits == 1) return rc;
   return launch_bf16_reduce(tl, false, ws, (int)splits, E, M, N, out, st);
 }
 
@@ -3273,9 +3316,9 @@ int sfp8_bf16_gemm_wgrad_rows(const void* a, const void* x, int x_rows, int64_t 
   const TrOp tra{kStage, ldt * kStage, (M / 32) * ldt * kStage}, trb{2 * N, kStage, T * 2 * N};
   const Tiling tl = tiling(M, N, splits);
   const auto launch = x_rows ? launch_wgrad<true, 0, 0, true, true> : launch_wgrad<true, 0, 0, true, false>;
-  const int rc = launch(tl, a, x, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr, ws, (int)splits, 1, tra,
-                        x_rows ? trb : TrOp{}, st);
-  if (rc) return rc;
+  const int rc = launch(tl, a, x, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr,
+                        splits > 1 ? ws : (float*)out, (int)splits, splits > 1, tra, x_rows ? trb : TrOp{}, st);
+  if (rc || splits == 1) return rc;
   return launch_bf16_reduce(tl, x_rows, ws, (int)splits, 1, M, N, out, st);
 }
 
@@ -3285,19 +3328,19 @@ int sfp8_bf16_moe_gemm_wgrad_rows(const void* a, const void* bt, int64_t M, int6
   if (M <= 0 || N <= 0 || E <= 0 || M % 32 || N % 4 || ldp <= 0 || ldp % kTile) return kErrBadShape;
   if (!fits32(slab_rows(M), 2 * ldp) || !fits32(slab_rows(N), 2 * ldp)) return kErrBadShape;
   if (!al16(a) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = sfp8_moe_wgrad_splits(M, N, E);
+  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, true);
   if (!ws || ws_floats < sfp8_bf16_moe_wgrad_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
-  const int rc = launch_moe_wgrad<true, 0, 0, true, false>(tl, a, bt, M, N, 2 * ldp, nullptr, nullptr, nullptr, ws,
-                                                           plan, (int)splits, st);
-  if (rc) return rc;
+  const int rc = launch_moe_wgrad<true, 0, 0, true, false>(tl, a, bt, M, N, 2 * ldp, nullptr, nullptr, (float*)out,
+                                                           ws, plan, (int)splits, st);
+  if (rc || splits == 1) return rc;
   return launch_bf16_reduce(tl, false, ws, (int)splits, E, M, N, out, st);
 }
 
 // ---- the weight gradient with row K-slab operands ----
 int64_t sfp8_wgrad_rows_workspace_floats(int64_t M, int64_t N, int64_t ldt) {
-  return sfp8_wgrad_splits(M, N, ldt) * (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * kTile * kTile;
+  return sfp8_wgrad_workspace_floats(M, N, ldt);
 }
 
 int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, int fmt_b, int b_rows, int64_t M,
@@ -3318,8 +3361,9 @@ int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, in
   const int splits = (int)sfp8_wgrad_splits(M, N, ldt);
   if (ws_floats < sfp8_wgrad_rows_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   const Tiling tl = tiling(M, N, splits);
-  const int rc = wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, st);
-  if (rc) return rc;
+  const int rc =
+      wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, splits > 1 ? ws : out, splits, splits > 1, st);
+  if (rc || splits == 1) return rc;
   return launch_reduce(tl, b_rows, ws, splits, 1, M, N, sa, sb, out, st);
 }
 
@@ -3345,7 +3389,7 @@ int sfp8_gemm_wgrad_momentum(const void* a, int fmt_a, int a_rows, const void* b
   }
   const Tiling tl = tiling(M, N, splits);
   if (ldt > 0) {
-    const int rc = wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, st);
+    const int rc = wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, ws, splits, 1, st);
     if (rc) return rc;
   }
   const auto kern = tl.small ? (b_rows ? splitk_momentum_kernel<true, true> : splitk_momentum_kernel<true, false>)

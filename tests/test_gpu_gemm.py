@@ -523,3 +523,38 @@ def test_persistent_swiglu_exact_path(dev, T, D, I):
         assert torch.equal(a, gu[i:i + 512]) and torch.equal(b, h[i:i + 512])
         most = torch.maximum(most, m)
     assert torch.equal(most, amax) and amax[1] > 0 and amax[2] > 0
+
+
+# With one split (fewer than 4096 tokens) the gradient is written from its tile:
+# 128 x 128 tiles up to 128 work-groups of 256 x 256 (32 x 4 of them at 8192 x
+# 1024), 256 x 256 above; M and N that end inside a tile, a pass or a wave.
+@pytest.mark.parametrize("M,N,T", [(64, 64, 1), (192, 320, 257), (448, 192, 900), (8192, 1024, 130),
+                                   (8256, 1088, 300), (8448, 1024, 3840)])
+def test_one_split_gradients(dev, M, N, T):
+    """Integer operands (at most 64 * 3840 < 2^24, exact in fp32): fp8 in every
+    layout pair and bf16, and nothing written past the gradient."""
+    from spark_gpt_amd import _lib
+
+    ops = sg.ops
+    g = torch.Generator(device=dev).manual_seed(M + N + T)
+    ldt = ops.ldt_of(T)
+    a, b = (torch.zeros(ldt, n, device=dev) for n in (M, N))
+    for v in (a, b):
+        v[:T] = torch.randint(-8, 9, (T, v.shape[1]), generator=g, device=dev).float()
+    ref, s = a.t() @ b, torch.tensor([4.0], device=dev)
+    rows = [ops.to_slab(a.to(E5)), ops.to_slab(b.to(E4))]
+    cols = [ops.to_slab(a.to(E5).t().contiguous()), ops.to_slab(b.to(E4).t().contiguous())]
+    for ar, br in ((True, True), (True, False), (False, True)):
+        out = ops.wgrad_rows(rows[0] if ar else cols[0], rows[1] if br else cols[1], M, N, s, s, a_rows=ar, b_rows=br)
+        assert torch.equal(out, ref / 16)
+    assert torch.equal(ops.wgrad(cols[0], cols[1], M, N, s, s), ref / 16)
+    buf = torch.full((M * N + 256,), 12345.0, device=dev)
+    ws = torch.empty(max(1, _lib.query("sfp8_wgrad_rows_workspace_floats", M, N, ldt)), device=dev)
+    _lib.call("sfp8_gemm_wgrad_rows", rows[0].data_ptr(), 1, 1, rows[1].data_ptr(), 0, 1, M, N, ldt, s.data_ptr(),
+              s.data_ptr(), buf.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(buf))
+    assert torch.equal(buf[: M * N].view(M, N), ref / 16) and bool((buf[M * N:] == 12345.0).all())
+    if T < 2048:
+        gs, x = ops.to_slab(a.bfloat16()), b[:T].bfloat16().contiguous()
+        assert torch.equal(ops.bf16_wgrad_rows(gs, x, M, N), ref.bfloat16())
+        at, bt = (ops.to_slab(v.bfloat16().t().contiguous()) for v in (a, b))
+        assert torch.equal(ops.bf16_wgrad(at, bt, M, N), ref.bfloat16())
