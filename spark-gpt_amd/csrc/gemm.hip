@@ -2906,6 +2906,50 @@ static int64_t wgrad_splits(int64_t M, int64_t N, int64_t kbytes) {
   return best;
 }
 
+// The modelled time (us) of `parts` M x N gradients (the experts') over
+// `stages` 64-byte K stages each, in s splits.  A stage of a 256 x 256 tile
+// takes 0.4 us, and up to 0.35 more the fuller the rounds are (the clock
+// falls); one of a 128 x 128 tile 0.3 us alone on its CU and 0.4 (bf16: 0.48)
+// beside another.  With one split the gradient is written by its own
+// work-group; several write and read 8 bytes per output each, at about 5
+// TB/s, and launch the reduction.  Measured against it (us, gradient and
+// reduction, 1 / 2 / 4 splits; the model's choice is marked): 8 experts, M =
+// 3072, N = 1024, 131072 rows 332* 362 410, 16384 rows 57* 124 181; M = 1536, N
+// = 512, 65536 rows fp8 52* 59 75, bf16 130 107* 128; 4 experts, M = 1024, N =
+// 512, 16384 rows bf16 38 31* 32; 16 experts, M = 512, N = 256 10* 19 25.
+static inline double wgrad_us(int64_t M, int64_t N, int64_t parts, double stages, int64_t s, bool bf16) {
+  const Tiling tl = tiling(M, N, parts * s);
+  const int64_t n = (int64_t)tl.m * tl.n * parts * s;
+  const int64_t rounds = cdiv(n, tl.small ? 2 * kCUs : kCUs);
+  const double us = !tl.small ? 0.4 + 0.35 * (double)n / (double)(rounds * kCUs) : n <= kCUs ? 0.3 : bf16 ? 0.48 : 0.4;
+  return (double)rounds * us * stages / (double)s +
+         (s > 1 ? 2.5 + (double)s * (double)parts * (double)M * (double)N * 8.0 / 5e6 : 0.0);
+}
+// The K splits that a dense call takes: those of wgrad_splits, which counts
+// rounds of 256 x 256 tiles only and sizes the workspace, or one or two splits
+// where this model, which knows the smaller tiles, gains a twentieth or so
+// (counts between, taken at 24 tiles and 49152 tokens, were no slower alone but
+// made the block's step 4 % slower).  Measured (us, gradient and reduction):
+// gate/up, D = 1024, I = 3072, 5003 tokens 51 -> 36 (2 -> 1 splits), 8192 67 ->
+// 52, 16384 109 -> 100; D = 2048, I = 6144, 16384 tokens 355 -> 329; bf16, D =
+// 1024, I = 3072, 16384 tokens 200 -> 182 (5 -> 2); within 3 % of each other
+// where the model is near even.
+static int64_t dense_splits(int64_t M, int64_t N, int64_t kbytes, bool bf16) {
+  const int64_t most = wgrad_splits(M, N, kbytes);
+  const double stages = (double)kbytes / (double)kStage;
+  int64_t best = most;
+  double best_us = 0.96 * wgrad_us(M, N, 1, stages, most, bf16);
+  for (int64_t s = 1; s <= 2 && s < most; ++s) {
+    if (!wgrad_split_ok(s, kbytes)) continue;
+    const double us = wgrad_us(M, N, 1, stages, s, bf16);
+    if (us < best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 int64_t sfp8_wgrad_splits(int64_t M, int64_t N, int64_t ldt) { return wgrad_splits(M, N, ldt); }
 
 int64_t sfp8_slab_bytes(int64_t rows, int64_t k) {
@@ -2930,7 +2974,7 @@ int sfp8_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_
   if (!fits32(slab_rows(M), ldt) || !fits32(slab_rows(N), ldt)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out)) return kErrBadAlignment;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t splits = sfp8_wgrad_splits(M, N, ldt);
+  const int64_t splits = dense_splits(M, N, ldt, false);
   if (splits > 1 && (!ws || ws_floats < sfp8_wgrad_workspace_floats(M, N, ldt))) return kErrWorkspaceTooSmall;
   if (ldt == 0) {
     // no tokens: the gradient is zero (a fill kernel, not a memset node, so
@@ -2950,25 +2994,6 @@ int sfp8_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_
 // ---- grouped (MoE expert) GEMMs over padded expert order (common.h) ----
 // ldp = padded rows (256 * sfp8_moe_padded_rows); plan from sfp8_moe_plan.
 namespace {
-// The modelled time (us) of `parts` M x N gradients (the experts') over
-// `stages` 64-byte K stages each, in s splits.  A stage of a 256 x 256 tile
-// takes 0.4 us, and up to 0.35 more the fuller the rounds are (the clock
-// falls); one of a 128 x 128 tile 0.3 us alone on its CU and 0.4 (bf16: 0.48)
-// beside another.  With one split the gradient is written by its own
-// work-group; several write and read 8 bytes per output each, at about 5
-// TB/s, and launch the reduction.  Measured against it (us, gradient and
-// reduction, 1 / 2 / 4 splits; the model's choice is marked): 8 experts, M =
-// 3072, N = 1024, 131072 rows 332* 362 410, 16384 rows 57* 124 181; M = 1536, N
-// = 512, 65536 rows fp8 52* 59 75, bf16 130 107* 128; 4 experts, M = 1024, N =
-// 512, 16384 rows bf16 38 31* 32; 16 experts, M = 512, N = 256 10* 19 25.
-inline double wgrad_us(int64_t M, int64_t N, int64_t parts, double stages, int64_t s, bool bf16) {
-  const Tiling tl = tiling(M, N, parts * s);
-  const int64_t n = (int64_t)tl.m * tl.n * parts * s;
-  const int64_t rounds = cdiv(n, tl.small ? 2 * kCUs : kCUs);
-  const double us = !tl.small ? 0.4 + 0.35 * (double)n / (double)(rounds * kCUs) : n <= kCUs ? 0.3 : bf16 ? 0.48 : 0.4;
-  return (double)rounds * us * stages / (double)s +
-         (s > 1 ? 2.5 + (double)s * (double)parts * (double)M * (double)N * 8.0 / 5e6 : 0.0);
-}
 // Most K splits of a grouped gradient, by which its workspace is sized before
 // its rows are known: at least 2, then doubling until the grid has 192
 // work-groups (8 at most).
@@ -3263,7 +3288,7 @@ int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, i
     hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, (float*)out, n);
     return status();
   }
-  const int64_t splits = sfp8_bf16_wgrad_splits(M, N, ldt);
+  const int64_t splits = dense_splits(M, N, 2 * ldt, true);
   if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   const Tiling tl = tiling(M, N, splits);
   const int rc = launch_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr,
@@ -3308,7 +3333,7 @@ int sfp8_bf16_gemm_wgrad_rows(const void* a, const void* x, int x_rows, int64_t 
     hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, (float*)out, n);
     return status();
   }
-  const int64_t splits = sfp8_bf16_wgrad_splits(M, N, ldt);
+  const int64_t splits = dense_splits(M, N, 2 * ldt, true);
   if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   // a: the bf16 K-slab of [ldt, M] (32 columns per 64-byte row); x (x_rows):
   // row-major [T, N] bf16, tokens T..ldt-1 read as zero through the range
@@ -3358,7 +3383,7 @@ int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, in
     hipLaunchKernelGGL(zero_fill_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, st, out, n);
     return status();
   }
-  const int splits = (int)sfp8_wgrad_splits(M, N, ldt);
+  const int splits = (int)dense_splits(M, N, ldt, false);
   if (ws_floats < sfp8_wgrad_rows_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   const Tiling tl = tiling(M, N, splits);
   const int rc =
@@ -3384,7 +3409,7 @@ int sfp8_gemm_wgrad_momentum(const void* a, int fmt_a, int a_rows, const void* b
   hipStream_t st = (hipStream_t)stream;
   int splits = 0;
   if (ldt > 0) {
-    splits = (int)sfp8_wgrad_splits(M, N, ldt);
+    splits = (int)dense_splits(M, N, ldt, false);
     if (ws_floats < sfp8_wgrad_momentum_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
   }
   const Tiling tl = tiling(M, N, splits);

@@ -525,13 +525,15 @@ def test_persistent_swiglu_exact_path(dev, T, D, I):
     assert torch.equal(most, amax) and amax[1] > 0 and amax[2] > 0
 
 
-# With one split (fewer than 4096 tokens) the gradient is written from its tile:
+# With one split (few tokens) the gradient is written from its tile:
 # 128 x 128 tiles up to 128 work-groups of 256 x 256 (32 x 4 of them at 8192 x
-# 1024), 256 x 256 above; M and N that end inside a tile, a pass or a wave.
+# 1024), 256 x 256 above; M and N that end inside a tile, a pass or a wave; from
+# 5003 tokens on sizes that take fewer splits than the most.
 @pytest.mark.parametrize("M,N,T", [(64, 64, 1), (192, 320, 257), (448, 192, 900), (8192, 1024, 130),
-                                   (8256, 1088, 300), (8448, 1024, 3840)])
+                                   (8256, 1088, 300), (8448, 1024, 3840), (6144, 1024, 5003),
+                                   (1024, 3072, 5003), (6144, 1024, 16384), (12288, 2048, 16384)])
 def test_one_split_gradients(dev, M, N, T):
-    """Integer operands (at most 64 * 3840 < 2^24, exact in fp32): fp8 in every
+    """Integer operands (at most 64 * 16384 < 2^24, exact in fp32): fp8 in every
     layout pair and bf16, and nothing written past the gradient."""
     from spark_gpt_amd import _lib
 
@@ -553,8 +555,7 @@ def test_one_split_gradients(dev, M, N, T):
     _lib.call("sfp8_gemm_wgrad_rows", rows[0].data_ptr(), 1, 1, rows[1].data_ptr(), 0, 1, M, N, ldt, s.data_ptr(),
               s.data_ptr(), buf.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(buf))
     assert torch.equal(buf[: M * N].view(M, N), ref / 16) and bool((buf[M * N:] == 12345.0).all())
-    if T < 2048:
-        gs, x = ops.to_slab(a.bfloat16()), b[:T].bfloat16().contiguous()
-        assert torch.equal(ops.bf16_wgrad_rows(gs, x, M, N), ref.bfloat16())
-        at, bt = (ops.to_slab(v.bfloat16().t().contiguous()) for v in (a, b))
-        assert torch.equal(ops.bf16_wgrad(at, bt, M, N), ref.bfloat16())
+    gs, x = ops.to_slab(a.bfloat16()), b[:T].bfloat16().contiguous()
+    assert torch.equal(ops.bf16_wgrad_rows(gs, x, M, N), ref.bfloat16())
+    at, bt = (ops.to_slab(v.bfloat16().t().contiguous()) for v in (a, b))
+    assert torch.equal(ops.bf16_wgrad(at, bt, M, N), ref.bfloat16())
