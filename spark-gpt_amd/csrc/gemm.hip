@@ -1612,17 +1612,13 @@ SFP8_DEV void store_grad_tile(uint8_t* lds, const floatx16 (&acc)[TS::kTB][2], f
   }
 }
 
-template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
-__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void wgrad_kernel(
-    const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldt,
+template <class TS, bool BF16, int FMT_A, int FMT_B, bool TRA, bool TRB>
+SFP8_DEV void wgrad_tile(
+    uint8_t* lds, int tm, int tn, int sp, const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldt,
     int64_t kchunk, const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out,
-    int tiles_m, int tiles_n, int splits, int partials, TrOp tra, TrOp trb) {
-  using TS = TileShape<SMALL>;
-  extern __shared__ __align__(16) uint8_t lds[];
-  int tm, tn, sp;
-  split_tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, splits, tm, tn, sp);
-  if (sp >= splits) return;  // grid padding (work-group uniform)
-  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+    int tiles_m, int tiles_n, int partials, TrOp tra, TrOp trb) {
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
+  if (m0 >= M) return;  // the second half of a tile past the last row (work-group uniform)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   floatx16 acc[TS::kTB][2];
@@ -1647,8 +1643,8 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   }
   if (partials) {
     // accumulator order: [split][tile][wave][tb][nb][i][lane][4]
-    float* frag = out + ((int64_t)sp * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kM) +
-                  wave * (TS::kM * TS::kM / (TS::kThreads / 64));
+    float* frag = out + ((int64_t)sp * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kN) +
+                  wave * (TS::kM * TS::kN / (TS::kThreads / 64));
 #pragma unroll
     for (int tb = 0; tb < TS::kTB; ++tb)
 #pragma unroll
@@ -1660,6 +1656,30 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     return;
   }
   store_grad_tile<TS, BF16, TRB>(lds, acc, BF16 ? 1.0f : 1.0f / (sa[0] * sb[0]), m0, n0, M, N, out);
+}
+template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void wgrad_kernel(
+    const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldt,
+    int64_t kchunk, const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out,
+    int tiles_m, int tiles_n, int splits, int partials, TrOp tra, TrOp trb) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  int tm, tn, sp = 0;
+  if (!SMALL && !partials) {
+    // one split: the last round in halves (tail_tile); a block's step, 16384
+    // tokens, D = 2048, I = 6144 (384 gate/up tiles), 1963 -> 1940 us
+    bool half;
+    if (!tail_tile(tiles_m, tiles_n, tm, tn, half)) return;
+    if (half) {
+      wgrad_tile<Tile<2, 4>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, 0, at, bt, M, N, ldt, kchunk, sa, sb, out,
+                                                           tiles_m, tiles_n, 0, tra, trb);
+      return;
+    }
+  } else {
+    split_tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, splits, tm, tn, sp);
+    if (sp >= splits) return;  // grid padding (work-group uniform)
+  }
+  wgrad_tile<TileShape<SMALL>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, sp, at, bt, M, N, ldt, kchunk, sa, sb, out,
+                                                             tiles_m, tiles_n, partials, tra, trb);
 }
 
 // Grouped (MoE) weight gradient: out[e, m, n] = sum over expert e's padded
@@ -1676,20 +1696,14 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // ws[e][sp][tile], summed in split order by splitk_reduce_kernel.
 // BF16: bf16 operands, 2 bytes per padded row (`ldp` counts K bytes), and a
 // bf16 gradient (bf16_wgrad_reduce_kernel).
-template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
-__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void moe_wgrad_kernel(
-    const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
+template <class TS, bool BF16, int FMT_A, int FMT_B, bool TRA, bool TRB>
+SFP8_DEV void moe_wgrad_tile(
+    uint8_t* lds, int tm, int tn, int e, int sp, const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
     const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out, float* __restrict__ ws,
     const int* __restrict__ plan, int tiles_m, int tiles_n, int splits) {
-  using TS = TileShape<SMALL>;
-  extern __shared__ __align__(16) uint8_t lds[];
   const MoePlan P{plan};
-  const int tiles = tiles_m * tiles_n;
-  const int lid = xcd_run(blockIdx.x, gridDim.x);
-  const int sp = (lid / tiles) % splits, e = lid / (tiles * splits);
-  int tm, tn;
-  raster(lid % tiles, tiles_m, tiles_n, tm, tn);
-  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kM;
+  const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
+  if (m0 >= M) return;  // the second half of a tile past the last row (work-group uniform)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   constexpr int64_t kBpe = BF16 ? 2 : 1;  // K bytes per padded row
@@ -1720,8 +1734,8 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
       TRB ? kRows * kStage : (int)(rpb * kStage), (int)nk, acc);
   if (splits > 1) {
     // accumulator order: [expert][split][tile][wave][tb][nb][i][lane][4]
-    float* frag = ws + (((int64_t)e * splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kM) +
-                  wave * (TS::kM * TS::kM / (TS::kThreads / 64));
+    float* frag = ws + (((int64_t)e * splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kN) +
+                  wave * (TS::kM * TS::kN / (TS::kThreads / 64));
 #pragma unroll
     for (int tb = 0; tb < TS::kTB; ++tb)
 #pragma unroll
@@ -1735,6 +1749,41 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
   const int64_t skip = (int64_t)e * M * N;
   store_grad_tile<TS, BF16, TRB>(lds, acc, BF16 ? 1.0f : 1.0f / (sa[0] * sb[0]), m0, n0, M, N,
                                  BF16 ? reinterpret_cast<float*>(reinterpret_cast<uint16_t*>(out) + skip) : out + skip);
+}
+template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TRB = false>
+__global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void moe_wgrad_kernel(
+    const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
+    const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out, float* __restrict__ ws,
+    const int* __restrict__ plan, int tiles_m, int tiles_n, int splits, int experts) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int tiles = tiles_m * tiles_n, n = tiles * splits * experts, pid = blockIdx.x;
+  int tm, tn;
+  if constexpr (!SMALL) {
+    // one split: the last round in halves, as tail_tile (the run of full tiles
+    // is the grid's without them); 8 experts, 131072 rows, D = 1024, I = 1536
+    // (384 gate/up tiles), the experts' step 2344 -> 2329 us
+    const int full = splits == 1 ? tail_full(n, kRound) : n;
+    if (pid >= full) {
+      const int lid = full + ((pid - full) >> 1);
+      if (lid >= n) return;
+      raster(lid % tiles, tiles_m, tiles_n, tm, tn);
+      moe_wgrad_tile<Tile<2, 4>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, 2 * tm + ((pid - full) & 1), tn, lid / tiles, 0, at,
+                                                               bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
+                                                               1);
+      return;
+    }
+    const int lid = xcd_run(pid, full);
+    raster(lid % tiles, tiles_m, tiles_n, tm, tn);
+    moe_wgrad_tile<Tile<4, 4>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, lid / (tiles * splits), (lid / tiles) % splits,
+                                                             at, bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
+                                                             splits);
+  } else {
+    const int lid = xcd_run(pid, gridDim.x);
+    raster(lid % tiles, tiles_m, tiles_n, tm, tn);
+    moe_wgrad_tile<Tile<2, 2>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, lid / (tiles * splits), (lid / tiles) % splits,
+                                                             at, bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
+                                                             splits);
+  }
 }
 
 // out[0, n) = 0: four floats per thread (n % 4 == 0, out 16-byte aligned).
@@ -2732,7 +2781,8 @@ int launch_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, int6
                              : wgrad_kernel<false, BF16, FMT_A, FMT_B, TRA, TRB>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  const dim3 grid = BF16 || tl.small ? tl.grid : dim3((unsigned)wgrad_grid(tl.m * tl.n, splits));
+  const dim3 grid = !partials ? with_tail(tl, false).grid
+                    : BF16 || tl.small ? tl.grid : dim3((unsigned)wgrad_grid(tl.m * tl.n, splits));
   hipLaunchKernelGGL(kern, grid, tl.block, tl.lds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldt, chunk, sa, sb,
                      out, tl.m, tl.n, splits, partials, tra, trb);
   return status();
@@ -2748,8 +2798,10 @@ int launch_moe_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, 
                              : moe_wgrad_kernel<false, BF16, FMT_A, FMT_B, TRA, TRB>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(kern, tl.grid, tl.block, tl.lds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out,
-                     ws, plan, tl.m, tl.n, splits);
+  const int n = (int)tl.grid.x, r = n % kRound;
+  const dim3 grid(!tl.small && splits == 1 && 2 * r <= kRound ? n + r : n);
+  hipLaunchKernelGGL(kern, grid, tl.block, tl.lds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out, ws,
+                     plan, tl.m, tl.n, splits, n / (tl.m * tl.n * splits));
   return status();
 }
 
@@ -2922,7 +2974,9 @@ static inline double wgrad_us(int64_t M, int64_t N, int64_t parts, double stages
   const int64_t n = (int64_t)tl.m * tl.n * parts * s;
   const int64_t rounds = cdiv(n, tl.small ? 2 * kCUs : kCUs);
   const double us = !tl.small ? 0.4 + 0.35 * (double)n / (double)(rounds * kCUs) : n <= kCUs ? 0.3 : bf16 ? 0.48 : 0.4;
-  return (double)rounds * us * stages / (double)s +
+  const int64_t r = n % kCUs;  // one split's last round in halves costs 0.6
+  const double cost = !tl.small && s == 1 && r > 0 && 2 * r <= kCUs ? (double)rounds - 0.4 : (double)rounds;
+  return cost * us * stages / (double)s +
          (s > 1 ? 2.5 + (double)s * (double)parts * (double)M * (double)N * 8.0 / 5e6 : 0.0);
 }
 // The K splits that a dense call takes: those of wgrad_splits, which counts

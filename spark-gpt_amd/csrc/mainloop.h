@@ -134,7 +134,7 @@ struct MainLoop {
   static constexpr int kWM = TM / (32 * TB);                // wave rows
   static constexpr int kStageA = TM * kStage;               // bytes of A per stage
   static constexpr int kWaves = kWM * WN;
-  static_assert(!(TR_A || TR_B) || (!PAIRED && 32 * NB * WN == TM), "transposing reads: plain, square tiles");
+  static_assert(!(TR_A || TR_B) || !PAIRED, "transposing reads: plain tiles");
   static constexpr bool kTr = TR_A || TR_B;
   using Rsrc = typename std::conditional<kTr, intx4, __amdgpu_buffer_rsrc_t>::type;
   static SFP8_DEV Rsrc rsrc(const void* base, int64_t bytes) {

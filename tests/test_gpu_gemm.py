@@ -527,11 +527,13 @@ def test_persistent_swiglu_exact_path(dev, T, D, I):
 
 # With one split (few tokens) the gradient is written from its tile:
 # 128 x 128 tiles up to 128 work-groups of 256 x 256 (32 x 4 of them at 8192 x
-# 1024), 256 x 256 above; M and N that end inside a tile, a pass or a wave; from
+# 1024), 256 x 256 above, a last round of up to 128 in halves;
+# M and N that end inside a tile, a half, a pass or a wave; from
 # 5003 tokens on sizes that take fewer splits than the most.
 @pytest.mark.parametrize("M,N,T", [(64, 64, 1), (192, 320, 257), (448, 192, 900), (8192, 1024, 130),
                                    (8256, 1088, 300), (8448, 1024, 3840), (6144, 1024, 5003),
-                                   (1024, 3072, 5003), (6144, 1024, 16384), (12288, 2048, 16384)])
+                                   (1024, 3072, 5003), (6144, 1024, 16384), (12288, 2048, 16384),
+                                   (16448, 1088, 300), (8256, 2304, 200)])
 def test_one_split_gradients(dev, M, N, T):
     """Integer operands (at most 64 * 16384 < 2^24, exact in fp32): fp8 in every
     layout pair and bf16, and nothing written past the gradient."""

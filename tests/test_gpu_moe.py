@@ -357,10 +357,12 @@ def test_moe_weight_cache_refresh(dev, monkeypatch):
 # 128 x 128 tiles up to 128 work-groups of 256 x 256 (tiles x splits x
 # experts), the larger ones from there on: both sides, widths that end inside
 # a tile of either shape, experts without rows and with one; few rows per
-# expert take one split (the gradient written from its tile), many several.
+# expert take one split (the gradient written from its tile, a last round of up
+# to 128 larger ones in halves), many several.
 @pytest.mark.parametrize("M_,N_,counts", [(320, 192, [300, 0, 513]), (64, 64, [1]), (512, 256, [256, 257] * 4),
                                           (576, 320, [129, 0, 700, 1] * 3), (64, 64, [3000, 0, 513]),
-                                          (320, 192, [20000, 1, 0, 9000]), (3072, 1024, [257] * 5)])
+                                          (320, 192, [20000, 1, 0, 9000]), (3072, 1024, [257] * 5),
+                                          (2880, 1088, [300, 0, 129, 700, 1])])
 def test_moe_wgrad_tile_shapes(dev, M_, N_, counts):
     """Integer operands: every product and partial sum is exact in fp32 (at
     most 64 * 20000 < 2^24), so each expert's gradient is known exactly."""
