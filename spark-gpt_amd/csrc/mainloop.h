@@ -114,8 +114,8 @@ SFP8_DEV void sched_interleave_valu() {
 // gradient reduces over -- and each fragment is assembled from four
 // transposing reads (ds_read_b64_tr_b8: 8 tokens of one column per lane;
 // ds_read_b64_tr_b16: 4 tokens) in the same (lane half, K) order as the plain
-// reads, so the MFMAs see the same values.  Only for a plain (unpaired) B of
-// 256 rows.  With TR_B the B tile is not permuted: accumulator v of block nb
+// reads, so the MFMAs see the same values.  Only for a plain (unpaired) B.
+// With TR_B the B tile is not permuted: accumulator v of block nb
 // in lane half g is column 32 nb + 8 (v / 4) + 4 g + v % 4 of the wave's
 // 32 NB.  These
 // instantiations issue their DMA as inline asm: the compiler treats a
