@@ -1979,86 +1979,122 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // bf16(x W^T), for up to 64 rows of x and W row-major [2I, D] bf16 as the
 // caller has it.  The call reads W once and little else, so it is bound by the
 // memory's bandwidth and latency: a work-group of 8 waves takes 16 gate and
-// the 16 up rows of W, the waves share K (wave w the 32-wide K steps w, w + 8,
-// ...), and each requests several steps' rows before it uses any.  The MFMA's
-// A operand is W (16 rows), its B operand 16 rows of x, so a lane ends with
-// four consecutive columns of one row of x; the waves' sums are added through
-// LDS in wave order.  NT = 16-row tiles of x; rows past T repeat the last and
-// are not written.  Measured (us, laying W out as K-slabs and the tiled kernel
-// -> this one): D = 1024, I = 3072, 8 rows 19 -> 4.4 (2.9 TB/s), 64 rows 19 ->
-// 7.8; D = 2048, I = 8192, 8 rows 41 -> 12.6 (5.3 TB/s).  From 65 rows on the
-// tiled kernel with row-major W takes over: 10.3 at 65, D = 1024 (and no slower
-// than on K-slabs: 29 against 32 at 2017 rows).
+// the 16 up rows of W (one MFMA's 32) against NT tiles of 32 rows of x.  K runs
+// in chunks of 128 through a ring of kRing LDS slots, kRing - 1 of them in
+// flight; all waves load, wave t multiplies x tile t.  One chain of MFMAs runs
+// over the whole K, 16 at a time, with the K values of MainLoop's fragments in
+// MainLoop's order, so that a row's h has the bytes of the tiled kernels,
+// training's and those from 65 rows on (K shared by the waves and their sums
+// added differed from them in the last bit now and then, and was no faster: us
+// at 1, 8 and 64 rows with weights out of the caches, D = 1024, I = 3072, 5.4 5.8
+// 9.6 -> 5.5 5.5 7.1 (2.3 TB/s at 8 rows); D = 2048, I = 8192, 17.2 18.5 29.5 ->
+// 17.5 17.9 21.5 (3.7 TB/s); D = 256, I = 1024, 2.8 3.0 3.9 -> 3.0 3.1 3.3).  At 65
+// rows the tiled kernel takes 16.4, 31.6 and 6.1.
+// LDS rows are 128 bytes (64 of K); row r keeps its 16-byte chunk c at c ^ ((r
+// >> 1) & 7), so that 16 lanes reading one chunk of 16 rows meet every bank
+// once.  Rows of x past T lie past the descriptor's records and cost no traffic.
 constexpr int kEvalRows = 64;  // most rows of x
+template <int NT>
+struct EvalShape {
+  static constexpr int kRows = 32 + 32 * NT;     // LDS rows of a 64-wide K step: W, then x
+  static constexpr int kSteps = 2;               // K steps of 64 in a chunk
+  static constexpr int kSlot = kSteps * kRows * 128;
+  static constexpr int kRing = NT == 1 ? 4 : 3;  // two work-groups fit a CU
+  static constexpr int kLds = kRing * kSlot;
+  static constexpr int kDma = 1 + NT;            // 1 KiB loads of each wave per chunk
+};
 template <int NT>
 __global__ __launch_bounds__(512) void bf16_swiglu_eval_kernel(const uint16_t* __restrict__ x,
                                                                const uint16_t* __restrict__ w, int T, int D, int I,
                                                                uint16_t* __restrict__ h) {
-  constexpr int kU = NT == 1 ? 4 : 2;  // K steps requested at once
-  __shared__ floatx4 part[8][NT][2][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int64_t n0 = (int64_t)blockIdx.x * 16;
-  const int steps = D / 32;
-  const uint16_t* wg = w + (n0 + r) * D + 8 * q;
-  const uint16_t* wu = w + (I + n0 + r) * D + 8 * q;
-  const uint16_t* xr[NT];
+  using S = EvalShape<NT>;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 31, g = lane >> 5;
+  const int n0 = (int)blockIdx.x * 16, ldx = 2 * D;
+  const int steps = D / 64, chunks = (steps + S::kSteps - 1) / S::kSteps;
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(w, (int64_t)2 * I * ldx), rx = make_rsrc(x, (int64_t)T * ldx);
+  // a load covers 8 rows of 128 bytes; this wave's: row group j of W in K step
+  // wave / 4, and of x (NT = 1: the same) in one (NT = 2: each) step
+  const auto chunk_of = [=](int row) { return (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) << 4); };
+  const int wj = wave & 3, wr = 8 * wj + (lane >> 3);
+  const int xj = NT == 1 ? wj : wave, xr = 8 * xj + (lane >> 3);
+  const uint32_t voff_w = (uint32_t)(((wr >> 4) * I + n0 + (wr & 15)) * ldx) + chunk_of(wr);
+  const uint32_t voff_x = (uint32_t)(xr * ldx) + chunk_of(xr);
+  const auto load = [&](int c) {  // chunk c; steps past the last are aimed out of range
+    uint8_t* slot = lds + (c % S::kRing) * S::kSlot;
+    const int s0 = c * S::kSteps + (wave >> 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(slot + (wave >> 2) * S::kRows * 128 + wj * 1024), 16,
+                                             s0 < steps ? voff_w + 128 * s0 : 0x80000000u, 0, 0, 0);
 #pragma unroll
-  for (int t = 0; t < NT; ++t) xr[t] = x + (int64_t)(16 * t + r < T ? 16 * t + r : T - 1) * D + 8 * q;
-  floatx4 ag[NT], au[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) ag[t] = au[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const auto at = [](const uint16_t* p, int s) { return *reinterpret_cast<const bf16x8*>(p + 32 * s); };
-  int s = wave;
-  for (; s + 8 * (kU - 1) < steps; s += 8 * kU) {
-    bf16x8 g[kU], u[kU], v[kU][NT];
-#pragma unroll
-    for (int k = 0; k < kU; ++k) {
-      g[k] = at(wg, s + 8 * k);
-      u[k] = at(wu, s + 8 * k);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) v[k][t] = at(xr[t], s + 8 * k);
+    for (int i = 0; i < NT; ++i) {
+      const int st = NT == 1 ? wave >> 2 : i, s = c * S::kSteps + st;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t)(slot + (st * S::kRows + 32) * 128 + xj * 1024), 16,
+                                               s < steps ? voff_x + 128 * s : 0x80000000u, 0, 0, 0);
     }
+  };
+  for (int c = 0; c < S::kRing - 1; ++c) load(c);
+  floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  // a chunk's operands, in the order of MainLoop's fragments: per 64 bytes of a
+  // row the lane half's first 16-byte chunk, then its second
+  struct Frag {
+    bf16x8 w[4 * S::kSteps], x[4 * S::kSteps];
+  };
+  const auto read = [&](Frag& f, int c) {
+    const uint8_t* pw = lds + (c % S::kRing) * S::kSlot + fr * 128;
 #pragma unroll
-    for (int k = 0; k < kU; ++k)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        ag[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g[k], v[k][t], ag[t], 0, 0, 0);
-        au[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u[k], v[k][t], au[t], 0, 0, 0);
-      }
-  }
-  for (; s < steps; s += 8) {
-    const bf16x8 g = at(wg, s), u = at(wu, s);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const bf16x8 v = at(xr[t], s);
-      ag[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g, v, ag[t], 0, 0, 0);
-      au[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u, v, au[t], 0, 0, 0);
+    for (int k = 0; k < 4 * S::kSteps; ++k) {
+      const int at = (k >> 2) * S::kRows * 128 + (((2 * (k & 2) + 2 * g + (k & 1)) ^ ((fr >> 1) & 7)) << 4);
+      f.w[k] = *reinterpret_cast<const bf16x8*>(pw + at);
+      f.x[k] = *reinterpret_cast<const bf16x8*>(pw + (32 + 32 * wave) * 128 + at);
     }
-  }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const auto multiply = [&](const Frag& f, int nk) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    part[wave][t][0][lane] = ag[t];
-    part[wave][t][1][lane] = au[t];
-  }
-  __syncthreads();
-  if (wave >= NT) return;
-  floatx4 g = part[0][wave][0][lane], u = part[0][wave][1][lane];
+    for (int st = 0; st < S::kSteps; ++st) {
+      if (st >= nk) break;
 #pragma unroll
-  for (int k = 1; k < 8; ++k) {
-    g += part[k][wave][0][lane];
-    u += part[k][wave][1][lane];
+      for (int k = 4 * st; k < 4 * st + 4; ++k)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[k], f.x[k], acc, 0, 0, 0);
+    }
+  };
+  // chunk c has landed, and every wave's reads of chunk c - 1, whose slot the
+  // next load fills, are done; its operands come while chunk c - 1 multiplies
+  const auto chunk = [&](int c, Frag& cur, const Frag& prev) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::kDma * (S::kRing - 2)) : "memory");
+    load(c + S::kRing - 1);
+    if (wave >= NT) return;
+    read(cur, c);
+    if (c) multiply(prev, S::kSteps);
+  };
+  Frag f0, f1;
+  for (int c = 0; c < chunks; c += 2) {
+    chunk(c, f0, f1);
+    if (c + 1 < chunks) chunk(c + 1, f1, f0);
   }
-  const int row = 16 * wave + r;
-  if (row >= T) return;
-  uint32_t o[2];
+  if (wave < NT) {
+    const int last = steps - (chunks - 1) * S::kSteps;
+    if (chunks & 1) multiply(f0, last);
+    else multiply(f1, last);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past the last chunk
+  // accumulator 4 q + i is W row 8 q + 4 g + i of the 32: gate for q < 2, up of
+  // the same columns for q + 2
+  const int row = 32 * wave + fr;
+  if (wave >= NT || row >= T) return;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    float g0 = g[2 * i], g1 = g[2 * i + 1], u0 = u[2 * i], u1 = u[2 * i + 1];
-    round2_bf16(g0, g1);
-    round2_bf16(u0, u1);
-    o[i] = pack2_bf16(g0 * sigmoid_fast(g0) * u0, g1 * sigmoid_fast(g1) * u1);
+  for (int q = 0; q < 2; ++q) {
+    uint32_t o[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int v = 4 * q + 2 * i;
+      float g0 = acc[v], g1 = acc[v + 1], u0 = acc[8 + v], u1 = acc[8 + v + 1];
+      round2_bf16(g0, g1);
+      round2_bf16(u0, u1);
+      o[i] = pack2_bf16(g0 * sigmoid_fast(g0) * u0, g1 * sigmoid_fast(g1) * u1);
+    }
+    *reinterpret_cast<intx2*>(h + (int64_t)row * I + n0 + 8 * q + 4 * g) = intx2{(int)o[0], (int)o[1]};
   }
-  *reinterpret_cast<intx2*>(h + (int64_t)row * I + n0 + 4 * q) = intx2{(int)o[0], (int)o[1]};
 }
 
 // The bf16 gate/up forward, persistent, with the SwiGLU of each tile under the
@@ -3273,12 +3309,11 @@ int sfp8_bf16_swiglu_eval(const void* x, const void* w, int64_t T, int64_t D, in
   if (T == 0) return kOk;
   hipStream_t st = (hipStream_t)stream;
   if (T <= kEvalRows) {
-    const auto kern = T <= 16   ? bf16_swiglu_eval_kernel<1>
-                      : T <= 32 ? bf16_swiglu_eval_kernel<2>
-                      : T <= 48 ? bf16_swiglu_eval_kernel<3>
-                                : bf16_swiglu_eval_kernel<4>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(I / 16)), dim3(512), 0, st, (const uint16_t*)x, (const uint16_t*)w, (int)T,
-                       (int)D, (int)I, (uint16_t*)h);
+    const auto kern = T <= 32 ? bf16_swiglu_eval_kernel<1> : bf16_swiglu_eval_kernel<2>;
+    const int lds = T <= 32 ? EvalShape<1>::kLds : EvalShape<2>::kLds, rc = prep(kern, lds);
+    if (rc) return rc;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(I / 16)), dim3(512), lds, st, (const uint16_t*)x, (const uint16_t*)w,
+                       (int)T, (int)D, (int)I, (uint16_t*)h);
     return status();
   }
   const Tiling tl = swiglu_tiling(T, I);

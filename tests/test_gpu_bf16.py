@@ -446,3 +446,26 @@ def test_eval_mlp(dev, T, D, I):
     assert torch.all((a - b).abs() <= 3 * 2 ** -8 * b.abs().clamp(min=1e-4))
     assert float((a != b).float().mean()) < 0.02
     assert O.rel_l2(y.float().cpu(), mlp(x).detach().float().cpu()) < 1e-2
+
+
+# up to 64 rows: one or two tiles of 32 rows of x, K in whole and half chunks of
+# 128, fewer chunks than the ring holds and more; from 65 on the tiled kernel
+@pytest.mark.parametrize("D,I", [(64, 64), (128, 192), (320, 128), (1024, 3072), (2048, 64)])
+@pytest.mark.parametrize("T", [1, 8, 31, 32, 33, 63, 64, 65])
+def test_eval_rows_equal_training_rows(dev, T, D, I):
+    """The evaluation kernels sum K as the training path's do: a row's h has the
+    same bytes with gradients on and off, whatever rows it is batched with,
+    NaN, infinite and huge values among them."""
+    torch.manual_seed(T + D)
+    x = torch.randn(T, D, device=dev).bfloat16()
+    w = (torch.randn(2 * I, D, device=dev) * D ** -0.5).bfloat16()
+    x[T // 2, D // 3] = float("nan")
+    x[T // 3, 0] = float("inf")
+    x[0] *= 1e18
+    offs = torch.full((1,), T, device=dev, dtype=torch.int32)
+    ref = sg._FusedSwiGLU.apply(x, w[None], offs)
+    with torch.no_grad():
+        h = sg.swiglu._EvalSwiGLU.apply(x, w)
+        alone = torch.cat([sg.swiglu._EvalSwiGLU.apply(r[None], w) for r in x])
+    bits = lambda t: t.view(torch.int16)  # noqa: E731
+    assert torch.equal(bits(h), bits(ref)) and torch.equal(bits(h), bits(alone))
