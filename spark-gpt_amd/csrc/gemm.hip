@@ -2320,7 +2320,11 @@ struct Bf16Pipe {
       write_all<RB, K + 1>(c);
     }
   }
+  // The last tile's epilogue.  The barrier first: EXACT tiles read row block 1
+  // of the tile before from the staging rows in their last stage, which another
+  // wave may still be in.
   static SFP8_DEV void tail(Ctx& c) {
+    __syncthreads();
     pieces<0, kPieces / 2>(c);
     block_stage<0>(c);
     __syncthreads();

@@ -473,3 +473,35 @@ def test_weight_cache_entry_dies_with_master(monkeypatch):
     del wgu
     gc.collect()
     assert len(TO._WCACHE) == 0
+
+
+@pytest.mark.parametrize("ke,exact", [(8, True), (8, False), (16, True), (16, False)])
+def test_bf16_pipe_staging_rows_are_ordered(ke, exact):
+    """The persistent bf16 SwiGLU kernel keeps one set of staging rows in LDS:
+    waves write their parts of them, then read each other's.  Along a wave's
+    program (three tiles, then the tail as the source has it) a barrier lies
+    between every write and the reads after it, and between every read and the
+    next write, so no wave overwrites rows that another still reads."""
+    src = open(os.path.join(ROOT, "spark-gpt_amd", "csrc", "gemm.hip")).read()
+    src = src[src.index("struct Bf16Pipe {"):src.index("constexpr int kBf16PipeRing")]
+    body = re.search(r"void tail\(Ctx& c\) \{(.*?)\n  \}", src, re.S).group(1)
+    kinds = {"__syncthreads()": "barrier", "block_stage": "write", "write_all": "read"}
+    tail = [kinds[t] for t in re.findall(r"__syncthreads\(\)|block_stage|write_all", body)]
+    assert tail.count("write") == tail.count("read") == 2
+    # Bf16Pipe: 48 pieces over the six slots of stages 0 .. ke - 2, 24 to a row block
+    slots = (ke - 1) * 6
+    done = lambda kt: (48 if (kt + 1) * 6 >= slots else (kt + 1) * 6 * 48 // slots) // 24 if kt >= 0 else 0  # noqa: E731
+    tile = []
+    for kt in range(ke):
+        tile.append("barrier")
+        tile += ["read"] * (kt > 0 and done(kt - 1) > done(kt - 2))
+        tile += ["write"] * (done(kt) > done(kt - 1))
+    tile += [] if exact else ["barrier"] * 4
+    assert tile.count("write") == tile.count("read") == 2
+    last, fenced = None, True
+    for event in tile * 3 + tail:
+        if event == "barrier":
+            fenced = True
+        elif event != last:
+            assert fenced or last is None, (last, event)
+            last, fenced = event, False
