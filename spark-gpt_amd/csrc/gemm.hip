@@ -587,13 +587,13 @@ struct SwigluPipe {
     if (c.prev) {
       // gu8 is a K-slab [2I/64][ldt][64], h8 one of [I/64][ldt][64]: the
       // tile's 64 gate, 64 up and 64 h columns are one block each (rows past
-      // T hold the zeros computed from x8's zero padding); the block's
-      // origin is the store's scalar offset
+      // T hold the zeros computed from x8's zero padding); the block's origin
+      // goes in the vector offset (Bf16Pipe::row_write says why)
       const uint32_t vo = (uint32_t)(row * 64 + col);
       __builtin_amdgcn_raw_buffer_store_b128(intx4{(int)c.gw[0], (int)c.gw[1], (int)c.gw[2], (int)c.gw[3]},
-                                             c.rgu, vo, (int)c.so_g, 0);
+                                             c.rgu, vo + c.so_g, 0, 0);
       __builtin_amdgcn_raw_buffer_store_b128(intx4{(int)c.uw[0], (int)c.uw[1], (int)c.uw[2], (int)c.uw[3]},
-                                             c.rgu, vo, (int)c.so_u, 0);
+                                             c.rgu, vo + c.so_u, 0, 0);
     }
     store16(c.hbuf + row * kPipeHStride + col, c.hw);
   }

@@ -505,3 +505,26 @@ def test_bf16_pipe_staging_rows_are_ordered(ke, exact):
         elif event != last:
             assert fenced or last is None, (last, event)
             last, fenced = event, False
+
+
+def test_wide_buffer_stores_have_no_scalar_offset():
+    """A 16-byte buffer store reads its data after it has issued: the compiler
+    keeps the next instruction from overwriting the data only if the store's
+    scalar offset is the literal zero (with a register there it sees no hazard).
+    Every such store of the sources has it so."""
+    csrc = os.path.join(ROOT, "spark-gpt_amd", "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        text = re.sub(r"//[^\n]*", "", open(os.path.join(csrc, name)).read())
+        for m in re.finditer(r"raw_(?:ptr_)?buffer_store_b(?:96|128)\(", text):
+            depth, args, start = 1, [], m.end()
+            for i in range(m.end(), len(text)):
+                depth += {"(": 1, "{": 1, "[": 1, ")": -1, "}": -1, "]": -1}.get(text[i], 0)
+                if depth == 0 or (depth == 1 and text[i] == ","):
+                    args.append(text[start:i].strip())
+                    start = i + 1
+                if depth == 0:
+                    break
+            assert len(args) == 5 and args[3] == "0", (name, args)
+            found += 1
+    assert found >= 10
