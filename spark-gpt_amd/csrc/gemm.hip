@@ -600,10 +600,11 @@ struct SwigluPipe {
 
   // Stage KT: the first kPre MFMAs, then the wait for stage KT+1 and the
   // barrier, then six slots (slot below), then the row-block stores the
-  // stage's unit completed.  Vector stores count in vmcnt too and may
-  // complete after later loads, so the wait allows only the kDma loads
-  // issued after stage KT+1's; stores still in flight can make it wait for
-  // those as well.
+  // stage's unit completed.  vmcnt counts loads and stores and falls in
+  // issue order.  The wait allows the kDma operations issued last: all of
+  // them the previous stage's loads, or after a stage that stored (which not
+  // every one does: c.prev) its stores and fewer of its loads, which are then
+  // waited for a stage early.
   template <int KT>
   static SFP8_DEV void stage(Ctx& c, int a_ss, int b_ss) {
     constexpr int cur = KT & 1, nxt = cur ^ 1;
@@ -2247,7 +2248,8 @@ struct Bf16Pipe {
     ML::template mfma_range<0, kPre>(c.f[PH & 1], c.acc);
     __builtin_amdgcn_sched_barrier(0);
     // what the stage before issued may still fly: its DMA and, after a write
-    // stage, its stores; block_stage's LDS writes must have landed
+    // stage, its stores (vmcnt counts both and falls in issue order; every wave
+    // issues the same number); block_stage's LDS writes must have landed
     constexpr int kFly = ML::kDma + (PREV >= 0 && written(PREV) >= 0 ? kWrites : 0);
     if constexpr (KT >= 0 && written(KT) >= 0)
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFly) : "memory");
