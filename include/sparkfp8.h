@@ -197,7 +197,7 @@ int64_t sfp8_wgrad_workspace_floats(int64_t M, int64_t N, int64_t ldt);
  * LDS reads: bytes equal to sfp8_gemm_wgrad on the copies, which the
  * producers then need not write.  M % 64 == 0 with
  * a_rows, N % 64 == 0 with b_rows, at least one set; ws: fp32 workspace of
- * sfp8_wgrad_rows_workspace_floats(M, N, ldt) floats. */
+ * sfp8_wgrad_rows_workspace_floats(M, N, ldt) floats (may be NULL when 0). */
 int64_t sfp8_wgrad_rows_workspace_floats(int64_t M, int64_t N, int64_t ldt);
 int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, int fmt_b, int b_rows, int64_t M,
                          int64_t N, int64_t ldt, const float* sa, const float* sb, float* out, float* ws,
@@ -314,9 +314,8 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
  * replaced by split partials summed in order: deterministic):
  * out[e] = sum over expert e's rows of at[:, t] bt[:, t]^T / (sa * sb),
  * fp32 [E, M, N]; experts without rows get zeros.  ws: fp32 workspace of
- * sfp8_moe_wgrad_workspace_floats(M, N, E) floats (may be NULL when 0), room
- * for the most splits that a call takes (sfp8_moe_wgrad_splits): with few rows
- * it takes fewer. */
+ * sfp8_moe_wgrad_workspace_floats(M, N, E) floats, room for the most splits
+ * that a call takes (sfp8_moe_wgrad_splits): with few rows it takes fewer. */
 int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E);
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E);
 int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_t M, int64_t N, int64_t E,
@@ -422,7 +421,8 @@ int sfp8_bf16_norm_dh(const void* p, const void* h, const float* rstd, int64_t T
  * out [M, N] = bf16(sum over ldt tokens of at[:, t] bt[:, t]^T), at / bt the
  * token-contiguous bf16 K-slabs of [M, ldt] / [N, ldt]; split partials summed
  * in order (deterministic).  ws: fp32 workspace of
- * sfp8_bf16_wgrad_workspace_floats(M, N, ldt) floats.  M N % 8 == 0. */
+ * sfp8_bf16_wgrad_workspace_floats(M, N, ldt) floats (may be NULL when 0).
+ * M N % 8 == 0. */
 int64_t sfp8_bf16_wgrad_splits(int64_t M, int64_t N, int64_t ldt);
 int64_t sfp8_bf16_wgrad_workspace_floats(int64_t M, int64_t N, int64_t ldt);
 int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, int64_t ldt, void* out, float* ws,

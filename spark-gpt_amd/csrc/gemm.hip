@@ -2847,6 +2847,13 @@ int launch_moe_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, 
   return status();
 }
 
+// Whether a weight gradient's workspace is missing or smaller than its size
+// query says.  The answer does not depend on the splits that the call takes,
+// which may be fewer than the query's; a size of 0 needs no pointer.
+inline bool no_workspace(const float* ws, int64_t have, int64_t floats) {
+  return floats > 0 && (!ws || have < floats);
+}
+
 // float4s of one split's partials, and the launches of the reductions over
 // them (E experts; tr_b: the partials of a transposed-read B).
 inline int64_t partial_quads(const Tiling& tl) { return (int64_t)tl.m * tl.n << (tl.small ? 12 : 14); }
@@ -3071,7 +3078,7 @@ int sfp8_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_
   if (!al16(at) || !al16(bt) || !al16(out)) return kErrBadAlignment;
   hipStream_t st = (hipStream_t)stream;
   const int64_t splits = dense_splits(M, N, ldt, false);
-  if (splits > 1 && (!ws || ws_floats < sfp8_wgrad_workspace_floats(M, N, ldt))) return kErrWorkspaceTooSmall;
+  if (no_workspace(ws, ws_floats, sfp8_wgrad_workspace_floats(M, N, ldt))) return kErrWorkspaceTooSmall;
   if (ldt == 0) {
     // no tokens: the gradient is zero (a fill kernel, not a memset node, so
     // that a captured graph replays it correctly)
@@ -3199,7 +3206,7 @@ int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, in
   if (!fits32(slab_rows(M), ldp) || !fits32(slab_rows(N), ldp)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
   const int64_t splits = moe_wgrad_splits(M, N, E, ldp, false);
-  if (splits > 1 && (!ws || ws_floats < sfp8_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
+  if (no_workspace(ws, ws_floats, sfp8_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
   const int rc = launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, false, false>(tl, at, bt, M, N, ldp, sa, sb, out, ws,
@@ -3384,7 +3391,7 @@ int sfp8_bf16_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t N, i
     return status();
   }
   const int64_t splits = dense_splits(M, N, 2 * ldt, true);
-  if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
+  if (no_workspace(ws, ws_floats, sfp8_bf16_wgrad_workspace_floats(M, N, ldt))) return kErrWorkspaceTooSmall;
   const Tiling tl = tiling(M, N, splits);
   const int rc = launch_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldt, wgrad_chunk(2 * ldt, splits), nullptr, nullptr,
                                                         splits > 1 ? ws : (float*)out, (int)splits, splits > 1, TrOp{},
@@ -3404,7 +3411,7 @@ int sfp8_bf16_moe_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t 
   if (!fits32(slab_rows(M), 2 * ldp) || !fits32(slab_rows(N), 2 * ldp)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
   const int64_t splits = moe_wgrad_splits(M, N, E, ldp, true);
-  if (!ws || ws_floats < sfp8_bf16_moe_wgrad_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
+  if (no_workspace(ws, ws_floats, sfp8_bf16_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
   const int rc = launch_moe_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldp, nullptr, nullptr, (float*)out,
@@ -3429,7 +3436,7 @@ int sfp8_bf16_gemm_wgrad_rows(const void* a, const void* x, int x_rows, int64_t 
     return status();
   }
   const int64_t splits = dense_splits(M, N, 2 * ldt, true);
-  if (!ws || ws_floats < sfp8_bf16_wgrad_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
+  if (no_workspace(ws, ws_floats, sfp8_bf16_wgrad_workspace_floats(M, N, ldt))) return kErrWorkspaceTooSmall;
   // a: the bf16 K-slab of [ldt, M] (32 columns per 64-byte row); x (x_rows):
   // row-major [T, N] bf16, tokens T..ldt-1 read as zero through the range
   // check, or else the token-contiguous bf16 K-slab of x^T over ldt tokens
@@ -3449,7 +3456,7 @@ int sfp8_bf16_moe_gemm_wgrad_rows(const void* a, const void* bt, int64_t M, int6
   if (!fits32(slab_rows(M), 2 * ldp) || !fits32(slab_rows(N), 2 * ldp)) return kErrBadShape;
   if (!al16(a) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
   const int64_t splits = moe_wgrad_splits(M, N, E, ldp, true);
-  if (!ws || ws_floats < sfp8_bf16_moe_wgrad_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
+  if (no_workspace(ws, ws_floats, sfp8_bf16_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
   const Tiling tl = tiling(M, N, E * splits);
   const int rc = launch_moe_wgrad<true, 0, 0, true, false>(tl, a, bt, M, N, 2 * ldp, nullptr, nullptr, (float*)out,
@@ -3466,7 +3473,7 @@ int64_t sfp8_wgrad_rows_workspace_floats(int64_t M, int64_t N, int64_t ldt) {
 int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, int fmt_b, int b_rows, int64_t M,
                          int64_t N, int64_t ldt, const float* sa, const float* sb, float* out, float* ws,
                          int64_t ws_floats, void* stream) {
-  if (!sa || !sb || !out || (ldt > 0 && (!a || !b || !ws))) return kErrNullPointer;
+  if (!sa || !sb || !out || (ldt > 0 && (!a || !b))) return kErrNullPointer;
   if (M <= 0 || N <= 0 || ldt < 0 || ldt % kTile || N % 4 || !(a_rows || b_rows)) return kErrBadShape;
   if ((a_rows && M % 64) || (b_rows && N % 64)) return kErrBadShape;
   if (fmt_a != kFmtE5M2 || fmt_b != kFmtE4M3) return kErrBadShape;
@@ -3479,7 +3486,8 @@ int sfp8_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b, in
     return status();
   }
   const int splits = (int)dense_splits(M, N, ldt, false);
-  if (ws_floats < sfp8_wgrad_rows_workspace_floats(M, N, ldt)) return kErrWorkspaceTooSmall;
+  const int64_t most = sfp8_wgrad_rows_workspace_floats(M, N, ldt);
+  if (no_workspace(ws, ws_floats, most)) return ws ? kErrWorkspaceTooSmall : kErrNullPointer;
   const Tiling tl = tiling(M, N, splits);
   const int rc =
       wgrad_partials(tl, a_rows, b_rows, a, b, M, N, ldt, sa, sb, splits > 1 ? ws : out, splits, splits > 1, st);

@@ -561,3 +561,33 @@ def test_one_split_gradients(dev, M, N, T):
     assert torch.equal(ops.bf16_wgrad_rows(gs, x, M, N), ref.bfloat16())
     at, bt = (ops.to_slab(v.bfloat16().t().contiguous()) for v in (a, b))
     assert torch.equal(ops.bf16_wgrad(at, bt, M, N), ref.bfloat16())
+
+
+def test_wgrads_without_workspace(dev):
+    """Where the size query says 0 floats a null workspace is taken."""
+    from spark_gpt_amd import _lib
+
+    ops = sg.ops
+    M, N, ldt = 128, 192, 512
+    g = torch.Generator(device=dev).manual_seed(3)
+    a, b = (torch.randint(-8, 9, (ldt, n), generator=g, device=dev).float() for n in (M, N))
+    ref, one, st = a.t() @ b, torch.ones(1, device=dev), _lib.stream_of(a)
+    for q in ("sfp8_wgrad_workspace_floats", "sfp8_wgrad_rows_workspace_floats", "sfp8_bf16_wgrad_workspace_floats"):
+        assert _lib.query(q, M, N, ldt) == 0
+    f = torch.empty(M, N, device=dev)
+    h = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    a8, b8 = ops.to_slab(a.to(E5)), ops.to_slab(b.to(E4))
+    _lib.call("sfp8_gemm_wgrad_rows", a8.data_ptr(), 1, 1, b8.data_ptr(), 0, 1, M, N, ldt, one.data_ptr(),
+              one.data_ptr(), f.data_ptr(), None, 0, st)
+    assert torch.equal(f, ref)
+    at, bt = ops.to_slab(a.to(E5).t().contiguous()), ops.to_slab(b.to(E4).t().contiguous())
+    _lib.call("sfp8_gemm_wgrad", at.data_ptr(), 1, bt.data_ptr(), 0, M, N, ldt, one.data_ptr(), one.data_ptr(),
+              f.zero_().data_ptr(), None, 0, st)
+    assert torch.equal(f, ref)
+    at, bt = ops.to_slab(a.bfloat16().t().contiguous()), ops.to_slab(b.bfloat16().t().contiguous())
+    _lib.call("sfp8_bf16_gemm_wgrad", at.data_ptr(), bt.data_ptr(), M, N, ldt, h.data_ptr(), None, 0, st)
+    assert torch.equal(h, ref.bfloat16())
+    gs, x = ops.to_slab(a.bfloat16()), b.bfloat16()
+    _lib.call("sfp8_bf16_gemm_wgrad_rows", gs.data_ptr(), x.data_ptr(), 1, M, N, ldt, ldt, h.zero_().data_ptr(), None,
+              0, st)
+    assert torch.equal(h, ref.bfloat16())

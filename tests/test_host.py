@@ -86,6 +86,14 @@ def test_invalid_arguments_rejected_before_launch():
     assert lib.sfp8_gemm_gateup_swiglu_fwd(16, 16, 100, 256, 384, 16, 16, 16, 16, 16, 16, 100, None) == -2
     assert lib.sfp8_gemm_down_dgrad_swiglu(16, 16, 16, 300, 256, 384, 16, 16, 16, 16, 768, None) == -2
     assert lib.sfp8_gemm_wgrad(16, 1, 16, 0, 256, 102, 256, 16, 16, 16, 16, 0, None) == -2  # N % 4
+    # a weight gradient needs the workspace that its size query asks for, also
+    # where the call takes one split and would not use it
+    assert _lib.query("sfp8_wgrad_workspace_floats", 6144, 1024, 5120) > 0
+    assert lib.sfp8_gemm_wgrad(16, 1, 16, 0, 6144, 1024, 5120, 16, 16, 16, None, 0, None) == -4
+    assert lib.sfp8_gemm_wgrad_rows(16, 1, 1, 16, 0, 1, 6144, 1024, 5120, 16, 16, 16, None, 0, None) == -1
+    assert lib.sfp8_gemm_wgrad_rows(16, 1, 1, 16, 0, 1, 6144, 1024, 5120, 16, 16, 16, 16, 64, None) == -4
+    assert lib.sfp8_bf16_gemm_wgrad(16, 16, 6144, 1024, 5120, 16, None, 0, None) == -4
+    assert lib.sfp8_moe_gemm_wgrad(16, 1, 16, 0, 3072, 1024, 8, 16, 4096, 16, 16, 16, None, 0, None) == -4
     # the allocation-free norm backward refuses shapes beyond its fixed scratch on the host
     assert lib.sfp8_norm_bwd_noalloc(16, 16, 16, 16, 16, 65536, 4096, 16, 16, 16, 16, 16, None, 65536, None) == -5
     assert lib.sfp8_norm_bwd_noalloc(None, 16, 16, 16, 16, 256, 1024, 16, 16, 16, 16, None, 16, 256, None) == -1
