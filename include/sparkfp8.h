@@ -315,9 +315,15 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
  * out[e] = sum over expert e's rows of at[:, t] bt[:, t]^T / (sa * sb),
  * fp32 [E, M, N]; experts without rows get zeros.  ws: fp32 workspace of
  * sfp8_moe_wgrad_workspace_floats(M, N, E) floats, room for the most splits
- * that a call takes (sfp8_moe_wgrad_splits): with few rows it takes fewer. */
+ * that a call takes (sfp8_moe_wgrad_splits); sfp8_wgrad_splits_of says how
+ * many it takes. */
 int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E);
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E);
+/* K splits that a weight gradient call takes, at most the count that sizes its
+ * workspace: dense (E = 0) over `rows` = ldt tokens, or grouped over `rows` =
+ * ldp padded rows of E experts; fp8, or bf16 operands (bf16 != 0).  -1 for sizes
+ * that no call accepts. */
+int64_t sfp8_wgrad_splits_of(int64_t M, int64_t N, int64_t E, int64_t rows, int bf16);
 int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_t M, int64_t N, int64_t E,
                         const int* plan, int64_t ldp, const float* sa, const float* sb, float* out, float* ws,
                         int64_t ws_floats, void* stream);

@@ -3014,7 +3014,7 @@ static int64_t wgrad_splits(int64_t M, int64_t N, int64_t kbytes) {
 // beside another.  With one split the gradient is written by its own
 // work-group; several write and read 8 bytes per output each, at about 5
 // TB/s, and launch the reduction.  Measured against it (us, gradient and
-// reduction, 1 / 2 / 4 splits; the model's choice is marked): 8 experts, M =
+// reduction, 1 / 2 / 4 splits of even rows; the model's choice is marked): 8 experts, M =
 // 3072, N = 1024, 131072 rows 332* 362 410, 16384 rows 57* 124 181; M = 1536, N
 // = 512, 65536 rows fp8 52* 59 75, bf16 130 107* 128; 4 experts, M = 1024, N =
 // 512, 16384 rows bf16 38 31* 32; 16 experts, M = 512, N = 256 10* 19 25.
@@ -3098,24 +3098,52 @@ int sfp8_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_
 // ldp = padded rows (256 * sfp8_moe_padded_rows); plan from sfp8_moe_plan.
 namespace {
 // Most K splits of a grouped gradient, by which its workspace is sized before
-// its rows are known: at least 2, then doubling until the grid has 192
+// its rows are known: at least 2, then doubling until the grid has 384
 // work-groups (8 at most).
 inline int64_t moe_splits_most(int64_t M, int64_t N, int64_t E) {
   const int64_t wgs = (int64_t)cdiv(M, kTile) * cdiv(N, kTile) * E;
   int64_t s = 2;
-  while (s < 8 && wgs * s < 192) s *= 2;
+  while (s < 8 && wgs * s < 384) s *= 2;
   return s;
 }
-// Its K splits (1, 2, 4 or 8) over ldp padded rows: more only where the model
-// gains a tenth.
+// The modelled time (us) of a grouped gradient whose rows all went to one
+// expert: `stages` K stages in s splits.  Its work-groups are one run of the
+// grid's, so they share the XCDs of that run (32 CUs each) and the others idle.
+// A stage takes 0.5 us for a 256 x 256 tile on a full XCD; 0.27 for a 128 x 128
+// one alone on its CU and 0.4 (bf16: 0.42) beside another.
+static inline double one_expert_us(int64_t M, int64_t N, int64_t E, double stages, int64_t s, bool bf16) {
+  const Tiling tl = tiling(M, N, E * s);
+  const int64_t w = (int64_t)tl.m * tl.n * s, n = w * E, r = n % kCUs;
+  const int64_t full = !tl.small && s == 1 && r < n && 2 * r <= kCUs ? n - r : n;  // as tail_full
+  const int64_t xcds = (8 * w + full - 1) / full, cus = 32 * (xcds < 8 ? xcds : 8);
+  const int64_t slots = tl.small ? 2 * cus : cus, rounds = (w + slots - 1) / slots;
+  const double fill = w <= cus ? 0.0 : w >= 2 * cus ? 1.0 : (double)(w - cus) / (double)cus;
+  const double us = !tl.small ? 0.5 : 0.27 + (bf16 ? 0.15 : 0.13) * fill;
+  return (double)rounds * us * stages / (double)s +
+         (s > 1 ? 2.5 + (double)s * (double)E * (double)M * (double)N * 8.0 / 5e6 : 0.0);
+}
+// Its K splits (1, 2, 4 or 8) over ldp padded rows.  The routing is known on
+// the device only, so the count has to do for all of them: of those that are no
+// slower than the most when one expert has every row, the one that is fastest
+// over even rows, more only where that gains a tenth.  Measured (us, fp8, even
+// rows / all on one expert, at 1, 2, 4 and 8 splits; the choice is marked): 8
+// experts, M = 3072, N = 1024, 131072 rows 352/1068* 395/1683; M = 1024, N = 1536
+// 173/1037* 219/1081; M = 1536, N = 512, 65536 rows 58/322 67/271* 86/280; 16
+// experts, M = 512, N = 256, 65536 rows 25/253 24/140 35/90* 44/93, 16384 rows
+// 11/71 21/48* 26/41 35/49; 4 experts, M = 1024, N = 512, 65536 rows 74/257 51/148
+// 48/110 53/101*.  (By the even rows alone the counts there were 1, 1, 1, 1, 1
+// and 4.)
 inline int64_t moe_wgrad_splits(int64_t M, int64_t N, int64_t E, int64_t ldp, bool bf16) {
-  const double stages = (double)ldp * (bf16 ? 2 : 1) / (double)kStage / (double)E;
-  const int64_t most = moe_splits_most(M, N, E);
-  int64_t best = 1;
-  double best_us = wgrad_us(M, N, E, stages, 1, bf16);
-  for (int64_t s = 2; s <= most; s *= 2) {
-    const double us = wgrad_us(M, N, E, stages, s, bf16);
-    if (us < 0.9 * best_us) {
+  const double per = (bf16 ? 2.0 : 1.0) / (double)kStage;  // stages per row
+  const int64_t most = moe_splits_most(M, N, E), pad = (int64_t)kTile * (E - 1);  // the other experts' padding
+  const double one = (double)(ldp - pad < kTile ? kTile : ldp - pad) * per;
+  const double bound = 1.05 * one_expert_us(M, N, E, one, most, bf16);
+  int64_t best = 0;
+  double best_us = 0.0;
+  for (int64_t s = 1; s <= most; s *= 2) {
+    if (s < most && one_expert_us(M, N, E, one, s, bf16) > bound) continue;
+    const double us = wgrad_us(M, N, E, (double)ldp * per / (double)E, s, bf16);
+    if (!best || us < 0.9 * best_us) {
       best = s;
       best_us = us;
     }
@@ -3191,6 +3219,11 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
 }
 
 int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E) { return moe_splits_most(M, N, E); }
+
+int64_t sfp8_wgrad_splits_of(int64_t M, int64_t N, int64_t E, int64_t rows, int bf16) {
+  if (M <= 0 || N <= 0 || E < 0 || rows <= 0 || rows % kTile) return -1;
+  return E ? moe_wgrad_splits(M, N, E, rows, bf16) : dense_splits(M, N, bf16 ? 2 * rows : rows, bf16);
+}
 
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E) {
   const int64_t s = sfp8_moe_wgrad_splits(M, N, E);
