@@ -321,9 +321,10 @@ int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E);
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E);
 /* K splits that a weight gradient call takes, at most the count that sizes its
  * workspace: dense (E = 0) over `rows` = ldt tokens, or grouped over `rows` =
- * ldp padded rows of E experts; fp8, or bf16 operands (bf16 != 0).  -1 for sizes
- * that no call accepts. */
-int64_t sfp8_wgrad_splits_of(int64_t M, int64_t N, int64_t E, int64_t rows, int bf16);
+ * ldp padded rows of E experts; fp8, or bf16 operands (bf16 != 0).  longest !=
+ * 0: those of an expert with more than one and a half times the average rows.
+ * -1 for sizes that no call accepts. */
+int64_t sfp8_wgrad_splits_of(int64_t M, int64_t N, int64_t E, int64_t rows, int bf16, int longest);
 int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, int64_t M, int64_t N, int64_t E,
                         const int* plan, int64_t ldp, const float* sa, const float* sb, float* out, float* ws,
                         int64_t ws_floats, void* stream);

@@ -48,7 +48,7 @@ SIGNATURES = {
     "sfp8_moe_gemm_down_dgrad_swiglu": (_INT, [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _P, _P]),
     "sfp8_moe_gemm_gateup_dgrad": (_INT, [_P, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _P]),
     "sfp8_moe_wgrad_splits": (_I64, [_I64, _I64, _I64]),
-    "sfp8_wgrad_splits_of": (_I64, [_I64, _I64, _I64, _I64, _INT]),
+    "sfp8_wgrad_splits_of": (_I64, [_I64, _I64, _I64, _I64, _INT, _INT]),
     "sfp8_moe_wgrad_workspace_floats": (_I64, [_I64, _I64, _I64]),
     "sfp8_moe_gemm_wgrad": (_INT, [_P, _INT, _P, _INT, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _P, _I64, _P]),
     "sfp8_moe_wgrad_rows_workspace_floats": (_I64, [_I64, _I64, _I64]),

@@ -1683,6 +1683,13 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
                                                              tiles_m, tiles_n, partials, tra, trb);
 }
 
+// K splits of expert e of a grouped gradient: `longest` for one with more than
+// one and a half times the average rows, else `even`.
+SFP8_DEV int moe_expert_splits(const int* __restrict__ plan, int e, int even, int longest) {
+  const MoePlan P{plan};
+  return 2 * (P.pcount(e) / kTile) * P.experts() > 3 * P.ntiles() ? longest : even;
+}
+
 // Grouped (MoE) weight gradient: out[e, m, n] = sum over expert e's padded
 // rows t of A[m, t] * B[n, t] / (sa * sb), A and B token-contiguous K-slab
 // copies over the padded expert order (zeros in padding rows).  Work-group
@@ -1697,11 +1704,14 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
 // ws[e][sp][tile], summed in split order by splitk_reduce_kernel.
 // BF16: bf16 operands, 2 bytes per padded row (`ldp` counts K bytes), and a
 // bf16 gradient (bf16_wgrad_reduce_kernel).
+// longest > splits: each expert has its own count (moe_expert_splits), read
+// from the plan; the work-groups past it exit, and the reductions skip experts
+// of one split.
 template <class TS, bool BF16, int FMT_A, int FMT_B, bool TRA, bool TRB>
 SFP8_DEV void moe_wgrad_tile(
     uint8_t* lds, int tm, int tn, int e, int sp, const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
     const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out, float* __restrict__ ws,
-    const int* __restrict__ plan, int tiles_m, int tiles_n, int splits) {
+    const int* __restrict__ plan, int tiles_m, int tiles_n, int splits, int ws_splits) {
   const MoePlan P{plan};
   const int64_t m0 = (int64_t)tm * TS::kM, n0 = (int64_t)tn * TS::kN;
   if (m0 >= M) return;  // the second half of a tile past the last row (work-group uniform)
@@ -1734,8 +1744,8 @@ SFP8_DEV void moe_wgrad_tile(
       [=](int r) { return TRB ? ((r / kRows) * ltok + (r % kRows)) * kStage : plain_col_nb<2>(r) * kStage; },
       TRB ? kRows * kStage : (int)(rpb * kStage), (int)nk, acc);
   if (splits > 1) {
-    // accumulator order: [expert][split][tile][wave][tb][nb][i][lane][4]
-    float* frag = ws + (((int64_t)e * splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kN) +
+    // accumulator order: [expert][split of ws_splits][tile][wave][tb][nb][i][lane][4]
+    float* frag = ws + (((int64_t)e * ws_splits + sp) * tiles_m * tiles_n + (int64_t)tm * tiles_n + tn) * (TS::kM * TS::kN) +
                   wave * (TS::kM * TS::kN / (TS::kThreads / 64));
 #pragma unroll
     for (int tb = 0; tb < TS::kTB; ++tb)
@@ -1755,36 +1765,44 @@ template <bool SMALL, bool BF16, int FMT_A, int FMT_B, bool TRA = false, bool TR
 __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinWaves) void moe_wgrad_kernel(
     const uint8_t* __restrict__ at, const uint8_t* __restrict__ bt, int64_t M, int64_t N, int64_t ldp,
     const float* __restrict__ sa, const float* __restrict__ sb, float* __restrict__ out, float* __restrict__ ws,
-    const int* __restrict__ plan, int tiles_m, int tiles_n, int splits, int experts) {
+    const int* __restrict__ plan, int tiles_m, int tiles_n, int splits, int longest, int experts) {
   extern __shared__ __align__(16) uint8_t lds[];
   const int tiles = tiles_m * tiles_n, n = tiles * splits * experts, pid = blockIdx.x;
-  int tm, tn;
-  if constexpr (!SMALL) {
-    // one split: the last round in halves, as tail_tile (the run of full tiles
-    // is the grid's without them); 8 experts, 131072 rows, D = 1024, I = 1536
-    // (384 gate/up tiles), the experts' step 2344 -> 2329 us
-    const int full = splits == 1 ? tail_full(n, kRound) : n;
-    if (pid >= full) {
-      const int lid = full + ((pid - full) >> 1);
-      if (lid >= n) return;
-      raster(lid % tiles, tiles_m, tiles_n, tm, tn);
-      moe_wgrad_tile<Tile<2, 4>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, 2 * tm + ((pid - full) & 1), tn, lid / tiles, 0, at,
-                                                               bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                                                               1);
-      return;
-    }
-    const int lid = xcd_run(pid, full);
-    raster(lid % tiles, tiles_m, tiles_n, tm, tn);
-    moe_wgrad_tile<Tile<4, 4>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, lid / (tiles * splits), (lid / tiles) % splits,
-                                                             at, bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                                                             splits);
+  int lid, e, sp, count = splits, tm, tn;
+  if (longest > splits) {
+    // the grid has `longest` splits, one after the other; a split's run over
+    // the XCDs is turned by its share of them, so that the splits of one expert
+    // lie on different XCDs
+    const int n0 = tiles * experts;
+    sp = pid / n0;
+    lid = (xcd_run(pid % n0, n0) + (int)((int64_t)n0 * sp / longest)) % n0;
+    e = lid / tiles;
+    count = moe_expert_splits(plan, e, splits, longest);
+    if (sp >= count) return;
   } else {
-    const int lid = xcd_run(pid, gridDim.x);
-    raster(lid % tiles, tiles_m, tiles_n, tm, tn);
-    moe_wgrad_tile<Tile<2, 2>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, lid / (tiles * splits), (lid / tiles) % splits,
-                                                             at, bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m, tiles_n,
-                                                             splits);
+    int full = n;
+    if constexpr (!SMALL) {
+      // one split: the last round in halves, as tail_tile (the run of full tiles
+      // is the grid's without them); 8 experts, 131072 rows, D = 1024, I = 1536
+      // (384 gate/up tiles), the experts' step 2344 -> 2329 us
+      if (splits == 1) full = tail_full(n, kRound);
+      if (pid >= full) {
+        lid = full + ((pid - full) >> 1);
+        if (lid >= n) return;
+        raster(lid % tiles, tiles_m, tiles_n, tm, tn);
+        moe_wgrad_tile<Tile<2, 4>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, 2 * tm + ((pid - full) & 1), tn, lid / tiles, 0,
+                                                                 at, bt, M, N, ldp, sa, sb, out, ws, plan, tiles_m,
+                                                                 tiles_n, 1, 1);
+        return;
+      }
+    }
+    lid = xcd_run(pid, full);
+    e = lid / (tiles * splits);
+    sp = (lid / tiles) % splits;
   }
+  raster(lid % tiles, tiles_m, tiles_n, tm, tn);
+  moe_wgrad_tile<TileShape<SMALL>, BF16, FMT_A, FMT_B, TRA, TRB>(lds, tm, tn, e, sp, at, bt, M, N, ldp, sa, sb, out, ws,
+                                                                 plan, tiles_m, tiles_n, count, longest);
 }
 
 // out[0, n) = 0: four floats per thread (n % 4 == 0, out 16-byte aligned).
@@ -1819,23 +1837,27 @@ template <bool SMALL, bool TR_B>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int splits,
                                                             int64_t n4, int tiles_n, int64_t M, int64_t N,
                                                             const float* __restrict__ sa,
-                                                            const float* __restrict__ sb, float* __restrict__ out) {
-  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (q >= n4) return;
-  // expert blockIdx.y of a grouped gradient: its splits' partials, its [M, N]
+                                                            const float* __restrict__ sb, float* __restrict__ out,
+                                                            const int* __restrict__ plan, int even) {
+  // expert blockIdx.y of a grouped gradient: its splits' partials, its [M, N];
+  // with a plan the splits that it has (one: the gradient is written)
   ws += (int64_t)blockIdx.y * splits * n4 * 4;
+  if (plan) splits = moe_expert_splits(plan, blockIdx.y, even, splits);
+  if (splits == 1) return;
   out += (int64_t)blockIdx.y * M * N;
   const floatx4* w4 = reinterpret_cast<const floatx4*>(ws);
-  floatx4 acc = __builtin_nontemporal_load(w4 + q);
-  for (int s = 1; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
-  int r, c;
-  acc_order_rc<SMALL, TR_B>((int)(q & ((1 << kTileQLog<SMALL>) - 1)), r, c);
-  const int64_t tile = q >> kTileQLog<SMALL>;
-  const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
-  const int64_t m = tm * TileShape<SMALL>::kM + r, n = tn * TileShape<SMALL>::kM + c;
-  if (m < M && n < N) {
-    const float deq = 1.0f / (sa[0] * sb[0]);
-    *reinterpret_cast<floatx4*>(out + m * N + n) = acc * deq;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n4; q += (int64_t)gridDim.x * 256) {
+    floatx4 acc = __builtin_nontemporal_load(w4 + q);
+    for (int s = 1; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
+    int r, c;
+    acc_order_rc<SMALL, TR_B>((int)(q & ((1 << kTileQLog<SMALL>) - 1)), r, c);
+    const int64_t tile = q >> kTileQLog<SMALL>;
+    const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
+    const int64_t m = tm * TileShape<SMALL>::kM + r, n = tn * TileShape<SMALL>::kM + c;
+    if (m < M && n < N) {
+      const float deq = 1.0f / (sa[0] * sb[0]);
+      *reinterpret_cast<floatx4*>(out + m * N + n) = acc * deq;
+    }
   }
 }
 
@@ -2532,21 +2554,25 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void bf16_gemm_kernel(
 template <bool SMALL, bool TR_B>
 __global__ __launch_bounds__(256) void bf16_wgrad_reduce_kernel(const float* __restrict__ ws, int splits, int64_t n4,
                                                                 int tiles_n, int64_t M, int64_t N,
-                                                                uint16_t* __restrict__ out) {
-  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (q >= n4) return;
+                                                                uint16_t* __restrict__ out,
+                                                                const int* __restrict__ plan, int even) {
   ws += (int64_t)blockIdx.y * splits * n4 * 4;
+  if (plan) splits = moe_expert_splits(plan, blockIdx.y, even, splits);  // as splitk_reduce_kernel
+  if (splits == 1) return;
   out += (int64_t)blockIdx.y * M * N;
   const floatx4* w4 = reinterpret_cast<const floatx4*>(ws);
-  floatx4 acc = __builtin_nontemporal_load(w4 + q);
-  for (int s = 1; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
-  int r, c;
-  acc_order_rc<SMALL, TR_B>((int)(q & ((1 << kTileQLog<SMALL>) - 1)), r, c);
-  const int64_t tile = q >> kTileQLog<SMALL>;
-  const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
-  const int64_t m = tm * TileShape<SMALL>::kM + r, n = tn * TileShape<SMALL>::kM + c;
-  if (m < M && n < N)  // N % 4 == 0: the 4 values are wholly inside or past the row
-    *reinterpret_cast<intx2*>(out + m * N + n) = intx2{(int)pack2_bf16(acc[0], acc[1]), (int)pack2_bf16(acc[2], acc[3])};
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n4; q += (int64_t)gridDim.x * 256) {
+    floatx4 acc = __builtin_nontemporal_load(w4 + q);
+    for (int s = 1; s < splits; ++s) acc += __builtin_nontemporal_load(w4 + (int64_t)s * n4 + q);
+    int r, c;
+    acc_order_rc<SMALL, TR_B>((int)(q & ((1 << kTileQLog<SMALL>) - 1)), r, c);
+    const int64_t tile = q >> kTileQLog<SMALL>;
+    const int64_t tm = tile / tiles_n, tn = tile % tiles_n;
+    const int64_t m = tm * TileShape<SMALL>::kM + r, n = tn * TileShape<SMALL>::kM + c;
+    if (m < M && n < N)  // N % 4 == 0: the 4 values are wholly inside or past the row
+      *reinterpret_cast<intx2*>(out + m * N + n) =
+          intx2{(int)pack2_bf16(acc[0], acc[1]), (int)pack2_bf16(acc[2], acc[3])};
+  }
 }
 
 // The weight gradient with the optimizer's momentum stage fused into its
@@ -2830,20 +2856,27 @@ int launch_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, int6
   return status();
 }
 
+// K splits of each expert of a grouped gradient, and of those with more than
+// one and a half times the average rows (moe_expert_splits).
+struct MoeSplits {
+  int even, longest;
+};
 // moe_wgrad_kernel over every expert's tiles and splits (tl of M x N and
-// E * splits parts).
+// E * splits.even parts).
 template <bool BF16, int FMT_A, int FMT_B, bool TRA, bool TRB>
 int launch_moe_wgrad(const Tiling& tl, const void* a, const void* b, int64_t M, int64_t N, int64_t ldp,
-                     const float* sa, const float* sb, float* out, float* ws, const int* plan, int splits,
+                     const float* sa, const float* sb, float* out, float* ws, const int* plan, MoeSplits splits,
                      hipStream_t st) {
   const auto kern = tl.small ? moe_wgrad_kernel<true, BF16, FMT_A, FMT_B, TRA, TRB>
                              : moe_wgrad_kernel<false, BF16, FMT_A, FMT_B, TRA, TRB>;
   const int rc = prep(kern, tl.lds);
   if (rc) return rc;
-  const int n = (int)tl.grid.x, r = n % kRound;
-  const dim3 grid(!tl.small && splits == 1 && 2 * r <= kRound ? n + r : n);
+  const int n = (int)tl.grid.x, r = n % kRound, n0 = n / splits.even;
+  const dim3 grid(splits.longest > splits.even                     ? n0 * splits.longest
+                  : !tl.small && splits.even == 1 && 2 * r <= kRound ? n + r
+                                                                     : n);
   hipLaunchKernelGGL(kern, grid, tl.block, tl.lds, st, (const uint8_t*)a, (const uint8_t*)b, M, N, ldp, sa, sb, out, ws,
-                     plan, tl.m, tl.n, splits, n / (tl.m * tl.n * splits));
+                     plan, tl.m, tl.n, splits.even, splits.longest, n0 / (tl.m * tl.n));
   return status();
 }
 
@@ -2855,26 +2888,31 @@ inline bool no_workspace(const float* ws, int64_t have, int64_t floats) {
 }
 
 // float4s of one split's partials, and the launches of the reductions over
-// them (E experts; tr_b: the partials of a transposed-read B).
+// them (E experts; tr_b: the partials of a transposed-read B; plan: the
+// experts' counts are `even` or `splits`, moe_expert_splits).
 inline int64_t partial_quads(const Tiling& tl) { return (int64_t)tl.m * tl.n << (tl.small ? 12 : 14); }
-inline dim3 reduce_grid(const Tiling& tl, int64_t E) {
-  return dim3((unsigned)((partial_quads(tl) + 255) / 256), (unsigned)E);
+inline dim3 reduce_grid(const Tiling& tl, int64_t E, bool few = false) {
+  // few: most experts have nothing to add, and work-groups that exit at once
+  // cost a launch's time too (16 experts, M = 2944, N = 896: 49152 of them 10 us,
+  // 6144 none); down to 512 an expert, which the others still need
+  const int64_t n = (partial_quads(tl) + 255) / 256;
+  return dim3((unsigned)(few && n > 512 ? (n > 4096 ? n / 8 : 512) : n), (unsigned)E);
 }
 int launch_reduce(const Tiling& tl, bool tr_b, const float* ws, int splits, int64_t E, int64_t M, int64_t N,
-                  const float* sa, const float* sb, float* out, hipStream_t st) {
+                  const float* sa, const float* sb, float* out, hipStream_t st, const int* plan = nullptr, int even = 0) {
   const auto kern = tl.small ? (tr_b ? splitk_reduce_kernel<true, true> : splitk_reduce_kernel<true, false>)
                              : (tr_b ? splitk_reduce_kernel<false, true> : splitk_reduce_kernel<false, false>);
-  hipLaunchKernelGGL(kern, reduce_grid(tl, E), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N, sa, sb,
-                     out);
+  hipLaunchKernelGGL(kern, reduce_grid(tl, E, plan && even == 1), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N, sa, sb,
+                     out, plan, even);
   return status();
 }
 int launch_bf16_reduce(const Tiling& tl, bool tr_b, const float* ws, int splits, int64_t E, int64_t M, int64_t N,
-                       void* out, hipStream_t st) {
+                       void* out, hipStream_t st, const int* plan = nullptr, int even = 0) {
   const auto kern = tl.small
                         ? (tr_b ? bf16_wgrad_reduce_kernel<true, true> : bf16_wgrad_reduce_kernel<true, false>)
                         : (tr_b ? bf16_wgrad_reduce_kernel<false, true> : bf16_wgrad_reduce_kernel<false, false>);
-  hipLaunchKernelGGL(kern, reduce_grid(tl, E), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N,
-                     (uint16_t*)out);
+  hipLaunchKernelGGL(kern, reduce_grid(tl, E, plan && even == 1), dim3(256), 0, st, ws, splits, partial_quads(tl), tl.n, M, N,
+                     (uint16_t*)out, plan, even);
   return status();
 }
 
@@ -3107,49 +3145,63 @@ inline int64_t moe_splits_most(int64_t M, int64_t N, int64_t E) {
   return s;
 }
 // The modelled time (us) of a grouped gradient whose rows all went to one
-// expert: `stages` K stages in s splits.  Its work-groups are one run of the
-// grid's, so they share the XCDs of that run (32 CUs each) and the others idle.
-// A stage takes 0.5 us for a 256 x 256 tile on a full XCD; 0.27 for a 128 x 128
-// one alone on its CU and 0.4 (bf16: 0.42) beside another.
-static inline double one_expert_us(int64_t M, int64_t N, int64_t E, double stages, int64_t s, bool bf16) {
-  const Tiling tl = tiling(M, N, E * s);
-  const int64_t w = (int64_t)tl.m * tl.n * s, n = w * E, r = n % kCUs;
-  const int64_t full = !tl.small && s == 1 && r < n && 2 * r <= kCUs ? n - r : n;  // as tail_full
-  const int64_t xcds = (8 * w + full - 1) / full, cus = 32 * (xcds < 8 ? xcds : 8);
-  const int64_t slots = tl.small ? 2 * cus : cus, rounds = (w + slots - 1) / slots;
-  const double fill = w <= cus ? 0.0 : w >= 2 * cus ? 1.0 : (double)(w - cus) / (double)cus;
+// expert: `stages` K stages in `longest` splits, with the tiles of E * even
+// parts.  With one count for all, its work-groups are one run of the grid's, so
+// they share the XCDs of that run (32 CUs each) and the others idle; with a
+// count of its own each split has such a run to itself.  A stage takes 0.5 us
+// for a 256 x 256 tile on a full XCD; 0.27 for a 128 x 128 one alone on its CU
+// and 0.4 (bf16: 0.42) beside another.
+static inline double one_expert_us(int64_t M, int64_t N, int64_t E, double stages, MoeSplits c, bool bf16) {
+  const Tiling tl = tiling(M, N, E * c.even);
+  const bool own = c.longest > c.even;
+  const int64_t w = (int64_t)tl.m * tl.n * (own ? 1 : c.even), n = w * E, r = n % kCUs;
+  const int64_t full = !own && !tl.small && c.even == 1 && r < n && 2 * r <= kCUs ? n - r : n;  // as tail_full
+  const int64_t wgs = own ? w * c.longest : w, xcds = (8 * w + full - 1) / full * (own ? c.longest : 1);
+  const int64_t cus = 32 * (xcds < 8 ? xcds : 8), slots = tl.small ? 2 * cus : cus, rounds = (wgs + slots - 1) / slots;
+  const double fill = wgs <= cus ? 0.0 : wgs >= 2 * cus ? 1.0 : (double)(wgs - cus) / (double)cus;
   const double us = !tl.small ? 0.5 : 0.27 + (bf16 ? 0.15 : 0.13) * fill;
-  return (double)rounds * us * stages / (double)s +
-         (s > 1 ? 2.5 + (double)s * (double)E * (double)M * (double)N * 8.0 / 5e6 : 0.0);
+  return (double)rounds * us * stages / (double)c.longest +
+         (c.longest > 1 ? 2.5 + (double)c.longest * (double)(own ? 1 : E) * (double)M * (double)N * 8.0 / 5e6 : 0.0);
 }
 // Its K splits (1, 2, 4 or 8) over ldp padded rows.  The routing is known on
-// the device only, so the count has to do for all of them: of those that are no
-// slower than the most when one expert has every row, the one that is fastest
-// over even rows, more only where that gains a tenth.  Measured (us, fp8, even
-// rows / all on one expert, at 1, 2, 4 and 8 splits; the choice is marked): 8
-// experts, M = 3072, N = 1024, 131072 rows 352/1068* 395/1683; M = 1024, N = 1536
-// 173/1037* 219/1081; M = 1536, N = 512, 65536 rows 58/322 67/271* 86/280; 16
-// experts, M = 512, N = 256, 65536 rows 25/253 24/140 35/90* 44/93, 16384 rows
-// 11/71 21/48* 26/41 35/49; 4 experts, M = 1024, N = 512, 65536 rows 74/257 51/148
-// 48/110 53/101*.  (By the even rows alone the counts there were 1, 1, 1, 1, 1
-// and 4.)
-inline int64_t moe_wgrad_splits(int64_t M, int64_t N, int64_t E, int64_t ldp, bool bf16) {
+// the device only, so they have to do for all of them: the count that is fastest
+// over even rows (more only where that gains a tenth), if it is no slower than
+// the most when one expert has every row; else the faster over even rows of two
+// ways to make it so, a larger count for all or one for the long experts only
+// (the fewest splits that do), which costs the reduction's launch.  Measured
+// (us, even rows / half on one expert / all on one; one split for all -> 1 and 2
+// to 4 for long ones): 16 experts, M = 512, N = 256, 16384 rows bf16 15/65/123
+// -> 17/28/40; M = 2944, N = 896, 68546 rows fp8 170/541/998 -> 173/374/542; 4
+// experts, M = 2048, N = 1024, 65536 rows fp8 117/181/325 -> 122/170/179.  The
+// most splits for all take 35/44/68, 311/630/993 and 142/203/325.
+inline MoeSplits moe_wgrad_splits(int64_t M, int64_t N, int64_t E, int64_t ldp, bool bf16) {
   const double per = (bf16 ? 2.0 : 1.0) / (double)kStage;  // stages per row
-  const int64_t most = moe_splits_most(M, N, E), pad = (int64_t)kTile * (E - 1);  // the other experts' padding
-  const double one = (double)(ldp - pad < kTile ? kTile : ldp - pad) * per;
-  const double bound = 1.05 * one_expert_us(M, N, E, one, most, bf16);
-  int64_t best = 0;
-  double best_us = 0.0;
-  for (int64_t s = 1; s <= most; s *= 2) {
-    if (s < most && one_expert_us(M, N, E, one, s, bf16) > bound) continue;
-    const double us = wgrad_us(M, N, E, (double)ldp * per / (double)E, s, bf16);
+  const int64_t pad = (int64_t)kTile * (E - 1);            // the other experts' padding
+  const double one = (double)(ldp - pad < kTile ? kTile : ldp - pad) * per, even = (double)ldp * per / (double)E;
+  const int most = (int)moe_splits_most(M, N, E);
+  const double bound = 1.05 * one_expert_us(M, N, E, one, {most, most}, bf16);
+  int best = 0, fixed = 0;  // of all counts; of those within the bound
+  double best_us = 0.0, fixed_us = 0.0;
+  for (int s = 1; s <= most; s *= 2) {
+    const double us = wgrad_us(M, N, E, even, s, bf16);
     if (!best || us < 0.9 * best_us) {
       best = s;
       best_us = us;
     }
+    if (s < most && one_expert_us(M, N, E, one, {s, s}, bf16) > bound) continue;
+    if (!fixed || us < 0.9 * fixed_us) {
+      fixed = s;
+      fixed_us = us;
+    }
   }
-  return best;
+  if (fixed == best) return {best, best};
+  for (int s = 2 * best; s <= most; s *= 2)
+    if (one_expert_us(M, N, E, one, {best, s}, bf16) <= bound)
+      return best_us + 3.0 < fixed_us ? MoeSplits{best, s} : MoeSplits{fixed, fixed};
+  return {fixed, fixed};
 }
+// The plan for the reductions when the experts' counts differ.
+inline const int* uneven(MoeSplits c, const int* plan) { return c.longest > c.even ? plan : nullptr; }
 inline bool moe_shape(int64_t E, int64_t D, int64_t I, int64_t ldp) {
   return E > 0 && D > 0 && I > 0 && D % 128 == 0 && I % 128 == 0 && ldp > 0 && ldp % kTile == 0;
 }
@@ -3220,9 +3272,11 @@ int sfp8_moe_gemm_gateup_dgrad(const void* dgu8, const void* w8t, int64_t E, int
 
 int64_t sfp8_moe_wgrad_splits(int64_t M, int64_t N, int64_t E) { return moe_splits_most(M, N, E); }
 
-int64_t sfp8_wgrad_splits_of(int64_t M, int64_t N, int64_t E, int64_t rows, int bf16) {
+int64_t sfp8_wgrad_splits_of(int64_t M, int64_t N, int64_t E, int64_t rows, int bf16, int longest) {
   if (M <= 0 || N <= 0 || E < 0 || rows <= 0 || rows % kTile) return -1;
-  return E ? moe_wgrad_splits(M, N, E, rows, bf16) : dense_splits(M, N, bf16 ? 2 * rows : rows, bf16);
+  if (!E) return dense_splits(M, N, bf16 ? 2 * rows : rows, bf16);
+  const MoeSplits s = moe_wgrad_splits(M, N, E, rows, bf16);
+  return longest ? s.longest : s.even;
 }
 
 int64_t sfp8_moe_wgrad_workspace_floats(int64_t M, int64_t N, int64_t E) {
@@ -3238,14 +3292,14 @@ int sfp8_moe_gemm_wgrad(const void* at, int fmt_a, const void* bt, int fmt_b, in
   if (fmt_a != kFmtE5M2 || fmt_b != kFmtE4M3) return kErrBadShape;
   if (!fits32(slab_rows(M), ldp) || !fits32(slab_rows(N), ldp)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, false);
+  const MoeSplits splits = moe_wgrad_splits(M, N, E, ldp, false);
   if (no_workspace(ws, ws_floats, sfp8_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const Tiling tl = tiling(M, N, E * splits);
+  const Tiling tl = tiling(M, N, E * splits.even);
   const int rc = launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, false, false>(tl, at, bt, M, N, ldp, sa, sb, out, ws,
-                                                                           plan, (int)splits, st);
-  if (rc || splits == 1) return rc;
-  return launch_reduce(tl, false, ws, (int)splits, E, M, N, sa, sb, out, st);
+                                                                           plan, splits, st);
+  if (rc || splits.longest == 1) return rc;
+  return launch_reduce(tl, false, ws, splits.longest, E, M, N, sa, sb, out, st, uneven(splits, plan), splits.even);
 }
 
 // ---- the grouped weight gradient with row K-slab operands ----
@@ -3262,16 +3316,16 @@ int sfp8_moe_gemm_wgrad_rows(const void* a, int fmt_a, int a_rows, const void* b
   if (fmt_a != kFmtE5M2 || fmt_b != kFmtE4M3) return kErrBadShape;
   if (!fits32(slab_rows(M), ldp) || !fits32(slab_rows(N), ldp)) return kErrBadShape;
   if (!al16(a) || !al16(b) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, false);
+  const MoeSplits splits = moe_wgrad_splits(M, N, E, ldp, false);
   if (ws_floats < sfp8_moe_wgrad_rows_workspace_floats(M, N, E)) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const Tiling tl = tiling(M, N, E * splits);
+  const Tiling tl = tiling(M, N, E * splits.even);
   const auto launch = a_rows ? (b_rows ? launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, true, true>
                                        : launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, true, false>)
                              : launch_moe_wgrad<false, kFmtE5M2, kFmtE4M3, false, true>;
-  const int rc = launch(tl, a, b, M, N, ldp, sa, sb, out, ws, plan, (int)splits, st);
-  if (rc || splits == 1) return rc;
-  return launch_reduce(tl, b_rows, ws, (int)splits, E, M, N, sa, sb, out, st);
+  const int rc = launch(tl, a, b, M, N, ldp, sa, sb, out, ws, plan, splits, st);
+  if (rc || splits.longest == 1) return rc;
+  return launch_reduce(tl, b_rows, ws, splits.longest, E, M, N, sa, sb, out, st, uneven(splits, plan), splits.even);
 }
 
 
@@ -3443,14 +3497,14 @@ int sfp8_bf16_moe_gemm_wgrad(const void* at, const void* bt, int64_t M, int64_t 
   if (M <= 0 || N <= 0 || E <= 0 || N % 4 || ldp <= 0 || ldp % kTile) return kErrBadShape;
   if (!fits32(slab_rows(M), 2 * ldp) || !fits32(slab_rows(N), 2 * ldp)) return kErrBadShape;
   if (!al16(at) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, true);
+  const MoeSplits splits = moe_wgrad_splits(M, N, E, ldp, true);
   if (no_workspace(ws, ws_floats, sfp8_bf16_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const Tiling tl = tiling(M, N, E * splits);
+  const Tiling tl = tiling(M, N, E * splits.even);
   const int rc = launch_moe_wgrad<true, 0, 0, false, false>(tl, at, bt, M, N, 2 * ldp, nullptr, nullptr, (float*)out,
-                                                           ws, plan, (int)splits, st);
-  if (rc || splits == 1) return rc;
-  return launch_bf16_reduce(tl, false, ws, (int)splits, E, M, N, out, st);
+                                                           ws, plan, splits, st);
+  if (rc || splits.longest == 1) return rc;
+  return launch_bf16_reduce(tl, false, ws, splits.longest, E, M, N, out, st, uneven(splits, plan), splits.even);
 }
 
 // ---- the bf16 weight gradients read through transposing LDS reads ----
@@ -3488,14 +3542,14 @@ int sfp8_bf16_moe_gemm_wgrad_rows(const void* a, const void* bt, int64_t M, int6
   if (M <= 0 || N <= 0 || E <= 0 || M % 32 || N % 4 || ldp <= 0 || ldp % kTile) return kErrBadShape;
   if (!fits32(slab_rows(M), 2 * ldp) || !fits32(slab_rows(N), 2 * ldp)) return kErrBadShape;
   if (!al16(a) || !al16(bt) || !al16(out) || !al16(ws)) return kErrBadAlignment;
-  const int64_t splits = moe_wgrad_splits(M, N, E, ldp, true);
+  const MoeSplits splits = moe_wgrad_splits(M, N, E, ldp, true);
   if (no_workspace(ws, ws_floats, sfp8_bf16_moe_wgrad_workspace_floats(M, N, E))) return kErrWorkspaceTooSmall;
   hipStream_t st = (hipStream_t)stream;
-  const Tiling tl = tiling(M, N, E * splits);
+  const Tiling tl = tiling(M, N, E * splits.even);
   const int rc = launch_moe_wgrad<true, 0, 0, true, false>(tl, a, bt, M, N, 2 * ldp, nullptr, nullptr, (float*)out,
-                                                           ws, plan, (int)splits, st);
-  if (rc || splits == 1) return rc;
-  return launch_bf16_reduce(tl, false, ws, (int)splits, E, M, N, out, st);
+                                                           ws, plan, splits, st);
+  if (rc || splits.longest == 1) return rc;
+  return launch_bf16_reduce(tl, false, ws, splits.longest, E, M, N, out, st, uneven(splits, plan), splits.even);
 }
 
 // ---- the weight gradient with row K-slab operands ----

@@ -337,21 +337,25 @@ def test_wgrad_ragged_columns_stay_in_bounds(dev, M, N):
     assert bool((buf[M * N:] == 12345.0).all())
 
 
-@pytest.mark.parametrize("M,N,T,splits", [(6144, 1024, 4096, 2), (1024, 3072, 16384, 5), (1024, 1024, 8192, 4),
-                                          (1024, 1024, 16384, 8), (320, 192, 1000, 1), (256, 256, 65536, 32)])
-def test_wgrad_rows_equals_token_contiguous(dev, M, N, T, splits):
+@pytest.mark.parametrize("M,N,T,splits,taken", [(6144, 1024, 4096, 2, 1), (2048, 3072, 32768, 5, 2),
+                                                (1024, 3072, 16384, 5, 5), (1024, 1024, 8192, 4, 4),
+                                                (1024, 1024, 16384, 8, 8), (320, 192, 1000, 1, 1),
+                                                (256, 256, 65536, 32, 32)])
+def test_wgrad_rows_equals_token_contiguous(dev, M, N, T, splits, taken):
     """The weight gradient read from the row K-slabs through transposing LDS
     reads gives the bytes of the one read from the token-contiguous copies
-    (same values in the same MFMA K positions, same split sums): one split
-    and several (2 and 4 splits: each split on 8 / splits XCDs; 5: uneven
-    splits, the last shorter, runs of the split-major order crossing split
-    boundaries; 8 and 32: whole splits per XCD), ragged tiles, and the same
-    operands in both layouts.  The result is also checked against a float64
+    (same values in the same MFMA K positions, same split sums): one split,
+    also where the workspace has room for more, and several (2 and 4 splits:
+    each split on 8 / splits XCDs; 5: uneven splits, the last shorter, runs of
+    the split-major order crossing split boundaries; 8 and 32: whole splits per
+    XCD; 2 and 5 in 256 x 256 tiles, the others in 128 x 128), ragged tiles,
+    and the same operands in both layouts.  The result is also checked against a float64
     matmul of the same operands, which no split mapping shares."""
     from spark_gpt_amd import _lib
 
     ops = sg.ops
     assert _lib.query("sfp8_wgrad_splits", M, N, ops.ldt_of(T)) == splits
+    assert _lib.query("sfp8_wgrad_splits_of", M, N, 0, ops.ldt_of(T), 0, 0) == taken
     g = torch.Generator(device=dev).manual_seed(M + N + T)
     a = (torch.randn(T, M, device=dev, generator=g) * 8).to(ops.E5M2)
     b = (torch.randn(T, N, device=dev, generator=g) * 8).to(ops.E4M3)
@@ -591,3 +595,26 @@ def test_wgrads_without_workspace(dev):
     _lib.call("sfp8_bf16_gemm_wgrad_rows", gs.data_ptr(), x.data_ptr(), 1, M, N, ldt, ldt, h.zero_().data_ptr(), None,
               0, st)
     assert torch.equal(h, ref.bfloat16())
+
+
+@pytest.mark.parametrize("M,N,T,fp8,bf16", [(1600, 2880, 20300, 3, 3), (3136, 1984, 6001, 1, 2),
+                                            (1024, 3072, 16384, 5, 5)])
+def test_split_gradients_of_large_tiles(dev, M, N, T, fp8, bf16):
+    """Several splits in 256 x 256 tiles, fp8 and bf16, ragged in both widths
+    and in the tokens: integer operands (at most 64 * 20300 < 2^24, exact in
+    fp32), so every partial and every sum is known."""
+    from spark_gpt_amd import _lib
+
+    ops = sg.ops
+    ldt = ops.ldt_of(T)
+    assert [_lib.query("sfp8_wgrad_splits_of", M, N, 0, ldt, b, 0) for b in (0, 1)] == [fp8, bf16]
+    g = torch.Generator(device=dev).manual_seed(M + N + T)
+    a, b = (torch.zeros(ldt, n, device=dev) for n in (M, N))
+    for v in (a, b):
+        v[:T] = torch.randint(-8, 9, (T, v.shape[1]), generator=g, device=dev).float()
+    ref, one = a.t() @ b, torch.ones(1, device=dev)
+    assert torch.equal(ops.wgrad_rows(ops.to_slab(a.to(E5)), ops.to_slab(b.to(E4)), M, N, one, one), ref)
+    gs, x = ops.to_slab(a.bfloat16()), b[:T].bfloat16().contiguous()
+    assert torch.equal(ops.bf16_wgrad_rows(gs, x, M, N), ref.bfloat16())
+    xt = ops.to_slab(b.bfloat16().t().contiguous())
+    assert torch.equal(ops.bf16_wgrad_rows(gs, xt, M, N, T=T), ref.bfloat16())

@@ -387,3 +387,58 @@ def test_moe_wgrad_tile_shapes(dev, M_, N_, counts):
     assert torch.equal(ops.moe_wgrad_rows(a8, bt8, M_, N_, E, plan, one, one, b_rows=False), ref)
     gs, bt = ops.to_slab(a.bfloat16()), ops.to_slab(b.bfloat16().t().contiguous())
     assert torch.equal(ops.bf16_wgrad_rows(gs, bt, M_, N_, plan=plan, E=E), ref.bfloat16())
+
+
+def _uneven(E, R):
+    """Rows per expert: one with half of them (more than one and a half times
+    the average), an empty one, a single row, the rest even and ragged."""
+    counts = [R // 2, 0, 1][:E]
+    left = R - sum(counts)
+    if E == 3:
+        return [R // 2, 0, left + 1]
+    each = left // (E - 3)
+    return counts + [each] * (E - 4) + [left - each * (E - 4)]
+
+
+# K splits (of an expert, of a long one) that the calls take; 128 x 128 tiles up
+# to 128 work-groups of 256 x 256 (tiles x experts x splits), else 256 x 256
+@pytest.mark.parametrize("bf16,M_,N_,E,R,splits", [
+    (0, 512, 256, 16, 12288, (1, 2)), (0, 512, 256, 6, 12288, (1, 4)), (0, 576, 320, 6, 24576, (2, 4)),
+    (0, 512, 256, 6, 24576, (4, 8)), (0, 512, 256, 4, 8192, (8, 8)),
+    (0, 1536, 320, 16, 8192, (1, 2)), (0, 1280, 256, 4, 65536, (8, 8)),  # 256 x 256
+    (1, 512, 256, 16, 16384, (1, 4)), (1, 576, 320, 6, 8192, (2, 4)), (1, 512, 256, 4, 4096, (8, 8)),
+    (1, 1536, 320, 16, 4096, (1, 2)), (1, 576, 1024, 8, 24576, (2, 2)), (1, 768, 1024, 6, 24576, (2, 4)),
+    (1, 2048, 320, 3, 16384, (4, 4)), (1, 768, 1024, 3, 16384, (4, 8)), (1, 576, 512, 4, 24576, (8, 8))])
+def test_moe_wgrad_splits(dev, bf16, M_, N_, E, R, splits):
+    """Every split count, with one count for all experts and with a larger one
+    for a long expert, in both tile shapes: integer operands (at most 64 *
+    32768 < 2^24), so each expert's gradient is known exactly."""
+    ops = sg.ops
+    counts = _uneven(E, R)
+    assert sum(counts) == R and min(counts) >= 0
+    ldp = ops.moe_padded_rows(R, E)
+    assert tuple(sg._lib.query("sfp8_wgrad_splits_of", M_, N_, E, ldp, bf16, i) for i in (0, 1)) == splits
+    g = torch.Generator(device=dev).manual_seed(M_ + N_ + R)
+    for order in (counts, counts[::-1]):  # the long expert first and last
+        plan = ops.moe_plan(torch.cumsum(torch.tensor(order), 0).to(torch.int32).to(dev), R)
+        a, b = torch.zeros(ldp, M_, device=dev), torch.zeros(ldp, N_, device=dev)
+        ref, row = [], 0
+        for c in order:
+            a[row:row + c] = torch.randint(-8, 9, (c, M_), generator=g, device=dev).float()
+            b[row:row + c] = torch.randint(-8, 9, (c, N_), generator=g, device=dev).float()
+            ref.append(a[row:row + c].t() @ b[row:row + c])
+            row += -(-c // 256) * 256
+        ref = torch.stack(ref)
+        if bf16:
+            gs, bt = ops.to_slab(a.bfloat16()), ops.to_slab(b.bfloat16().t().contiguous())
+            at = ops.to_slab(a.bfloat16().t().contiguous())
+            assert torch.equal(ops.bf16_wgrad_rows(gs, bt, M_, N_, plan=plan, E=E), ref.bfloat16())
+            assert torch.equal(ops.bf16_wgrad(at, bt, M_, N_, plan=plan, E=E), ref.bfloat16())
+        else:
+            one = torch.ones(1, device=dev)
+            a8, b8 = ops.to_slab(a.to(ops.E5M2)), ops.to_slab(b.to(ops.E4M3))
+            at8, bt8 = ops.to_slab(a.to(ops.E5M2).t().contiguous()), ops.to_slab(b.to(ops.E4M3).t().contiguous())
+            assert torch.equal(ops.moe_wgrad_rows(a8, b8, M_, N_, E, plan, one, one), ref)
+            assert torch.equal(ops.moe_wgrad_rows(a8, bt8, M_, N_, E, plan, one, one, b_rows=False), ref)
+            assert torch.equal(ops.moe_wgrad_rows(at8, b8, M_, N_, E, plan, one, one, a_rows=False), ref)
+            assert torch.equal(ops.moe_wgrad(at8, bt8, M_, N_, E, plan, one, one), ref)

@@ -108,11 +108,14 @@ def _wgrad_operands(dev, M, N, T, seed):
     return at, bt, sa, sb
 
 
-@pytest.mark.parametrize("M,N,T", [(256, 256, 16384), (768, 320, 1000), (6144, 1024, 4096)])
-def test_wgrad_momentum_matches_wgrad_then_stage(dev, M, N, T):
+@pytest.mark.parametrize("M,N,T,splits", [(256, 256, 16384, 8), (768, 320, 1000, 1), (6144, 1024, 4096, 1),
+                                          (2048, 3072, 32768, 2)])
+def test_wgrad_momentum_matches_wgrad_then_stage(dev, M, N, T, splits):
     """Fused == ops.wgrad followed by the momentum stage, bytes equal, with
-    and without the gradient output; one split and several."""
+    and without the gradient output; one split and several, in 128 x 128 and
+    (the last) 256 x 256 tiles."""
     ops = sg.ops
+    assert sg._lib.query("sfp8_wgrad_splits_of", M, N, 0, ops.ldt_of(T), 0, 0) == splits
     at, bt, sa, sb = _wgrad_operands(dev, M, N, T, M + T)
     dw = ops.wgrad(at, bt, M, N, sa, sb)
     v0 = torch.randn(M, N, device=dev) * 1e-2

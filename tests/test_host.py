@@ -73,19 +73,21 @@ def test_size_queries_need_no_gpu():
 
 @pytest.mark.parametrize("E,M,N,R,fp8,bf16", [
     # more splits are no faster with every row on one expert: one, by the even rows
-    (8, 3072, 1024, 131072, 1, 1), (8, 1024, 1536, 131072, 1, 1), (8, 3072, 1024, 16384, 1, 1),
-    (8, 1536, 512, 16384, 1, 1), (16, 2048, 1024, 16384, 1, 1),
-    # one split would take that expert up to three times as long as the most
-    (8, 1536, 512, 65536, 2, 2), (4, 2048, 1024, 65536, 2, 2), (16, 512, 256, 16384, 2, 4),
-    (16, 512, 256, 65536, 4, 4), (4, 1024, 512, 65536, 8, 8), (4, 1280, 512, 32768, 2, 4),
+    (8, 3072, 1024, 131072, (1, 1), (1, 1)), (8, 1024, 1536, 131072, (1, 1), (1, 1)),
+    (8, 1536, 512, 16384, (1, 1), (1, 1)), (16, 2048, 1024, 16384, (1, 1), (1, 1)),
+    # one split (four) would take that expert up to three times as long as the most
+    (8, 1536, 512, 65536, (1, 2), (2, 2)), (4, 2048, 1024, 65536, (1, 2), (2, 2)),
+    (16, 512, 256, 16384, (1, 2), (1, 4)), (16, 512, 256, 65536, (4, 4), (4, 4)),
+    (4, 1024, 512, 65536, (4, 8), (8, 8)), (16, 2944, 896, 68546, (1, 2), (1, 2)),
 ])
 def test_grouped_splits_bound_uneven_routing(E, M, N, R, fp8, bf16):
-    """The K splits of a grouped gradient suit even rows and, since the routing
-    is not known on the host, all rows on one expert."""
+    """The K splits of a grouped gradient (of an expert, of a long one) suit
+    even rows and, since the routing is not known on the host, all rows on one
+    expert."""
     ldp = _lib.query("sfp8_moe_padded_rows", R, E)
-    assert _lib.query("sfp8_wgrad_splits_of", M, N, E, ldp, 0) == fp8
-    assert _lib.query("sfp8_wgrad_splits_of", M, N, E, ldp, 1) == bf16
-    assert max(fp8, bf16) <= _lib.query("sfp8_moe_wgrad_splits", M, N, E)
+    for b, want in ((0, fp8), (1, bf16)):
+        assert tuple(_lib.query("sfp8_wgrad_splits_of", M, N, E, ldp, b, i) for i in (0, 1)) == want
+    assert max(fp8 + bf16) <= _lib.query("sfp8_moe_wgrad_splits", M, N, E)
 
 
 def test_invalid_arguments_rejected_before_launch():
