@@ -355,7 +355,7 @@ def test_compiled_norm_swiglu_matches_eager(dev):
 
 
 def test_bf16_ops_opcheck(dev):
-    """Fake implementations of the four bf16 operators against real runs."""
+    """Fake implementations of the five bf16 operators against real runs."""
     utils = ("test_faketensor",)
     T, D, I = 300, 256, 384
     h, norm_w, w_gu, _ = _norm_case(dev, T, D, I, 7)
@@ -371,6 +371,34 @@ def test_bf16_ops_opcheck(dev):
     hh, gu2, plan = torch.ops.sparkfp8.swiglu_fwd(*fargs)
     torch.library.opcheck(torch.ops.sparkfp8.swiglu_bwd.default, (probe.to(dev), fargs[0], fargs[1], gu2, plan),
                           test_utils=utils)
+    for rows in (0, 7, 300):
+        torch.library.opcheck(torch.ops.sparkfp8.swiglu_eval.default, (fargs[0][:rows], fargs[1][0].contiguous()),
+                              test_utils=utils)
+
+
+@pytest.mark.parametrize("T", [5, 300])
+def test_compiled_eval_mlp_matches_eager(dev, T):
+    """torch.compile traces MLP.forward while gradients are off as one custom
+    operator and the down projection, no graph break; h has eager's bytes."""
+    torch.manual_seed(3)
+    mlp = sg.MLP(256, 384).to(dev).to(torch.bfloat16)
+    x = torch.randn(T, 256, device=dev).bfloat16()
+    w = mlp.gate_up_proj.weight
+
+    def both(v):
+        return sg.swiglu._EvalSwiGLU.apply(v, w), mlp(v)
+
+    with torch.no_grad():
+        h, y = both(x)
+        explain = torch._dynamo.explain(both)(x)
+        assert explain.graph_break_count == 0, explain.break_reasons
+        torch._dynamo.reset()
+        compiled = torch.compile(both, mode="default", dynamic=False)
+        for _ in range(2):
+            hc, yc = compiled(x)
+            assert torch.equal(hc, h)
+            assert O.rel_l2(yc.float().cpu(), y.float().cpu()) < 1e-2
+    torch._dynamo.reset()
 
 
 @pytest.mark.parametrize("T,M,N", [(4096, 1536, 1024), (1000, 768, 512), (65536, 6144, 1024), (1, 256, 256)])
@@ -469,3 +497,28 @@ def test_eval_rows_equal_training_rows(dev, T, D, I):
         alone = torch.cat([sg.swiglu._EvalSwiGLU.apply(r[None], w) for r in x])
     bits = lambda t: t.view(torch.int16)  # noqa: E731
     assert torch.equal(bits(h), bits(ref)) and torch.equal(bits(h), bits(alone))
+
+
+@pytest.mark.parametrize("T,D,I", [(10241, 256, 1024), (10241, 512, 1152), (5121, 640, 2048)])
+def test_persistent_bf16_swiglu_special_values(dev, T, D, I):
+    """Rows are independent: NaN, infinite and huge rows through the persistent
+    kernel (several tiles per work-group, with and without the row scale) have
+    the bytes that the one-tile kernel gives them in a batch of 512, and the
+    rows beside them those of ordinary rows."""
+    ops = sg.ops
+    torch.manual_seed(T + D)
+    x = torch.randn(T, D, device=dev).bfloat16()
+    x[::97, 3] = float("nan")
+    x[5::89, D - 1] = float("inf")
+    x[7::83] *= 1e19
+    w = (torch.randn(2 * I, D, device=dev) * D ** -0.5).bfloat16()
+    ws, _ = ops.bf16_weight_slabs(w[None], transposed=False)
+    scale = torch.rand(T, device=dev) + 0.5
+    bits = lambda t: t.view(torch.int16)  # noqa: E731
+    for rstd in (None, scale):
+        gu, h = ops.bf16_swiglu_fwd(x, ws, I, rstd=rstd)
+        for a in range(0, T, 512):
+            b = min(T, a + 512)
+            g1, h1 = ops.bf16_swiglu_fwd(x[a:b], ws, I, rstd=None if rstd is None else rstd[a:b].contiguous())
+            assert torch.equal(bits(gu[a:b]), bits(g1)) and torch.equal(bits(h[a:b]), bits(h1))
+    assert bool(h.isnan().any()) and bool(gu.isinf().any()) and float(h.isnan().any(1).float().mean()) < 0.1

@@ -321,3 +321,79 @@ def test_block_vs_bf16_mlp(dev, T, D, I, capsys):
         print("\nrel-L2 of the FP8 block vs the bf16 MLP:", {k: round(v, 4) for k, v in errs.items()})
     for name, e in errs.items():
         assert e < 0.12, (name, e)
+
+
+def _all_paths(dev, seed):
+    """One pass of every path whose calls are native: the FP8 block with its
+    post-step hook, the bf16 sub-block, evaluation and the grouped experts."""
+    norm, mlp = _setup(dev, 700, 256, 512, seed)
+    g = torch.Generator(device=dev).manual_seed(seed)
+    h = torch.randn(700, 256, device=dev, generator=g).to(torch.bfloat16)
+    probe = torch.randn(700, 256, device=dev, generator=g)
+    offs = torch.tensor([300, 300, 700], device=dev, dtype=torch.int32)
+    w = (torch.randn(3, 1024, 256, device=dev, generator=g) / 16).to(torch.bfloat16)
+
+    def run():
+        mlp.fp8_scale.fill_(1.0)
+        mlp.fp8_amax.zero_()
+        out = list(_step(h, probe, norm, mlp))
+        sg.fp8_update_scales(mlp)
+        out.append(mlp.fp8_scale.clone())
+        x, nw, wg = (t.detach().clone().requires_grad_(True) for t in (h, norm.weight, mlp.gate_up_proj.weight))
+        y = sg._NormSwiGLU.apply(x, nw, wg, 1e-6)
+        out += [y.detach(), *torch.autograd.grad(y, [x, nw, wg], y.detach())]
+        x, we = h.clone().requires_grad_(True), w.clone().requires_grad_(True)
+        y = sg._FusedSwiGLU.apply(x, we, offs)
+        out += [y.detach(), *torch.autograd.grad(y, [x, we], y.detach())]
+        with torch.no_grad():
+            out.append(sg.swiglu._EvalSwiGLU.apply(h[:40], w[0]))
+        return [t.detach() for t in out]
+
+    return run
+
+
+def test_native_calls_run_on_the_current_stream(dev):
+    """On a side stream behind other work of that stream, the calls (and the
+    backward's, made from autograd's thread) give the bytes of the default
+    stream."""
+    run = _all_paths(dev, 11)
+    ref = run()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    a = torch.randn(4096, 4096, device=dev)
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            for _ in range(4):
+                a = a @ a * 1e-3  # the stream is busy when the calls are made
+            got = run()
+        side.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, ref, strict=True))
+
+
+def test_native_calls_from_threads(dev):
+    """Two threads at once, each on a stream of its own with weights of its own."""
+    import threading
+
+    runs = [_all_paths(dev, s) for s in (21, 22)]
+    refs = [r() for r in runs]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            for _ in range(5):
+                with torch.cuda.stream(stream):
+                    got = runs[i]()
+                stream.synchronize()
+                if not all(torch.equal(x, y) for x, y in zip(got, refs[i], strict=True)):
+                    bad.append(i)
+        except Exception as e:  # noqa: BLE001
+            bad.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad

@@ -140,19 +140,37 @@ def test_ops_reject_host_tensors():
 
 
 def test_native_wrappers_refuse_host_tensors():
-    """The native wrappers check before they launch: a host tensor raises
-    ValueError, a wrong keyword or a non-tensor TypeError."""
+    """Every native wrapper checks before it launches: a host tensor raises
+    ValueError (RuntimeError where only its stream is asked for), a wrong keyword
+    or a non-tensor TypeError."""
     b = torch.zeros(4, 128, dtype=torch.bfloat16)
     f, s = torch.zeros(256, 128), torch.ones(5)
     x8, g8 = torch.zeros(2, 256, 64).to(ops.E4M3), torch.zeros(2, 256, 64).to(ops.E5M2)
-    for fn, args in ((ops.block_weight_quant, (f, f)), (ops.weight_quant_experts, (f[None], s)),
-                     (ops.gateup_swiglu_fwd, (x8, x8, s, s, s, 4, 128)), (ops.down_fwd, (x8, x8, b, s, s)),
-                     (ops.down_dgrad_swiglu, (b, x8, x8, s, s)), (ops.gateup_dgrad, (g8, x8, s, s, 4, 128)),
-                     (ops.wgrad_rows, (g8, x8, 128, 128, s, s)), (ops.norm_bwd, (b, s, b, b, s, s, s)),
-                     (ops.moe_plan, (torch.ones(2, dtype=torch.int32), 4)), (ops.moe_topk_sum, (b, s, 2, 2)),
-                     (ops.bf16_weight_slabs, (f[None],)), (ops.bf16_norm_dh, (b, b, s))):
+    plan = torch.zeros(64, dtype=torch.int32)
+    b3 = torch.zeros(4, 256, 32, dtype=torch.bfloat16)
+    x83, g83 = x8[None], g8[None]
+    calls = {"norm_quant": (b, s, s, s, 1e-6), "block_weight_quant": (f, f), "weight_quant_experts": (f[None], s),
+             "gateup_swiglu_fwd": (x8, x8, s, s, s, 4, 128), "down_fwd": (x8, x8, b, s, s),
+             "down_dgrad_swiglu": (b, x8, x8, s, s), "gateup_dgrad": (g8, x8, s, s, 4, 128),
+             "wgrad_rows": (g8, x8, 128, 128, s, s), "norm_bwd": (b, s, b, b, s, s, s),
+             "moe_plan": (torch.ones(2, dtype=torch.int32), 4),
+             "moe_rows_quant": (b, None, plan, 256, s, 0, s, 0, 0, True),
+             "moe_wgrad_rows": (g8, x8, 128, 128, 2, plan, s, s), "moe_topk_sum": (b, s, 2, 2),
+             "moe_down_dgrad_swiglu": (b, b3[None], x8, plan, s, s), "bf16_weight_slabs": (f[None],),
+             "bf16_rows_prep": (b, None, 256), "bf16_swiglu_fwd": (b, b3[None], 128), "bf16_swiglu_eval": (b, b),
+             "bf16_swiglu_bwd": (b, b, None, None, 256), "bf16_norm_dh": (b, b, s),
+             "bf16_wgrad_rows": (b3, b, 128, 128)}
+    for name, args in calls.items():
         with pytest.raises(ValueError):
-            fn(*args)
+            getattr(ops, name)(*args)
+    # no operand of these is checked by itself: the stream is refused
+    late = {"moe_gateup_swiglu_fwd": (x8, x83, plan, s, s, s, 128), "moe_down_fwd": (x8, x83, plan, s, s, 4, 128),
+            "moe_gateup_dgrad": (g8, g83, plan, s, s, 4, 128), "bf16_gemm": (b3, b3, 4, 128, 128),
+            "bf16_fold_grads": (b, f, s)}
+    for name, args in late.items():
+        with pytest.raises(RuntimeError):
+            getattr(ops, name)(*args)
+    assert set(calls) | set(late) == set(ops._NATIVE)
     with pytest.raises(TypeError):
         ops.norm_quant(b, s, s, s, 1e-6, rows=True)
     with pytest.raises(TypeError):
