@@ -3,10 +3,10 @@
 // Every GEMM here is C[m, n] = sum_k A[m, k] * B[n, k]: both operands are
 // K-contiguous rows in HBM, except that a weight gradient (K = tokens) may
 // read either operand as the token-major activation its producer wrote,
-// through transposing LDS reads (MainLoop TR_A / TR_B).  One work-group (256 threads = 4 waves, one wave
-// per SIMD) computes a 256 x 256 output tile with the pipelined main loop of
-// mainloop.h; each wave owns 128 x 128 as 4 x 4 blocks of 32 x 32 MFMA
-// accumulators.
+// through transposing LDS reads (MainLoop TR_A / TR_B).  One work-group
+// computes an output tile with the pipelined main loop of mainloop.h: 256 x 256
+// by 8 waves of 128 x 64, 192 x 256 or 128 x 256 by 8, 128 x 128 by 4 of 64 x 64
+// (Tile below), each wave's share as blocks of 32 x 32 MFMA accumulators.
 //
 // MFMA: v_mfma_f32_32x32x64_f8f6f4 (e4m3/e5m2 chosen per operand) or
 // v_mfma_f32_32x32x16_bf16.  The B fragment is passed as the instruction's
@@ -17,9 +17,9 @@
 // placement of K inside a fragment gives the same dot product.
 //
 // Output-column permutation: the B tile is filled with its rows permuted
-// (plain_col / paired_col below), so that accumulator v of block nb of the
-// lane in half g is output column  base + 16*nb + v  -- 16 (and across blocks
-// 64 or 32) consecutive columns per lane.  Every epilogue access is then a
+// (plain_col_nb, paired_col8 and paired_col64 below), so that accumulator v of
+// block nb of the lane in half g is output column  base + 16*nb + v  -- 16 (and
+// across blocks 32) consecutive columns per lane.  Every epilogue access is then a
 // 16-byte vector; LDS staging remains only for the transposed copies.
 #include "common.h"
 #include "mainloop.h"
@@ -79,17 +79,10 @@ SFP8_DEV void split_tile_coords(int pid, int nwg, int tiles_m, int tiles_n, int 
   raster(lid % tiles, tiles_m, tiles_n, tm, tn);
 }
 
-// Output column (within the 256-column tile) held in B-tile row r, plain
-// layout: wave column wn owns rows 128*wn.., lane half g of block nb element
-// v (row 32*nb + 8*(v/4) + 4*g + v%4) gets column 128*wn + 64*g + 16*nb + v.
-SFP8_DEV int plain_col(int r) {
-  const int rl = r & 127;
-  return (r & 128) + 64 * ((rl >> 2) & 1) + 16 * (rl >> 5) + 4 * ((rl >> 3) & 3) + (rl & 3);
-}
-
-// The same for a 64*NB-row B tile (NB blocks of 32 per wave): B row r holds
-// column 32*NB*wn + 16*NB*g + 16*nb + v, so a lane's NB blocks cover 16*NB
-// consecutive columns.  plain_col_nb<4> == plain_col.
+// Output column (within the tile) held in B-tile row r, plain layout of NB
+// blocks of 32 rows per wave: wave column wn owns rows 32*NB*wn.., lane half g
+// of block nb element v (row 32*nb + 8*(v/4) + 4*g + v%4) gets column 32*NB*wn +
+// 16*NB*g + 16*nb + v, so a lane's NB blocks cover 16*NB consecutive columns.
 template <int NB>
 SFP8_DEV int plain_col_nb(int r) {
   const int wn = r / (32 * NB), rl = r % (32 * NB);
@@ -153,7 +146,7 @@ struct Tile {
   static constexpr int kThreads = 128 * WN;
   static constexpr int kMinWaves = WN == 2 ? 2 : 1;  // per SIMD: two work-groups of 4 waves fit a CU
   template <bool BF16, int FA, int FB, bool TRA = false, bool TRB = false, bool PAIRED = false>
-  using Loop = MainLoop<BF16, FA, FB, PAIRED, 2, kStages, 0, TRA, TRB, WN, TB, TB == 3 ? 256 : kM>;
+  using Loop = MainLoop<BF16, FA, FB, PAIRED, 2, kStages, TRA, TRB, WN, TB, TB == 3 ? 256 : kM>;
   static constexpr int kLds = Loop<true, 0, 0>::kLds;
   static constexpr int kOutStride = 2 * kN + 16;        // a staged bf16 row
   static constexpr int kPieces = kM * kN / 8 / kThreads;  // 16-byte pieces of it per thread
@@ -405,7 +398,7 @@ SFP8_DEV void pipe_h8_rows(const uint8_t* hbuf, uint8_t* dst) {
 // MFMAs).
 template <int NK, int TB>
 struct SwigluPipe {
-  using ML = MainLoop<false, kFmtE4M3, kFmtE4M3, true, 2, 4, 0, false, false, 2, TB>;
+  using ML = MainLoop<false, kFmtE4M3, kFmtE4M3, true, 2, 4, false, false, 2, TB>;
   static constexpr int kWaves = ML::kWaves, kWM = ML::kWM;
   static constexpr int kUnits = 4 * TB;  // 4 pairs each: unit u = row block u/4, pairs 4*(u%4) ..
   static constexpr int kSt = 4;          // LDS ring stages
@@ -886,31 +879,8 @@ __global__ __launch_bounds__(TB == 4 ? 256 : 512, 1) void swiglu_pipe_kernel(
 // whole rows.  Pass P holds tile rows 64P..64P+63 and 128+64P..128+64P+63.
 constexpr int kBf16Stride = 528;
 
-template <int P>
-SFP8_DEV void stage_bf16_half(uint8_t* lds, const floatx16 (&acc)[4][4], float s) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
-  const int fr = lane & 31, g = lane >> 5, cb = 128 * wn + 64 * g;
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt) {
-    const int lr = 64 * wm + 32 * tt + fr;
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      uint32_t w0[4], w1[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        w0[i] = pack2_bf16(acc[2 * P + tt][nb][2 * i] * s, acc[2 * P + tt][nb][2 * i + 1] * s);
-        w1[i] = pack2_bf16(acc[2 * P + tt][nb][8 + 2 * i] * s, acc[2 * P + tt][nb][8 + 2 * i + 1] * s);
-      }
-      uint8_t* q = lds + lr * kBf16Stride + (cb + 16 * nb) * 2;
-      store16(q, w0);
-      store16(q + 16, w1);
-    }
-  }
-}
-
-// The same for the 8-wave tile layout (wave (wm, wn), wn = 0..3, owns A rows
-// 128 wm.. and output columns 64 wn.. as 4 x 2 blocks; lane half g of block
-// nb holds columns 64 wn + 32 g + 16 nb + v).
+// Wave (wm, wn), wn = 0..3, owns A rows 128 wm.. and output columns 64 wn.. as 4
+// x 2 blocks; lane half g of block nb holds columns 64 wn + 32 g + 16 nb + v.
 template <int P>
 SFP8_DEV void stage_bf16_half8(uint8_t* lds, const floatx16 (&acc)[4][2], float s) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
@@ -1298,7 +1268,7 @@ __global__ __launch_bounds__(TileShape<SMALL>::kThreads, TileShape<SMALL>::kMinW
     Loop::run(base, o.a, o.a_bytes, arow, kStage, o.b, o.b_bytes, brow, (int)(ip * kStage), nk, acc);
   }
   // Row-order epilogue, in two passes (128-row tiles: one) of 128 tile rows (the rows
-  // of stage_bf16_half<P>): dh staged in LDS as bf16, then each thread takes
+  // of stage_bf16_half8<P>): dh staged in LDS as bf16, then each thread takes
   // 16-column chunks of one row, reading gu8 and writing dgu8 as whole K-slab
   // rows; with dgu8t the codes also go to LDS for the token-contiguous copy.
   const __amdgpu_buffer_rsrc_t rgu = make_rsrc(gu8 + m0 * 64, 2 * I * ldt - m0 * 64);
@@ -1545,7 +1515,7 @@ __global__ __launch_bounds__(TS::kThreads, TS::kMinWaves) void gateup_dgrad_kern
 // K bytes [sp * kchunk, min((sp + 1) * kchunk, ldt)) (the last split may be
 // shorter; every split is a whole number of 128-byte stage pairs); with splits > 1
 // each split writes its raw fp32 accumulators to ws in accumulator order
-// (frag_offset below: each wave store instruction is one contiguous 1 KiB
+// (acc_order_rc: each wave store instruction is one contiguous 1 KiB
 // run) and splitk_reduce_kernel sums them in split order (deterministic) and
 // scatters them to [M, N].
 // With `partials` the raw partials go to `out` as the workspace, also for one
@@ -2138,7 +2108,7 @@ __global__ __launch_bounds__(512) void bf16_swiglu_eval_kernel(const uint16_t* _
 // bf16_swiglu_fwd_kernel.
 template <int KE, bool EXACT>
 struct Bf16Pipe {
-  using ML = MainLoop<true, 0, 0, true, 2, kStages, 0, false, false, 2, 2>;
+  using ML = MainLoop<true, 0, 0, true, 2, kStages, false, false, 2, 2>;
   static constexpr int kUnits = 8, kPre = 2, kSlots = ML::kMfma - kPre;
   // the pieces fill the slots of stages 0 .. KE - 2; a row block staged at the
   // end of a stage is written in the next

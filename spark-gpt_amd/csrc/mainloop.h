@@ -6,9 +6,9 @@
 // accumulators (fp32, 16*TB*NB registers per lane).  The GEMMs here use
 // 8 waves (two per SIMD) of 128 x 64 (TB = 4, NB = 2, WN = 4) per 256 x 256
 // tile, or of 64 x 64 (TB = 2, NB = 2, WN = 2) per 256 x 128 tile, so that
-// one wave's stage waits and barriers are covered by the other's MFMAs; 4
-// waves of 128 x 128 (NB = 4, WN = 2) remain available.  The 128 x 128 tile
-// (TM = 128: 4 waves of 64 x 64, a 64 KiB ring) lets two work-groups share a
+// one wave's stage waits and barriers are covered by the other's MFMAs.  The
+// 128 x 128 tile (TM = 128: 4 waves of 64 x 64, a 64 KiB ring) lets two
+// work-groups share a
 // CU, one's epilogue and waits under the other's MFMAs: a quarter of the
 // work per tile, for shapes with too few 256 x 256 tiles or a short K.  Every
 // tile shape adds the same products in the same K order to each output.
@@ -77,37 +77,6 @@ struct BLayout {
   }
 };
 
-// Interleave N_MFMA MFMAs with N_DS LDS reads (spread over all of them) and
-// N_VM DMA issues (spread over the first half).
-template <int N_MFMA, int N_DS, int N_VM, int I = 0>
-SFP8_DEV void sched_interleave() {
-  if constexpr (I < N_MFMA) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-    constexpr int ds = (N_DS * (I + 1) + N_MFMA - 1) / N_MFMA - (N_DS * I + N_MFMA - 1) / N_MFMA;
-    if constexpr (ds > 0) __builtin_amdgcn_sched_group_barrier(0x100, ds, 0);  // DS read
-    constexpr int half = N_MFMA / 2;
-    constexpr int vm = I < half ? (N_VM * (I + 1) + half - 1) / half - (N_VM * I + half - 1) / half : 0;
-    if constexpr (vm > 0) __builtin_amdgcn_sched_group_barrier(0x020, vm, 0);  // VMEM (DMA)
-    sched_interleave<N_MFMA, N_DS, N_VM, I + 1>();
-  }
-}
-
-// The same with up to N_VALU vector-ALU instructions (other work of the wave,
-// such as a deferred epilogue) placed after each MFMA.
-template <int N_MFMA, int N_VALU, int N_DS, int N_VM, int I = 0>
-SFP8_DEV void sched_interleave_valu() {
-  if constexpr (I < N_MFMA) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-    __builtin_amdgcn_sched_group_barrier(0x002, N_VALU, 0);  // VALU
-    constexpr int ds = (N_DS * (I + 1) + N_MFMA - 1) / N_MFMA - (N_DS * I + N_MFMA - 1) / N_MFMA;
-    if constexpr (ds > 0) __builtin_amdgcn_sched_group_barrier(0x100, ds, 0);  // DS read
-    constexpr int half = N_MFMA / 2;
-    constexpr int vm = I < half ? (N_VM * (I + 1) + half - 1) / half - (N_VM * I + half - 1) / half : 0;
-    if constexpr (vm > 0) __builtin_amdgcn_sched_group_barrier(0x020, vm, 0);  // VMEM (DMA)
-    sched_interleave_valu<N_MFMA, N_VALU, N_DS, N_VM, I + 1>();
-  }
-}
-
 // TR_A / TR_B: the operand's tile arrives as blocks of 64 (fp8) or 32 (bf16)
 // rows, each [tokens of the K stage][64 bytes of 64 (32) M or N values] -- a
 // row K-slab (or the row-major rows) of the token-major activation a weight
@@ -127,8 +96,8 @@ SFP8_DEV void sched_interleave_valu() {
 // DMA is aimed out of range) or 2 (two wave rows of 64 of a TM = 128 tile, or
 // four of a TM = 256 one: then only the fragment, DMA and MFMA pieces, not
 // run()).
-template <bool BF16, int FMT_A, int FMT_B, bool PAIRED, int NB = 4, int STAGES = kStages, int PRE = 0,
-          bool TR_A = false, bool TR_B = false, int WN = 2, int TB = 4, int TM = kTile>
+template <bool BF16, int FMT_A, int FMT_B, bool PAIRED, int NB = 2, int STAGES = kStages, bool TR_A = false,
+          bool TR_B = false, int WN = 2, int TB = 4, int TM = kTile>
 struct MainLoop {
   static_assert(TB >= 2 && TB <= 4, "2 to 4 A blocks per wave");
   static constexpr int kWM = TM / (32 * TB);                // wave rows
@@ -151,7 +120,7 @@ struct MainLoop {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, 0);
     }
   }
-  static_assert(NB == 2 || NB == 4, "2 or 4 B blocks per wave");
+  static_assert(NB == 2, "the stages are scheduled for 2 B blocks per wave");
   static_assert(STAGES >= 3, "at least three LDS stages");
   static constexpr int kTileN = 32 * NB * WN;             // B rows per tile
   static constexpr int kStageB = kTileN * kStage;
@@ -251,9 +220,6 @@ struct MainLoop {
   }
 
   static constexpr int kMfma = (BF16 ? 2 : 1) * TB * NB;  // MFMAs per stage
-  // MFMAs of a stage issued before its barrier: they need only registers, and
-  // keep the matrix pipe busy while the waves meet.
-  static constexpr int kPre = PRE;
 
   // MFMAs [LO, HI) of one stage, in (h, tb, nb) order.
   template <int LO, int HI>
@@ -277,9 +243,6 @@ struct MainLoop {
       }
     }
   }
-
-  // Per stage after the barrier: kMfma - kPre MFMAs, 2*(4+NB) LDS reads, 4+NB DMAs.
-  static SFP8_DEV void schedule() { sched_interleave<kMfma - kPre, 2 * (4 + NB), kDma>(); }
 
   // MFMA M of the stage, then fragment reads [R0, R1) of the next stage, as
   // one group the scheduler may not reorder with its neighbours.
@@ -314,10 +277,9 @@ struct MainLoop {
   //   every wave finished reading it before this barrier), all within the
   //   first 10-16 MFMAs so the reads land long before stage kt+1 starts;
   //   the remaining MFMAs.
-  // The grouping depends on the MFMA length: fp8 256 x 256 alternates
-  // fragments and DMA over 10 MFMAs of 64 cycles, bf16 alternates one
-  // fragment and one DMA over 16 MFMAs of 32 cycles, NB = 2 issues the
-  // fragments over 3 MFMAs and then the DMA over 3.
+  // The grouping depends on the MFMA length: bf16 alternates one fragment and
+  // one DMA over MFMAs of 32 cycles, fp8 issues the fragments over 3 MFMAs of 64
+  // cycles and then the DMA over 2.
   static constexpr int kSchedPre = 2;
   static_assert(TB != 4 || kMfma >= kSchedPre + (4 + NB) / 2 + (4 + NB) / 2, "stage too short for the schedule");
   static SFP8_DEV void stage_large(uint8_t* lds, const Frag& cur, Frag& nxt, Acc& acc, int dma_buf, int ld, int rd_buf,
@@ -330,32 +292,6 @@ struct MainLoop {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kDma * (STAGES - 3)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     const int sa = ld * a_sstride, sb = ld * b_sstride;
-    constexpr int H = (4 + NB) / 2;  // MFMAs carrying reads (and DMA issues)
-    if constexpr (BF16 && NB == 4) {
-      // bf16: 32 MFMAs of 32 cycles per stage.  Two reads after each of 4
-      // MFMAs would crowd 16 KiB of LDS reads per wave into 128 cycles; one
-      // fragment and one DMA instruction after alternate MFMAs spread them
-      // over 16 (5 % faster on the down dgrad than the fp8 order).
-      mfma_then_reads<P + 0, 0, 1>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 1, 0, 1>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 2, 1, 2>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 3, 1, 2>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 4, 2, 3>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 5, 2, 3>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 6, 3, 4>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 7, 3, 4>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 8, 4, 5>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 9, 4, 5>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 10, 5, 6>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 11, 5, 6>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 12, 6, 7>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 13, 6, 7>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 14, 7, 8>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 15, 7, 8>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_range<P + 16, kMfma>(cur, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      return;
-    }
     if constexpr (TB == 3 && BF16) {
       // 8 waves of 96 x 64: 12 bf16 MFMAs, five fragments and four DMA issues
       mfma_then_reads<P + 0, 0, 1>(lds, cur, nxt, acc, rd_buf, aoff, boff);
@@ -368,7 +304,6 @@ struct MainLoop {
       mfma_then_reads<P + 7, 4, 5>(lds, cur, nxt, acc, rd_buf, aoff, boff);
       mfma_range<P + 8, kMfma>(cur, acc);
       __builtin_amdgcn_sched_barrier(0);
-      return;
     } else if constexpr (TB == 3) {
       // the same with 6 fp8 MFMAs
       mfma_then_reads<P + 0, 0, 2>(lds, cur, nxt, acc, rd_buf, aoff, boff);
@@ -379,9 +314,7 @@ struct MainLoop {
       load_one(1, lds, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
       __builtin_amdgcn_sched_barrier(0);
       mfma_then_dma<P + 3, 2, 4>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      return;
-    } else {
-    if constexpr (BF16 && NB == 2) {
+    } else if constexpr (BF16) {
       // bf16, 8 waves of 128 x 64: 16 MFMAs of 32 cycles; six fragments and
       // four DMA issues alternate over 10 of them
       mfma_then_reads<P + 0, 0, 1>(lds, cur, nxt, acc, rd_buf, aoff, boff);
@@ -396,26 +329,7 @@ struct MainLoop {
       mfma_then_reads<P + 9, 5, 6>(lds, cur, nxt, acc, rd_buf, aoff, boff);
       mfma_range<P + 10, kMfma>(cur, acc);
       __builtin_amdgcn_sched_barrier(0);
-      return;
-    }
-    if constexpr (!BF16 && NB == 4) {
-      // fp8, 256 x 256: fragments and DMA issues alternate over 10 MFMAs
-      // (2-3 % faster than 4 MFMAs of reads followed by 4 of DMA)
-      mfma_then_reads<P + 0, 0, 1>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 1, 0, 1>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 2, 1, 3>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 3, 1, 3>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 4, 3, 5>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 5, 3, 5>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 6, 5, 7>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 7, 5, 7>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_then_reads<P + 8, 7, 8>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-      mfma_then_dma<P + 9, 7, 8>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-      mfma_range<P + 10, kMfma>(cur, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      return;
-    }
-    if constexpr (!BF16 && NB == 2 && kDma == 4 && TR_A && TR_B) {
+    } else if constexpr (TR_A && TR_B) {
       // fp8, 8 waves of 128 x 64, both operands through transposing reads
       // (four per fragment): two fragments and two DMA issues alternate over
       // 5 MFMAs (2 % faster on the gate/up weight gradient than the order
@@ -427,9 +341,7 @@ struct MainLoop {
       mfma_then_reads<P + 4, 4, 6>(lds, cur, nxt, acc, rd_buf, aoff, boff);
       mfma_range<P + 5, kMfma>(cur, acc);
       __builtin_amdgcn_sched_barrier(0);
-      return;
-    }
-    if constexpr (!BF16 && NB == 2 && kDma == 4) {
+    } else {
       // fp8, 8 waves of 128 x 64: 8 MFMAs of 64 cycles; two fragments after
       // each of 3, then two DMA issues after each of 2
       mfma_then_reads<P + 0, 0, 2>(lds, cur, nxt, acc, rd_buf, aoff, boff);
@@ -439,18 +351,6 @@ struct MainLoop {
       mfma_then_dma<P + 4, 2, 4>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
       mfma_range<P + 5, kMfma>(cur, acc);
       __builtin_amdgcn_sched_barrier(0);
-      return;
-    }
-    // NB = 2: two fragments after each of 3 MFMAs, then two DMA issues after
-    // each of 3
-    mfma_then_reads<P + 0, 0, 2>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-    mfma_then_reads<P + 1, 2, 4>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-    mfma_then_reads<P + 2, 4, 6>(lds, cur, nxt, acc, rd_buf, aoff, boff);
-    mfma_then_dma<P + H + 0, 0, 2>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-    mfma_then_dma<P + H + 1, 2, 4>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-    mfma_then_dma<P + H + 2, 4, 6>(lds, cur, acc, dma_buf, ra, rb, voff_a, voff_b, sa, sb, wave);
-    mfma_range<P + 2 * H, kMfma>(cur, acc);
-    __builtin_amdgcn_sched_barrier(0);
     }
   }
 
