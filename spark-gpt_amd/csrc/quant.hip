@@ -1082,7 +1082,9 @@ static int allow_lds(K kernel, size_t bytes) {
 // when their usual row blocks are fewer than the 256 CUs.  At T = 5003, D =
 // 1024 (80 blocks of 64 rows) norm_quant 12.2 -> 8.7 us and norm_bwd 18.7 ->
 // 16.0.  Narrower rows leave each work-group too little: T = 8192, D = 256 (128
-// blocks) 7.0 -> 8.5 and 11.2 -> 11.9.  (At D = 4096 a block is 16 rows anyway.)
+// blocks) 7.0 -> 8.5 and 11.2 -> 11.9.  D = 512 lies between, and is left with 64:
+// norm_quant 6.9 -> 4.6 at T = 5003 and 8.2 -> 7.2 at 16000, norm_bwd 11.7 -> 10.7
+// and 19.2 -> 24.2.  (At D = 4096 a block is 16 rows anyway.)
 template <int D>
 static bool few_rows(int64_t ldt) {
   return (D == 1024 || D == 2048) && ldt / NormCfg<D>::RT < 256;
